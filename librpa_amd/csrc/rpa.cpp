@@ -8,12 +8,11 @@
 //      stored side by side per atom column block: Gpm[R][row][2*ao(J) + s*nb(J) + j].
 //   2. W(K, J, S)[k, (j, nu)] = sum_{(L,R2) in N(J)} G(S+R2)_KL C^J(L,R2): one GEMM
 //      per (J, S, sign) on a gathered G panel, written as W[(s, j)][(K, k)][nu].
-//   3. T(I,J,R)[(K,R1,k,i)][nu] = G_KJ(R-R1) W(I,J,R) + G_IJ(R) W(K,J,R-R1): two row-
-//      indirect GEMM batches with K = 2 nb(J) (both signs at once).
-//   4. chi0s(I,J,R) = Cfin_I * T: one GEMM per output block, K = sum_K nb(I) nb(K).
+//   3. chi0s(I,J,R) = sum_(K,R1,k) C^I [G_IJ W(K,J,R-R1)] + W(I,-R)^T W(J,R), one launch per tile
+//      class (chi0.hip): the bracket is formed in registers and never stored.
 // The four terms of LibRI's labels a1b1_a2b2 and a1b2_a2b1 called with
 // (G+, G-) and (G-, G+) (thirdparty/LibRI/include/RI/physics/RPA.hpp:104-138)
-// are the four (sign, term) products of steps 3-4.
+// are the four (sign, term) products of step 3.
 //
 // chi0s(R, tau) of every tau stays resident; the tau -> omega cosine transform
 // and the R -> q sum (chi_libri_ft_ct, chi0.cpp:507-596) are fused into the
@@ -54,9 +53,9 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     ec_prec = pe;
     planned_ntau = ntau;
     ts = (prec == Prec::F64) ? 8 : 4;
-    // K parts of each contraction problem (LIBRPA_AMD_SPLITK, default 4; 1 = one plain write)
-    int nsk = 4;
-    if (const char *e = std::getenv("LIBRPA_AMD_SPLITK")) nsk = std::max(1, std::atoi(e));
+    // parts of each contraction (LIBRPA_AMD_SPLITK; default: by load; 1 = one plain write)
+    int splitk = 0;
+    if (const char *e = std::getenv("LIBRPA_AMD_SPLITK")) splitk = std::max(1, std::atoi(e));
     const auto &mf = ds.mf;
     natom = (int)ds.nb_wfc.size();
     if (natom == 0 || ds.nb_aux.size() != (size_t)natom) LRA_THROW("atomic basis sizes not set");
@@ -113,7 +112,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     }
     // packed Cs in the two GEMM layouts
     {
-        std::vector<double> cfin(cfin_off[natom]), cwb(cwb_off[natom]);
+        std::vector<double> cfin(cfin_off[natom] + kChi0Pad), cwb(cwb_off[natom]);
         cnorm.assign(natom, 0.0);
         for (int I = 0; I < natom; ++I) {
             for (size_t n = 0; n < nbrs[I].size(); ++n) {
@@ -157,7 +156,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     for (int J = 0; J < natom; ++J)
         for (int I = 0; I <= J; ++I)
             for (int r = 0; r < nR; ++r) {
-                outs.push_back({I, J, r, E_tot, 0});
+                outs.push_back({I, J, r, E_tot});
                 E_tot += (long long)na[I] * na[J];
             }
     std::vector<int> out_index((size_t)natom * natom * nR, -1);
@@ -179,7 +178,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     for (int J = 0; J < natom; ++J)
         for (int S = 0; S < nR; ++S)
             w_off[(size_t)J * nR + S + 1] = w_off[(size_t)J * nR + S] + 2LL * nb[J] * NAO * na[J];
-    // ---- chunking over J by memory budget (gathered G panels and T) ----
+    // ---- chunking over J by memory budget (gathered G panels) ----
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
     // chi0(R, tau) of every tau beside the W slabs, or staged through pinned host memory
@@ -196,40 +195,28 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     }
     chunks.clear();
     {
-        int j = 0, o = 0;
+        int j = 0;
         while (j < natom) {
             Chunk c;
             c.j_begin = j;
-            c.o_begin = o;
-            long long g = 0, t = 0;
-            int jj = j, oo = o;
+            long long g = 0;
+            int jj = j;
             while (jj < natom) {
-                long long g1 = (long long)nR * 2 * NAO * lsum[jj];
-                long long t1 = 0;
-                int o2 = oo;
-                while (o2 < (int)outs.size() && outs[o2].J == jj) { t1 += ksum[outs[o2].I] * na[jj]; ++o2; }
-                const double bytes = (double)(g + g1 + t + t1) * ts;
-                if (jj > j && bytes > budget) break;
-                g += g1; t += t1; oo = o2; ++jj;
+                const long long g1 = (long long)nR * 2 * NAO * lsum[jj];
+                if (jj > j && (double)(g + g1) * ts > budget) break;
+                g += g1;
+                ++jj;
             }
             c.j_end = jj;
-            c.o_end = oo;
-            c.ghat_elems = g; c.t_elems = t;
+            c.ghat_elems = g;
             chunks.push_back(std::move(c));
             j = jj;
-            o = oo;
         }
     }
 
     const long long gpm_r = (long long)NAO * 2 * NAO;  // elements per cell of Gpm
     flops_chi0_exec = 0;
-    // reverse neighbour lists: for each K the (I, n) with nbrs[I][n].K == K
-    std::vector<std::vector<std::pair<int, int>>> rev(natom);
-    for (int I = 0; I < natom; ++I)
-        for (size_t n = 0; n < nbrs[I].size(); ++n) rev[nbrs[I][n].K].push_back({I, (int)n});
-    std::set<int> classes(nb.begin(), nb.end());
-    std::map<std::tuple<int, int, int, int>, int> kt_pos;  // K-table start per species pair (per chunk)
-
+    ghat_max = 0;
     auto say = [&](const char *what, size_t a, size_t b) {
         if (!verbose) return;
         fprintf(stderr, "[librpa-mi355x] plan: %s %zu / %zu\n", what, a, b);
@@ -238,13 +225,11 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
     say("outputs (I <= J, R) and chunks", outs.size(), chunks.size());
     for (auto &c : chunks) {
         say("problem lists of chunk", (size_t)(&c - chunks.data()) + 1, chunks.size());
-        kt_pos.clear();
         // offsets inside the chunk buffers
-        long long go = 0, to = 0;
+        long long go = 0;
         for (int J = c.j_begin; J < c.j_end; ++J)
             for (int S = 0; S < nR; ++S)
                 for (int sg = 0; sg < 2; ++sg) { c.ghat_off.push_back(go); go += (long long)NAO * lsum[J]; }
-        for (int o = c.o_begin; o < c.o_end; ++o) { outs[o].toff = to; to += ksum[outs[o].I] * na[outs[o].J]; }
         auto ghat_at = [&](int J, int S, int sg) { return c.ghat_off[((size_t)(J - c.j_begin) * nR + S) * 2 + sg]; };
         auto w_at = [&](int J, int S) { return w_off[(size_t)J * nR + S]; };
 
@@ -276,122 +261,69 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
                                             w_at(J, S) + (long long)sp * nb[J] * NAO * na[J], na[J]);
                     pr.ncb = na[J];
                     pr.cbs = (long long)NAO * na[J];
-                    if (pr.K > 0) c.wb.add(pr);
+                    c.wb.add(pr);  // K = 0 (an atom without Cs) writes zeros
                 }
-        // G_KJ(R - R1) W(I, J, R) contracted with C^I directly: with
-        // X(I, J, R)[mu][(j, i)] = sum_(K,R1) C^I(K,R1)(mu, i, k) G_KJ(R - R1)(k, j) = W(J, -R)-block of I,
-        // chi0s(I, J, R) += sum_(s', j, i) W(I, -R)[(1 - s', i)][(J, j)][mu] W(J, R)[(s', j)][(I, i)][nu]
-        for (int o = c.o_begin; o < c.o_end; ++o) {
+        c.wb.finalize(big_tile(prec), stream);
+        c.d_jobs = upload(c.jobs, stream);
+        c.d_colsrc = upload(c.colsrc, stream);
+        flops_chi0_exec += c.wb.flops;
+        ghat_max = std::max(ghat_max, c.ghat_elems);
+    }
+    // ---- the contraction: every output block (chi0.hip) ----
+    {
+        std::vector<Chi0Seg> segs;
+        std::vector<int> segtab((size_t)natom * nR);
+        for (int I = 0; I < natom; ++I)
+            for (int r = 0; r < nR; ++r) {
+                const size_t first = segs.size();
+                segtab[(size_t)I * nR + r] = (int)first;
+                int at = 0;
+                for (const auto &n : nbrs[I]) {
+                    const auto &R1 = cells[n.r];
+                    const int S = fold_index(cells[r][0] - R1[0], cells[r][1] - R1[1], cells[r][2] - R1[2]);
+                    for (int k = 0; k < nb[n.K]; ++k) segs.push_back({S, (int)ao[n.K] + k, at++, 0});
+                }
+                std::sort(segs.begin() + first, segs.end(), [](const Chi0Seg &a, const Chi0Seg &b) {
+                    return std::make_pair(a.cell, a.row) < std::make_pair(b.cell, b.row);
+                });
+            }
+        std::vector<Chi0Out> co(outs.size());
+        out_flops.assign(outs.size(), 0.0);
+        contract_flops = contract_bytes = 0;
+        for (size_t o = 0; o < outs.size(); ++o) {
             const auto &O = outs[o];
             const auto &Rv = cells[O.r];
             const int mr = fold_index(-Rv[0], -Rv[1], -Rv[2]);
-            const int ni = nb[O.I], nj = nb[O.J];
-            const auto key = std::make_tuple(ni, na[O.I], nj, na[O.J]);
-            auto it = kt_pos.find(key);
-            if (it == kt_pos.end()) {
-                it = kt_pos.emplace(key, (int)(c.xb.ktab.size() / 2)).first;
-                for (int sp = 0; sp < 2; ++sp)
-                    for (int j = 0; j < nj; ++j)
-                        for (int i = 0; i < ni; ++i) {
-                            c.xb.ktab.push_back(((long long)(1 - sp) * ni + i) * NAO * na[O.I] + (long long)j * na[O.I]);
-                            c.xb.ktab.push_back(((long long)sp * nj + j) * NAO * na[O.J] + (long long)i * na[O.J]);
-                        }
-            }
-            GemmProb pr = make_prob(na[O.I], na[O.J], 2 * ni * nj, w_at(O.I, mr) + ao[O.J] * na[O.I], 0,
-                                    w_at(O.J, O.r) + ao[O.I] * na[O.J], 0, O.eoff, na[O.J]);
-            pr.kt_off = it->second;
-            c.xb.add(pr);
-            c.x_owner.push_back(o);
+            Chi0Out &c = co[o];
+            c.cfin = cfin_off[O.I];
+            c.gpm = O.r * gpm_r + ao[O.I] * 2LL * NAO + 2 * ao[O.J];
+            c.wseg = w_off[(size_t)O.J * nR];
+            c.xa = w_off[(size_t)O.I * nR + mr] + ao[O.J] * na[O.I];
+            c.xb = w_off[(size_t)O.J * nR + O.r] + ao[O.I] * na[O.J];
+            c.eoff = O.eoff;
+            c.I = O.I; c.J = O.J; c.r = O.r;
+            c.ni = nb[O.I]; c.nj = nb[O.J]; c.ai = na[O.I]; c.aj = na[O.J];
+            c.lsum = (int)lsum[O.I];
+            c.segtab = segtab[(size_t)O.I * nR + O.r];
+            // T, its contraction with C^I, and the direct term
+            const double ni = c.ni, nj = c.nj, ai = c.ai, aj = c.aj;
+            out_flops[o] = 4.0 * ni * nj * lsum[O.I] * aj + 2.0 * ai * ni * lsum[O.I] * aj + 4.0 * ai * aj * ni * nj;
+            contract_flops += out_flops[o];
+            contract_bytes += 2.0 * ts * ai * aj;
         }
-        // T_A: per (J, S, K, class of I), rows (I, n, i) from G_IJ(S + R1), B = W(K, J, S)
-        for (int J = c.j_begin; J < c.j_end; ++J)
-            for (int S = 0; S < nR; ++S)
-                for (int K = 0; K < natom; ++K)
-                    for (int cls : classes) {
-                        GemmProb pr = make_prob(0, nb[K] * na[J], 2 * nb[J], 0, 0, w_at(J, S) + ao[K] * na[J],
-                                                NAO * na[J], 0, 0);
-                        pr.ncb = na[J];
-                        pr.cbs = (long long)cls * na[J];
-                        pr.rt_off = (int)(c.ta.rowtab.size() / 2);
-                        int m = 0;
-                        const size_t owners0 = c.ta_outs.size();
-                        const auto &Sv = cells[S];
-                        for (const auto &in : rev[K]) {
-                            const int I = in.first, n = in.second;
-                            if (I > J || nb[I] != cls) continue;
-                            const auto &R1 = cells[nbrs[I][n].r];
-                            const int rr = fold_index(Sv[0] + R1[0], Sv[1] + R1[1], Sv[2] + R1[2]);
-                            const int o = out_index[((size_t)I * natom + J) * nR + rr];
-                            if (c.ta_outs.size() == owners0 || c.ta_outs.back() != o) c.ta_outs.push_back(o);
-                            for (int i = 0; i < nb[I]; ++i) {
-                                c.ta.rowtab.push_back(rr * gpm_r + (ao[I] + i) * 2LL * NAO + 2 * ao[J]);
-                                c.ta.rowtab.push_back(outs[o].toff + (koff[I][n] + i) * na[J]);
-                                ++m;
-                            }
-                        }
-                        if (m == 0) {
-                            c.ta.rowtab.resize((size_t)pr.rt_off * 2);
-                            c.ta_outs.resize(owners0);
-                            continue;
-                        }
-                        pr.M = m;
-                        c.ta.add(pr);
-                        if (c.ta_ptr.empty()) c.ta_ptr.push_back(0);
-                        c.ta_ptr.push_back((int)c.ta_outs.size());
-                    }
-        // final: chi0s(o) = Cfin_I (na_I x ksum_I) * T_o (ksum_I x na_J), K split in nsk parts that
-        // accumulate atomically: each output block has few, long tiles (K ~ 25k), and shorter ones
-        // fill the last wave of a launch better
-        for (int o = c.o_begin; o < c.o_end; ++o) {
-            const auto &O = outs[o];
-            if (ksum[O.I] == 0) continue;
-            const int cls = (na[O.I] > 64 ? 2 : 0) + (na[O.J] > 64 ? 1 : 0);
-            const int kt = (int)ksum[O.I];
-            const int step = std::max(32, (kt / nsk + 31) / 32 * 32);
-            for (int k0 = 0; k0 < kt; k0 += step) {
-                const int kl = std::min(step, kt - k0);
-                c.fin[cls].add(make_prob(na[O.I], na[O.J], kl, cfin_off[O.I] + (long long)k0 * na[O.I], na[O.I],
-                                         O.toff + (long long)k0 * na[O.J], na[O.J], O.eoff, na[O.J]));
-                c.fin_owner[cls].push_back(o);
-            }
-        }
-        c.wb.finalize(big_tile(prec), stream);
-        c.xb.trans_a = true;
-        c.xb.finalize(T64x64, stream);
-        c.ta.tag = 4;
-        c.ta.finalize(T64x128, stream);
-        c.fin_flops = 0;
-        for (auto &f : c.fin) {
-            f.tag = 3;
-            f.atomic = nsk > 1;
-            f.trans_a = true;  // Cfin_I is stored k-major, so A tiles load along mu
-            f.finalize(T64x64, stream);
-            c.fin_flops += f.flops;
-        }
-        c.d_jobs = upload(c.jobs, stream);
-        c.d_colsrc = upload(c.colsrc, stream);
-        flops_chi0_exec += c.wb.flops + c.xb.flops + c.ta.flops + c.fin_flops;
-        // algorithmic HBM bytes of each contraction launch: Cfin_I and T read once, chi0s read and written
-        for (int k = 0; k < 4; ++k) {
-            c.fin_bytes[k] = 0;
-            for (const auto &p : c.fin[k].probs)
-                c.fin_bytes[k] += (double)ts * ((double)p.M * p.K + (double)p.K * p.N + 2.0 * p.M * p.N);
-        }
-        c.ta_bytes = 0;
-        for (const auto &p : c.ta.probs)
-            c.ta_bytes += (double)ts * ((double)p.M * p.K + (double)p.K * p.N + (double)p.M * p.N);
+        // what the contraction has to move: W and Cs read once, chi0s read and written
+        contract_bytes += (double)ts * (w_off.back() + cfin_off[natom]);
+        flops_chi0_exec += contract_flops;
+        d_segs = upload(segs, stream);
+        d_couts = upload(co, stream);
+        d_skip.alloc(std::max<size_t>(1, outs.size()));
+        ctasks[0].build(co, prec == Prec::F64, 1, splitk, stream);
+        if (mixed) ctasks[1].build(co, false, 1, splitk, stream);
+        HIP_CHECK(hipStreamSynchronize(stream));
     }
     flops_chi0_exec *= ntau;
-    size_t max_g = 0, max_t = 0;
-    for (auto &c : chunks) {
-        max_g = std::max(max_g, (size_t)c.ghat_elems);
-        max_t = std::max(max_t, (size_t)c.t_elems);
-    }
-    ghat_max = max_g;
-    t_max = max_t;
-    d_Ghat.alloc(max_g * ts);
-    d_W.alloc((size_t)w_off.back() * ts);
-    d_T.alloc(max_t * ts);
+    d_Ghat.alloc(ghat_max * ts);
+    d_W.alloc((size_t)(w_off.back() + kChi0Pad) * ts);
     screen_plan(ds);
 
     // ---- G build data ----
@@ -540,29 +472,14 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
     if (host_staged) d_chiw.release();  // its room goes back to W and T (reformed for Ec)
     prepare_gf(mf, nbands_g);
     d_Ghat.reserve(ghat_max * ts);
-    d_W.reserve((size_t)w_off.back() * ts);
-    d_T.reserve(t_max * ts);
+    d_W.reserve((size_t)(w_off.back() + kChi0Pad) * ts);
     if (mixed) {
         if (prec != Prec::F64) LRA_THROW("mixed chi0 precision needs the FP64 plan");
         if (const char *e = std::getenv("LIBRPA_AMD_MIXED_AMAX")) mixed_amax = std::atof(e);
-        // the low-weight tau points run in mixed_low, FP32 or BF16x3 (both read the FP32 copies)
-        d_chi32.reserve(sizeof(float) * (size_t)E_tot);
     }
     cur = prec;
-    if (const char *ov = std::getenv("LIBRPA_AMD_OVERLAP")) overlap_ta = std::atoi(ov) != 0;
     // LIBRPA_AMD_AUTOTUNE=0 keeps the default tile shapes (no timing runs on first use)
     if (const char *at = std::getenv("LIBRPA_AMD_AUTOTUNE")) autotune = std::atoi(at) != 0;
-    if (overlap_ta && chunks.size() > 1) {
-        if (!s2) {
-            HIP_CHECK(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking));
-            for (hipEvent_t *e : {&ev_ready, &ev_s2, &ev_ta[0], &ev_ta[1], &ev_c[0], &ev_c[1]})
-                HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming));
-        }
-        // a second T buffer when the device has room for it (else the chunks run in sequence)
-        size_t free_b = 0, total_b = 0;
-        HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-        if (d_T2.bytes() < t_max * ts && free_b > t_max * ts + (size_t)4e9) d_T2.reserve(t_max * ts);
-    }
     HIP_CHECK(hipMemsetAsync(d_chi0s.get(), 0, d_chi0s.bytes(), stream));
     if (screen_mode != 0 && nspin > 1) LRA_THROW("chi0 block screening needs nspin = 1");
     if (host_staged && collect) LRA_THROW("screening samples need the device-resident chi0 store (too large here)");
@@ -572,10 +489,6 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
     }
     scr_blocks = scr_skipped = scr_flops = scr_flops_skipped = 0;
     if (collect) features.assign((size_t)ntau * MLP_NFEAT * outs.size(), 0.0f);
-    for (auto &c : chunks) {
-        c.xb.use_skip = c.ta.use_skip = false;
-        for (auto &f : c.fin) f.use_skip = false;
-    }
     bool tuned_chi0[2] = {false, false};  // [plan precision, FP32 of the mixed mode]
     n_lowp_tau = 0;
     for (int it = 0; it < ntau; ++it) {
@@ -590,31 +503,18 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
         }
         const bool lowp = cur != prec;
         n_lowp_tau += lowp ? 1 : 0;
-        // the small-K GEMMs (X: K = 2 n_b(I) n_b(J) in a K table; T_A: K = 2 n_b(J)) stay in FP32 when
-        // the tau point runs in BF16x3, whose 32-deep K slices would pad them and cost more than FP32
-        const Prec small = cur == Prec::BF16X3 ? Prec::F32 : cur;
         // low-precision tau points time under their own region names
         const char *lsuf = cur == Prec::BF16X3 ? "_bf16x3" : "_f32";
         auto rn = [lowp, lsuf](const char *r) { return lowp ? std::string(r) + lsuf : std::string(r); };
-        auto rs = [&rn, small, cur_ = cur](const char *r) {  // regions of the small-K GEMMs
-            return small == cur_ ? rn(r) : std::string(r) + "_f32";
-        };
         const double bsc = lowp ? 4.0 / ts : 1.0;  // algorithmic bytes scale with the element size
-        const void *Cfin_p = lowp ? d_Cfin32.get() : d_Cfin.get();
         const void *CWb_p = lowp ? d_CWb32.get() : d_CWb.get();
-        if (lowp) HIP_CHECK(hipMemsetAsync(d_chi32.get(), 0, d_chi32.bytes(), stream));
+        // the one slice of a host-staged store starts from zero at every tau
+        if (host_staged) HIP_CHECK(hipMemsetAsync(d_chi0s.get(), 0, d_chi0s.bytes(), stream));
         if (mixed)
-            for (auto &c : chunks) {
-                c.wb.use_tiles(cur, stream);
-                c.xb.use_tiles(small, stream);
-                c.ta.use_tiles(small, stream);
-                for (auto &f : c.fin) f.use_tiles(cur, stream);
-            }
+            for (auto &c : chunks) c.wb.use_tiles(cur, stream);
         for (int s = 0; s < nspin; ++s) {
             build_gf(mf, tau, s);
             if (s == 0 && (screen_mode != 0 || collect)) screen_tau(it, tau);
-            char *chi_base =
-                lowp ? d_chi32.as<char>() : d_chi0s.as<char>() + (host_staged ? 0 : (size_t)it * E_tot * ts);
             // tiles are tuned per precision on the first tau point built at it
             const bool tune_now = autotune && s == 0 && !tuned_chi0[lowp];
             for (auto &c : chunks) {
@@ -636,64 +536,26 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
                 gemm_run(cur, c.wb, d_Ghat.get(), CWb_p, d_W.get(), 1.0, 0.0, stream);
                 prof.end(rn("chi0_W"), stream, c.wb.flops);
             }
-            // T_A of chunk c + 1 (second stream, second T buffer) overlaps the contraction of chunk c
-            const bool overlap = overlap_ta && !tune_now && chunks.size() > 1 && d_T2.bytes() >= t_max * ts;
-            if (overlap) {
-                HIP_CHECK(hipEventRecord(ev_ready, stream));  // G and W of this tau written
-                HIP_CHECK(hipStreamWaitEvent(s2, ev_ready, 0));
-                for (size_t ci = 0; ci < chunks.size(); ++ci) {
-                    auto &c = chunks[ci];
-                    void *Tb = (ci % 2) ? d_T2.get() : d_T.get();
-                    // the contraction two chunks back has finished reading this buffer
-                    if (ci >= 2) HIP_CHECK(hipStreamWaitEvent(s2, ev_c[ci % 2], 0));
-                    prof.begin(rs("chi0_TA"), s2);
-                    gemm_run(small, c.ta, d_Gpm.get(), d_W.get(), Tb, 1.0, 0.0, s2);
-                    prof.end(rs("chi0_TA"), s2, c.ta.flops, c.ta_bytes * bsc);
-                    HIP_CHECK(hipEventRecord(ev_ta[ci % 2], s2));
-                    prof.begin(rs("chi0_X"), stream);
-                    gemm_run(small, c.xb, d_W.get(), d_W.get(), chi_base, 1.0, s == 0 ? 0.0 : 1.0, stream);
-                    prof.end(rs("chi0_X"), stream, c.xb.flops);
-                    HIP_CHECK(hipStreamWaitEvent(stream, ev_ta[ci % 2], 0));
-                    for (int k = 0; k < 4; ++k) {
-                        if (c.fin[k].total_tiles == 0) continue;
-                        prof.begin(rn("chi0_contract"), stream);
-                        gemm_run(cur, c.fin[k], Cfin_p, Tb, chi_base, 1.0, 1.0, stream);
-                        prof.end(rn("chi0_contract"), stream, c.fin[k].flops, c.fin_bytes[k] * bsc);
-                    }
-                    HIP_CHECK(hipEventRecord(ev_c[ci % 2], stream));
-                }
-                // the next G and W builds overwrite what T_A reads
-                HIP_CHECK(hipEventRecord(ev_s2, s2));
-                HIP_CHECK(hipStreamWaitEvent(stream, ev_s2, 0));
-                continue;
-            }
-            for (auto &c : chunks) {
-                if (tune_now && verbose) {
-                    fprintf(stderr, "[librpa-mi355x] chi0: tuning T_A and the contraction of chunk %d / %zu\n",
-                            (int)(&c - chunks.data()) + 1, chunks.size());
-                    fflush(stderr);
-                }
-                if (tune_now && c.ta.cfg_by_prec[(int)cur] < 0) {
-                    // TA overwrites T; the contraction trials accumulate into chi0s before the X
-                    // term below resets it (beta = 0) for this tau
-                    c.ta.tune(small, d_Gpm.get(), d_W.get(), d_T.get(), 1.0, 0.0, stream);
-                    gemm_run(small, c.ta, d_Gpm.get(), d_W.get(), d_T.get(), 1.0, 0.0, stream);
-                    for (auto &f : c.fin) f.tune(cur, Cfin_p, d_T.get(), chi_base, 1.0, 1.0, stream);
-                }
-                prof.begin(rs("chi0_X"), stream);
-                gemm_run(small, c.xb, d_W.get(), d_W.get(), chi_base, 1.0, s == 0 ? 0.0 : 1.0, stream);
-                prof.end(rs("chi0_X"), stream, c.xb.flops);
-                prof.begin(rs("chi0_TA"), stream);
-                gemm_run(small, c.ta, d_Gpm.get(), d_W.get(), d_T.get(), 1.0, 0.0, stream);
-                prof.end(rs("chi0_TA"), stream, c.ta.flops, c.ta_bytes * bsc);
-                // one timing region per launch (per block-shape class)
-                for (int k = 0; k < 4; ++k) {
-                    if (c.fin[k].total_tiles == 0) continue;
-                    prof.begin(rn("chi0_contract"), stream);
-                    gemm_run(cur, c.fin[k], Cfin_p, d_T.get(), chi_base, 1.0, 1.0, stream);
-                    prof.end(rn("chi0_contract"), stream, c.fin[k].flops, c.fin_bytes[k] * bsc);
-                }
-            }
+            // the contraction; a BF16x3 tau point contracts in FP32 (the kernel is bound by its
+            // operand reads there, and FP32 keeps more digits)
+            const size_t coff = host_staged ? 0 : (size_t)it * E_tot;
+            const unsigned char *skip = screen_mode != 0 ? d_skip.as<unsigned char>() : nullptr;
+            const std::string region = cur == Prec::F64 || prec == Prec::F32 ? "chi0_contract" : "chi0_contract_f32";
+            const int nout = (int)outs.size();
+            prof.begin(region, stream);
+            if (cur == Prec::F64)
+                launch_chi0_contract<double, double>(ctasks[0], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
+                                                     d_Gpm.as<double>(), 0, d_W.as<double>(), 0, d_Cfin.as<double>(),
+                                                     d_chi0s.as<double>() + coff, 0, NAO, 1, skip, stream);
+            else if (lowp)
+                launch_chi0_contract<float, double>(ctasks[1], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
+                                                    d_Gpm.as<float>(), 0, d_W.as<float>(), 0, d_Cfin32.as<float>(),
+                                                    d_chi0s.as<double>() + coff, 0, NAO, 1, skip, stream);
+            else
+                launch_chi0_contract<float, float>(ctasks[0], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
+                                                   d_Gpm.as<float>(), 0, d_W.as<float>(), 0, d_Cfin.as<float>(),
+                                                   d_chi0s.as<float>() + coff, 0, NAO, 1, skip, stream);
+            prof.end(region, stream, contract_flops, contract_bytes * bsc);
         }
         tuned_chi0[lowp] = tuned_chi0[lowp] || autotune;
         if (verbose) {
@@ -701,10 +563,6 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
             fprintf(stderr, "[librpa-mi355x] chi0: tau %d / %d (%.1f s)\n", it + 1, ntau, now_s() - t0);
             fflush(stderr);
         }
-        // the FP32 result of a low-precision tau point goes into the FP64 chi0(R, tau) store
-        if (lowp)
-            launch_convert<float, double>(d_chi32.as<float>(), d_chi0s.as<double>() + (host_staged ? 0 : (size_t)it * E_tot),
-                                          E_tot, stream);
         // a host-staged build keeps its slice in pageable host memory (stream order makes the next
         // tau's kernels wait for the copy)
         if (host_staged)
@@ -1082,8 +940,6 @@ void RpaEngine::release_ec() {
 void RpaEngine::release_work() {
     d_Ghat.release();
     d_W.release();
-    d_T.release();
-    d_T2.release();
 }
 
 void RpaEngine::free_host_store() {
@@ -1093,12 +949,6 @@ void RpaEngine::free_host_store() {
 
 RpaEngine::~RpaEngine() {
     free_host_store();
-    if (s2) {
-        (void)hipStreamSynchronize(s2);
-        for (hipEvent_t e : {ev_ready, ev_s2, ev_ta[0], ev_ta[1], ev_c[0], ev_c[1]})
-            if (e) (void)hipEventDestroy(e);
-        (void)hipStreamDestroy(s2);
-    }
 }
 
 void RpaEngine::chi0s_block(int it, int I, int J, int r, double *out) {

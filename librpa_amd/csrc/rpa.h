@@ -6,6 +6,7 @@
 #include <tuple>
 #include <vector>
 
+#include "chi0.h"
 #include "dataset.h"
 #include "gemm.h"
 #include "kernels.h"
@@ -29,34 +30,32 @@ struct RpaEngine {
 
     struct Nbr { int K, r; };
     std::vector<std::vector<Nbr>> nbrs;           // folded Cs neighbours of each atom
-    std::vector<std::vector<long long>> koff;     // row offset (in T / Cfin columns) per neighbour
+    std::vector<std::vector<long long>> koff;     // row offset (in Cfin) per neighbour
     std::vector<std::vector<long long>> loff;     // row offset in CWb per neighbour
     std::vector<long long> ksum, lsum, cfin_off, cwb_off;
     long long n_cs_blocks = 0;
 
-    struct Out { int I, J, r; long long eoff, toff; };
+    struct Out { int I, J, r; long long eoff; };
     std::vector<Out> outs;
     long long E_tot = 0;
 
     struct Chunk {
         int j_begin, j_end;          // atoms J in [j_begin, j_end)
-        int o_begin, o_end;          // outputs
-        long long ghat_elems = 0, t_elems = 0;
-        double fin_bytes[4] = {0, 0, 0, 0}, ta_bytes = 0;  // algorithmic HBM bytes per launch
+        long long ghat_elems = 0;
         std::vector<long long> ghat_off;  // per (J - j_begin, S, sigma)
         std::vector<GatherJob> jobs;
         std::vector<long long> colsrc;
         DevBuf d_jobs, d_colsrc;
         int max_gcol = 0;
-        // contraction batches by (na(I) > 64, na(J) > 64), so that each shape class gets its own
-        // tile (a tile covering all of na(I) reads T once)
-        GemmBatch wb, xb, ta, fin[4];
-        double fin_flops = 0;
-        // screening maps: output of each X / contraction problem, outputs written by each T_A problem
-        std::vector<int> x_owner, fin_owner[4], ta_ptr, ta_outs;
+        GemmBatch wb;
     };
     std::vector<Chunk> chunks;
     std::vector<long long> w_off;  // W(K, J, S) block of (J, S) in d_W
+    // the contraction (chi0.hip): task lists at the plan's precision and, in the mixed modes, FP32
+    Chi0Tasks ctasks[2];
+    DevBuf d_couts, d_segs, d_skip;
+    std::vector<double> out_flops;  // per output and tau point
+    double contract_flops = 0, contract_bytes = 0;
 
     // G build
     int band_lo[2] = {0, 0}, band_hi[2] = {0, 0};  // per sign (0: +tau, 1: -tau)
@@ -72,17 +71,10 @@ struct RpaEngine {
     int n_lowp_tau = 0;  // tau points of the last build that ran in FP32 (mixed mode)
     Prec mixed_low = Prec::F32;  // precision of those tau points
     Prec cur = Prec::F64;  // precision of the tau point being built
-    DevBuf d_Cfin32, d_CWb32, d_chi32;
-    DevBuf d_Cfin, d_CWb, d_ZZ, d_Zs, d_Mst, d_Gpm, d_Ghat, d_W, d_T, d_T2, d_chi0s;
+    DevBuf d_Cfin32, d_CWb32;
+    DevBuf d_Cfin, d_CWb, d_ZZ, d_Zs, d_Mst, d_Gpm, d_Ghat, d_W, d_chi0s;
     DevBuf d_wre, d_wim, d_eps, d_wg, d_cs, d_sn, d_gcol;
     hipStream_t stream = 0;
-    // T_A of the next chunk on a second stream (default priority, non-blocking) into a second
-    // T buffer, overlapping the current chunk's contraction.  Off unless LIBRPA_AMD_OVERLAP=1:
-    // on the 128-atom cell it saves 1.5% of the wall time, but the two kernels then share the
-    // memory system and each one's own timing no longer describes it.
-    bool overlap_ta = false;
-    hipStream_t s2 = nullptr;
-    hipEvent_t ev_ready = nullptr, ev_s2 = nullptr, ev_ta[2] = {nullptr, nullptr}, ev_c[2] = {nullptr, nullptr};
     RpaEngine() = default;
     RpaEngine(const RpaEngine &) = delete;
     RpaEngine &operator=(const RpaEngine &) = delete;
@@ -142,7 +134,7 @@ struct RpaEngine {
     void prepare_gf(const MeanField &mf, int nbands_g);
     void build_gf(const MeanField &mf, double tau, int s);
     void build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g);
-    void release_work();  // free the gathered-G, W and T work buffers (rebuilt by build_chi0)
+    void release_work();  // free the gathered-G and W work buffers (rebuilt by build_chi0)
     void release_ec();    // free the Ec work buffers (rebuilt by ec)
     // chi0(R, omega) = sum_tau (2 / nspin) gamma_c(omega, tau) chi0(R, tau) of the last build, FP64
     // [omega][E], formed once per Ec / W evaluation when it fits in max_bytes (returns whether it
@@ -160,7 +152,7 @@ struct RpaEngine {
     // kChi0RqMaxQ q points
     void assemble_dense_q(const TFGrid &g, const std::vector<const double *> &kfs, int w0, int cnt, void *dense,
                           bool f64, long long nn, bool embed, hipStream_t s);
-    long long ghat_max = 0, t_max = 0;
+    long long ghat_max = 0;
     RpaResult ec(const Dataset &ds, const TFGrid &g);
     // dense chi0(q, omega) block for verification
     void chi0q_block(const Dataset &ds, const TFGrid &g, int iw, int iq, int I, int J, double *re, double *im);

@@ -54,21 +54,6 @@ void RpaEngine::screen_plan(const Dataset &ds) {
     d_gnorm.alloc(sizeof(double) * 2 * std::max(1, nout));
     d_feat.alloc(sizeof(float) * MLP_NFEAT * std::max(1, nout));
     d_pred.alloc(sizeof(float) * std::max(1, nout));
-    for (auto &c : chunks) {
-        if (c.x_owner.size() != c.xb.probs.size() || (!c.ta.probs.empty() && c.ta_ptr.size() != c.ta.probs.size() + 1))
-            LRA_THROW("screening maps out of step with the problem lists");
-        for (int k = 0; k < 4; ++k)
-            if (c.fin_owner[k].size() != c.fin[k].probs.size()) LRA_THROW("screening maps out of step");
-        auto prep = [&](GemmBatch &b, bool zero) {
-            b.skipv.assign(b.probs.size(), 0);
-            b.d_skip.alloc(std::max<size_t>(1, b.probs.size()));
-            b.skip_zero = zero;
-            b.use_skip = false;
-        };
-        prep(c.xb, true);
-        prep(c.ta, false);
-        for (auto &f : c.fin) prep(f, false);
-    }
 }
 
 void RpaEngine::screen_tau(int it, double tau) {
@@ -128,32 +113,13 @@ void RpaEngine::screen_tau(int it, double tau) {
         for (int o = 0; o < nout; ++o)
             if ((double)pred_h[o] * tscale + tmean < lthr) skip_out[o] = 1;
     }
-    // per-problem flags of every batch that writes or reads an output block
     double fl = 0, fls = 0, nsk = 0;
-    auto flops_of = [](const GemmProb &p) { return 2.0 * p.M * p.N * (double)p.K; };
-    for (auto &c : chunks) {
-        for (size_t p = 0; p < c.xb.probs.size(); ++p) c.xb.skipv[p] = skip_out[c.x_owner[p]];
-        for (size_t p = 0; p < c.ta.probs.size(); ++p) {
-            unsigned char all = 1;
-            for (int q = c.ta_ptr[p]; q < c.ta_ptr[p + 1] && all; ++q) all = skip_out[c.ta_outs[q]];
-            c.ta.skipv[p] = all;
-        }
-        for (int k = 0; k < 4; ++k)
-            for (size_t p = 0; p < c.fin[k].probs.size(); ++p) c.fin[k].skipv[p] = skip_out[c.fin_owner[k][p]];
-        auto push = [&](GemmBatch &b) {
-            for (size_t p = 0; p < b.probs.size(); ++p) {
-                fl += flops_of(b.probs[p]);
-                if (b.skipv[p]) fls += flops_of(b.probs[p]);
-            }
-            if (!b.probs.empty())
-                HIP_CHECK(hipMemcpyAsync(b.d_skip.get(), b.skipv.data(), b.skipv.size(), hipMemcpyHostToDevice, stream));
-            b.use_skip = true;
-        };
-        push(c.xb);
-        push(c.ta);
-        for (auto &f : c.fin) push(f);
+    for (int o = 0; o < nout; ++o) {
+        fl += out_flops[o];
+        if (skip_out[o]) fls += out_flops[o];
+        nsk += skip_out[o];
     }
-    for (int o = 0; o < nout; ++o) nsk += skip_out[o];
+    HIP_CHECK(hipMemcpyAsync(d_skip.get(), skip_out.data(), nout, hipMemcpyHostToDevice, stream));
     scr_blocks += nout;
     scr_skipped += nsk;
     scr_flops += fl;
