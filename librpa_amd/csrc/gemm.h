@@ -12,9 +12,9 @@
 //   * column table on C: the within-block part c % ncb may be replaced by an
 //     entry of a table of element offsets (scattered output columns);
 //   * atomic epilogue: C += alpha A B with atomic adds, for outputs that several
-//     problems of one launch accumulate into;
-//   * K table: the inner index k may address A and B through a table of element
-//     offsets (a_k, b_k), for contractions whose summed index spans several strides.
+//     problems of one launch accumulate into.
+// A batch may run nz times in one launch on operands za, zb, zc elements apart (the tau points of a
+// small system), so that few problems still fill the device.
 #pragma once
 
 #include <functional>
@@ -41,7 +41,6 @@ struct GemmProb {
     int rt_off;    // offset into the row table, -1 if not row-indirect
     int kmode;     // triangular operand: 0 none, 1 B lower (k < n is zero), 2 A = L^T (k < m is zero)
     int ct_off;    // offset into the column table, -1 if none
-    int kt_off;    // offset (in pairs) into the K table, -1 if none
 };
 
 // Tile configurations (BM x BN; 256 threads, the w8 shapes 512).
@@ -69,21 +68,16 @@ struct GemmBatch {
     std::vector<GemmProb> probs;
     std::vector<long long> rowtab;  // pairs (a_row_off, c_row_off)
     std::vector<long long> coltab;  // C column offsets (within a column-split block)
-    std::vector<long long> ktab;    // pairs (a_k, b_k): offsets of inner index k in A and B
     int cfg = T64x64;
     bool trans_a = false;  // A stored as A^T (element (m,k) at a_off + k*lda + m)
     bool trans_b = false;  // B stored as B^T (element (k,n) at b_off + n*ldb + k)
     bool lower_only = false;
     bool atomic = false;   // C += alpha A B by atomic adds (beta must be 1)
-    // per-problem skip flags (screening): skipped problems return, or with skip_zero write
-    // alpha * 0 + beta * C; d_skip is filled by the owner before a launch with use_skip set
-    bool use_skip = false, skip_zero = false;
-    std::vector<unsigned char> skipv;
-    DevBuf d_skip;
-    int tag = 0;           // 3 / 4: launch under a separately named (traceable) plain instantiation
+    int nz = 1;                        // copies of the batch in one launch
+    long long za = 0, zb = 0, zc = 0;  // operand distances of a copy, in elements
     int total_tiles = 0;
     double flops = 0;      // flops of one launch: 2 M N K summed, less the skipped triangular work
-    DevBuf d_probs, d_rowtab, d_coltab, d_ktab;
+    DevBuf d_probs, d_rowtab, d_coltab;
 
     bool tuned = false;
     float tuned_ms = 0;    // time of the chosen tile shape in the tuning run

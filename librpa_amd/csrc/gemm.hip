@@ -64,10 +64,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int G) {
     return x < rem ? x * (per + 1) + idx : rem * (per + 1) + (x - rem) * per + idx;
 }
 
-// VAR selects the addressing extras compiled in: 0 plain, 1 K table, 2 column table and
-// atomic epilogue (kept out of the plain kernels, where they cost registers), 3 and 4 plain
-// code under separate symbols (the chi0 contraction and T_A, so that kernel traces can
-// isolate them).
+// VAR selects the addressing extras compiled in: 0 plain, 2 column table and atomic epilogue
+// (kept out of the plain kernels, where they cost registers).  blockIdx.y is the copy of the batch.
 template <int MODE, int BM, int BN, int WM, int WN, bool TA, bool TB, int VAR>
 __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__restrict__ probs, int nprob, int total,
                                                     const typename ModeTraits<MODE>::T *__restrict__ A,
@@ -75,17 +73,13 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
                                                     typename ModeTraits<MODE>::T *__restrict__ C,
                                                     const long long *__restrict__ rowtab,
                                                     const long long *__restrict__ coltab,
-                                                    const long long *__restrict__ ktab,
                                                     typename ModeTraits<MODE>::T alpha,
                                                     typename ModeTraits<MODE>::T beta, int lower_only, int atomic,
-                                                    const unsigned char *__restrict__ skip, int skip_zero) {
+                                                    long long za, long long zb, long long zc) {
     using T = typename ModeTraits<MODE>::T;
     using V = typename ModeTraits<MODE>::V;
     constexpr int NT = WM * WN * 64;
-    // the chi0 contraction (VAR 3, K ~ 25k) runs with a 32-deep K slice: half the barriers per
-    // flop; T_A (VAR 4, K = 2 n_basis(J), e.g. 40) with an 8-deep one, which pads K by at most 7
-    constexpr bool bk8 = VAR == 4 && MODE != 2 && (BM * 8) % NT == 0 && (BN * 8) % NT == 0;
-    constexpr int BK = (VAR == 3 && MODE != 2) ? 32 : bk8 ? 8 : ModeTraits<MODE>::BK;
+    constexpr int BK = ModeTraits<MODE>::BK;
     constexpr int PAD = ModeTraits<MODE>::PAD;
     constexpr int LDK = BK + PAD;
     static_assert(WM * WN == 4 || WM * WN == 8, "4 or 8 waves");
@@ -106,9 +100,9 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
     if (tile >= total) return;
     const int pi = find_prob(probs, nprob, tile);
     const GemmProb P = probs[pi];
-    // a screened-out problem: return, or (skip_zero) write alpha * 0 + beta * C without the K loop
-    const bool dead = skip != nullptr && skip[pi] != 0;
-    if (dead && !skip_zero) return;
+    A += blockIdx.y * za;
+    B += blockIdx.y * zb;
+    C += blockIdx.y * zc;
     const int lt = tile - P.tile0;
     const int tm = lt / P.tiles_n, tn = lt % P.tiles_n;
     const int m0 = tm * BM, n0 = tn * BN;
@@ -152,14 +146,13 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
             for (int r = 0; r < 4; ++r) acc[a][b][r] = 0;
 
     T ra[LA], rb[LB];
-    constexpr bool kt = VAR == 1;
     auto gload = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
             const int gk = k0 + ak[i];
             T v = 0;
             if (arow[i] >= 0 && gk < P.K) {
-                const long long ko = kt ? ktab[2ll * (P.kt_off + gk)] : (TA ? (long long)gk * P.lda : (long long)gk);
+                const long long ko = TA ? (long long)gk * P.lda : (long long)gk;
                 v = A[arow[i] + ko];
             }
             ra[i] = v;
@@ -169,8 +162,7 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
             const int gk = k0 + bk[i], gn = n0 + bn[i];
             T v = 0;
             if (gk < P.K && gn < P.N) {
-                const long long ko =
-                    kt ? ktab[2ll * (P.kt_off + gk) + 1] : (TB ? (long long)gk : (long long)gk * P.ldb);
+                const long long ko = TB ? (long long)gk : (long long)gk * P.ldb;
                 v = TB ? B[P.b_off + (long long)gn * P.ldb + ko] : B[P.b_off + ko + gn];
             }
             rb[i] = v;
@@ -206,7 +198,6 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
     int kbeg = 0;
     if (P.kmode == 1) kbeg = (n0 / BK) * BK;
     else if (P.kmode == 2) kbeg = (m0 / BK) * BK;
-    if (dead) kbeg = P.K;
     gload(kbeg);
     for (int k0 = kbeg; k0 < P.K; k0 += BK) {
         __syncthreads();
@@ -279,13 +270,9 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
             ccol[b] = col;
         }
     }
-    // a full tile with alpha = 1, beta = 0 and plain stores (the chi0 build's W, X and T_A GEMMs):
-    // no per-element checks, scaling or reads of C
-    // T_A (tag 4) writes the contraction's T operand, gigabytes per launch that no cache keeps
-    // until the contraction reads them: in FP64 streamed past the caches with non-temporal stores
-    // (6% faster on the 128-atom cell). 16 lanes then write whole 128-byte lines; with 4-byte
-    // elements they write half lines, and non-temporal stores made the FP32 T_A 17% slower.
-    const bool plain = !((VAR == 2 || VAR == 3) && atomic) && alpha == T(1) && beta == T(0);
+    // a full tile with alpha = 1, beta = 0 and plain stores (the chi0 build's W GEMMs): no
+    // per-element checks, scaling or reads of C
+    const bool plain = !(VAR == 2 && atomic) && alpha == T(1) && beta == T(0);
     if (plain && m0 + BM <= P.M && n0 + BN <= P.N) {
 #pragma unroll
         for (int a = 0; a < FM; ++a) {
@@ -294,10 +281,7 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
                 const int gm = m0 + wm * WTM + a * 16 + (MODE == 0 ? 4 * r + kq : 4 * kq + r);
                 const long long crow = rt ? rowtab[2ll * (P.rt_off + gm) + 1] : P.c_off + (long long)gm * P.ldc;
 #pragma unroll
-                for (int b = 0; b < FN; ++b) {
-                    if constexpr (VAR == 4 && sizeof(T) == 8) __builtin_nontemporal_store(acc[a][b][r], C + crow + ccol[b]);
-                    else C[crow + ccol[b]] = acc[a][b][r];
-                }
+                for (int b = 0; b < FN; ++b) C[crow + ccol[b]] = acc[a][b][r];
             }
         }
         return;
@@ -316,13 +300,12 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
                 if (ccol[b] < 0) continue;
                 T *dst = C + crow + ccol[b];
                 const T v0 = alpha * acc[a][b][r];
-                if ((VAR == 2 || VAR == 3) && atomic) {
+                if (VAR == 2 && atomic) {
                     atomicAdd(dst, v0);
                 } else {
                     T v = v0;
                     if (beta != T(0)) v += beta * *dst;
-                    if constexpr (VAR == 4 && sizeof(T) == 8) __builtin_nontemporal_store(v, dst);
-                    else *dst = v;
+                    *dst = v;
                 }
             }
         }
@@ -348,7 +331,6 @@ GemmProb make_prob(int M, int N, int K, long long a_off, int lda, long long b_of
     p.a_off = a_off; p.lda = lda; p.b_off = b_off; p.ldb = ldb; p.c_off = c_off; p.ldc = ldc;
     p.rt_off = -1;
     p.ct_off = -1;
-    p.kt_off = -1;
     return p;
 }
 
@@ -378,7 +360,6 @@ void GemmBatch::finalize(int cfg_, hipStream_t s) {
     // the tables do not depend on the tile shape: upload once
     if (!rowtab.empty() && d_rowtab.bytes() != rowtab.size() * sizeof(long long)) d_rowtab = upload(rowtab, s);
     if (!coltab.empty() && d_coltab.bytes() != coltab.size() * sizeof(long long)) d_coltab = upload(coltab, s);
-    if (!ktab.empty() && d_ktab.bytes() != ktab.size() * sizeof(long long)) d_ktab = upload(ktab, s);
 }
 
 template <int MODE, int CFG, bool TA, bool TB, int VAR>
@@ -392,12 +373,12 @@ static void launch_one(const GemmBatch &b, const void *A, const void *B, void *C
     // 8-wave tiles: 128x128 as 2 x 4 waves of 64x32, 128x64 as 4 x 2 waves of 32x32
     constexpr int WM = (CFG == 2 || CFG == 5) ? 1 : (CFG == 8) ? 4 : 2;
     constexpr int WN = (CFG == 7) ? 4 : (CFG == 8) ? 2 : 4 / WM;
-    hipLaunchKernelGGL((ggemm_kernel<MODE, BM, BN, WM, WN, TA, TB, VAR>), dim3(b.total_tiles), dim3(WM * WN * 64), 0, s,
+    hipLaunchKernelGGL((ggemm_kernel<MODE, BM, BN, WM, WN, TA, TB, VAR>), dim3(b.total_tiles, b.nz),
+                       dim3(WM * WN * 64), 0, s,
                        b.d_probs.as<GemmProb>(), (int)b.probs.size(), b.total_tiles, static_cast<const T *>(A),
                        static_cast<const T *>(B), static_cast<T *>(C), b.d_rowtab.as<long long>(),
-                       b.d_coltab.as<long long>(), b.d_ktab.as<long long>(), (T)alpha, (T)beta,
-                       (int)b.lower_only, (int)b.atomic, b.use_skip ? b.d_skip.as<unsigned char>() : nullptr,
-                       (int)b.skip_zero);
+                       b.d_coltab.as<long long>(), (T)alpha, (T)beta, (int)b.lower_only, (int)b.atomic, b.za, b.zb,
+                       b.zc);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -421,22 +402,6 @@ static void launch_cfg(const GemmBatch &b, const void *A, const void *B, void *C
 template <int MODE>
 static void launch_mode(const GemmBatch &b, const void *A, const void *B, void *C, double alpha, double beta,
                         hipStream_t s) {
-    if (!b.ktab.empty()) {
-        // K-table batches: transposed A, plain B, 64x64 tiles
-        if (!b.trans_a || b.trans_b || b.cfg != T64x64 || b.atomic || !b.coltab.empty())
-            LRA_THROW("K-table GEMM: transposed A, plain B, 64x64 tiles, plain epilogue");
-        launch_one<MODE, 0, true, false, 1>(b, A, B, C, alpha, beta, s);
-        return;
-    }
-    if (b.tag == 3 || b.tag == 4) {
-        // same code as the plain kernel, instantiated separately so that traces can tell it apart
-        if (b.trans_b || (b.trans_a && b.tag == 4) || !b.coltab.empty() || (b.atomic && b.tag == 4))
-            LRA_THROW("tagged GEMM: plain B, no column table (and plain A, plain epilogue for tag 4)");
-        if (b.tag == 3 && b.trans_a) launch_cfg<MODE, true, false, 3>(b, A, B, C, alpha, beta, s);
-        else if (b.tag == 3) launch_cfg<MODE, false, false, 3>(b, A, B, C, alpha, beta, s);
-        else launch_cfg<MODE, false, false, 4>(b, A, B, C, alpha, beta, s);
-        return;
-    }
     if (b.atomic || !b.coltab.empty()) {
         // column-table / atomic batches: plain A and B, 64x64 or 128x128 tiles
         if (b.trans_a || b.trans_b || (b.cfg != T128x128 && b.cfg != T64x64))
@@ -461,8 +426,8 @@ std::map<std::vector<long long>, std::pair<int, float>> &tune_cache() {
     return c;
 }
 std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
-    std::vector<long long> k = {(long long)prec, b.tag, b.trans_a, b.trans_b, b.lower_only,
-                                (long long)b.rowtab.size(), (long long)b.coltab.size(), (long long)b.ktab.size()};
+    std::vector<long long> k = {(long long)prec, b.nz, b.trans_a, b.trans_b, b.lower_only,
+                                (long long)b.rowtab.size(), (long long)b.coltab.size()};
     k.reserve(k.size() + 8 * b.probs.size());
     for (const auto &p : b.probs) {
         k.push_back(p.M);
@@ -471,7 +436,7 @@ std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
         k.push_back(p.lda);
         k.push_back(p.ldb);
         k.push_back(p.ldc);
-        k.push_back(p.kmode + 4 * (p.rt_off >= 0) + 8 * (p.ct_off >= 0) + 16 * (p.kt_off >= 0));
+        k.push_back(p.kmode + 4 * (p.rt_off >= 0) + 8 * (p.ct_off >= 0));
         k.push_back(p.ncb < p.N ? p.ncb : 0);
     }
     return k;
@@ -480,7 +445,7 @@ std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
 
 int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alpha, double beta, hipStream_t s,
                     const std::function<void()> &before) {
-    if (probs.empty() || (atomic && tag != 3)) return cfg;
+    if (probs.empty() || atomic) return cfg;
     const auto key = tune_key(prec, *this);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -493,11 +458,8 @@ int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alp
             return cfg;
         }
     }
-    const bool was_skip = use_skip;
-    use_skip = false;
     std::vector<int> cands;
-    if (!ktab.empty()) cands = {T64x64};
-    else if (!coltab.empty()) cands = {T64x64, T128x128};
+    if (!coltab.empty()) cands = {T64x64, T128x128};
     else for (int c = 0; c < NUM_TILE_CFG; ++c) cands.push_back(c);
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
@@ -526,7 +488,6 @@ int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alp
     HIP_CHECK(hipEventDestroy(e0));
     HIP_CHECK(hipEventDestroy(e1));
     finalize(bc, s);
-    use_skip = was_skip;
     tuned = true;
     tuned_ms = best;
     cfg_by_prec[(int)prec] = bc;

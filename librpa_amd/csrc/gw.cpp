@@ -845,7 +845,7 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
         DevBuf dcw = upload(cw, st), dsw = upload(sw, st);
         if (verbose) { fprintf(stderr, "[librpa-mi355x] Sigma_c: tau %d / %d (%.1f s)\n", it + 1, g.n, now_s() - t0); fflush(stderr); }
         for (int s = 0; s < nspin; ++s) {
-            R0.build_gf(ds.mf, g.tau[it], s);
+            R0.build_gf(ds.mf, &g.tau[it], 1, s);
             for (int sg = 0; sg < 2; ++sg) {
                 HIP_CHECK(hipMemsetAsync(d_sig[sg].get(), 0, d_sig[sg].bytes(), st));
                 HIP_CHECK(hipMemsetAsync(d_extA.get(), 0, d_extA.bytes(), st));

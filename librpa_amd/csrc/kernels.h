@@ -6,20 +6,25 @@
 namespace lra {
 
 // G(R, +-tau) build ----------------------------------------------------------------
-// Zs[(2b + c)][j] = s_b * (c == 0 ? Re U[b][j] : Im U[b][j]) for b in [b0, b1),
-// s_b = exp(min(0, -tau (eps_b - mu))) * w_b with the occupation weights of
+// For every tau point z < taus.n and sign sg (0: +tau, 1: -tau):
+// Zs[z][sg][k][(2b + c)][j] = s_b * (c == 0 ? Re U[b][j] : Im U[b][j]) for b in [b0[sg], b1[sg]),
+// s_b = exp(min(0, -t (eps_b - mu))) * w_b with the occupation weights of
 // build_gf_Rt_libri_serial (src/core/chi0.cpp:333-355).  U, eps, wg per k.
-void launch_scale_bands(const double *wre, const double *wim, const double *eps, const double *wg,
-                        double *Zs, int nk, int nbands, int nbasis, int b0, int b1, double tau, double efermi,
+constexpr int kTauMax = 34;  // the largest minimax grid
+struct TauList { int n; double t[kTauMax]; };
+void launch_scale_bands(const double *wre, const double *wim, const double *eps, const double *wg, double *Zs, int nk,
+                        int nbands, int nbasis, const int b0[2], const int b1[2], const TauList &taus, double efermi,
                         int nspin, int nbands_g, hipStream_t s);
 
-// Gpm[R][row][gcol[col]] = sgn * sum_k (cs[R][k] Mre_k[row][col] + sn[R][k] Mim_k[row][col]),
-// Mstack per k laid out [Re rows; Im rows] (2 nbasis x nbasis).  T = double or float.
+// Gpm[z][R][row][gcol[sg][col]] = (sg ? -1 : 1) sum_k (cs[R][k] Mre_k[row][col] + sn[R][k] Mim_k[row][col]),
+// Mstack[z][sg][k] laid out [Re rows; Im rows] (2 nbasis x nbasis), for nz tau points and both
+// signs.  T = double or float.
 template <class T>
 void launch_k2r(const double *Mstack, const double *cs, const double *sn, const int *gcol, T *Gpm, int nk, int nR,
-                int nbasis, double sgn, hipStream_t s);
+                int nbasis, int nz, hipStream_t s);
 
-// Column gather: dst[job][row][c] = src[colsrc[job_cols + c] + row * src_ld] for row < nrows.
+// Column gather: dst[job][row][c] = src[colsrc[job_cols + c] + row * src_ld] for row < nrows, for nz
+// sources zs and destinations zd elements apart.
 struct GatherJob {
     long long dst_off;
     int ncol;
@@ -27,7 +32,8 @@ struct GatherJob {
 };
 template <class T>
 void launch_gather_cols(const T *src, long long src_ld, T *dst, const GatherJob *jobs, int njobs,
-                        const long long *colsrc, int nrows, int maxcol, hipStream_t s);
+                        const long long *colsrc, int nrows, int maxcol, hipStream_t s, int nz = 1, long long zs = 0,
+                        long long zd = 0);
 
 // tau -> omega and R -> q of chi0s into dense Hermitian matrices ---------------------
 // For each pair p = (I <= J) with element count na_I * na_J and each omega w of the
@@ -48,7 +54,7 @@ void launch_chi0_assemble(const TS *chi0s, long long E_tot, int ntau, const Pair
 // The same in two passes, when a chi0(R, omega) store fits: chiw[w][i] = sum_t coef[w][t]
 // chi0s[t][i] once for all q (coef = (2 / nspin) gamma_c, nw x ntau, row-major), then per q and
 // frequency chunk the R -> q phase sum ph[r] = (cos, sin)(2 pi q.R_r) into dense matrices.
-constexpr int kTauOmegaMax = 34;  // the largest minimax grid
+constexpr int kTauOmegaMax = kTauMax;
 void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
                          hipStream_t s);
 void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,

@@ -12,14 +12,18 @@ namespace lra {
 // ------------------------------------------------------------------------------------
 // G build helpers
 // ------------------------------------------------------------------------------------
-__global__ void scale_bands_kernel(const double *__restrict__ wre, const double *__restrict__ wim,
-                                   const double *__restrict__ eps, const double *__restrict__ wg,
-                                   double *__restrict__ Zs, int nk, int nbands, int nbasis, int b0, int b1,
-                                   double tau, double efermi, int nspin, int nbands_g) {
+__global__ __launch_bounds__(256) void scale_bands_kernel(const double *__restrict__ wre,
+                                                          const double *__restrict__ wim,
+                                                          const double *__restrict__ eps,
+                                                          const double *__restrict__ wg, double *__restrict__ Zs,
+                                                          int nk, int nbands, int nbasis, int lo0, int hi0, int lo1,
+                                                          int hi1, TauList taus, double efermi, int nspin,
+                                                          int nbands_g) {
+    const int k = blockIdx.y, sg = blockIdx.z & 1, b0 = sg ? lo1 : lo0, b1 = sg ? hi1 : hi0;
     const long long per_k = (long long)(b1 - b0) * nbasis;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (idx >= per_k || k >= nk) return;
+    if (idx >= per_k) return;
+    const double tau = sg ? -taus.t[blockIdx.z >> 1] : taus.t[blockIdx.z >> 1];
     const int b = b0 + (int)(idx / nbasis);
     const int j = (int)(idx % nbasis);
     const double e = eps[(long long)k * nbands + b];
@@ -36,60 +40,73 @@ __global__ void scale_bands_kernel(const double *__restrict__ wre, const double 
     double sb = exp(sc) * w;
     if (nbands_g >= 0 && b >= nbands_g) sb = 0;
     const long long src = ((long long)k * nbands + b) * nbasis + j;
-    double *z = Zs + (long long)k * 2 * nbands * nbasis;
+    double *z = Zs + ((long long)blockIdx.z * nk + k) * 2 * nbands * nbasis;
     z[(2ll * b) * nbasis + j] = sb * wre[src];
     z[(2ll * b + 1) * nbasis + j] = sb * wim[src];
 }
 
-void launch_scale_bands(const double *wre, const double *wim, const double *eps, const double *wg, double *Zs,
-                        int nk, int nbands, int nbasis, int b0, int b1, double tau, double efermi, int nspin,
-                        int nbands_g, hipStream_t s) {
-    if (b1 <= b0) return;
-    const long long per_k = (long long)(b1 - b0) * nbasis;
-    dim3 grid(ceil_div(per_k, 256), nk);
-    hipLaunchKernelGGL(scale_bands_kernel, grid, dim3(256), 0, s, wre, wim, eps, wg, Zs, nk, nbands, nbasis, b0,
-                       b1, tau, efermi, nspin, nbands_g);
+void launch_scale_bands(const double *wre, const double *wim, const double *eps, const double *wg, double *Zs, int nk,
+                        int nbands, int nbasis, const int b0[2], const int b1[2], const TauList &taus, double efermi,
+                        int nspin, int nbands_g, hipStream_t s) {
+    const long long per_k = (long long)std::max(b1[0] - b0[0], b1[1] - b0[1]) * nbasis;
+    if (per_k <= 0 || taus.n <= 0) return;
+    hipLaunchKernelGGL(scale_bands_kernel, dim3(ceil_div(per_k, 256), nk, 2 * taus.n), dim3(256), 0, s, wre, wim, eps,
+                       wg, Zs, nk, nbands, nbasis, b0[0], b1[0], b0[1], b1[1], taus, efermi, nspin, nbands_g);
     HIP_CHECK(hipGetLastError());
 }
 
+// k -> R: a thread holds one (row, column) of kK2rCells cells, so that M is read once per group of
+// cells and a small basis (17 functions on 27 k) still spreads over the device.  With one thread for
+// all cells that case took 0.2 ms per tau point and sign on two workgroups.
+constexpr int kK2rCells = 4;
 template <class T>
-__global__ void k2r_kernel(const double *__restrict__ M, const double *__restrict__ cs, const double *__restrict__ sn,
-                           const int *__restrict__ gcol, T *__restrict__ G, int nk, int nR, int nbasis, double sgn) {
+__global__ __launch_bounds__(256) void k2r_kernel(const double *__restrict__ M, const double *__restrict__ cs,
+                                                  const double *__restrict__ sn, const int *__restrict__ gcol,
+                                                  T *__restrict__ G, int nk, int nR, int nbasis) {
     const long long nn = (long long)nbasis * nbasis;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nn) return;
+    const int r0 = blockIdx.y * kK2rCells, z = blockIdx.z >> 1, sg = blockIdx.z & 1;
+    M += (long long)blockIdx.z * nk * 2 * nn;
+    G += (long long)z * nR * 2 * nn;
     const int row = (int)(idx / nbasis), col = (int)(idx % nbasis);
-    const long long kstride = 2 * nn;
-    const long long dst = (long long)row * 2 * nbasis + gcol[col];
-    for (int r = 0; r < nR; ++r) {
-        double acc = 0;
-        for (int k = 0; k < nk; ++k) {
-            const double re = M[k * kstride + idx];
-            const double im = M[k * kstride + nn + idx];
-            acc += cs[r * nk + k] * re + sn[r * nk + k] * im;
+    const long long dst = (long long)row * 2 * nbasis + gcol[sg * nbasis + col];
+    double acc[kK2rCells];
+#pragma unroll
+    for (int i = 0; i < kK2rCells; ++i) acc[i] = 0;
+    for (int k = 0; k < nk; ++k) {
+        const double re = M[k * 2 * nn + idx], im = M[k * 2 * nn + nn + idx];
+#pragma unroll
+        for (int i = 0; i < kK2rCells; ++i) {
+            const int r = min(r0 + i, nR - 1);
+            acc[i] += cs[r * nk + k] * re + sn[r * nk + k] * im;
         }
-        G[(long long)r * 2 * nn + dst] = static_cast<T>(sgn * acc);
     }
+#pragma unroll
+    for (int i = 0; i < kK2rCells; ++i)
+        if (r0 + i < nR) G[(long long)(r0 + i) * 2 * nn + dst] = static_cast<T>(sg ? -acc[i] : acc[i]);
 }
 
 template <class T>
 void launch_k2r(const double *Mstack, const double *cs, const double *sn, const int *gcol, T *Gpm, int nk, int nR,
-                int nbasis, double sgn, hipStream_t s) {
+                int nbasis, int nz, hipStream_t s) {
     const long long nn = (long long)nbasis * nbasis;
-    hipLaunchKernelGGL((k2r_kernel<T>), dim3(ceil_div(nn, 256)), dim3(256), 0, s, Mstack, cs, sn, gcol, Gpm, nk,
-                       nR, nbasis, sgn);
+    hipLaunchKernelGGL((k2r_kernel<T>), dim3(ceil_div(nn, 256), ceil_div(nR, kK2rCells), 2 * nz), dim3(256), 0, s,
+                       Mstack, cs, sn, gcol, Gpm, nk, nR, nbasis);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_k2r<double>(const double *, const double *, const double *, const int *, double *, int, int,
-                                 int, double, hipStream_t);
+                                 int, int, hipStream_t);
 template void launch_k2r<float>(const double *, const double *, const double *, const int *, float *, int, int,
-                                int, double, hipStream_t);
+                                int, int, hipStream_t);
 
 template <class T>
 __global__ void gather_cols_kernel(const T *__restrict__ src, long long src_ld, T *__restrict__ dst,
                                    const GatherJob *__restrict__ jobs, const long long *__restrict__ colsrc,
-                                   int nrows) {
+                                   int nrows, long long zs, long long zd) {
     const GatherJob J = jobs[blockIdx.y];
+    src += blockIdx.z * zs;
+    dst += blockIdx.z * zd;
     const long long n = (long long)nrows * J.ncol;
     for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
          idx += (long long)gridDim.x * blockDim.x) {
@@ -100,18 +117,19 @@ __global__ void gather_cols_kernel(const T *__restrict__ src, long long src_ld, 
 
 template <class T>
 void launch_gather_cols(const T *src, long long src_ld, T *dst, const GatherJob *jobs, int njobs,
-                        const long long *colsrc, int nrows, int maxcol, hipStream_t s) {
+                        const long long *colsrc, int nrows, int maxcol, hipStream_t s, int nz, long long zs,
+                        long long zd) {
     if (njobs == 0) return;
     const long long n = (long long)nrows * maxcol;
     const int bx = std::min(ceil_div(n, 256), 2048);
-    hipLaunchKernelGGL((gather_cols_kernel<T>), dim3(bx, njobs), dim3(256), 0, s, src, src_ld, dst, jobs, colsrc,
-                       nrows);
+    hipLaunchKernelGGL((gather_cols_kernel<T>), dim3(bx, njobs, nz), dim3(256), 0, s, src, src_ld, dst, jobs, colsrc,
+                       nrows, zs, zd);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_gather_cols<double>(const double *, long long, double *, const GatherJob *, int,
-                                         const long long *, int, int, hipStream_t);
+                                         const long long *, int, int, hipStream_t, int, long long, long long);
 template void launch_gather_cols<float>(const float *, long long, float *, const GatherJob *, int,
-                                        const long long *, int, int, hipStream_t);
+                                        const long long *, int, int, hipStream_t, int, long long, long long);
 
 // ------------------------------------------------------------------------------------
 // chi0 (R, tau) -> dense chi0 (q, omega)

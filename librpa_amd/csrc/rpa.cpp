@@ -316,14 +316,26 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
         flops_chi0_exec += contract_flops;
         d_segs = upload(segs, stream);
         d_couts = upload(co, stream);
-        d_skip.alloc(std::max<size_t>(1, outs.size()));
-        ctasks[0].build(co, prec == Prec::F64, 1, splitk, stream);
-        if (mixed) ctasks[1].build(co, false, 1, splitk, stream);
+        // tau points per launch: one tau point of a small system leaves the device idle between its
+        // launches, so several run as copies of one batch, up to about 120 GFLOP (2 ms) and 8 GB
+        double wflops = 0;
+        for (const auto &c : chunks) wflops += c.wb.flops;
+        const double per_tau = 8.0 * (2.0 * nk * (2.0 * nbands * NAO + 2.0 * NAO * NAO)) +
+                               ts * ((double)nR * 2 * NAO * NAO + ghat_max + (double)w_off.back());
+        nbatch = 1;
+        if (!host_staged && chunks.size() == 1)
+            nbatch = (int)std::max(1.0, std::min({(double)ntau, std::ceil(1.2e11 / std::max(1.0, contract_flops + wflops)),
+                                                  std::min(8e9, 0.1 * (double)free_b) / per_tau}));
+        if (const char *e = std::getenv("LIBRPA_AMD_TAU_BATCH")) nbatch = std::max(1, std::min(nbatch, std::atoi(e)));
+        nbatch = ceil_div(ntau, ceil_div(ntau, nbatch));
+        ctasks[0].build(co, prec == Prec::F64, nbatch, splitk, stream);
+        if (mixed) ctasks[1].build(co, false, nbatch, splitk, stream);
+        d_skip.alloc(std::max<size_t>(1, outs.size()) * nbatch);
         HIP_CHECK(hipStreamSynchronize(stream));
     }
     flops_chi0_exec *= ntau;
-    d_Ghat.alloc(ghat_max * ts);
-    d_W.alloc((size_t)(w_off.back() + kChi0Pad) * ts);
+    d_Ghat.alloc(ghat_max * nbatch * ts);
+    d_W.alloc((size_t)(w_off.back() * nbatch + kChi0Pad) * ts);
     screen_plan(ds);
 
     // ---- G build data ----
@@ -357,9 +369,9 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
             HIP_CHECK(hipMemcpy(d_wre.as<double>() + wre.size() * s, wre.data(), wre.size() * 8, hipMemcpyHostToDevice));
             HIP_CHECK(hipMemcpy(d_wim.as<double>() + wim.size() * s, wim.data(), wim.size() * 8, hipMemcpyHostToDevice));
         }
-        d_Zs.alloc(sizeof(double) * (size_t)nk * 2 * nbands * NAO);
-        d_Mst.alloc(sizeof(double) * (size_t)nk * 2 * NAO * NAO);
-        d_Gpm.alloc(ts * (size_t)nR * NAO * 2 * NAO);
+        d_Zs.alloc(sizeof(double) * (size_t)nbatch * 2 * nk * 2 * nbands * NAO);
+        d_Mst.alloc(sizeof(double) * (size_t)nbatch * 2 * nk * 2 * NAO * NAO);
+        d_Gpm.alloc(ts * (size_t)nbatch * nR * NAO * 2 * NAO);
         std::vector<double> cs((size_t)nR * nk), sn((size_t)nR * nk);
         for (int r = 0; r < nR; ++r)
             for (int k = 0; k < nk; ++k) {
@@ -422,45 +434,45 @@ void RpaEngine::prepare_gf(const MeanField &mf, int nbands_g) {
         if (hi <= lo) { lo = 0; hi = 0; }
         band_lo[sg] = lo;
         band_hi[sg] = hi;
-        GemmBatch &b = gb[sg];
-        b = GemmBatch();
-        b.trans_a = true;
-        if (hi > lo)
-            for (int k = 0; k < nk; ++k)
-                b.add(make_prob(2 * NAO, NAO, 2 * (hi - lo), (long long)k * 2 * nbands * 2 * NAO + 2LL * lo * 2 * NAO,
-                                2 * NAO, (long long)k * 2 * nbands * NAO + 2LL * lo * NAO, NAO,
-                                (long long)k * 2 * NAO * NAO, NAO));
-        b.finalize(T64x64, stream);
     }
+    // both signs in one batch; a sign without bands has K = 0 and gets zeros
+    gb = GemmBatch();
+    gb.trans_a = true;
+    const long long zs_k = 2LL * nbands * NAO, mst_k = 2LL * NAO * NAO;
+    for (int sg = 0; sg < 2; ++sg)
+        for (int k = 0; k < nk; ++k)
+            gb.add(make_prob(2 * NAO, NAO, 2 * (band_hi[sg] - band_lo[sg]), k * 2 * zs_k + 4LL * band_lo[sg] * NAO, 2 * NAO,
+                             ((long long)sg * nk + k) * zs_k + 2LL * band_lo[sg] * NAO, NAO,
+                             ((long long)sg * nk + k) * mst_k, NAO));
+    gb.zb = 2 * nk * zs_k;
+    gb.zc = 2 * nk * mst_k;
+    gb.finalize(T64x64, stream);
     gf_nbands = nbands_g;
 }
 
-void RpaEngine::build_gf(const MeanField &mf, double tau, int s) {
+void RpaEngine::build_gf(const MeanField &mf, const double *taus, int nz, int s) {
     auto &prof = profiler();
     const size_t zz_s = (size_t)nk * 2 * nbands * 2 * NAO * s;
     const size_t w_s = (size_t)nk * nbands * NAO * s;
     const size_t e_s = (size_t)nk * nbands * s;
-    const long long gpm_bytes = (long long)nR * NAO * 2 * NAO * ts;
+    const long long gpm_bytes = (long long)nz * nR * NAO * 2 * NAO * ts;
+    if (nz > nbatch || nz > kTauMax) LRA_THROW("G build: more tau points than the buffers hold");
+    TauList tl;
+    tl.n = nz;
+    for (int z = 0; z < nz; ++z) tl.t[z] = taus[z];
     prof.begin("gf_build", stream);
-    for (int sg = 0; sg < 2; ++sg) {
-        const double t = sg == 0 ? tau : -tau;
-        if (band_hi[sg] > band_lo[sg]) {
-            launch_scale_bands(d_wre.as<double>() + w_s, d_wim.as<double>() + w_s, d_eps.as<double>() + e_s,
-                               d_wg.as<double>() + e_s, d_Zs.as<double>(), nk, nbands, NAO, band_lo[sg], band_hi[sg],
-                               t, mf.efermi, nspin, gf_nbands, stream);
-            gemm_run(Prec::F64, gb[sg], d_ZZ.as<double>() + zz_s, d_Zs.get(), d_Mst.get(), 1.0, 0.0, stream);
-        } else {
-            HIP_CHECK(hipMemsetAsync(d_Mst.get(), 0, d_Mst.bytes(), stream));
-        }
-        const double sgn = t < 0 ? -1.0 : 1.0;
-        if (cur == Prec::F64)
-            launch_k2r<double>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(),
-                               d_gcol.as<int>() + (size_t)sg * NAO, d_Gpm.as<double>(), nk, nR, NAO, sgn, stream);
-        else
-            launch_k2r<float>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(),
-                              d_gcol.as<int>() + (size_t)sg * NAO, d_Gpm.as<float>(), nk, nR, NAO, sgn, stream);
-    }
-    prof.end("gf_build", stream, gb[0].flops + gb[1].flops, (double)gpm_bytes);
+    launch_scale_bands(d_wre.as<double>() + w_s, d_wim.as<double>() + w_s, d_eps.as<double>() + e_s,
+                       d_wg.as<double>() + e_s, d_Zs.as<double>(), nk, nbands, NAO, band_lo, band_hi, tl, mf.efermi,
+                       nspin, gf_nbands, stream);
+    gb.nz = nz;
+    gemm_run(Prec::F64, gb, d_ZZ.as<double>() + zz_s, d_Zs.get(), d_Mst.get(), 1.0, 0.0, stream);
+    if (cur == Prec::F64)
+        launch_k2r<double>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(), d_gcol.as<int>(),
+                           d_Gpm.as<double>(), nk, nR, NAO, nz, stream);
+    else
+        launch_k2r<float>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(), d_gcol.as<int>(), d_Gpm.as<float>(),
+                          nk, nR, NAO, nz, stream);
+    prof.end("gf_build", stream, nz * gb.flops, (double)gpm_bytes);
 }
 
 void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
@@ -471,8 +483,8 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
     chiw_ok = false;  // chi0(R, omega) of an earlier build is stale
     if (host_staged) d_chiw.release();  // its room goes back to W and T (reformed for Ec)
     prepare_gf(mf, nbands_g);
-    d_Ghat.reserve(ghat_max * ts);
-    d_W.reserve((size_t)(w_off.back() + kChi0Pad) * ts);
+    d_Ghat.reserve(ghat_max * nbatch * ts);
+    d_W.reserve((size_t)(w_off.back() * nbatch + kChi0Pad) * ts);
     if (mixed) {
         if (prec != Prec::F64) LRA_THROW("mixed chi0 precision needs the FP64 plan");
         if (const char *e = std::getenv("LIBRPA_AMD_MIXED_AMAX")) mixed_amax = std::atof(e);
@@ -491,18 +503,21 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
     if (collect) features.assign((size_t)ntau * MLP_NFEAT * outs.size(), 0.0f);
     bool tuned_chi0[2] = {false, false};  // [plan precision, FP32 of the mixed mode]
     n_lowp_tau = 0;
-    for (int it = 0; it < ntau; ++it) {
-        const double tau = g.tau[it];
-        // mixed precision: FP32 contractions for the tau points whose column of the cosine t->f
-        // matrix is small (the transform amplifies chi0(R, tau) errors by that column's entries)
-        cur = prec;
-        if (mixed) {
-            double amax = 0;
-            for (int w = 0; w < g.n; ++w) amax = std::max(amax, std::fabs(g.cos_t2f[(size_t)w * g.n + it]));
-            if (amax <= mixed_amax) cur = mixed_low;
-        }
+    // mixed precision: FP32 contractions for the tau points whose column of the cosine t->f matrix is
+    // small (the transform amplifies chi0(R, tau) errors by that column's entries)
+    std::vector<Prec> tau_prec(ntau, prec);
+    for (int it = 0; mixed && it < ntau; ++it) {
+        double amax = 0;
+        for (int w = 0; w < g.n; ++w) amax = std::max(amax, std::fabs(g.cos_t2f[(size_t)w * g.n + it]));
+        if (amax <= mixed_amax) tau_prec[it] = mixed_low;
+    }
+    const long long zg = (long long)nR * NAO * 2 * NAO, zw = w_off.back();
+    for (int it = 0, nz = 1; it < ntau; it += nz) {
+        // tau points [it, it + nz) of one precision in one pass
+        cur = tau_prec[it];
+        for (nz = 1; nz < nbatch && it + nz < ntau && tau_prec[it + nz] == cur; ++nz) {}
         const bool lowp = cur != prec;
-        n_lowp_tau += lowp ? 1 : 0;
+        n_lowp_tau += lowp ? nz : 0;
         // low-precision tau points time under their own region names
         const char *lsuf = cur == Prec::BF16X3 ? "_bf16x3" : "_f32";
         auto rn = [lowp, lsuf](const char *r) { return lowp ? std::string(r) + lsuf : std::string(r); };
@@ -513,8 +528,8 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
         if (mixed)
             for (auto &c : chunks) c.wb.use_tiles(cur, stream);
         for (int s = 0; s < nspin; ++s) {
-            build_gf(mf, tau, s);
-            if (s == 0 && (screen_mode != 0 || collect)) screen_tau(it, tau);
+            build_gf(mf, &g.tau[it], nz, s);
+            if (s == 0 && (screen_mode != 0 || collect)) screen_taus(it, &g.tau[it], nz);
             // tiles are tuned per precision on the first tau point built at it
             const bool tune_now = autotune && s == 0 && !tuned_chi0[lowp];
             for (auto &c : chunks) {
@@ -526,15 +541,20 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
                 prof.begin(rn("chi0_gather"), stream);
                 if (cur == Prec::F64)
                     launch_gather_cols<double>(d_Gpm.as<double>(), 2LL * NAO, d_Ghat.as<double>(), c.d_jobs.as<GatherJob>(),
-                                               (int)c.jobs.size(), c.d_colsrc.as<long long>(), NAO, c.max_gcol, stream);
+                                               (int)c.jobs.size(), c.d_colsrc.as<long long>(), NAO, c.max_gcol, stream, nz, zg,
+                                               c.ghat_elems);
                 else
                     launch_gather_cols<float>(d_Gpm.as<float>(), 2LL * NAO, d_Ghat.as<float>(), c.d_jobs.as<GatherJob>(),
-                                              (int)c.jobs.size(), c.d_colsrc.as<long long>(), NAO, c.max_gcol, stream);
-                prof.end(rn("chi0_gather"), stream, 0, 2.0 * c.ghat_elems * (lowp ? 4 : ts));
+                                              (int)c.jobs.size(), c.d_colsrc.as<long long>(), NAO, c.max_gcol, stream, nz, zg,
+                                               c.ghat_elems);
+                prof.end(rn("chi0_gather"), stream, 0, 2.0 * nz * c.ghat_elems * (lowp ? 4 : ts));
+                c.wb.nz = nz;
+                c.wb.za = c.ghat_elems;
+                c.wb.zc = zw;
                 if (tune_now && c.wb.cfg_by_prec[(int)cur] < 0) c.wb.tune(cur, d_Ghat.get(), CWb_p, d_W.get(), 1.0, 0.0, stream);
                 prof.begin(rn("chi0_W"), stream);
                 gemm_run(cur, c.wb, d_Ghat.get(), CWb_p, d_W.get(), 1.0, 0.0, stream);
-                prof.end(rn("chi0_W"), stream, c.wb.flops);
+                prof.end(rn("chi0_W"), stream, nz * c.wb.flops);
             }
             // the contraction; a BF16x3 tau point contracts in FP32 (the kernel is bound by its
             // operand reads there, and FP32 keeps more digits)
@@ -545,22 +565,22 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
             prof.begin(region, stream);
             if (cur == Prec::F64)
                 launch_chi0_contract<double, double>(ctasks[0], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
-                                                     d_Gpm.as<double>(), 0, d_W.as<double>(), 0, d_Cfin.as<double>(),
-                                                     d_chi0s.as<double>() + coff, 0, NAO, 1, skip, stream);
+                                                     d_Gpm.as<double>(), zg, d_W.as<double>(), zw, d_Cfin.as<double>(),
+                                                     d_chi0s.as<double>() + coff, E_tot, NAO, nz, skip, stream);
             else if (lowp)
                 launch_chi0_contract<float, double>(ctasks[1], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
-                                                    d_Gpm.as<float>(), 0, d_W.as<float>(), 0, d_Cfin32.as<float>(),
-                                                    d_chi0s.as<double>() + coff, 0, NAO, 1, skip, stream);
+                                                    d_Gpm.as<float>(), zg, d_W.as<float>(), zw, d_Cfin32.as<float>(),
+                                                    d_chi0s.as<double>() + coff, E_tot, NAO, nz, skip, stream);
             else
                 launch_chi0_contract<float, float>(ctasks[0], d_couts.as<Chi0Out>(), nout, d_segs.as<Chi0Seg>(),
-                                                   d_Gpm.as<float>(), 0, d_W.as<float>(), 0, d_Cfin.as<float>(),
-                                                   d_chi0s.as<float>() + coff, 0, NAO, 1, skip, stream);
-            prof.end(region, stream, contract_flops, contract_bytes * bsc);
+                                                   d_Gpm.as<float>(), zg, d_W.as<float>(), zw, d_Cfin.as<float>(),
+                                                   d_chi0s.as<float>() + coff, E_tot, NAO, nz, skip, stream);
+            prof.end(region, stream, nz * contract_flops, nz * contract_bytes * bsc);
         }
         tuned_chi0[lowp] = tuned_chi0[lowp] || autotune;
         if (verbose) {
             HIP_CHECK(hipStreamSynchronize(stream));
-            fprintf(stderr, "[librpa-mi355x] chi0: tau %d / %d (%.1f s)\n", it + 1, ntau, now_s() - t0);
+            fprintf(stderr, "[librpa-mi355x] chi0: tau %d / %d (%.1f s)\n", it + nz, ntau, now_s() - t0);
             fflush(stderr);
         }
         // a host-staged build keeps its slice in pageable host memory (stream order makes the next

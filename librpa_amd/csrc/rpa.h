@@ -53,6 +53,7 @@ struct RpaEngine {
     std::vector<long long> w_off;  // W(K, J, S) block of (J, S) in d_W
     // the contraction (chi0.hip): task lists at the plan's precision and, in the mixed modes, FP32
     Chi0Tasks ctasks[2];
+    int nbatch = 1;  // tau points per pass: G, gathered G and W are held for that many
     DevBuf d_couts, d_segs, d_skip;
     std::vector<double> out_flops;  // per output and tau point
     double contract_flops = 0, contract_bytes = 0;
@@ -60,7 +61,7 @@ struct RpaEngine {
     // G build
     int band_lo[2] = {0, 0}, band_hi[2] = {0, 0};  // per sign (0: +tau, 1: -tau)
     int gf_nbands = -1;
-    GemmBatch gb[2];
+    GemmBatch gb;  // both signs, every k; a copy per tau point of a pass
 
     // ---- device data ----
     size_t ts = 8;  // storage element size (8 fp64, 4 fp32)
@@ -126,13 +127,13 @@ struct RpaEngine {
     std::vector<float> pred_h, feat_h;
     double scr_blocks = 0, scr_skipped = 0, scr_flops = 0, scr_flops_skipped = 0;
     void screen_plan(const Dataset &ds);
-    void screen_tau(int it, double tau);            // features and skip flags after build_gf
+    void screen_taus(int it, const double *taus, int nz);  // features and skip flags after build_gf
     void chi0_norms(std::vector<double> &out);      // ||chi0s(o, tau)||_F, [tau][output]
 
     void plan(const Dataset &ds, Prec p, Prec pe, int ntau);
-    // G(R, +-tau) of spin s into d_Gpm (prepare_gf once per band cut first)
+    // G(R, +-tau) of spin s and nz tau points into d_Gpm (prepare_gf once per band cut first)
     void prepare_gf(const MeanField &mf, int nbands_g);
-    void build_gf(const MeanField &mf, double tau, int s);
+    void build_gf(const MeanField &mf, const double *taus, int nz, int s);
     void build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g);
     void release_work();  // free the gathered-G and W work buffers (rebuilt by build_chi0)
     void release_ec();    // free the Ec work buffers (rebuilt by ec)

@@ -51,76 +51,81 @@ void RpaEngine::screen_plan(const Dataset &ds) {
     d_gblocks = upload(gblocks, stream);
     d_eoff = upload(eo, stream);
     d_esize = upload(es, stream);
-    d_gnorm.alloc(sizeof(double) * 2 * std::max(1, nout));
-    d_feat.alloc(sizeof(float) * MLP_NFEAT * std::max(1, nout));
-    d_pred.alloc(sizeof(float) * std::max(1, nout));
+    d_gnorm.alloc(sizeof(double) * 2 * std::max(1, nout) * nbatch);
+    d_feat.alloc(sizeof(float) * MLP_NFEAT * std::max(1, nout) * nbatch);
+    d_pred.alloc(sizeof(float) * std::max(1, nout) * nbatch);
 }
 
-void RpaEngine::screen_tau(int it, double tau) {
+void RpaEngine::screen_taus(int it, const double *taus, int nz) {
     const int nout = (int)outs.size();
     if (nout == 0) return;
     auto &prof = profiler();
     prof.begin("chi0_screen", stream);
-    if (cur == Prec::F64)
-        launch_block_norms<double>(d_Gpm.as<double>(), 2LL * NAO, d_gblocks.as<BlockRef>(), 2 * nout,
-                                   d_gnorm.as<double>(), stream);
-    else
-        launch_block_norms<float>(d_Gpm.as<float>(), 2LL * NAO, d_gblocks.as<BlockRef>(), 2 * nout,
-                                  d_gnorm.as<double>(), stream);
-    gnorm_h.resize(2 * (size_t)nout);
-    HIP_CHECK(hipMemcpyAsync(gnorm_h.data(), d_gnorm.get(), sizeof(double) * 2 * nout, hipMemcpyDeviceToHost, stream));
+    const long long zg = (long long)nR * NAO * 2 * NAO;
+    for (int z = 0; z < nz; ++z) {
+        double *gn = d_gnorm.as<double>() + (size_t)z * 2 * nout;
+        if (cur == Prec::F64)
+            launch_block_norms<double>(d_Gpm.as<double>() + z * zg, 2LL * NAO, d_gblocks.as<BlockRef>(), 2 * nout, gn, stream);
+        else
+            launch_block_norms<float>(d_Gpm.as<float>() + z * zg, 2LL * NAO, d_gblocks.as<BlockRef>(), 2 * nout, gn, stream);
+    }
+    gnorm_h.resize(2 * (size_t)nout * nz);
+    HIP_CHECK(hipMemcpyAsync(gnorm_h.data(), d_gnorm.get(), sizeof(double) * gnorm_h.size(), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
-    double gpx = 0, gmx = 0;
-    for (int o = 0; o < nout; ++o) {
-        gpx = std::max(gpx, gnorm_h[2 * (size_t)o]);
-        gmx = std::max(gmx, gnorm_h[2 * (size_t)o + 1]);
+    feat_h.resize((size_t)MLP_NFEAT * nout * nz);
+    skip_out.assign((size_t)nout * nz, 0);
+    for (int z = 0; z < nz; ++z) {
+        const double *gn = gnorm_h.data() + (size_t)z * 2 * nout;
+        float *fz = feat_h.data() + (size_t)z * MLP_NFEAT * nout;
+        double gpx = 0, gmx = 0;
+        for (int o = 0; o < nout; ++o) {
+            gpx = std::max(gpx, gn[2 * (size_t)o]);
+            gmx = std::max(gmx, gn[2 * (size_t)o + 1]);
+        }
+        const float ltau = (float)std::log(taus[z]), lgm = (float)std::log(gpx * gmx + 1e-300);
+        for (int o = 0; o < nout; ++o) {
+            const float *fs = &feat_static[5 * (size_t)o];
+            float *f = fz + (size_t)MLP_NFEAT * o;
+            f[0] = fs[0]; f[1] = fs[1]; f[2] = fs[2]; f[3] = ltau; f[4] = fs[3]; f[5] = fs[4];
+            f[6] = (float)std::log(gn[2 * (size_t)o] * gn[2 * (size_t)o + 1] + 1e-300);
+            f[7] = lgm;
+        }
+        if (collect) std::copy(fz, fz + (size_t)MLP_NFEAT * nout, features.begin() + (size_t)(it + z) * MLP_NFEAT * nout);
+        if (screen_mode == 0) continue;
+        for (int o = 0; o < nout; ++o) {
+            const auto &O = outs[o];
+            const double bound = cnorm[O.I] * cnorm[O.J] *
+                                 (gn[2 * (size_t)o] * gmx + gn[2 * (size_t)o + 1] * gpx + 2.0 * gpx * gmx);
+            if (bound < screen_thr) skip_out[(size_t)z * nout + o] = 1;
+        }
     }
-    feat_h.resize((size_t)MLP_NFEAT * nout);
-    const float ltau = (float)std::log(tau), lgm = (float)std::log(gpx * gmx + 1e-300);
-    for (int o = 0; o < nout; ++o) {
-        const float *fs = &feat_static[5 * (size_t)o];
-        float *f = &feat_h[(size_t)MLP_NFEAT * o];
-        f[0] = fs[0]; f[1] = fs[1]; f[2] = fs[2]; f[3] = ltau; f[4] = fs[3]; f[5] = fs[4];
-        f[6] = (float)std::log(gnorm_h[2 * (size_t)o] * gnorm_h[2 * (size_t)o + 1] + 1e-300);
-        f[7] = lgm;
-    }
-    if (collect) std::copy(feat_h.begin(), feat_h.end(), features.begin() + (size_t)it * MLP_NFEAT * nout);
     if (screen_mode == 0) {
         prof.end("chi0_screen", stream);
         return;
-    }
-    skip_out.assign(nout, 0);
-    for (int o = 0; o < nout; ++o) {
-        const auto &O = outs[o];
-        const double bound = cnorm[O.I] * cnorm[O.J] *
-                             (gnorm_h[2 * (size_t)o] * gmx + gnorm_h[2 * (size_t)o + 1] * gpx + 2.0 * gpx * gmx);
-        if (bound < screen_thr) skip_out[o] = 1;
     }
     if (screen_mode == 2) {
         // standardise with the model's scaling, predict ln ||chi0s|| on the device
         const float *mean = screen_model.data() + MLP_NPARAM, *scale = mean + MLP_NFEAT;
         const float tmean = screen_model[MLP_NPARAM + 2 * MLP_NFEAT], tscale = screen_model[MLP_NPARAM + 2 * MLP_NFEAT + 1];
         std::vector<float> xs(feat_h.size());
-        for (int o = 0; o < nout; ++o)
-            for (int k = 0; k < MLP_NFEAT; ++k)
-                xs[(size_t)MLP_NFEAT * o + k] = (feat_h[(size_t)MLP_NFEAT * o + k] - mean[k]) / scale[k];
+        for (size_t i = 0; i < xs.size(); ++i) xs[i] = (feat_h[i] - mean[i % MLP_NFEAT]) / scale[i % MLP_NFEAT];
         HIP_CHECK(hipMemcpyAsync(d_feat.get(), xs.data(), sizeof(float) * xs.size(), hipMemcpyHostToDevice, stream));
-        launch_mlp_forward(d_model.as<float>(), d_feat.as<float>(), nout, d_pred.as<float>(), stream);
-        pred_h.resize(nout);
-        HIP_CHECK(hipMemcpyAsync(pred_h.data(), d_pred.get(), sizeof(float) * nout, hipMemcpyDeviceToHost, stream));
+        launch_mlp_forward(d_model.as<float>(), d_feat.as<float>(), nout * nz, d_pred.as<float>(), stream);
+        pred_h.resize((size_t)nout * nz);
+        HIP_CHECK(hipMemcpyAsync(pred_h.data(), d_pred.get(), sizeof(float) * pred_h.size(), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
         const double lthr = std::log(screen_thr);
-        for (int o = 0; o < nout; ++o)
-            if ((double)pred_h[o] * tscale + tmean < lthr) skip_out[o] = 1;
+        for (size_t i = 0; i < pred_h.size(); ++i)
+            if ((double)pred_h[i] * tscale + tmean < lthr) skip_out[i] = 1;
     }
     double fl = 0, fls = 0, nsk = 0;
-    for (int o = 0; o < nout; ++o) {
-        fl += out_flops[o];
-        if (skip_out[o]) fls += out_flops[o];
-        nsk += skip_out[o];
+    for (size_t i = 0; i < skip_out.size(); ++i) {
+        fl += out_flops[i % nout];
+        if (skip_out[i]) fls += out_flops[i % nout];
+        nsk += skip_out[i];
     }
-    HIP_CHECK(hipMemcpyAsync(d_skip.get(), skip_out.data(), nout, hipMemcpyHostToDevice, stream));
-    scr_blocks += nout;
+    HIP_CHECK(hipMemcpyAsync(d_skip.get(), skip_out.data(), skip_out.size(), hipMemcpyHostToDevice, stream));
+    scr_blocks += (double)nout * nz;
     scr_skipped += nsk;
     scr_flops += fl;
     scr_flops_skipped += fls;
