@@ -12,7 +12,9 @@
 //   * column table on C: the within-block part c % ncb may be replaced by an
 //     entry of a table of element offsets (scattered output columns);
 //   * atomic epilogue: C += alpha A B with atomic adds, for outputs that several
-//     problems of one launch accumulate into.
+//     problems of one launch accumulate into;
+//   * second segment: A B may be followed by sgn2 A2 B2 of the same shape and strides in the same
+//     accumulators (the real or imaginary part of a complex product, from separate planes).
 // A batch may run nz times in one launch on operands za, zb, zc elements apart (the tau points of a
 // small system), so that few problems still fill the device.
 #pragma once
@@ -41,6 +43,8 @@ struct GemmProb {
     int rt_off;    // offset into the row table, -1 if not row-indirect
     int kmode;     // triangular operand: 0 none, 1 B lower (k < n is zero), 2 A = L^T (k < m is zero)
     int ct_off;    // offset into the column table, -1 if none
+    int sgn2;      // +1 / -1: sign of the second segment, 0 = none
+    long long a_off2, b_off2;
 };
 
 // Tile configurations (BM x BN; 256 threads, the w8 shapes 512).
@@ -73,6 +77,7 @@ struct GemmBatch {
     bool trans_b = false;  // B stored as B^T (element (k,n) at b_off + n*ldb + k)
     bool lower_only = false;
     bool atomic = false;   // C += alpha A B by atomic adds (beta must be 1)
+    bool two_segments = false;         // every problem has a second segment (set by finalize)
     int nz = 1;                        // copies of the batch in one launch
     long long za = 0, zb = 0, zc = 0;  // operand distances of a copy, in elements
     int total_tiles = 0;

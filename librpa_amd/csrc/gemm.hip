@@ -64,8 +64,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int G) {
     return x < rem ? x * (per + 1) + idx : rem * (per + 1) + (x - rem) * per + idx;
 }
 
-// VAR selects the addressing extras compiled in: 0 plain, 2 column table and atomic epilogue
-// (kept out of the plain kernels, where they cost registers).  blockIdx.y is the copy of the batch.
+// VAR selects the extras compiled in: 0 plain, 1 second segment, 2 column table and atomic epilogue
+// (kept out of the plain kernels, where they cost registers and 5% of the time).  blockIdx.y is the copy of the batch.
 template <int MODE, int BM, int BN, int WM, int WN, bool TA, bool TB, int VAR>
 __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__restrict__ probs, int nprob, int total,
                                                     const typename ModeTraits<MODE>::T *__restrict__ A,
@@ -146,6 +146,7 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
             for (int r = 0; r < 4; ++r) acc[a][b][r] = 0;
 
     T ra[LA], rb[LB];
+    T sg = 1;
     auto gload = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
                 const long long ko = TA ? (long long)gk * P.lda : (long long)gk;
                 v = A[arow[i] + ko];
             }
-            ra[i] = v;
+            ra[i] = VAR == 1 ? sg * v : v;
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
@@ -199,11 +200,20 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
     if (P.kmode == 1) kbeg = (n0 / BK) * BK;
     else if (P.kmode == 2) kbeg = (m0 / BK) * BK;
     gload(kbeg);
-    for (int k0 = kbeg; k0 < P.K; k0 += BK) {
+    bool second = VAR == 1;
+    for (int k0 = kbeg; k0 < P.K;) {
         __syncthreads();
         sstore();
         __syncthreads();
-        if (k0 + BK < P.K) gload(k0 + BK);
+        k0 += BK;
+        if (VAR == 1 && k0 >= P.K && second) {  // the second segment: the same shape from other planes
+            second = false;
+            k0 = kbeg;
+            sg = static_cast<T>(P.sgn2);
+            A += P.a_off2 - P.a_off;
+            B += P.b_off2 - P.b_off;
+        }
+        if (k0 < P.K) gload(k0);
         if constexpr (MODE == 0 || MODE == 1) {
 #pragma unroll
             for (int kk = 0; kk < BK; kk += 4) {
@@ -339,19 +349,22 @@ void GemmBatch::finalize(int cfg_, hipStream_t s) {
     const int bm = tile_bm(cfg), bn = tile_bn(cfg);
     int t0 = 0;
     flops = 0;
+    two_segments = !probs.empty() && probs[0].sgn2 != 0;
     for (auto &p : probs) {
+        if ((p.sgn2 != 0) != two_segments) LRA_THROW("GEMM batch: one or two segments, the same for all problems");
         p.tiles_n = ceil_div(p.N, bn);
         p.tile0 = t0;
         t0 += ceil_div(p.M, bm) * p.tiles_n;
         if (p.kmode == 0 && !lower_only) {
-            flops += 2.0 * p.M * p.N * (double)p.K;
+            flops += (p.sgn2 ? 4.0 : 2.0) * p.M * p.N * (double)p.K;
         } else {
             // executed work: tiles above the diagonal skipped, K started at the tile's diagonal
             for (int m0 = 0; m0 < p.M; m0 += bm)
                 for (int n0 = 0; n0 < p.N; n0 += bn) {
                     if (lower_only && n0 > m0 + bm - 1) continue;
                     const int kb = p.kmode == 1 ? n0 : (p.kmode == 2 ? m0 : 0);
-                    flops += 2.0 * std::min(bm, p.M - m0) * std::min(bn, p.N - n0) * (double)std::max(0, p.K - kb);
+                    flops += (p.sgn2 ? 4.0 : 2.0) * std::min(bm, p.M - m0) * std::min(bn, p.N - n0) *
+                             (double)std::max(0, p.K - kb);
                 }
         }
     }
@@ -410,6 +423,13 @@ static void launch_mode(const GemmBatch &b, const void *A, const void *B, void *
         else launch_one<MODE, 1, false, false, 2>(b, A, B, C, alpha, beta, s);
         return;
     }
+    if (b.two_segments) {
+        if (b.trans_a && b.trans_b) LRA_THROW("two-segment GEMM: at most one operand transposed");
+        if (b.trans_a) launch_cfg<MODE, true, false, 1>(b, A, B, C, alpha, beta, s);
+        else if (b.trans_b) launch_cfg<MODE, false, true, 1>(b, A, B, C, alpha, beta, s);
+        else launch_cfg<MODE, false, false, 1>(b, A, B, C, alpha, beta, s);
+        return;
+    }
     if (b.trans_a && b.trans_b) launch_cfg<MODE, true, true>(b, A, B, C, alpha, beta, s);
     else if (b.trans_a) launch_cfg<MODE, true, false>(b, A, B, C, alpha, beta, s);
     else if (b.trans_b) launch_cfg<MODE, false, true>(b, A, B, C, alpha, beta, s);
@@ -436,7 +456,7 @@ std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
         k.push_back(p.lda);
         k.push_back(p.ldb);
         k.push_back(p.ldc);
-        k.push_back(p.kmode + 4 * (p.rt_off >= 0) + 8 * (p.ct_off >= 0));
+        k.push_back(p.kmode + 4 * (p.rt_off >= 0) + 8 * (p.ct_off >= 0) + 16 * (p.sgn2 != 0));
         k.push_back(p.ncb < p.N ? p.ncb : 0);
     }
     return k;

@@ -539,7 +539,7 @@ void stage_coulomb(const RpaEngine &R0, const std::map<std::tuple<int, int, int>
                 out.vmax[k] = std::max(out.vmax[k], std::abs(v));
                 out.imax[k] = std::max(out.imax[k], std::fabs(v.imag()));
             }
-            desc.push_back({(long long)vals.size(), (int)R0.abf[I], (int)R0.abf[J], R0.na[I], R0.na[J], I == J ? 1 : 0});
+            desc.push_back({(long long)vals.size(), (int)R0.abf[I], (int)R0.abf[J], R0.na[I], R0.na[J], I == J ? 1 : 0, 0});
             vals.insert(vals.end(), kv.second.begin(), kv.second.end());
         }
         out.first.push_back((int)desc.size());
@@ -554,7 +554,7 @@ void dense_coulomb(const CoulombStage &cs, int kq, int n, int n2, bool embed, bo
                    hipStream_t st) {
     HIP_CHECK(hipMemsetAsync(V, 0, sizeof(double) * (size_t)n2 * n2, st));
     launch_v_scatter(cs.blk.as<double>(), cs.desc.as<VBlock>() + cs.first[kq], cs.first[kq + 1] - cs.first[kq], V, n,
-                     n2, embed ? 1 : 0, real_part ? 1 : 0, st);
+                     embed ? kEmbedded : kReal, real_part ? 1 : 0, 0, 0, st);
 }
 }  // namespace
 
@@ -743,7 +743,7 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
         for (int w0 = 0; w0 < nw; w0 += WCH) {
             const int cnt = std::min(WCH, nw - w0);
             prof.begin("gw_w_chi0q", st);
-            R0.assemble_dense(g, kf, w0, cnt, dD.get(), true, (long long)nn, embed, st);
+            R0.assemble_dense(g, kf, w0, cnt, dD.get(), true, (long long)nn, embed ? kEmbedded : kReal, st);
             prof.end("gw_w_chi0q", st);
             auto &bb = get_batches(cnt, chol);
             prof.begin("gw_w_gemm", st);

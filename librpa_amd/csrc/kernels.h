@@ -38,7 +38,9 @@ void launch_gather_cols(const T *src, long long src_ld, T *dst, const GatherJob 
 // tau -> omega and R -> q of chi0s into dense Hermitian matrices ---------------------
 // For each pair p = (I <= J) with element count na_I * na_J and each omega w of the
 // chunk: val = (2 / nspin) sum_t sum_r gamma[w][t] e^{i 2 pi q.R_r} chi0s[t][eoff[p][r] + e].
-// Output: real (Gamma) n x n, or the real embedding [[Re, -Im], [Im, Re]] (2n x 2n).
+// Output by layout: real (Gamma) n x n, the real embedding [[Re, -Im], [Im, Re]] (2n x 2n), or the
+// planes Re and Im (n x n each).
+enum DenseLayout : int { kReal = 0, kEmbedded = 1, kPlanar = 2 };
 struct PairDesc {
     int I, J;
     int naI, naJ;
@@ -49,7 +51,7 @@ constexpr int kChi0AssembleMaxW = 8;  // frequencies per launch (nw <= this)
 template <class TS, class TD>
 void launch_chi0_assemble(const TS *chi0s, long long E_tot, int ntau, const PairDesc *pairs, int npairs,
                           long long n_pair_elems, const long long *eoff, int nR, const double *gam_ph,
-                          int nw, TD *dense, long long dense_stride, int n, bool embed, hipStream_t s);
+                          int nw, TD *dense, long long dense_stride, int n, DenseLayout lay, hipStream_t s);
 
 // The same in two passes, when a chi0(R, omega) store fits: chiw[w][i] = sum_t coef[w][t]
 // chi0s[t][i] once for all q (coef = (2 / nspin) gamma_c, nw x ntau, row-major), then per q and
@@ -63,44 +65,43 @@ void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const do
 template <class TS>
 void launch_tau_accumulate(const TS *slice, long long E_tot, int t, int ntau, const double *coef, int nw, double *chiw,
                            hipStream_t s);
-template <class TD>
-void launch_chi0_rq(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs, long long n_pair_elems,
-                    const long long *eoff, int nR, const double *ph, int nw, TD *dense, long long dense_stride, int n,
-                    bool embed, hipStream_t s);
-// chi0_rq for nq <= kChi0RqMaxQ q points at once (phases ph[q][r] as (cos, sin)); q point qi writes
+// for nq <= kChi0RqMaxQ q points at once (phases ph[q][r] as (cos, sin)); q point qi writes
 // its nw matrices at dense + qi * q_stride
 constexpr int kChi0RqMaxQ = 8;
 template <class TD>
 void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs,
                           long long n_pair_elems, const long long *eoff, int nR, const double *ph, int nq, int nw,
-                          TD *dense, long long dense_stride, long long q_stride, int n, bool embed, hipStream_t s);
+                          TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s);
 
 // Dense helpers --------------------------------------------------------------------
-// A = I, or diag(d) when d (n device doubles) is given
-template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s, const double *d = nullptr);
-template <class T> void launch_zero_upper(T *A, int n, int lda, hipStream_t s);
+template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s);
 template <class TS, class TD> void launch_convert(const TS *src, TD *dst, long long n, hipStream_t s);
-void launch_copy_lower_f2d(const float *src, double *dst, int n, int lda, hipStream_t s);
+// lower triangles of nmat n x n matrices, stride elements apart (pitch n)
+void launch_copy_lower_f2d(const float *src, double *dst, int n, long long nmat, long long stride, hipStream_t s);
 
 // One upper atom-pair block V_IJ(q) (I <= J) of the Coulomb matrix, complex, na_I x na_J
-// row-major at element offset off of the block store; r0 / c0 are the ABF offsets of I and J.
+// row-major at element offset off of the block store; r0 / c0 are the ABF offsets of I and J, q
+// counts the matrices.
 struct VBlock {
     long long off;
-    int r0, c0, na, nb, diag;
+    int r0, c0, na, nb, diag, q;
 };
-// Dense real V(q) (n2 = n, Gamma) or its real embedding [[Re, -Im], [Im, Re]] (n2 = 2n) from the
-// upper blocks, Hermitian fill; V must be zeroed first.  Every dense entry is written by at most
-// one (block, element), so the blocks run in parallel.  drop_imag embeds Re V only.
-void launch_v_scatter(const double *blk, const VBlock *d, int nblk, double *V, int n, int n2, int embed,
-                      int drop_imag, hipStream_t s);
-// *acc += sum_i A_ii, or sum_i signs_i A_ii when signs (n device doubles) is given
-void launch_trace_acc(const double *A, int n, int lda, double *acc, hipStream_t s, const double *signs = nullptr);
+// Dense V(q) from the upper blocks, Hermitian fill, in one of the layouts: block b goes to the matrix
+// at V + (b.q - q0) * stride.  V must be zeroed first.  Every dense entry is written by at most one
+// (block, element), so the blocks run in parallel.  drop_imag takes Re V only.
+void launch_v_scatter(const double *blk, const VBlock *d, int nblk, double *V, int n, DenseLayout lay, int drop_imag,
+                      int q0, long long stride, hipStream_t s);
+// For matrix u of nmat (stride elements apart, pitch n): A_ii += S_i, acc[2u] += sum_i S_i A_ii with
+// S = signs + (u / per) * n
+void launch_add_signs_trace(double *A, int n, long long nmat, long long stride, const double *signs, int per, double *acc,
+                            hipStream_t s);
 void launch_copy_block(const double *src, int lds, double *dst, int ldd, int rows, int cols, hipStream_t s);
 
-// Blocked Cholesky with signed pivots (lower, row-major, FP64): A = L S L^T in place,
-// S = diag(+-1); equal to Cholesky for positive-definite A.  logdet (device scalar)
-// += ln |det A|; *flag set to 1 on a zero / NaN pivot.  When keep_L is false only the
-// log-determinant is produced.  signs (n device doubles, optional) receives S.
+// Blocked Cholesky with signed pivots (lower, row-major, FP64): A = L S L^H in place, S = diag(+-1);
+// equal to Cholesky for positive-definite A.  A is real, or Hermitian with its imaginary plane im
+// elements after the real one (im = 0: real).  logdet (device scalar) += ln |det A|; *flag set to 1
+// on a zero / NaN pivot.  When keep_L is false only the log-determinant is produced.  signs (n
+// device doubles, optional) receives S.
 struct CholWork {
     DevBuf linv, panel;
 };
@@ -113,6 +114,6 @@ void cholesky_logdet(double *A, int n, int lda, double *logdet, int *flag, bool 
 // Matrix b writes its pivot signs to signs[b * sstride + j] when signs is given.
 void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, int lda, double *logdet,
                              long long ld_stride, int *flag, bool keep_L, CholWork &w, hipStream_t s,
-                             int ncols = -1, double *signs = nullptr, long long sstride = 0);
+                             int ncols = -1, double *signs = nullptr, long long sstride = 0, long long im = 0);
 
 }  // namespace lra

@@ -134,13 +134,39 @@ template void launch_gather_cols<float>(const float *, long long, float *, const
 // ------------------------------------------------------------------------------------
 // chi0 (R, tau) -> dense chi0 (q, omega)
 // ------------------------------------------------------------------------------------
+// chi0(q, omega) element (row, col) and its Hermitian mirror in one of the dense layouts
+template <class TD>
+__device__ __forceinline__ void put_dense(TD *__restrict__ D, long long n, long long row, long long col, double re,
+                                          double im, bool mirror, int lay) {
+    if (lay != kEmbedded) {
+        D[row * n + col] = static_cast<TD>(re);
+        if (mirror) D[col * n + row] = static_cast<TD>(re);
+        if (lay == kPlanar) {
+            D[(n + row) * n + col] = static_cast<TD>(im);
+            if (mirror) D[(n + col) * n + row] = static_cast<TD>(-im);
+        }
+        return;
+    }
+    const long long ld = 2 * n;
+    D[row * ld + col] = static_cast<TD>(re);
+    D[(n + row) * ld + n + col] = static_cast<TD>(re);
+    D[(n + row) * ld + col] = static_cast<TD>(im);
+    D[row * ld + n + col] = static_cast<TD>(-im);
+    if (mirror) {
+        D[col * ld + row] = static_cast<TD>(re);
+        D[(n + col) * ld + n + row] = static_cast<TD>(re);
+        D[(n + col) * ld + row] = static_cast<TD>(-im);
+        D[col * ld + n + row] = static_cast<TD>(im);
+    }
+}
+
 // NW accumulators per thread (a multiple of 8 covering the chunk): one pass over chi0(R, tau) per
 // chunk of up to kChi0AssembleMaxW frequencies
 template <class TS, class TD, int NW>
 __global__ void chi0_assemble_kernel(const TS *__restrict__ chi0s, long long E_tot, int ntau,
                                      const PairDesc *__restrict__ pairs, int npairs, long long nelem,
                                      const long long *__restrict__ eoff, int nR, const double *__restrict__ gp,
-                                     int nw, TD *__restrict__ dense, long long dstride, int n, int embed) {
+                                     int nw, TD *__restrict__ dense, long long dstride, int n, int lay) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nelem) return;
     int lo = 0, hi = npairs - 1;
@@ -174,49 +200,32 @@ __global__ void chi0_assemble_kernel(const TS *__restrict__ chi0s, long long E_t
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         if (w >= nw) break;
-        TD *D = dense + w * dstride;
-        if (!embed) {
-            const long long ld = n;
-            D[row * ld + col] = static_cast<TD>(re[w]);
-            if (mirror) D[col * ld + row] = static_cast<TD>(re[w]);
-        } else {
-            const long long ld = 2ll * n;
-            D[row * ld + col] = static_cast<TD>(re[w]);
-            D[(n + row) * ld + n + col] = static_cast<TD>(re[w]);
-            D[(n + row) * ld + col] = static_cast<TD>(im[w]);
-            D[row * ld + n + col] = static_cast<TD>(-im[w]);
-            if (mirror) {
-                D[col * ld + row] = static_cast<TD>(re[w]);
-                D[(n + col) * ld + n + row] = static_cast<TD>(re[w]);
-                D[(n + col) * ld + row] = static_cast<TD>(-im[w]);
-                D[col * ld + n + row] = static_cast<TD>(im[w]);
-            }
-        }
+        put_dense(dense + w * dstride, n, row, col, re[w], im[w], mirror, lay);
     }
 }
 
 template <class TS, class TD>
 void launch_chi0_assemble(const TS *chi0s, long long E_tot, int ntau, const PairDesc *pairs, int npairs,
                           long long n_pair_elems, const long long *eoff, int nR, const double *gam_ph, int nw,
-                          TD *dense, long long dense_stride, int n, bool embed, hipStream_t s) {
+                          TD *dense, long long dense_stride, int n, DenseLayout lay, hipStream_t s) {
     if (nw < 1 || nw > kChi0AssembleMaxW) LRA_THROW("omega chunk too large");
     hipLaunchKernelGGL((chi0_assemble_kernel<TS, TD, kChi0AssembleMaxW>), dim3(ceil_div(n_pair_elems, 256)), dim3(256),
                        0, s, chi0s, E_tot, ntau, pairs, npairs, n_pair_elems, eoff, nR, gam_ph, nw, dense, dense_stride,
-                       n, (int)embed);
+                       n, (int)lay);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_chi0_assemble<double, double>(const double *, long long, int, const PairDesc *, int, long long,
                                                    const long long *, int, const double *, int, double *, long long,
-                                                   int, bool, hipStream_t);
+                                                   int, DenseLayout, hipStream_t);
 template void launch_chi0_assemble<float, float>(const float *, long long, int, const PairDesc *, int, long long,
                                                  const long long *, int, const double *, int, float *, long long,
-                                                 int, bool, hipStream_t);
+                                                 int, DenseLayout, hipStream_t);
 template void launch_chi0_assemble<float, double>(const float *, long long, int, const PairDesc *, int, long long,
                                                   const long long *, int, const double *, int, double *, long long,
-                                                  int, bool, hipStream_t);
+                                                  int, DenseLayout, hipStream_t);
 template void launch_chi0_assemble<double, float>(const double *, long long, int, const PairDesc *, int, long long,
                                                   const long long *, int, const double *, int, float *, long long,
-                                                  int, bool, hipStream_t);
+                                                  int, DenseLayout, hipStream_t);
 
 // chiw[w][i] = sum_t coef[w][t] chi0s[t][i] for every element i of the chi0(R, tau) store: the
 // cosine tau -> omega transform, done once for all q.  Coefficients in LDS; each thread owns one
@@ -291,15 +300,19 @@ template void launch_tau_accumulate<double>(const double *, long long, int, int,
 template void launch_tau_accumulate<float>(const float *, long long, int, int, const double *, int, double *,
                                            hipStream_t);
 
-// dense chi0(q, omega) of nw frequencies from chi0(R, omega): per pair element and frequency,
-// sum_r (cos_r + i sin_r) chiw[w][eoff[p][r] + e], written like chi0_assemble (Hermitian fill,
-// real or embedded).  Reads chiw once per (element, R, frequency).
-template <class TD>
+// dense chi0(q, omega) of nw frequencies from chi0(R, omega) for up to NQ q points at once: per pair
+// element, sum_r (cos_r + i sin_r) chiw[w][eoff[p][r] + e] with the phases ph[q][r] as (cos, sin); each
+// chiw value read feeds every q of the launch.  A thread does wper frequencies, one when the elements
+// alone are under 1024 workgroups: with all 16 in the loop the 2-atom cell (120 functions, 43
+// workgroups) took 168 us where its bytes take 15; with one each the 64-atom cell takes 6.2 ms, not 4.7.
+// q point qi writes its nw matrices at dense + qi * qstride.
+template <class TD, int NQ>
 __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__ chiw, long long E_tot,
                                                       const PairDesc *__restrict__ pairs, int npairs, long long nelem,
                                                       const long long *__restrict__ eoff, int nR,
-                                                      const double *__restrict__ ph, int nw, TD *__restrict__ dense,
-                                                      long long dstride, int n, int embed) {
+                                                      const double *__restrict__ ph, int nq, int nw, int wper,
+                                                      TD *__restrict__ dense, long long dstride, long long qstride,
+                                                      int n, int lay) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nelem) return;
     int lo = 0, hi = npairs - 1;
@@ -310,70 +323,17 @@ __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__
     const PairDesc P = pairs[lo];
     const long long e = idx - P.e0;
     const int mu = (int)(e / P.naJ), nu = (int)(e % P.naJ);
-    const long long row = P.rowI + mu, col = P.colJ + nu;
-    const bool mirror = P.I != P.J;
-    for (int w = 0; w < nw; ++w) {
-        double re = 0, im = 0;
-        const double *cw = chiw + (long long)w * E_tot + e;
-        for (int r = 0; r < nR; ++r) {
-            const long long off = eoff[(long long)lo * nR + r];
-            if (off < 0) continue;
-            const double v = cw[off];
-            re += ph[2 * r] * v;
-            im += ph[2 * r + 1] * v;
-        }
-        TD *D = dense + w * dstride;
-        if (!embed) {
-            D[row * n + col] = static_cast<TD>(re);
-            if (mirror) D[col * n + row] = static_cast<TD>(re);
-        } else {
-            const long long ld = 2ll * n;
-            D[row * ld + col] = static_cast<TD>(re);
-            D[(n + row) * ld + n + col] = static_cast<TD>(re);
-            D[(n + row) * ld + col] = static_cast<TD>(im);
-            D[row * ld + n + col] = static_cast<TD>(-im);
-            if (mirror) {
-                D[col * ld + row] = static_cast<TD>(re);
-                D[(n + col) * ld + n + row] = static_cast<TD>(re);
-                D[(n + col) * ld + row] = static_cast<TD>(-im);
-                D[col * ld + n + row] = static_cast<TD>(im);
-            }
-        }
-    }
-}
-
-// The same for up to kChi0RqMaxQ q points at once: each chiw value read feeds every q of the launch
-// (phases ph[q][r] as (cos, sin)); q point qi writes its nw matrices at dense + qi * qstride.
-template <class TD>
-__global__ __launch_bounds__(256) void chi0_rq_multi_kernel(const double *__restrict__ chiw, long long E_tot,
-                                                            const PairDesc *__restrict__ pairs, int npairs,
-                                                            long long nelem, const long long *__restrict__ eoff,
-                                                            int nR, const double *__restrict__ ph, int nq, int nw,
-                                                            TD *__restrict__ dense, long long dstride,
-                                                            long long qstride, int n, int embed) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nelem) return;
-    int lo = 0, hi = npairs - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (pairs[mid].e0 <= idx) lo = mid; else hi = mid - 1;
-    }
-    const PairDesc P = pairs[lo];
-    const long long e = idx - P.e0;
-    const int mu = (int)(e / P.naJ), nu = (int)(e % P.naJ);
-    const long long row = P.rowI + mu, col = P.colJ + nu;
-    const bool mirror = P.I != P.J;
-    for (int w = 0; w < nw; ++w) {
-        double re[kChi0RqMaxQ], im[kChi0RqMaxQ];
+    for (int w = blockIdx.y * wper; w < min(nw, (int)(blockIdx.y + 1) * wper); ++w) {
+        double re[NQ], im[NQ];
 #pragma unroll
-        for (int q = 0; q < kChi0RqMaxQ; ++q) re[q] = im[q] = 0.0;
+        for (int q = 0; q < NQ; ++q) re[q] = im[q] = 0.0;
         const double *cw = chiw + (long long)w * E_tot + e;
         for (int r = 0; r < nR; ++r) {
             const long long off = eoff[(long long)lo * nR + r];
             if (off < 0) continue;
             const double v = cw[off];
 #pragma unroll
-            for (int q = 0; q < kChi0RqMaxQ; ++q) {
+            for (int q = 0; q < NQ; ++q) {
                 if (q < nq) {
                     re[q] += ph[2 * ((long long)q * nR + r)] * v;
                     im[q] += ph[2 * ((long long)q * nR + r) + 1] * v;
@@ -381,25 +341,9 @@ __global__ __launch_bounds__(256) void chi0_rq_multi_kernel(const double *__rest
             }
         }
 #pragma unroll
-        for (int q = 0; q < kChi0RqMaxQ; ++q) {
+        for (int q = 0; q < NQ; ++q) {
             if (q >= nq) break;
-            TD *D = dense + q * qstride + w * dstride;
-            if (!embed) {
-                D[row * n + col] = static_cast<TD>(re[q]);
-                if (mirror) D[col * n + row] = static_cast<TD>(re[q]);
-            } else {
-                const long long ld = 2ll * n;
-                D[row * ld + col] = static_cast<TD>(re[q]);
-                D[(n + row) * ld + n + col] = static_cast<TD>(re[q]);
-                D[(n + row) * ld + col] = static_cast<TD>(im[q]);
-                D[row * ld + n + col] = static_cast<TD>(-im[q]);
-                if (mirror) {
-                    D[col * ld + row] = static_cast<TD>(re[q]);
-                    D[(n + col) * ld + n + row] = static_cast<TD>(re[q]);
-                    D[(n + col) * ld + row] = static_cast<TD>(-im[q]);
-                    D[col * ld + n + row] = static_cast<TD>(im[q]);
-                }
-            }
+            put_dense(dense + q * qstride + w * dstride, n, P.rowI + mu, P.colJ + nu, re[q], im[q], P.I != P.J, lay);
         }
     }
 }
@@ -407,63 +351,47 @@ __global__ __launch_bounds__(256) void chi0_rq_multi_kernel(const double *__rest
 template <class TD>
 void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs,
                           long long n_pair_elems, const long long *eoff, int nR, const double *ph, int nq, int nw,
-                          TD *dense, long long dense_stride, long long q_stride, int n, bool embed, hipStream_t s) {
+                          TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s) {
     if (nq < 1 || nq > kChi0RqMaxQ) LRA_THROW("chi0_rq_multi: 1 to kChi0RqMaxQ q points per launch");
-    hipLaunchKernelGGL((chi0_rq_multi_kernel<TD>), dim3(ceil_div(n_pair_elems, 256)), dim3(256), 0, s, chiw, E_tot,
-                       pairs, npairs, n_pair_elems, eoff, nR, ph, nq, nw, dense, dense_stride, q_stride, n, (int)embed);
+    const int bx = ceil_div(n_pair_elems, 256), wper = bx >= 1024 ? nw : 1;
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chiw, E_tot, pairs, npairs,
+                           n_pair_elems, eoff, nR, ph, nq, nw, wper, dense, dense_stride, q_stride, n, (int)lay);
+    };
+    if (nq == 1) go(chi0_rq_kernel<TD, 1>);
+    else go(chi0_rq_kernel<TD, kChi0RqMaxQ>);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_chi0_rq_multi<double>(const double *, long long, const PairDesc *, int, long long,
                                            const long long *, int, const double *, int, int, double *, long long,
-                                           long long, int, bool, hipStream_t);
+                                           long long, int, DenseLayout, hipStream_t);
 template void launch_chi0_rq_multi<float>(const double *, long long, const PairDesc *, int, long long,
                                           const long long *, int, const double *, int, int, float *, long long,
-                                          long long, int, bool, hipStream_t);
-
-template <class TD>
-void launch_chi0_rq(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs, long long n_pair_elems,
-                    const long long *eoff, int nR, const double *ph, int nw, TD *dense, long long dense_stride, int n,
-                    bool embed, hipStream_t s) {
-    hipLaunchKernelGGL((chi0_rq_kernel<TD>), dim3(ceil_div(n_pair_elems, 256)), dim3(256), 0, s, chiw, E_tot, pairs,
-                       npairs, n_pair_elems, eoff, nR, ph, nw, dense, dense_stride, n, (int)embed);
-    HIP_CHECK(hipGetLastError());
-}
-template void launch_chi0_rq<double>(const double *, long long, const PairDesc *, int, long long, const long long *,
-                                     int, const double *, int, double *, long long, int, bool, hipStream_t);
-template void launch_chi0_rq<float>(const double *, long long, const PairDesc *, int, long long, const long long *, int,
-                                    const double *, int, float *, long long, int, bool, hipStream_t);
+                                          long long, int, DenseLayout, hipStream_t);
 
 // ------------------------------------------------------------------------------------
 // dense helpers
 // ------------------------------------------------------------------------------------
 template <class T>
-__global__ void set_identity_kernel(T *A, int n, int lda, const double *__restrict__ diag) {
+__global__ void set_identity_kernel(T *A, int n, int lda) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)n * n) return;
     const int i = (int)(idx / n), j = (int)(idx % n);
-    A[(long long)i * lda + j] = (i == j) ? (diag ? static_cast<T>(diag[i]) : T(1)) : T(0);
+    A[(long long)i * lda + j] = i == j ? T(1) : T(0);
 }
-template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s, const double *diag) {
-    hipLaunchKernelGGL((set_identity_kernel<T>), dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, A, n, lda,
-                       diag);
+template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s) {
+    hipLaunchKernelGGL((set_identity_kernel<T>), dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, A, n, lda);
     HIP_CHECK(hipGetLastError());
 }
-template void launch_set_identity<double>(double *, int, int, hipStream_t, const double *);
-template void launch_set_identity<float>(float *, int, int, hipStream_t, const double *);
+template void launch_set_identity<double>(double *, int, int, hipStream_t);
 
-template <class T>
-__global__ void zero_upper_kernel(T *A, int n, int lda) {
+// zero above the diagonal; the diagonal too on odd planes (blockIdx.y counts matrices, .z planes im apart)
+__global__ void zero_upper_kernel(double *A, int n, int lda, long long stride, long long im) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)n * n) return;
     const int i = (int)(idx / n), j = (int)(idx % n);
-    if (j > i) A[(long long)i * lda + j] = T(0);
+    if (j > i || (j == i && blockIdx.z)) A[blockIdx.y * stride + blockIdx.z * im + (long long)i * lda + j] = 0.0;
 }
-template <class T> void launch_zero_upper(T *A, int n, int lda, hipStream_t s) {
-    hipLaunchKernelGGL((zero_upper_kernel<T>), dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, A, n, lda);
-    HIP_CHECK(hipGetLastError());
-}
-template void launch_zero_upper<double>(double *, int, int, hipStream_t);
-template void launch_zero_upper<float>(float *, int, int, hipStream_t);
 
 template <class TS, class TD>
 __global__ void convert_kernel(const TS *__restrict__ src, TD *__restrict__ dst, long long n) {
@@ -479,65 +407,69 @@ template void launch_convert<double, float>(const double *, float *, long long, 
 template void launch_convert<float, double>(const float *, double *, long long, hipStream_t);
 template void launch_convert<double, double>(const double *, double *, long long, hipStream_t);
 
-__global__ void copy_lower_f2d_kernel(const float *__restrict__ src, double *__restrict__ dst, int n, int lda) {
+__global__ void copy_lower_f2d_kernel(const float *__restrict__ src, double *__restrict__ dst, int n, long long stride) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)n * n) return;
     const int i = (int)(idx / n), j = (int)(idx % n);
-    if (j <= i) dst[(long long)i * lda + j] = static_cast<double>(src[(long long)i * lda + j]);
+    const long long o = blockIdx.y * stride + idx;
+    if (j <= i) dst[o] = static_cast<double>(src[o]);
 }
-void launch_copy_lower_f2d(const float *src, double *dst, int n, int lda, hipStream_t s) {
-    hipLaunchKernelGGL(copy_lower_f2d_kernel, dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, src, dst, n,
-                       lda);
-    HIP_CHECK(hipGetLastError());
+void launch_copy_lower_f2d(const float *src, double *dst, int n, long long nmat, long long stride, hipStream_t s) {
+    for (long long m0 = 0; m0 < nmat; m0 += 32768) {
+        hipLaunchKernelGGL(copy_lower_f2d_kernel, dim3(ceil_div((long long)n * n, 256), (unsigned)std::min(32768LL, nmat - m0)),
+                           dim3(256), 0, s, src + m0 * stride, dst + m0 * stride, n, stride);
+        HIP_CHECK(hipGetLastError());
+    }
 }
 
-__global__ void v_scatter_kernel(const double2 *__restrict__ blk, const VBlock *__restrict__ desc, double *V,
-                                 long long n, long long n2, int embed, int drop_imag) {
+__global__ __launch_bounds__(256) void v_scatter_kernel(const double2 *__restrict__ blk, const VBlock *__restrict__ desc,
+                                                        double *V, long long n, int lay, int drop_imag, int q0,
+                                                        long long stride) {
     const VBlock b = desc[blockIdx.x];
+    V += (b.q - q0) * stride;
     const int tot = b.na * b.nb;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < tot; e += gridDim.y * blockDim.x) {
         const int mu = e / b.nb, nu = e % b.nb;
         double2 v = blk[b.off + e];
         if (drop_imag) v.y = 0.0;
-        const long long r = b.r0 + mu, c = b.c0 + nu;
-        V[r * n2 + c] = v.x;
-        if (!b.diag) V[c * n2 + r] = v.x;
-        if (embed) {
-            V[(n + r) * n2 + n + c] = v.x;
-            V[(n + r) * n2 + c] = v.y;
-            V[r * n2 + n + c] = -v.y;
-            if (!b.diag) {
-                V[(n + c) * n2 + n + r] = v.x;
-                V[(n + c) * n2 + r] = -v.y;
-                V[c * n2 + n + r] = v.y;
-            }
-        }
+        put_dense(V, n, b.r0 + mu, b.c0 + nu, v.x, v.y, !b.diag, lay);
     }
 }
 
-void launch_v_scatter(const double *blk, const VBlock *d, int nblk, double *V, int n, int n2, int embed,
-                      int drop_imag, hipStream_t s) {
+void launch_v_scatter(const double *blk, const VBlock *d, int nblk, double *V, int n, DenseLayout lay, int drop_imag,
+                      int q0, long long stride, hipStream_t s) {
     if (nblk == 0) return;
-    hipLaunchKernelGGL(v_scatter_kernel, dim3(nblk), dim3(256), 0, s, reinterpret_cast<const double2 *>(blk), d, V,
-                       (long long)n, (long long)n2, embed, drop_imag);
+    // a molecule has a handful of blocks of up to 10^4 elements: several workgroups each
+    const int split = nblk >= 2048 ? 1 : nblk >= 256 ? 4 : 16;
+    hipLaunchKernelGGL(v_scatter_kernel, dim3(nblk, split), dim3(256), 0, s, reinterpret_cast<const double2 *>(blk), d, V,
+                       (long long)n, (int)lay, drop_imag, q0, stride);
     HIP_CHECK(hipGetLastError());
 }
 
-__global__ void trace_kernel(const double *__restrict__ A, int n, int lda, double *acc,
-                             const double *__restrict__ signs) {
+__global__ __launch_bounds__(256) void add_signs_trace_kernel(double *A, int n, long long stride,
+                                                              const double *__restrict__ signs, int per, double *acc) {
     __shared__ double red[256];
+    const long long u = blockIdx.x;
+    double *M = A + u * stride;
+    const double *S = signs + (u / per) * n;
     double v = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) v += (signs ? signs[i] : 1.0) * A[(long long)i * lda + i];
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const double m = M[(long long)i * n + i] + S[i];
+        M[(long long)i * n + i] = m;
+        v += S[i] * m;
+    }
     red[threadIdx.x] = v;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *acc += red[0];
+    if (threadIdx.x == 0) acc[2 * u] += red[0];
 }
-void launch_trace_acc(const double *A, int n, int lda, double *acc, hipStream_t s, const double *signs) {
-    hipLaunchKernelGGL(trace_kernel, dim3(1), dim3(256), 0, s, A, n, lda, acc, signs);
+void launch_add_signs_trace(double *A, int n, long long nmat, long long stride, const double *signs, int per, double *acc,
+                            hipStream_t s) {
+    if (nmat <= 0) return;
+    hipLaunchKernelGGL(add_signs_trace_kernel, dim3((unsigned)nmat), dim3(256), 0, s, A, n, stride, signs, per, acc);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -558,8 +490,6 @@ void launch_copy_block(const double *src, int lds, double *dst, int ldd, int row
 // ------------------------------------------------------------------------------------
 // Blocked Cholesky with log-determinant
 // ------------------------------------------------------------------------------------
-constexpr int CHOL_NB = 64;
-
 // A double of another lane (lane is wave-uniform).
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
     const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
@@ -568,135 +498,254 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
     return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
-// Factor the nb x nb diagonal block at (j0, j0) of matrix blockIdx.x as L S L^T with
-// S = diag(+-1) (a Cholesky factorisation that tolerates negative pivots), write L11 back, write
-// Linv = L11^{-1} (row-major, CHOL_NB pitch) and the pivot signs, and accumulate
-// sum log|d_j| = ln |det| of the block.  A zero or NaN pivot sets *flag.
+typedef double v4d __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4d mfma16(double a, double b, v4d c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+constexpr int chol_nb(bool cplx) { return cplx ? 32 : 64; }  // columns of a diagonal block
+// per matrix: Linv, then Linv with row c times the pivot sign of c, each in planes
+constexpr long long chol_work(bool cplx) { return 2LL * (cplx ? 2 : 1) * chol_nb(cplx) * chol_nb(cplx); }
+
+// Factor the nb x nb diagonal block at (j0, j0) of matrix blockIdx.x as L S L^H with S = diag(+-1) (a
+// Cholesky factorisation that tolerates negative pivots), write L11 back, write L11^{-1} and
+// S L11^{-1} (row-major) and the pivot signs, and accumulate sum log|d_j| = ln |det| of the block.  A
+// zero or NaN pivot sets *flag.
 //
-// One wave per matrix; lane t keeps row t of the unit-padded 64 x 64 block in registers (the
-// loops are unrolled so every index is static).  At step j every lane takes the pivot from lane j
-// with readlane and forms s_j and sqrt|d_j| itself, lane t > j scales its entry, and each lane
-// updates its row with the scaled column read lane by lane.  The inverse is then formed with lane c
-// holding column c, again from readlane of the rows.  (Rows in LDS with lane-local loops took
-// three times as long: every step then waits on LDS round trips.)
-__global__ __launch_bounds__(64) void potrf_diag_kernel(double *A0, long long strideA, int lda, int j0, int nb,
-                                                        double *work, double *logdet0, long long ld_stride,
-                                                        int *flag, double *signs, long long sstride) {
-    __shared__ double L[CHOL_NB][CHOL_NB + 1];
-    const int t = threadIdx.x;
+// One workgroup per matrix, the block in LDS, 64 real or 32 complex columns in panels of 16.  A panel
+// is factored by one wave: lane t holds its 16 entries of row t (complex: lanes t and t + 32 the real
+// and imaginary parts), takes the pivot and the other rows' entries by readlane.  The four waves then
+// update the rest with MFMA.  The inverse goes from the 16 x 16 diagonal blocks, a wave each, outwards:
+// X_ij = -X_ii sum_k L_ik X_kj with the sum's accumulators as the next MFMA's operand.  (With all 64
+// columns in one wave's registers, every pivot step updates 64 columns lane by lane: 62 us a block.)
+template <bool CPLX>
+__global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long strideA, long long im, int lda, int j0,
+                                                          int nb, double *work, double *logdet0, long long ld_stride,
+                                                          int *flag, double *signs, long long sstride) {
+    constexpr int NB = chol_nb(CPLX), PL = CPLX ? 2 : 1, PN = NB / 16, NX = PN * (PN + 1) / 2;
+    __shared__ double L[PL][NB][NB + 1];
+    __shared__ double X[PL][NX][16][17];
+    __shared__ double sg[NB];
     double *A = A0 + strideA * blockIdx.x;
-    double *Linv = work + (long long)blockIdx.x * (CHOL_NB * CHOL_NB + CHOL_NB);
-    double *sgn = Linv + CHOL_NB * CHOL_NB;
-    // coalesced row loads through LDS into row t of lane t
-    for (int r = 0; r < CHOL_NB; ++r)
-        L[r][t] = (r < nb && t < nb) ? A[(long long)(j0 + r) * lda + j0 + t] : (r == t ? 1.0 : 0.0);
+    double *Linv = work + chol_work(CPLX) * blockIdx.x, *SLinv = Linv + (long long)PL * NB * NB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
+    for (int e = tid; e < PL * NB * NB; e += 256) {
+        const int h = e / (NB * NB), r = (e / NB) % NB, q = e % NB;
+        L[h][r][q] = (r < nb && q <= r) ? A[h * im + (long long)(j0 + r) * lda + j0 + q] : (r == q && h == 0 ? 1.0 : 0.0);
+    }
     __syncthreads();
-    double a[CHOL_NB];
-#pragma unroll
-    for (int k = 0; k < CHOL_NB; ++k) a[k] = L[t][k];
+    const int t = lane % NB, half = lane / NB;  // row and plane of a panel lane
+    double my_r = 1.0;
     bool bad = false;
-    double my_s = 1.0, my_r = 1.0;
+    for (int p = 0; p < PN; ++p) {
+        if (wave == 0) {
+            double a[16];
 #pragma unroll
-    for (int j = 0; j < CHOL_NB; ++j) {
-        double d = readlane_f64(a[j], j);
-        if (!(fabs(d) > 0.0)) { bad = true; d = 1.0; }
-        const double s = d > 0 ? 1.0 : -1.0;
-        const double r = sqrt(fabs(d));
-        // L_tj = a_tj / (s_j sqrt|d_j|), so that A = L S L^T also for a negative pivot; the update
-        // a_tk -= s_j L_tj L_kj then equals a_tk - a_tj a_kj / d_j
-        const double l = a[j] * (s / r);
-        if (t == j) { a[j] = r; my_s = s; my_r = r; }
-        if (t > j) a[j] = l;
-        const double f = t > j ? s * l : 0.0;
-        // entries k > t (upper triangle) are updated too and never used: no lane mask needed
+            for (int k = 0; k < 16; ++k) a[k] = L[half][t][16 * p + k];
 #pragma unroll
-        for (int k = j + 1; k < CHOL_NB; ++k) a[k] -= f * readlane_f64(a[j], k);
+            for (int j = 0; j < 16; ++j) {
+                const int jj = 16 * p + j;
+                double d = readlane_f64(a[j], jj);
+                if (!(fabs(d) > 0.0)) { bad = true; d = 1.0; }
+                const double s = d > 0 ? 1.0 : -1.0, r = sqrt(fabs(d));
+                // L_tj = a_tj / (s r), so that A = L S L^H also for a negative pivot
+                const double l = t > jj ? a[j] * (s / r) : 0.0;
+                if (t == jj) { a[j] = half ? 0.0 : r; if (!half) { my_r = r; sg[t] = s; } }
+                if (t > jj) a[j] = l;
+                const double f1 = s * l;
+                if constexpr (CPLX) {
+                    // a_tk -= s L_tj conj(L_kj): real lanes lr lr' + li li', imaginary lanes li lr' - lr li'
+                    const double lp = __shfl_xor(l, 32, 64), f2 = half ? -s * lp : s * lp;
+#pragma unroll
+                    for (int k = j + 1; k < 16; ++k)
+                        a[k] -= f1 * readlane_f64(a[j], 16 * p + k) + f2 * readlane_f64(a[j], 32 + 16 * p + k);
+                } else {
+#pragma unroll
+                    for (int k = j + 1; k < 16; ++k) a[k] -= f1 * readlane_f64(a[j], 16 * p + k);
+                }
+            }
+            if (t >= 16 * p)
+#pragma unroll
+                for (int k = 0; k < 16; ++k) L[half][t][16 * p + k] = a[k];
+        }
+        __syncthreads();
+        // tiles right of the panel: L_ij -= L_ip S L_jp^H
+        int n = 0;
+        for (int i = p + 1; i < PN; ++i)
+            for (int j = p + 1; j <= i; ++j)
+                for (int h = 0; h < PL; ++h, ++n) {
+                    if ((n & 3) != wave) continue;
+                    v4d acc;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[r] = L[h][16 * i + 4 * r + kq][16 * j + c];
+#pragma unroll
+                    for (int st = 0; st < 4; ++st) {
+                        const int k = 16 * p + 4 * st + kq;
+                        const double s = sg[k];
+                        if constexpr (!CPLX) {
+                            acc = mfma16(-s * L[0][16 * i + c][k], L[0][16 * j + c][k], acc);
+                        } else {
+                            const double ar = L[0][16 * i + c][k], ai = L[PL - 1][16 * i + c][k];
+                            acc = mfma16(-s * (h ? ai : ar), L[0][16 * j + c][k], acc);
+                            acc = mfma16(h ? s * ar : -s * ai, L[PL - 1][16 * j + c][k], acc);
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) L[h][16 * i + 4 * r + kq][16 * j + c] = acc[r];
+                }
+        __syncthreads();
     }
-    // L back through LDS as coalesced rows (lower triangle)
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < CHOL_NB; ++k) L[t][k] = a[k];
-    __syncthreads();
-    for (int r = 0; r < nb; ++r)
-        if (t <= r) A[(long long)(j0 + r) * lda + j0 + t] = L[r][t];
-    // column t of L^{-1}: x_r = (delta_rt - sum_{k < r} L_rk x_k) / L_rr (x_k = 0 for k < t)
-    double x[CHOL_NB];
-    const double dinv = 1.0 / my_r;
-#pragma unroll
-    for (int r = 0; r < CHOL_NB; ++r) {
-        double acc = r == t ? 1.0 : 0.0;
-#pragma unroll
-        for (int k = 0; k < r; ++k) acc -= readlane_f64(a[k], r) * x[k];
-        x[r] = acc * readlane_f64(dinv, r);
+    for (int e = tid; e < PL * NB * NB; e += 256) {
+        const int h = e / (NB * NB), r = (e / NB) % NB, q = e % NB;
+        if (r < nb && q <= r) A[h * im + (long long)(j0 + r) * lda + j0 + q] = L[h][r][q];
     }
+    // inverses of the diagonal blocks: lane c (complex: c and c + 16) holds column c
+    if (wave < PN) {
+        const int hx = CPLX ? kq & 1 : 0, b = 16 * wave;
+        double x[16];
 #pragma unroll
-    for (int r = 0; r < CHOL_NB; ++r) Linv[r * CHOL_NB + t] = (r < nb && t < nb) ? x[r] : 0.0;
-    sgn[t] = t < nb ? my_s : 1.0;
-    if (signs != nullptr && t < nb) signs[sstride * blockIdx.x + j0 + t] = my_s;
-    double v = t < nb ? 2.0 * log(my_r) : 0.0;
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (t == 0) {
-        logdet0[ld_stride * blockIdx.x] += v;
-        if (bad) *flag = 1;
+        for (int r = 0; r < 16; ++r) x[r] = (r == c && hx == 0) ? 1.0 : 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            x[r] *= 1.0 / L[0][b + r][b + r];
+            double xp = 0;
+            if constexpr (CPLX) {
+                xp = __shfl_xor(x[r], 16, 64);
+                if (!hx) xp = -xp;
+            }
+#pragma unroll
+            for (int q = r + 1; q < 16; ++q) {
+                x[q] -= L[0][b + q][b + r] * x[r];
+                if constexpr (CPLX) x[q] -= L[PL - 1][b + q][b + r] * xp;
+            }
+        }
+        if (kq < PL)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) X[kq][wave * (wave + 3) / 2][r][c] = x[r];
+    }
+    __syncthreads();
+    for (int dist = 1; dist < PN; ++dist) {
+        const int i = dist + wave, j = wave;
+        if (i < PN) {
+            v4d tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0};
+            for (int k = j; k < i; ++k) {
+                const int xb = k * (k + 1) / 2 + j;
+#pragma unroll
+                for (int st = 0; st < 4; ++st) {
+                    const int q = 4 * st + kq;
+                    const double lr = L[0][16 * i + c][16 * k + q], xr = X[0][xb][q][c];
+                    tr = mfma16(lr, xr, tr);
+                    if constexpr (CPLX) {
+                        const double li = L[PL - 1][16 * i + c][16 * k + q], xi = X[PL - 1][xb][q][c];
+                        tr = mfma16(-li, xi, tr);
+                        ti = mfma16(lr, xi, ti);
+                        ti = mfma16(li, xr, ti);
+                    }
+                }
+            }
+            v4d yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0};
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                const double xr = -X[0][i * (i + 3) / 2][c][4 * st + kq];
+                yr = mfma16(xr, tr[st], yr);
+                if constexpr (CPLX) {
+                    const double xi = -X[PL - 1][i * (i + 3) / 2][c][4 * st + kq];
+                    yr = mfma16(-xi, ti[st], yr);
+                    yi = mfma16(xr, ti[st], yi);
+                    yi = mfma16(xi, tr[st], yi);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                X[0][i * (i + 1) / 2 + j][4 * r + kq][c] = yr[r];
+                if constexpr (CPLX) X[PL - 1][i * (i + 1) / 2 + j][4 * r + kq][c] = yi[r];
+            }
+        }
+        __syncthreads();
+    }
+    for (int e = tid; e < PL * NB * NB; e += 256) {
+        const int h = e / (NB * NB), r = (e / NB) % NB, q = e % NB, bi = r / 16, bj = q / 16;
+        const double v = (q <= r && r < nb) ? X[h][bi * (bi + 1) / 2 + bj][r % 16][q % 16] : 0.0;
+        Linv[e] = v;
+        SLinv[e] = sg[r] * v;
+    }
+    if (signs != nullptr && tid < nb) signs[sstride * blockIdx.x + j0 + tid] = sg[tid];
+    if (wave == 0) {
+        double v = (half == 0 && t < nb) ? 2.0 * log(my_r) : 0.0;
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (lane == 0) {
+            logdet0[ld_stride * blockIdx.x] += v;
+            if (bad) *flag = 1;
+        }
     }
 }
 
-// Qs[r][c] = Q[r][c] * sgn[c] for matrix blockIdx.y of the batch; Q and Qs are m x nb regions of
-// the given pitch inside that matrix's pair of wide panels
-constexpr int CHOL_PW = 8 * CHOL_NB;   // middle panel: its update of the outer panel runs with K = 512
-constexpr int CHOL_PO = 4 * CHOL_PW;   // outer panel of large matrices: the trailing update has K = 2048
-
-__global__ void scale_cols_kernel(double *__restrict__ Q, double *__restrict__ Qs, long long pstride, int pitch,
-                                  const double *__restrict__ work, int m, int nb) {
+// m x nb blocks of nmat matrices (blockIdx.y) and their planes (.z)
+__global__ void copy_panel_kernel(const double *__restrict__ src, int lds, long long sstride, long long splane,
+                                  double *__restrict__ dst, int ldd, long long dstride, long long dplane, int m, int nb) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)m * nb) return;
-    const long long r = idx / nb, c = idx % nb;
-    const double *sgn = work + (long long)blockIdx.y * (CHOL_NB * CHOL_NB + CHOL_NB) + CHOL_NB * CHOL_NB;
-    const long long o = (long long)blockIdx.y * pstride + r * pitch + c;
-    Qs[o] = Q[o] * sgn[c];
+    const long long r = idx / nb, q = idx % nb;
+    dst[blockIdx.y * dstride + blockIdx.z * dplane + r * ldd + q] = src[blockIdx.y * sstride + blockIdx.z * splane + r * lds + q];
 }
 
 struct CholPlan {
     std::vector<int> j0s, nbs;
-    std::vector<GemmBatch> trsm, inpanel;  // per 64-column step
-    std::vector<GemmBatch> mid;            // per step: the K = CHOL_PW update of the outer panel's other columns
+    std::vector<GemmBatch> trsm, inpanel;  // per step of one diagonal block
+    std::vector<GemmBatch> mid;            // per step: the middle panel's update of the outer panel's other columns
     std::vector<GemmBatch> trail;          // per step: the trailing update after an outer panel
 };
 
-static std::map<std::tuple<int, int, int, long long, hipStream_t, int>, CholPlan> &chol_plans() {
-    static std::map<std::tuple<int, int, int, long long, hipStream_t, int>, CholPlan> p;
+static std::map<std::tuple<int, int, int, long long, hipStream_t, int, long long>, CholPlan> &chol_plans() {
+    static std::map<std::tuple<int, int, int, long long, hipStream_t, int, long long>, CholPlan> p;
     return p;
 }
 
-// Right-looking blocked L S L^T factorisation in three levels.  64-column steps (diagonal block
-// by potrf_diag_kernel, Q = A21 L11^-T by GEMM, signs applied) update only the rest of their
-// 512-column middle panel (K = 64); after each middle panel one GEMM with K = 512 updates the
-// remaining columns of its outer panel; after each outer panel one lower-triangular GEMM updates
-// the trailing matrix with K = the outer panel width (2048 for n >= 4096, else 512, when the
-// middle level is the outer one).  Few, deep trailing updates read and write the trailing matrix
-// four times less often than 512-wide ones.  Q and Q S of the outer panel's columns are kept in
-// two wide buffers per matrix (pitch = outer panel width, indexed by global row).
+// Right-looking blocked L S L^H factorisation in three levels.  Steps of one diagonal block (64 real
+// or 32 complex columns, by potrf_block_kernel; Q = A21 L11^-H and Q S by one GEMM launch) update only
+// the rest of their middle panel (512 real or 256 complex columns); after each middle panel one GEMM
+// updates the remaining columns of its outer panel; after each outer panel one lower-triangular GEMM
+// updates the trailing matrix (2048 real or 1024 complex columns for n >= 4096 / 2048, else the middle
+// level is the outer one).  Few, deep trailing updates read and write the trailing matrix four times
+// less often.  Q and Q S of the outer panel's columns are kept in wide buffers per matrix (pitch =
+// outer panel width, indexed by global row).
+//
+// A Hermitian matrix is factored as such, from its two planes, each product as two real segments:
+// 4/3 n^3 real multiply-adds, where the real embedding [[Re, -Im], [Im, Re]] (2n x 2n) needs 8/3 n^3.
 void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, int lda, double *logdet,
                              long long ld_stride, int *flag, bool keep_L, CholWork &w, hipStream_t s, int ncols,
-                             double *signs, long long sstride) {
+                             double *signs, long long sstride, long long im) {
+    const bool cplx = im != 0;
     const int nf = (ncols > 0 && ncols < n) ? ncols : n;
-    const int PO = n >= 4096 ? CHOL_PO : CHOL_PW;
-    const long long wstride = CHOL_NB * CHOL_NB + CHOL_NB;
-    const long long pstride = 2LL * n * PO;  // Q then Q S, each n x PO
+    const int NB = chol_nb(cplx), PW = 8 * NB, PO = n >= 64 * NB ? 4 * PW : PW, PL = cplx ? 2 : 1;
+    const long long wstride = chol_work(cplx), wplane = (long long)NB * NB;
+    const long long qplane = (long long)n * PO, qs_off = PL * qplane, pstride = 2 * qs_off;  // Q planes, then Q S planes
     w.linv.reserve(sizeof(double) * wstride * nbatch);
     w.panel.reserve(sizeof(double) * pstride * nbatch);
-    const long long qs_off = (long long)n * PO;
-    auto key = std::make_tuple(n, lda, nbatch, strideA, s, nf);
+    auto key = std::make_tuple(n, lda, nbatch, strideA, s, nf, im);
     auto &plans = chol_plans();
     auto it = plans.find(key);
     if (it == plans.end()) {
         CholPlan cp;
+        // C (+)= A B^H: one real problem, or its real and imaginary parts as two segments each
+        auto add = [&](GemmBatch &b, int M, int N, int K, long long ao, long long ap, int la, long long bo, long long bp,
+                       int lb, long long co, long long cpl, int lc) {
+            GemmProb p = make_prob(M, N, K, ao, la, bo, lb, co, lc);
+            if (cplx) { p.sgn2 = 1; p.a_off2 = ao + ap; p.b_off2 = bo + bp; }
+            b.add(p);
+            if (!cplx) return;
+            p = make_prob(M, N, K, ao + ap, la, bo, lb, co + cpl, lc);
+            p.sgn2 = -1;
+            p.a_off2 = ao;
+            p.b_off2 = bo + bp;
+            b.add(p);
+        };
         for (int o0 = 0; o0 < nf; o0 += PO) {
             const int oend = std::min(o0 + PO, nf);
-            for (int p0 = o0; p0 < oend; p0 += CHOL_PW) {
-                const int pend = std::min(p0 + CHOL_PW, oend);
-                for (int j0 = p0; j0 < pend; j0 += CHOL_NB) {
-                    const int nb = std::min(CHOL_NB, pend - j0);
+            for (int p0 = o0; p0 < oend; p0 += PW) {
+                const int pend = std::min(p0 + PW, oend);
+                for (int j0 = p0; j0 < pend; j0 += NB) {
+                    const int nb = std::min(NB, pend - j0);
                     const int m = n - j0 - nb;
                     const int wcols = pend - j0 - nb;  // middle panel columns right of this step
                     cp.j0s.push_back(j0);
@@ -707,38 +756,39 @@ void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, in
                         ip.trans_b = true;
                         for (int b = 0; b < nbatch; ++b) {
                             const long long wq = pstride * b + (long long)(j0 + nb) * PO + (j0 - o0);
-                            // Q = A21 * Linv^T  (A21: m x nb at (j0+nb, j0)) into the wide buffer
-                            tr.add(make_prob(m, nb, nb, strideA * b + (long long)(j0 + nb) * lda + j0, lda,
-                                             wstride * b, CHOL_NB, wq, PO));
-                            // A[j0+nb:, j0+nb:pend] -= (Q S) Q[0:wcols]^T
+                            const long long a21 = strideA * b + (long long)(j0 + nb) * lda + j0;
+                            // Q = A21 Linv^H and Q S (A21: m x nb at (j0+nb, j0)) into the wide buffers
+                            add(tr, m, nb, nb, a21, im, lda, wstride * b, wplane, NB, wq, qplane, PO);
+                            add(tr, m, nb, nb, a21, im, lda, wstride * b + PL * wplane, wplane, NB, wq + qs_off, qplane, PO);
+                            // A[j0+nb:, j0+nb:pend] -= (Q S) Q[0:wcols]^H
                             if (wcols > 0)
-                                ip.add(make_prob(m, wcols, nb, wq + qs_off, PO, wq, PO,
-                                                 strideA * b + (long long)(j0 + nb) * lda + (j0 + nb), lda));
+                                add(ip, m, wcols, nb, wq + qs_off, qplane, PO, wq, qplane, PO,
+                                    strideA * b + (long long)(j0 + nb) * lda + (j0 + nb), im, lda);
                         }
                         tr.finalize(T64x64, s);
                         if (wcols > 0) ip.finalize(T64x64, s);
                     }
                     if (j0 + nb == pend && pend < oend) {
-                        // the middle panel's update of the outer panel: A[pend:, pend:oend] -= (Q S) Q^T
+                        // the middle panel's update of the outer panel: A[pend:, pend:oend] -= (Q S) Q^H
                         // over its pend - p0 columns (rectangular; the upper part of the diagonal
                         // block is not read)
                         md.trans_b = true;
                         for (int b = 0; b < nbatch; ++b) {
                             const long long wq = pstride * b + (long long)pend * PO + (p0 - o0);
-                            md.add(make_prob(n - pend, oend - pend, pend - p0, wq + qs_off, PO, wq, PO,
-                                             strideA * b + (long long)pend * lda + pend, lda));
+                            add(md, n - pend, oend - pend, pend - p0, wq + qs_off, qplane, PO, wq, qplane, PO,
+                                strideA * b + (long long)pend * lda + pend, im, lda);
                         }
                         md.finalize(T128x128w8, s);
                     }
                     const int mt = n - oend;
                     if (j0 + nb == oend && mt > 0) {
-                        // trailing update of the outer panel: A22 -= (Q S) Q^T over its oend - o0 columns
+                        // trailing update of the outer panel: A22 -= (Q S) Q^H over its oend - o0 columns
                         tl.trans_b = true;
                         tl.lower_only = true;
                         for (int b = 0; b < nbatch; ++b) {
                             const long long wq = pstride * b + (long long)oend * PO;
-                            tl.add(make_prob(mt, mt, oend - o0, wq + qs_off, PO, wq, PO,
-                                             strideA * b + (long long)oend * lda + oend, lda));
+                            add(tl, mt, mt, oend - o0, wq + qs_off, qplane, PO, wq, qplane, PO,
+                                strideA * b + (long long)oend * lda + oend, im, lda);
                         }
                         tl.finalize(T128x128w8, s);
                     }
@@ -757,27 +807,32 @@ void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, in
     for (size_t b = 0; b < cp.j0s.size(); ++b) {
         const int j0 = cp.j0s[b], nb = cp.nbs[b];
         const int o0 = (j0 / PO) * PO;
-        hipLaunchKernelGGL(potrf_diag_kernel, dim3(nbatch), dim3(CHOL_NB), 0, s, A, strideA, lda, j0, nb, work,
-                           logdet, ld_stride, flag, signs, sstride);
+        if (cplx)
+            hipLaunchKernelGGL(potrf_block_kernel<true>, dim3(nbatch), dim3(256), 0, s, A, strideA, im, lda, j0, nb, work,
+                               logdet, ld_stride, flag, signs, sstride);
+        else
+            hipLaunchKernelGGL(potrf_block_kernel<false>, dim3(nbatch), dim3(256), 0, s, A, strideA, im, lda, j0, nb, work,
+                               logdet, ld_stride, flag, signs, sstride);
         HIP_CHECK(hipGetLastError());
         const int m = n - j0 - nb;
         if (m > 0) {
-            double *wq = panel + (long long)(j0 + nb) * PO + (j0 - o0);
             gemm_run(Prec::F64, cp.trsm[b], A, work, panel, 1.0, 0.0, s);
-            hipLaunchKernelGGL(scale_cols_kernel, dim3(ceil_div((long long)m * nb, 256), nbatch), dim3(256), 0, s, wq,
-                               wq + qs_off, pstride, PO, work, m, nb);
-            HIP_CHECK(hipGetLastError());
-            if (keep_L)
-                for (int bb = 0; bb < nbatch; ++bb)
-                    launch_copy_block(wq + pstride * bb + qs_off, PO, A + strideA * bb + (long long)(j0 + nb) * lda + j0,
-                                      lda, m, nb, s);
+            if (keep_L) {
+                const double *qs = panel + qs_off + (long long)(j0 + nb) * PO + (j0 - o0);
+                hipLaunchKernelGGL(copy_panel_kernel, dim3(ceil_div((long long)m * nb, 256), nbatch, PL), dim3(256), 0, s,
+                                   qs, PO, pstride, qplane, A + (long long)(j0 + nb) * lda + j0, lda, strideA, im, m, nb);
+                HIP_CHECK(hipGetLastError());
+            }
             gemm_run(Prec::F64, cp.inpanel[b], panel, panel, A, -1.0, 1.0, s);
         }
         gemm_run(Prec::F64, cp.mid[b], panel, panel, A, -1.0, 1.0, s);
         gemm_run(Prec::F64, cp.trail[b], panel, panel, A, -1.0, 1.0, s);
     }
-    if (keep_L)
-        for (int bb = 0; bb < nbatch; ++bb) launch_zero_upper<double>(A + strideA * bb, n, lda, s);
+    if (keep_L) {
+        hipLaunchKernelGGL(zero_upper_kernel, dim3(ceil_div((long long)n * n, 256), nbatch, PL), dim3(256), 0, s, A, n, lda,
+                           strideA, im);
+        HIP_CHECK(hipGetLastError());
+    }
 }
 
 void cholesky_logdet(double *A, int n, int lda, double *logdet, int *flag, bool keep_L, CholWork &w, hipStream_t s,

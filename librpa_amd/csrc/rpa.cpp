@@ -616,9 +616,13 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     auto &prof = profiler();
     const double t0 = now_s();
     RpaResult res;
-    const bool embed = nk > 1;
-    const int n = NABF, n2 = embed ? 2 * NABF : NABF;
-    const size_t nn = (size_t)n2 * n2;
+    // a Hermitian matrix of a k point is its real and imaginary plane (n x n each), every product two
+    // real segments: half the work and the bytes of the real embedding [[Re, -Im], [Im, Re]]
+    const bool herm = nk > 1;
+    const DenseLayout lay = herm ? kPlanar : kReal;
+    const int n = NABF;
+    const long long plane = (long long)n * n;
+    const size_t nn = (size_t)plane * (herm ? 2 : 1);
     std::vector<int> ibz;
     std::vector<double> wq;
     ibz_list(ds, nk, ibz, wq);
@@ -652,7 +656,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     for (const DevBuf *b : {&ec_V, &ec_L32, &ec_D, &ec_X, &ec_M, &ec_M64, &ec_S, &ec_Vld, &ec_acc, &ec_cw.linv,
                             &ec_cw.panel})
         held += (double)b->bytes();
-    const double panel_w = 16.0 * n2 * (n2 >= 4096 ? 2048 : 512);  // Cholesky panels per matrix
+    const double panel_w = 16.0 * n * (n >= (herm ? 2048 : 4096) ? 2048 : 512);  // Cholesky panels per matrix
     const double per_w = (double)nn * (3 * es + (f64 ? 0 : 8)) + panel_w;
     const double per_q = (double)nn * 12 + panel_w;
     const double budget = std::min(96e9, 0.6 * ((double)free_b + held)) - (double)nn * 12;
@@ -673,7 +677,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     // pivot signs S of V = L S L^T: a Coulomb matrix that is not positive definite keeps
     // det(1 - V chi0) = det(S) det(S - L^T chi0 L) and Tr(V chi0) = n - sum_i S_i M_ii with
     // M = S - L^T chi0 L, so Ec is exact for any V (as the LU of epsilon.cpp:600-693 is)
-    dS.reserve((size_t)n2 * 8 * QG);
+    dS.reserve((size_t)n * 8 * QG);
     if (!f64) { dL32.reserve(nn * 4 * QG); dM64.reserve(nn * 8 * UCH); }
     const size_t acc_bytes = sizeof(double) * 2 * nq * nw + 64;
     dacc.reserve(acc_bytes);
@@ -690,7 +694,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
                 const int ik = std::get<0>(kv.first), I = std::get<1>(kv.first), J = std::get<2>(kv.first);
                 if (ik != ibz[iq] || I > J) continue;
                 if (kv.second.size() != (size_t)na[I] * na[J]) LRA_THROW("Coulomb block of the wrong size");
-                desc.push_back({(long long)store.size(), (int)abf[I], (int)abf[J], na[I], na[J], I == J ? 1 : 0});
+                desc.push_back({(long long)store.size(), (int)abf[I], (int)abf[J], na[I], na[J], I == J ? 1 : 0, iq});
                 store.insert(store.end(), kv.second.begin(), kv.second.end());
             }
             vdesc_q.push_back((int)desc.size());
@@ -703,7 +707,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     // (q per pass, omega per q, order, precision) -> (X = D L, M = S - L^T X) over the pass's
     // matrices u = qi * cnt + w, whose L is that of q qi; kept with their tuned tiles
     auto get_batches = [&](int qg, int cnt) -> std::pair<GemmBatch, GemmBatch> & {
-        const auto key = std::make_tuple(qg, cnt, n2, (int)ec_prec);
+        const auto key = std::make_tuple(qg, cnt, n, (int)ec_prec);
         auto it = ec_batches.find(key);
         if (it != ec_batches.end()) return it->second;
         auto &pr = ec_batches[key];
@@ -712,30 +716,33 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
         bm.lower_only = true;
         for (int qi = 0; qi < qg; ++qi)
             for (int w = 0; w < cnt; ++w) {
-                const long long u = (long long)qi * cnt + w;
-                GemmProb px = make_prob(n2, n2, n2, u * nn, n2, (long long)qi * nn, n2, u * nn, n2);
-                px.kmode = 1;  // L is lower triangular: column tile n0 needs k >= n0 only
-                bx.add(px);
-                GemmProb pm = make_prob(n2, n2, n2, (long long)qi * nn, n2, u * nn, n2, u * nn, n2);
-                pm.kmode = 2;  // A = L^T: row tile m0 needs k >= m0 only
-                bm.add(pm);
+                const long long u = ((long long)qi * cnt + w) * (long long)nn, l = (long long)qi * (long long)nn;
+                // plane h of X = D L (no conjugate) and of M = L^H X
+                for (int h = 0; h < (herm ? 2 : 1); ++h) {
+                    GemmProb px = make_prob(n, n, n, u, n, l + h * plane, n, u + h * plane, n);
+                    px.kmode = 1;  // L is lower triangular: column tile n0 needs k >= n0 only
+                    GemmProb pm = make_prob(n, n, n, l, n, u + h * plane, n, u + h * plane, n);
+                    pm.kmode = 2;  // A = L^T: row tile m0 needs k >= m0 only
+                    if (herm) {
+                        px.sgn2 = h ? 1 : -1;
+                        px.a_off2 = u + plane;
+                        px.b_off2 = l + (1 - h) * plane;
+                        pm.sgn2 = h ? -1 : 1;
+                        pm.a_off2 = l + plane;
+                        pm.b_off2 = u + (1 - h) * plane;
+                    }
+                    bx.add(px);
+                    bm.add(pm);
+                }
             }
-        const int cfg = n2 >= 1024 ? big_tile(ec_prec) : T64x64;
+        const int cfg = n >= 1024 ? big_tile(ec_prec) : T64x64;
         bx.finalize(cfg, stream);
         bm.finalize(cfg, stream);
         // executed flops of the triangular products
-        bx.flops = 2.0 * qg * cnt * (double)n2 * n2 * n2 / 2.0;
-        bm.flops = 2.0 * qg * cnt * (double)n2 * n2 * n2 / 6.0;
+        const double c = (herm ? 4.0 : 1.0) * qg * cnt * (double)n * n * n;
+        bx.flops = c;
+        bm.flops = c / 3.0;
         return pr;
-    };
-    auto set_m_identity = [&](int qg, int cnt) {
-        for (int qi = 0; qi < qg; ++qi)
-            for (int w = 0; w < cnt; ++w) {
-                const size_t u = (size_t)qi * cnt + w;
-                const double *sg = dS.as<double>() + (size_t)qi * n2;
-                if (f64) launch_set_identity<double>(dM.as<double>() + u * nn, n2, n2, stream, sg);
-                else launch_set_identity<float>(dM.as<float>() + u * nn, n2, n2, stream, sg);
-            }
     };
     for (int iq0 = 0; iq0 < nq; iq0 += QG) {
         const int qg = std::min(QG, nq - iq0);
@@ -747,16 +754,13 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
         // dense V(q) from the staged upper atom-pair blocks (Hermitian fill, utils_matrix_m_mpi.h:430-441)
         prof.begin("ec_v_fill", stream);
         HIP_CHECK(hipMemsetAsync(dV.get(), 0, (size_t)qg * nn * 8, stream));
-        for (int qi = 0; qi < qg; ++qi) {
-            const int iq = iq0 + qi;
-            launch_v_scatter(d_vblk.as<double>(), d_vdesc.as<VBlock>() + vdesc_q[iq], vdesc_q[iq + 1] - vdesc_q[iq],
-                             dV.as<double>() + (size_t)qi * nn, n, n2, embed ? 1 : 0, 0, stream);
-        }
+        launch_v_scatter(d_vblk.as<double>(), d_vdesc.as<VBlock>() + vdesc_q[iq0], vdesc_q[iq0 + qg] - vdesc_q[iq0],
+                         dV.as<double>(), n, lay, 0, iq0, (long long)nn, stream);
         prof.end("ec_v_fill", stream, 0, (double)qg * nn * 8);
         prof.begin("ec_chol_v", stream);
-        cholesky_logdet_batched(dV.as<double>(), (long long)nn, qg, n2, n2, dVld.as<double>(), 1, dflag + 1, true, cw,
-                                stream, -1, dS.as<double>(), n2);
-        prof.end("ec_chol_v", stream, (double)qg * n2 * n2 * n2 / 3.0);
+        cholesky_logdet_batched(dV.as<double>(), (long long)nn, qg, n, n, dVld.as<double>(), 1, dflag + 1, true, cw,
+                                stream, -1, dS.as<double>(), n, herm ? plane : 0);
+        prof.end("ec_chol_v", stream, (herm ? 4.0 : 1.0) * qg * n * n * n / 3.0);
         const void *Lp = dV.get();
         if (!f64) {
             launch_convert<double, float>(dV.as<double>(), dL32.as<float>(), (long long)qg * nn, stream);
@@ -770,7 +774,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
             prof.begin("chi0_transform", stream);
             std::vector<const double *> kfs(qg);
             for (int qi = 0; qi < qg; ++qi) kfs[qi] = &ds.kfrac[(size_t)ibz[iq0 + qi] * 3];
-            assemble_dense_q(g, kfs, w0, cnt, dD.get(), f64, (long long)nn, embed, stream);
+            assemble_dense_q(g, kfs, w0, cnt, dD.get(), f64, (long long)nn, lay, stream);
             const double tbytes = chiw_ok ? 8.0 * E_tot * cnt * ceil_div(qg, kChi0RqMaxQ) + (double)es * cnt * nn * qg
                                           : ((double)ts * E_tot * ntau_done * ceil_div(cnt, kChi0AssembleMaxW) +
                                              (double)es * cnt * nn) * qg;
@@ -779,31 +783,28 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
             if (autotune && !bb.first.tuned) {
                 bb.first.tune(ec_prec, dD.get(), Lp, dX.get(), 1.0, 0.0, stream);
                 gemm_run(ec_prec, bb.first, dD.get(), Lp, dX.get(), 1.0, 0.0, stream);
-                bb.second.tune(ec_prec, Lp, dX.get(), dM.get(), -1.0, 1.0, stream, [&]() { set_m_identity(qg, cnt); });
+                bb.second.tune(ec_prec, Lp, dX.get(), dM.get(), -1.0, 0.0, stream);
             }
             prof.begin("ec_gemm_x", stream);
             gemm_run(ec_prec, bb.first, dD.get(), Lp, dX.get(), 1.0, 0.0, stream);
             prof.end("ec_gemm_x", stream, bb.first.flops);
-            set_m_identity(qg, cnt);
             prof.begin("ec_gemm_m", stream);
-            gemm_run(ec_prec, bb.second, Lp, dX.get(), dM.get(), -1.0, 1.0, stream);
+            gemm_run(ec_prec, bb.second, Lp, dX.get(), dM.get(), -1.0, 0.0, stream);
             prof.end("ec_gemm_m", stream, bb.second.flops);
             double *M64 = dM.as<double>();
             if (!f64) {
-                for (int u = 0; u < nu; ++u)
-                    launch_copy_lower_f2d(dM.as<float>() + (size_t)u * nn, dM64.as<double>() + (size_t)u * nn, n2, n2,
-                                          stream);
+                launch_copy_lower_f2d(dM.as<float>(), dM64.as<double>(), n, (long long)nu * (herm ? 2 : 1), plane, stream);
                 M64 = dM64.as<double>();
             }
             // accumulators of (q, omega) at 2 (q nw + omega): the pass's matrices are consecutive
             // there (one q per pass, or all omega of each q)
             double *acc0 = dacc.as<double>() + 2 * ((size_t)iq0 * nw + w0);
             prof.begin("ec_logdet", stream);
-            for (int u = 0; u < nu; ++u)
-                launch_trace_acc(M64 + (size_t)u * nn, n2, n2, acc0 + 2 * u, stream,
-                                 dS.as<double>() + (size_t)(u / cnt) * n2);
-            cholesky_logdet_batched(M64, (long long)nn, nu, n2, n2, acc0 + 1, 2, dflag, false, cw, stream);
-            prof.end("ec_logdet", stream, (double)nu * n2 * n2 * n2 / 3.0);
+            // S joins -L^H X here, in FP64 whatever the precision of the products
+            launch_add_signs_trace(M64, n, nu, (long long)nn, dS.as<double>(), cnt, acc0, stream);
+            cholesky_logdet_batched(M64, (long long)nn, nu, n, n, acc0 + 1, 2, dflag, false, cw, stream, -1, nullptr, 0,
+                                    herm ? plane : 0);
+            prof.end("ec_logdet", stream, (herm ? 4.0 : 1.0) * nu * n * n * n / 3.0);
         }
     }
     std::vector<double> hacc(2 * (size_t)nq * nw);
@@ -813,13 +814,11 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     HIP_CHECK(hipStreamSynchronize(stream));
     if (hflag[1]) LRA_THROW("Coulomb matrix is singular or not finite (zero pivot in its factorisation)");
     if (hflag[0]) LRA_THROW("1 - V chi0 is singular or not finite at some (q, omega)");
-    const double half = embed ? 0.5 : 1.0;
     for (int iq = 0; iq < nq; ++iq)
         for (int iw = 0; iw < nw; ++iw) {
             const double tr = hacc[2 * ((size_t)iq * nw + iw)];
             const double ld = hacc[2 * ((size_t)iq * nw + iw) + 1];
-            const double trpi = (n2 - tr) * half;
-            const double val = trpi + ld * half;
+            const double val = (n - tr) + ld;
             res.qcontrib[iq] += cplx(val * g.omega_w[iw] * wq[iq] / (2 * M_PI), 0.0);
         }
     for (auto &c : res.qcontrib) res.ec_re += c.real();
@@ -864,11 +863,11 @@ bool RpaEngine::form_chiw(const TFGrid &g, double max_bytes, hipStream_t s) {
 }
 
 void RpaEngine::assemble_dense_q(const TFGrid &g, const std::vector<const double *> &kfs, int w0, int cnt,
-                                 void *dense, bool f64, long long nn, bool embed, hipStream_t s) {
+                                 void *dense, bool f64, long long nn, DenseLayout lay, hipStream_t s) {
     const size_t es = f64 ? 8 : 4;
     if (!chiw_ok) {
         for (size_t qi = 0; qi < kfs.size(); ++qi)
-            assemble_dense(g, kfs[qi], w0, cnt, static_cast<char *>(dense) + qi * cnt * nn * es, f64, nn, embed, s);
+            assemble_dense(g, kfs[qi], w0, cnt, static_cast<char *>(dense) + qi * cnt * nn * es, f64, nn, lay, s);
         return;
     }
     const int n = NABF;
@@ -889,35 +888,27 @@ void RpaEngine::assemble_dense_q(const TFGrid &g, const std::vector<const double
         if (f64)
             launch_chi0_rq_multi<double>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
                                          d_pair_eoff.as<long long>(), nR, dph.as<double>(), nq, cnt, (double *)Dd, nn,
-                                         (long long)cnt * nn, n, embed, s);
+                                         (long long)cnt * nn, n, lay, s);
         else
             launch_chi0_rq_multi<float>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
                                         d_pair_eoff.as<long long>(), nR, dph.as<double>(), nq, cnt, (float *)Dd, nn,
-                                        (long long)cnt * nn, n, embed, s);
+                                        (long long)cnt * nn, n, lay, s);
         HIP_CHECK(hipStreamSynchronize(s));  // dph is freed on return
     }
 }
 
 void RpaEngine::assemble_dense(const TFGrid &g, const double *kf, int w0, int cnt, void *dense, bool f64, long long nn,
-                               bool embed, hipStream_t s) {
+                               DenseLayout lay, hipStream_t s) {
+    if (chiw_ok) {
+        assemble_dense_q(g, {kf}, w0, cnt, dense, f64, nn, lay, s);
+        return;
+    }
     const int n = NABF;
     std::vector<double> ph((size_t)nR * 2);
     for (int r = 0; r < nR; ++r) {
         const double ang = 2 * M_PI * (kf[0] * cells[r][0] + kf[1] * cells[r][1] + kf[2] * cells[r][2]);
         ph[2 * r] = std::cos(ang);
         ph[2 * r + 1] = std::sin(ang);
-    }
-    if (chiw_ok) {
-        DevBuf dph = upload(ph, s);
-        const double *cw = d_chiw.as<double>() + (size_t)w0 * E_tot;
-        if (f64)
-            launch_chi0_rq<double>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
-                                   d_pair_eoff.as<long long>(), nR, dph.as<double>(), cnt, (double *)dense, nn, n, embed, s);
-        else
-            launch_chi0_rq<float>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
-                                  d_pair_eoff.as<long long>(), nR, dph.as<double>(), cnt, (float *)dense, nn, n, embed, s);
-        HIP_CHECK(hipStreamSynchronize(s));  // dph is freed on return
-        return;
     }
     const size_t es = f64 ? 8 : 4;
     for (int a0 = 0; a0 < cnt; a0 += kChi0AssembleMaxW) {
@@ -935,19 +926,19 @@ void RpaEngine::assemble_dense(const TFGrid &g, const double *kf, int w0, int cn
         if (prec == Prec::F64 && f64)
             launch_chi0_assemble<double, double>(d_chi0s.as<double>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                                  (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                                 dgp.as<double>(), cw_n, (double *)Dd, nn, n, embed, s);
+                                                 dgp.as<double>(), cw_n, (double *)Dd, nn, n, lay, s);
         else if (prec == Prec::F64)
             launch_chi0_assemble<double, float>(d_chi0s.as<double>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                                 (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                                dgp.as<double>(), cw_n, (float *)Dd, nn, n, embed, s);
+                                                dgp.as<double>(), cw_n, (float *)Dd, nn, n, lay, s);
         else if (f64)
             launch_chi0_assemble<float, double>(d_chi0s.as<float>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                                 (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                                dgp.as<double>(), cw_n, (double *)Dd, nn, n, embed, s);
+                                                dgp.as<double>(), cw_n, (double *)Dd, nn, n, lay, s);
         else
             launch_chi0_assemble<float, float>(d_chi0s.as<float>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                                (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                               dgp.as<double>(), cw_n, (float *)Dd, nn, n, embed, s);
+                                               dgp.as<double>(), cw_n, (float *)Dd, nn, n, lay, s);
         HIP_CHECK(hipStreamSynchronize(s));  // dgp is freed on return
     }
 }
@@ -1001,9 +992,11 @@ void RpaEngine::chi0s_block(int it, int I, int J, int r, double *out) {
 void RpaEngine::chi0q_block(const Dataset &ds, const TFGrid &g, int iw, int iq, int I, int J, double *re,
                             double *im) {
     if (host_staged) LRA_THROW("chi0(q, omega) blocks are not kept with the host-staged chi0 store");
-    const bool embed = nk > 1;
-    const int n = NABF, n2 = embed ? 2 * NABF : NABF;
-    DevBuf dD((size_t)n2 * n2 * 8);
+    const bool herm = nk > 1;
+    const DenseLayout lay = herm ? kPlanar : kReal;
+    const int n = NABF;
+    const size_t nn = (size_t)n * n * (herm ? 2 : 1);
+    DevBuf dD(nn * 8);
     std::vector<double> gp((size_t)nR * ntau_done * 2);
     const double *kf = &ds.kfrac[(size_t)iq * 3];
     for (int r = 0; r < nR; ++r) {
@@ -1018,19 +1011,19 @@ void RpaEngine::chi0q_block(const Dataset &ds, const TFGrid &g, int iw, int iq, 
     if (prec == Prec::F64)
         launch_chi0_assemble<double, double>(d_chi0s.as<double>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                              (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                             dgp.as<double>(), 1, dD.as<double>(), 0, n, embed, stream);
+                                             dgp.as<double>(), 1, dD.as<double>(), 0, n, lay, stream);
     else
         launch_chi0_assemble<float, double>(d_chi0s.as<float>(), E_tot, ntau_done, d_pairs.as<PairDesc>(),
                                             (int)pairs.size(), n_pair_elems, d_pair_eoff.as<long long>(), nR,
-                                            dgp.as<double>(), 1, dD.as<double>(), 0, n, embed, stream);
-    std::vector<double> h((size_t)n2 * n2);
+                                            dgp.as<double>(), 1, dD.as<double>(), 0, n, lay, stream);
+    std::vector<double> h(nn);
     HIP_CHECK(hipMemcpyAsync(h.data(), dD.get(), h.size() * 8, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     for (int mu = 0; mu < na[I]; ++mu)
         for (int nu = 0; nu < na[J]; ++nu) {
             const size_t r = abf[I] + mu, c = abf[J] + nu;
-            re[(size_t)mu * na[J] + nu] = h[r * n2 + c];
-            im[(size_t)mu * na[J] + nu] = embed ? h[(n + r) * n2 + c] : 0.0;
+            re[(size_t)mu * na[J] + nu] = h[r * n + c];
+            im[(size_t)mu * na[J] + nu] = herm ? h[(n + r) * n + c] : 0.0;
         }
 }
 

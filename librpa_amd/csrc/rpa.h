@@ -145,14 +145,14 @@ struct RpaEngine {
     bool chiw_ok = false;
     bool form_chiw(const TFGrid &g, double max_bytes, hipStream_t s);
     // dense chi0(q, omega) of the frequencies [w0, w0 + cnt) at fractional q into cnt matrices of nn
-    // elements (FP64 or FP32), real at Gamma or the real embedding
+    // elements (FP64 or FP32) in one of the dense layouts
     void assemble_dense(const TFGrid &g, const double *kf, int w0, int cnt, void *dense, bool f64, long long nn,
-                        bool embed, hipStream_t s);
+                        DenseLayout lay, hipStream_t s);
     // the same for several q points at once (chi0(R, omega) formed): q point qi of kfs writes its
     // cnt matrices at dense + qi * cnt * nn elements; chi0(R, omega) is read once per
     // kChi0RqMaxQ q points
     void assemble_dense_q(const TFGrid &g, const std::vector<const double *> &kfs, int w0, int cnt, void *dense,
-                          bool f64, long long nn, bool embed, hipStream_t s);
+                          bool f64, long long nn, DenseLayout lay, hipStream_t s);
     long long ghat_max = 0;
     RpaResult ec(const Dataset &ds, const TFGrid &g);
     // dense chi0(q, omega) block for verification
