@@ -116,8 +116,8 @@ int librpa_amd_mlp_loss_grad(const float *params, const float *X, const float *t
  * memory (code under HIP graph capture, tight retraining loops): the same kernels on
  * device-resident arrays d_params [4801], d_X [n][8], d_t [n] (in) and d_grad [4801], d_loss
  * [1 double] (out), enqueued on stream (a hipStream_t; NULL = the null stream) without
- * synchronising.  The per-sample activations and chunk partial sums live in a static device
- * array of the library (35 MB, held by each GPU it runs on until the process ends), so
+ * synchronising.  The partial sums live in a static device array of the library (10 MB, held
+ * by each GPU it runs on until the process ends), and
  * n <= LIBRPA_AMD_MLP_NOALLOC_MAX; a larger n is an error.  Every call on one GPU shares that
  * array: calls that overlap on one GPU (other streams, other threads) race.  Returns 0 when
  * the work is enqueued, nonzero on error. */

@@ -32,7 +32,7 @@ void launch_chi0_block_norms(const T *chi0s, long long E_tot, int ntau, const lo
 void launch_mlp_forward(const float *params, const float *X, int n, float *y, hipStream_t s);
 
 struct MlpWork {
-    DevBuf acts, part, r2, grad, m, v;
+    DevBuf part, grad, m, v;
 };
 // mean squared error of the MLP on (X, t) and its gradient (layout of the parameter vector);
 // grad and loss are device pointers (loss: one double)
@@ -42,7 +42,7 @@ void mlp_loss_grad(const float *params, const float *X, const float *t, int n, f
 // library (kMlpNoallocScratchBytes per GPU), for n <= kMlpNoallocMax; larger n throws.  Calls that
 // overlap on one GPU share that array and race.
 constexpr int kMlpNoallocMax = 32768;
-constexpr size_t kMlpNoallocScratchBytes = 35176704;  // activations + dy, r2, 64 chunk partials
+constexpr size_t kMlpNoallocScratchBytes = 9836544;  // 512 partial gradients and losses
 void mlp_loss_grad_noalloc(const float *params, const float *X, const float *t, int n, float *grad, double *loss,
                            hipStream_t s);
 // Device address of the static work array on the current device (resolved once per device).

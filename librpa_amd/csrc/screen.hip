@@ -2,14 +2,15 @@
 //
 // MLP, FP32: z1 = x W1 + b1, h1 = silu(z1), z2 = h1 W2 + b2, h2 = silu(z2), y = h2 w3 + b3.
 // Parameter vector: W1[8][64], b1[64], W2[64][64], b2[64], w3[64], b3.
-// Training: full-batch mean squared error; one thread per sample computes the forward pass and
-// the per-sample deltas (dz1, dz2, dy); a second kernel reduces them to the parameter gradient
-// over sample chunks, a third sums the chunks; Adam updates the parameters in place.
+// Training: full-batch mean squared error; one kernel takes tiles of 64 samples from the forward pass
+// to partial parameter gradients, a second sums those; Adam updates the parameters in place.
 #include "screen.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 namespace lra {
 
@@ -17,9 +18,7 @@ namespace {
 constexpr int OW1 = 0, OB1 = MLP_NFEAT * MLP_H, OW2 = OB1 + MLP_H, OB2 = OW2 + MLP_H * MLP_H, OW3 = OB2 + MLP_H,
               OB3 = OW3 + MLP_H;
 static_assert(OB3 + 1 == MLP_NPARAM, "parameter layout");
-constexpr int ACT = 4 * MLP_H;  // per-sample activations: h1, dz1, h2, dz2
-constexpr int NROW = MLP_NFEAT + 1 + MLP_H + 1 + 1 + 1;  // gradient rows: W1, b1, W2, b2, w3, b3
-constexpr int GCHUNKS = 64;
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float sig(float z) { return 1.0f / (1.0f + expf(-z)); }
 
@@ -123,142 +122,253 @@ void launch_mlp_forward(const float *params, const float *X, int n, float *y, hi
     HIP_CHECK(hipGetLastError());
 }
 
-// per sample: forward pass, r = y - t, dy = 2 r / n, dz2 = dy w3 silu'(z2), dz1 = (W2 dz2) silu'(z1);
-// act[s] = [h1 | dz1 | h2 | dz2], dy[s], r2[s] = r^2.  The silu' factors are parked in the dz
-// slots of act (each thread re-reads only what it wrote), so that at most one 64-vector
-// (h1, then dz2) lives in registers.
-__global__ __launch_bounds__(256) void mlp_fwdbwd_kernel(const float *__restrict__ params,
-                                                         const float *__restrict__ X, const float *__restrict__ t,
-                                                         int n, float *__restrict__ act, float *__restrict__ dyo,
-                                                         double *__restrict__ r2) {
-    __shared__ float P[MLP_NPARAM];
-    for (int i = threadIdx.x; i < MLP_NPARAM; i += blockDim.x) P[i] = params[i];
-    __syncthreads();
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    float *a = act + (long long)s * ACT;
-    float x[MLP_NFEAT];
-#pragma unroll
-    for (int i = 0; i < MLP_NFEAT; ++i) x[i] = X[(long long)s * MLP_NFEAT + i];
-    float h1[MLP_H];
-#pragma unroll
-    for (int j = 0; j < MLP_H; ++j) {
-        float z = P[OB1 + j];
-#pragma unroll
-        for (int i = 0; i < MLP_NFEAT; ++i) z += x[i] * P[OW1 + i * MLP_H + j];
-        const float g = sig(z);
-        h1[j] = z * g;
-        a[j] = h1[j];
-        a[MLP_H + j] = g * (1.0f + z * (1.0f - g));  // silu'(z1), scaled below
-    }
-    float y = P[OB3];
-    for (int j = 0; j < MLP_H; ++j) {
-        float z = P[OB2 + j];
-#pragma unroll
-        for (int k = 0; k < MLP_H; ++k) z += h1[k] * P[OW2 + k * MLP_H + j];
-        const float g = sig(z);
-        const float h2 = z * g;
-        a[2 * MLP_H + j] = h2;
-        a[3 * MLP_H + j] = g * (1.0f + z * (1.0f - g));  // silu'(z2), scaled below
-        y += h2 * P[OW3 + j];
-    }
-    const float r = y - t[s];
-    const float dy = 2.0f * r / (float)n;
-    float d2[MLP_H];
-#pragma unroll
-    for (int j = 0; j < MLP_H; ++j) {
-        d2[j] = a[3 * MLP_H + j] * dy * P[OW3 + j];
-        a[3 * MLP_H + j] = d2[j];
-    }
-    for (int k = 0; k < MLP_H; ++k) {
-        float dh = 0;
-#pragma unroll
-        for (int j = 0; j < MLP_H; ++j) dh += d2[j] * P[OW2 + k * MLP_H + j];
-        a[MLP_H + k] *= dh;
-    }
-    dyo[s] = dy;
-    r2[s] = (double)r * (double)r;
+// Loss and gradient in two launches.  The first keeps a tile of 64 samples on chip from the forward
+// pass to its share of every parameter's gradient, all products on the FP32 matrix units: a wave
+// holds 16 samples as the columns of Z1^T, Z2^T and the deltas.  The forward pass takes its terms in
+// the order of the hidden units (h1 and h2 through LDS): z2 and y are then the sums that one thread
+// per sample would form, bit by bit.  In the backward pass the result registers of one product
+// (register r of lane group kq: hidden unit 16 f + 4 kq + r of fragment f) are the next one's B
+// operand with W2's columns taken in that order, and no value crosses a lane.  The products over
+// samples (W1, b1, W2) read h1 and the deltas back from LDS across the four waves; b2 and w3 are
+// summed in registers.  A workgroup takes tiles blockIdx.x, + gridDim.x, ... and writes one
+// partial gradient; the second launch adds the partials in FP64.
+//
+// Bound by the chain of one tile (232 MFMAs a wave, 3 us, and its loads); a thread per sample with
+// activations in memory (two launches over 20 MB of them, 79 workgroups) took 168 us for 20000
+// samples.  Rows of 68 floats keep the lanes of a step on different banks
+// (the forward products' W2 rows 4 st + kq apart, two to a bank).
+constexpr int TS = 64, LDH = MLP_H + 4, LDX = 20;
+
+__device__ __forceinline__ v4f mfma_f32(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// sum over the 16 lanes of a lane group (every lane gets it)
+__device__ __forceinline__ float row_sum(float v) {
+    const auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v += dpp(v, std::integral_constant<int, 0xB1>());   // lane ^ 1
+    v += dpp(v, std::integral_constant<int, 0x4E>());   // lane ^ 2
+    v += dpp(v, std::integral_constant<int, 0x141>());  // mirror of 8 lanes
+    v += dpp(v, std::integral_constant<int, 0x140>());  // mirror of 16 lanes
+    return v;
 }
 
-// part[chunk][param] = sum over the chunk's samples of the per-sample gradient, one gradient row
-// (64 or 1 columns) per blockIdx.x
-__global__ __launch_bounds__(256) void mlp_grad_rows_kernel(const float *__restrict__ X,
-                                                            const float *__restrict__ act,
-                                                            const float *__restrict__ dy, int n, int chunk,
-                                                            float *__restrict__ part) {
-    __shared__ float red[4][MLP_H];
-    const int row = blockIdx.x, ch = blockIdx.y;
-    const int g = threadIdx.x >> 6, j = threadIdx.x & 63;
-    // row -> (A source, B source, output offset, columns)
-    int asrc, bsrc, out, ncol = MLP_H;
-    if (row < MLP_NFEAT) { asrc = row; bsrc = 1; out = OW1 + row * MLP_H; }
-    else if (row == MLP_NFEAT) { asrc = -1; bsrc = 1; out = OB1; }
-    else if (row < MLP_NFEAT + 1 + MLP_H) { asrc = 100 + (row - MLP_NFEAT - 1); bsrc = 3; out = OW2 + (row - MLP_NFEAT - 1) * MLP_H; }
-    else if (row == MLP_NFEAT + 1 + MLP_H) { asrc = -1; bsrc = 3; out = OB2; }
-    else if (row == MLP_NFEAT + 2 + MLP_H) { asrc = -2; bsrc = 2; out = OW3; }
-    else { asrc = -1; bsrc = -2; out = OB3; ncol = 1; }
-    const int s0 = ch * chunk, s1 = min(n, s0 + chunk);
-    float acc = 0;
-    if (j < ncol)
-        for (int s = s0 + g; s < s1; s += 4) {
-            const float *as = act + (long long)s * ACT;
-            const float av = asrc >= 100 ? as[asrc - 100] : asrc >= 0 ? X[(long long)s * MLP_NFEAT + asrc]
-                                                           : asrc == -2 ? dy[s] : 1.0f;
-            const float bv = bsrc == -2 ? dy[s] : as[bsrc * MLP_H + j];
-            acc += av * bv;
+__global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restrict__ params, const float *__restrict__ X,
+                                                            const float *__restrict__ t, int n, int ntile,
+                                                            float *__restrict__ part, double *__restrict__ lossp) {
+    __shared__ __align__(16) float W2s[MLP_H * LDH], H1[TS * LDH], D1[TS * LDH], D2[TS * LDH], Xs[TS * LDX];
+    __shared__ float red[2][4][MLP_H], red3[4];
+    __shared__ double redl[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
+    for (int i = tid; i < MLP_H * MLP_H; i += 256) W2s[(i / MLP_H) * LDH + i % MLP_H] = params[OW2 + i];
+    // columns 8 to 15 of X: the ones of b1, then zeros
+    for (int i = tid; i < TS * 8; i += 256) Xs[(i >> 3) * LDX + 8 + (i & 7)] = (i & 7) == 0 ? 1.0f : 0.0f;
+    float w1[2][4], b1[4][4], b2[4][4], w3[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st) w1[st][m] = params[OW1 + (4 * st + kq) * MLP_H + 16 * m + c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * m + 4 * kq + r;
+            b1[m][r] = params[OB1 + j];
+            b2[m][r] = params[OB2 + j];
+            w3[m][r] = params[OW3 + j];
         }
-    red[g][j] = acc;
+    }
+    float w3k[16];  // w3 in the order of the products over hidden units
+#pragma unroll
+    for (int st = 0; st < 16; ++st) w3k[st] = params[OW3 + 4 * st + kq];
+    const float b3 = params[OB3];
+    v4f g2[4], g1 = {0, 0, 0, 0}, gb2[4], gw3[4];  // W2 rows of this wave, W1 and b1 columns of it, b2, w3
+#pragma unroll
+    for (int m = 0; m < 4; ++m) g2[m] = gb2[m] = gw3[m] = v4f{0, 0, 0, 0};
+    float gb3 = 0;
+    double loss = 0;
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int s = tile * TS + 16 * wave + c;
+        float xb[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            xb[st] = s < n ? X[(long long)s * MLP_NFEAT + 4 * st + kq] : 0.0f;
+            Xs[(16 * wave + c) * LDX + 4 * st + kq] = xb[st];
+        }
+        const float ts = s < n ? t[s] : 0.0f;
+        v4f s1[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            v4f z = {b1[m][0], b1[m][1], b1[m][2], b1[m][3]};
+#pragma unroll
+            for (int st = 0; st < 2; ++st) z = mfma_f32(w1[st][m], xb[st], z);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float g = sig(z[r]);
+                s1[m][r] = g * (1.0f + z[r] * (1.0f - g));
+                z[r] *= g;
+            }
+            *reinterpret_cast<v4f *>(&H1[(16 * wave + c) * LDH + 16 * m + 4 * kq]) = z;
+        }
+        __syncthreads();
+        v4f d[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) d[m] = v4f{b2[m][0], b2[m][1], b2[m][2], b2[m][3]};
+#pragma unroll
+        for (int st = 0; st < 16; ++st) {
+            const float h = H1[(16 * wave + c) * LDH + 4 * st + kq];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) d[m] = mfma_f32(W2s[(4 * st + kq) * LDH + 16 * m + c], h, d[m]);
+        }
+        v4f h2[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float z = d[m][r], g = sig(z);
+                h2[m][r] = z * g;
+                d[m][r] = g * (1.0f + z * (1.0f - g));
+            }
+            *reinterpret_cast<v4f *>(&D1[(16 * wave + c) * LDH + 16 * m + 4 * kq]) = h2[m];
+        }
+        __syncthreads();
+        v4f y = {b3, b3, b3, b3};  // the same in all four rows
+#pragma unroll
+        for (int st = 0; st < 16; ++st) y = mfma_f32(w3k[st], D1[(16 * wave + c) * LDH + 4 * st + kq], y);
+        const float res = s < n ? y[0] - ts : 0.0f;
+        const float dy = 2.0f * res / (float)n;
+        if (kq == 0) {
+            gb3 += dy;
+            loss += (double)res * (double)res;
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                gw3[m][r] += dy * h2[m][r];
+                d[m][r] = s < n ? d[m][r] * dy * w3[m][r] : 0.0f;
+                gb2[m][r] += d[m][r];
+            }
+            *reinterpret_cast<v4f *>(&D2[(16 * wave + c) * LDH + 16 * m + 4 * kq]) = d[m];
+        }
+        // dz1 = (W2 dz2) silu'(z1)
+        v4f e[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) e[m] = v4f{0, 0, 0, 0};
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const v4f w = *reinterpret_cast<const v4f *>(&W2s[(16 * m + c) * LDH + 16 * f + 4 * kq]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e[m] = mfma_f32(w[r], d[f][r], e[m]);
+            }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) e[m][r] *= s1[m][r];
+            *reinterpret_cast<v4f *>(&D1[(16 * wave + c) * LDH + 16 * m + 4 * kq]) = e[m];
+        }
+        __syncthreads();
+        // products over the tile's samples, step (q, u) over samples 16 q + 4 kq + u
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = 16 * q + 4 * kq + u;
+                const float a = H1[k * LDH + 16 * wave + c];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) g2[m] = mfma_f32(a, D2[k * LDH + 16 * m + c], g2[m]);
+                g1 = mfma_f32(Xs[k * LDX + c], D1[k * LDH + 16 * wave + c], g1);
+            }
+        __syncthreads();
+    }
+    float *out = part + (long long)blockIdx.x * MLP_NPARAM;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int i = 4 * kq + r;  // rows 0 to 7 of W1, then b1
+        if (i <= MLP_NFEAT) out[(i < MLP_NFEAT ? OW1 + i * MLP_H : OB1) + 16 * wave + c] = g1[r];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            out[OW2 + (16 * wave + 4 * kq + r) * MLP_H + 16 * m + c] = g2[m][r];
+            const float x = row_sum(gb2[m][r]), z = row_sum(gw3[m][r]);
+            if (c == 0) {
+                red[0][wave][16 * m + 4 * kq + r] = x;
+                red[1][wave][16 * m + 4 * kq + r] = z;
+            }
+        }
+    }
+    gb3 = row_sum(gb3);
+    for (int o = 8; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
+    if (lane == 0) {
+        red3[wave] = gb3;
+        redl[wave] = loss;
+    }
     __syncthreads();
-    if (g == 0 && j < ncol) part[(long long)ch * MLP_NPARAM + out + j] = red[0][j] + red[1][j] + red[2][j] + red[3][j];
+    if (tid < 2 * MLP_H) {
+        const int w = tid / MLP_H, j = tid % MLP_H;
+        out[(w ? OW3 : OB2) + j] = red[w][0][j] + red[w][1][j] + red[w][2][j] + red[w][3][j];
+    }
+    if (tid == 0) {
+        out[OB3] = red3[0] + red3[1] + red3[2] + red3[3];
+        lossp[blockIdx.x] = redl[0] + redl[1] + redl[2] + redl[3];
+    }
 }
 
-__global__ void mlp_grad_sum_kernel(const float *__restrict__ part, int nch, float *__restrict__ grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= MLP_NPARAM) return;
-    float s = 0;
-    for (int c = 0; c < nch; ++c) s += part[(long long)c * MLP_NPARAM + p];
-    grad[p] = s;
-}
-
-__global__ __launch_bounds__(1024) void mean_kernel(const double *__restrict__ v, int n, double *out) {
-    __shared__ double red[16];
+// grad = sum of the partials, 64 parameters a workgroup, wave w the partials w, w + 16, ...; the last
+// workgroup: the mean loss
+__global__ __launch_bounds__(1024) void mlp_grad_sum_kernel(const float *__restrict__ part,
+                                                            const double *__restrict__ lossp, int npart, int n,
+                                                            float *__restrict__ grad, double *__restrict__ loss) {
+    __shared__ double red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double s = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += v[i];
-    const double tot = block_sum(s, red);
-    if (threadIdx.x == 0) out[0] = tot / (double)n;
+    if (blockIdx.x == gridDim.x - 1) {
+        for (int i = threadIdx.x; i < npart; i += 1024) s += lossp[i];
+        const double v = block_sum(s, &red[0][0]);
+        if (threadIdx.x == 0) *loss = v / (double)n;
+        return;
+    }
+    const int p = blockIdx.x * 64 + lane;
+    if (p < MLP_NPARAM) {
+#pragma unroll 8
+        for (int i = wave; i < npart; i += 16) s += part[(long long)i * MLP_NPARAM + p];
+    }
+    red[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && p < MLP_NPARAM) {
+        s = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) s += red[w][lane];
+        grad[p] = (float)s;
+    }
 }
 
 namespace {
-// The loss and gradient launches on caller-provided work memory: act [n][ACT] followed by dy [n],
-// r2 [n], part [GCHUNKS][MLP_NPARAM].  Every entry the later launches read is written by an earlier
-// one in the same call, so the work memory needs no clearing.
+// at most two workgroups (of 78 KB of LDS) on each of the 256 CUs: one round, one partial each
+constexpr int kMlpParts = 512;
+constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
+constexpr size_t kPartBytes = align256(sizeof(float) * (size_t)kMlpParts * MLP_NPARAM);
+
+// The two launches on caller-provided work memory of kMlpNoallocScratchBytes: partial gradients, then
+// partial losses.  Every entry the second launch reads is written by the first, so the work memory
+// needs no clearing.
 void loss_grad_launches(const float *params, const float *X, const float *t, int n, float *grad, double *loss,
-                        float *act, double *r2, float *part, hipStream_t s) {
-    float *dy = act + (size_t)n * ACT;
-    hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, params, X, t, n, act, dy, r2);
+                        char *work, hipStream_t s) {
+    float *part = reinterpret_cast<float *>(work);
+    double *lossp = reinterpret_cast<double *>(work + kPartBytes);
+    const int ntile = ceil_div(n, TS), npart = std::min(ntile, kMlpParts);
+    hipLaunchKernelGGL(mlp_tile_grad_kernel, dim3(npart), dim3(256), 0, s, params, X, t, n, ntile, part, lossp);
     HIP_CHECK(hipGetLastError());
-    const int chunk = ceil_div(n, GCHUNKS);
-    const int nch = ceil_div(n, chunk);
-    hipLaunchKernelGGL(mlp_grad_rows_kernel, dim3(NROW, nch), dim3(256), 0, s, X, act, dy, n, chunk, part);
-    HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3(ceil_div(MLP_NPARAM, 256)), dim3(256), 0, s, part, nch, grad);
-    HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(mean_kernel, dim3(1), dim3(1024), 0, s, r2, n, loss);
+    hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3(ceil_div(MLP_NPARAM, 64) + 1), dim3(1024), 0, s, part, lossp, npart, n,
+                       grad, loss);
     HIP_CHECK(hipGetLastError());
 }
-
-constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-constexpr size_t kActBytes = align256(sizeof(float) * (size_t)kMlpNoallocMax * (ACT + 1));
-constexpr size_t kR2Bytes = align256(sizeof(double) * (size_t)kMlpNoallocMax);
-constexpr size_t kPartBytes = align256(sizeof(float) * (size_t)GCHUNKS * MLP_NPARAM);
-constexpr size_t kScratchBytes = kActBytes + kR2Bytes + kPartBytes;
-static_assert(kScratchBytes == kMlpNoallocScratchBytes, "scratch size");
+static_assert(kPartBytes + align256(sizeof(double) * kMlpParts) == kMlpNoallocScratchBytes, "scratch size");
 }  // namespace
 
-// Work memory of the allocation-free loss and gradient (about 35 MB): each GPU the library runs
+// Work memory of the allocation-free loss and gradient (about 10 MB): each GPU the library runs
 // on holds its own copy from the code object's load until the process ends.  Host code reaches it
 // only through the per-device address from hipGetSymbolAddress below, never through this name.
-static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
+static __device__ __align__(256) double scratch[kMlpNoallocScratchBytes / sizeof(double)];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -286,19 +396,14 @@ void mlp_loss_grad_noalloc(const float *params, const float *X, const float *t, 
         LRA_THROW("allocation-free MLP loss/gradient: " + std::to_string(n) + " samples exceed the maximum of " +
                   std::to_string(kMlpNoallocMax));
     if (!params || !X || !t || !grad || !loss) LRA_THROW("allocation-free MLP loss/gradient: null device pointer");
-    char *base = mlp_noalloc_setup();
-    loss_grad_launches(params, X, t, n, grad, loss, reinterpret_cast<float *>(base),
-                       reinterpret_cast<double *>(base + kActBytes), reinterpret_cast<float *>(base + kActBytes + kR2Bytes),
-                       s);
+    loss_grad_launches(params, X, t, n, grad, loss, mlp_noalloc_setup(), s);
 }
 
 void mlp_loss_grad(const float *params, const float *X, const float *t, int n, float *grad, double *loss,
                    MlpWork &w, hipStream_t s) {
     if (n <= 0) LRA_THROW("mlp: no samples");
-    w.acts.reserve(sizeof(float) * ((size_t)n * ACT + n));
-    w.r2.reserve(sizeof(double) * n);
-    w.part.reserve(sizeof(float) * (size_t)GCHUNKS * MLP_NPARAM);
-    loss_grad_launches(params, X, t, n, grad, loss, w.acts.as<float>(), w.r2.as<double>(), w.part.as<float>(), s);
+    w.part.reserve(kMlpNoallocScratchBytes);
+    loss_grad_launches(params, X, t, n, grad, loss, w.part.as<char>(), s);
 }
 
 __global__ void adam_kernel(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
