@@ -124,19 +124,18 @@ void launch_mlp_forward(const float *params, const float *X, int n, float *y, hi
 
 // Loss and gradient in two launches.  The first keeps a tile of 64 samples on chip from the forward
 // pass to its share of every parameter's gradient, all products on the FP32 matrix units: a wave
-// holds 16 samples as the columns of Z1^T, Z2^T and the deltas.  The forward pass takes its terms in
-// the order of the hidden units (h1 and h2 through LDS): z2 and y are then the sums that one thread
-// per sample would form, bit by bit.  In the backward pass the result registers of one product
-// (register r of lane group kq: hidden unit 16 f + 4 kq + r of fragment f) are the next one's B
-// operand with W2's columns taken in that order, and no value crosses a lane.  The products over
-// samples (W1, b1, W2) read h1 and the deltas back from LDS across the four waves; b2 and w3 are
-// summed in registers.  A workgroup takes tiles blockIdx.x, + gridDim.x, ... and writes one
-// partial gradient; the second launch adds the partials in FP64.
+// holds 16 samples as the columns of Z1^T, Z2^T and the deltas, and passes them from product to
+// product through its own rows in LDS.  The terms are taken in the order of the hidden units: z2 and
+// y are the sums that one thread per sample would form, bit by bit.  The products over samples (W1,
+// b1, W2) read h1 and the deltas of all four waves; b2 and w3 are summed in registers.  A workgroup
+// takes tiles blockIdx.x, + gridDim.x, ... and writes one partial gradient; the second launch adds the
+// partials in FP64.
 //
-// Bound by the chain of one tile (232 MFMAs a wave, 3 us, and its loads); a thread per sample with
-// activations in memory (two launches over 20 MB of them, 79 workgroups) took 168 us for 20000
-// samples.  Rows of 68 floats keep the lanes of a step on different banks
-// (the forward products' W2 rows 4 st + kq apart, two to a bank).
+// Bound by the chain of one tile: 232 MFMAs a wave are 3 us, the rest is the latency of the first
+// loads and of the code itself, so the products are loops.  A call on 20000 samples takes 25 us;
+// with all products unrolled and registers for one workgroup a CU 31, with a thread per sample and
+// activations in memory (two launches over 20 MB of them) 168.  Rows of 68 floats keep the lanes of a step
+// on different banks (W2 rows in the forward product: two to a bank).
 constexpr int TS = 64, LDH = MLP_H + 4, LDX = 20;
 
 __device__ __forceinline__ v4f mfma_f32(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -153,14 +152,16 @@ __device__ __forceinline__ float row_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restrict__ params, const float *__restrict__ X,
+__global__ __launch_bounds__(256, 2) void mlp_tile_grad_kernel(const float *__restrict__ params, const float *__restrict__ X,
                                                             const float *__restrict__ t, int n, int ntile,
                                                             float *__restrict__ part, double *__restrict__ lossp) {
     __shared__ __align__(16) float W2s[MLP_H * LDH], H1[TS * LDH], D1[TS * LDH], D2[TS * LDH], Xs[TS * LDX];
+    __shared__ float w3s[MLP_H];
     __shared__ float red[2][4][MLP_H], red3[4];
     __shared__ double redl[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
     for (int i = tid; i < MLP_H * MLP_H; i += 256) W2s[(i / MLP_H) * LDH + i % MLP_H] = params[OW2 + i];
+    if (tid < MLP_H) w3s[tid] = params[OW3 + tid];
     // columns 8 to 15 of X: the ones of b1, then zeros
     for (int i = tid; i < TS * 8; i += 256) Xs[(i >> 3) * LDX + 8 + (i & 7)] = (i & 7) == 0 ? 1.0f : 0.0f;
     float w1[2][4], b1[4][4], b2[4][4], w3[4][4];
@@ -176,9 +177,6 @@ __global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restr
             w3[m][r] = params[OW3 + j];
         }
     }
-    float w3k[16];  // w3 in the order of the products over hidden units
-#pragma unroll
-    for (int st = 0; st < 16; ++st) w3k[st] = params[OW3 + 4 * st + kq];
     const float b3 = params[OB3];
     v4f g2[4], g1 = {0, 0, 0, 0}, gb2[4], gw3[4];  // W2 rows of this wave, W1 and b1 columns of it, b2, w3
 #pragma unroll
@@ -212,7 +210,7 @@ __global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restr
         v4f d[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) d[m] = v4f{b2[m][0], b2[m][1], b2[m][2], b2[m][3]};
-#pragma unroll
+#pragma unroll 4
         for (int st = 0; st < 16; ++st) {
             const float h = H1[(16 * wave + c) * LDH + 4 * st + kq];
 #pragma unroll
@@ -231,8 +229,8 @@ __global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restr
         }
         __syncthreads();
         v4f y = {b3, b3, b3, b3};  // the same in all four rows
-#pragma unroll
-        for (int st = 0; st < 16; ++st) y = mfma_f32(w3k[st], D1[(16 * wave + c) * LDH + 4 * st + kq], y);
+#pragma unroll 4
+        for (int st = 0; st < 16; ++st) y = mfma_f32(w3s[4 * st + kq], D1[(16 * wave + c) * LDH + 4 * st + kq], y);
         const float res = s < n ? y[0] - ts : 0.0f;
         const float dy = 2.0f * res / (float)n;
         if (kq == 0) {
@@ -249,18 +247,17 @@ __global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restr
             }
             *reinterpret_cast<v4f *>(&D2[(16 * wave + c) * LDH + 16 * m + 4 * kq]) = d[m];
         }
+        __syncthreads();
         // dz1 = (W2 dz2) silu'(z1)
         v4f e[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) e[m] = v4f{0, 0, 0, 0};
+#pragma unroll 4
+        for (int st = 0; st < 16; ++st) {
+            const float x = D2[(16 * wave + c) * LDH + 4 * st + kq];
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const v4f w = *reinterpret_cast<const v4f *>(&W2s[(16 * m + c) * LDH + 16 * f + 4 * kq]);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) e[m] = mfma_f32(w[r], d[f][r], e[m]);
-            }
+            for (int m = 0; m < 4; ++m) e[m] = mfma_f32(W2s[(16 * m + c) * LDH + 4 * st + kq], x, e[m]);
+        }
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
 #pragma unroll
@@ -269,7 +266,7 @@ __global__ __launch_bounds__(256) void mlp_tile_grad_kernel(const float *__restr
         }
         __syncthreads();
         // products over the tile's samples, step (q, u) over samples 16 q + 4 kq + u
-#pragma unroll
+#pragma unroll 1
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
