@@ -416,11 +416,11 @@ template <int MODE>
 static void launch_mode(const GemmBatch &b, const void *A, const void *B, void *C, double alpha, double beta,
                         hipStream_t s) {
     if (b.atomic || !b.coltab.empty()) {
-        // column-table / atomic batches: plain A and B, 64x64 or 128x128 tiles
-        if (b.trans_a || b.trans_b || (b.cfg != T128x128 && b.cfg != T64x64))
-            LRA_THROW("column-table GEMM: plain A and B, 64x64 or 128x128 tiles");
-        if (b.cfg == T64x64) launch_one<MODE, 0, false, false, 2>(b, A, B, C, alpha, beta, s);
-        else launch_one<MODE, 1, false, false, 2>(b, A, B, C, alpha, beta, s);
+        // column-table / atomic batches: plain A and B^T, 64x64 or 128x128 tiles
+        if (b.trans_a || !b.trans_b || (b.cfg != T128x128 && b.cfg != T64x64))
+            LRA_THROW("column-table GEMM: plain A and transposed B, 64x64 or 128x128 tiles");
+        if (b.cfg == T64x64) launch_one<MODE, 0, false, true, 2>(b, A, B, C, alpha, beta, s);
+        else launch_one<MODE, 1, false, true, 2>(b, A, B, C, alpha, beta, s);
         return;
     }
     if (b.two_segments) {

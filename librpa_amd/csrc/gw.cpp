@@ -17,15 +17,18 @@
 // W = S_c eps^{-1} S_c - S_c S_c, the Schur complement of [[eps, S_c], [S_c, S_c S_c]].
 //
 // Self-energy (RI::GW::cal_Sigmas, thirdparty/LibRI/include/RI/physics/GW.hpp:102-122,
-// called from G0W0::build_spacetime, src/core/gw.cpp:217-875), per tau, spin and sign:
-//   U_J(S)[(X,x)][(j,nu)] = sum_{(L,Rb) in N(J)} G_XL(S+Rb) C^J(L,Rb)           (GEMM per (J,S))
-//   T_I[(n,mu,k)][(R,J,j)] = sum_nu W_IJ(R)(mu,nu) U_J(R-Ra_n)[(K_n,k)][(j,nu)]    (rows gathered)
-//   label a0b0_a2b2: Sigma_IJ(R)(i,j) = sum_(n,mu,k) C^I(n)(mu,i,k) T_I[(n,mu,k)][(R,J,j)]
-//   label a0b0_a1b2: Sigma_KJ(R-Ra)(k,j) += sum_(mu,i) C^I(n)(mu,i,k) T_I[(on-site,mu,i)][(R,J,j)]
-//   label a0b0_a1b1: Y_I[(mu,i)][(S,L,l)] = sum_{J,R} W_IJ(R) G_IJ(R) C^J(L,S-R)  (two GEMMs per (J,R))
-//                    Sigma_KL(S-Ra)(k,l) += sum_(mu,i) C^I(n)(mu,i,k) Y_I[(mu,i)][(S,L,l)]
+// called from G0W0::build_spacetime, src/core/gw.cpp:217-875), per tau and spin, both signs at once:
+//   U_J(S)[(X,x)][j][nu] = sum_{(L,Rb) in N(J)} G_XL(S+Rb) C^J(L,Rb)           (GEMM per (J,S,sign))
+//   CW_IJ(R)[c][i][nu] = sum_mu C^I[(c,i)][mu] W_IJ(R)(mu,nu), c = (n,k) in N(I)  (GEMM per (I,J,R))
+//   label a0b0_a2b2: Sigma_IJ(R)(i,j) = sum_(c,nu) CW_IJ(R)[c][i][nu] U_J(R-Ra_c)[c][j][nu]
+//   label a0b0_a1b2: Sigma_KJ(R-Ra)(k,j) += sum_(i,nu) CW_IJ(R)[c][i][nu] U_J(R)[(I,i)][j][nu]
+//   label a0b0_a1b1: Y_I[(S,L,l)][i][mu] = sum_{J,R,j} G_IJ(R)(i,j) CW_JI(-R)[(L,S-R,l)][j][mu]
+//                    Sigma_KL(S-Ra)(k,l) += sum_(i,mu) C^I[c][i][mu] Y_I[(S,L,l)][i][mu]
 //   label a0b0_a2b1: the transpose of a0b0_a1b2, Sigma_XY(R) += [a1b2]_YX(-R)^T.
-// Outputs indexed by a cell difference go through an extended (2p-1)^3 cell grid with
+// CW holds neither sign nor spin and serves three labels (the third by W_IJ(R) = W_JI(-R)^T), where W
+// against U and against G C^J would be two products of its size per sign: 1 + 2 * 5/4.6 of its flops
+// a tau point, not 2 + 2 * 2 (n_aux = 4.6 n_ao).  It takes the room that T = W U would.
+// Y's outputs are indexed by a cell difference: they go through an extended (2p-1)^3 cell grid with
 // atomic accumulation and are folded back to the BvK cell afterwards.  Sigma(R, i w) =
 // sum_tau 0.5 (S+ + S-) gamma_c + i 0.5 (S+ - S-) gamma_s (gw.cpp:681-797).
 #include "gw.h"
@@ -49,19 +52,6 @@ namespace lra {
 namespace {
 double now_s() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
-}
-inline int bvk_mod(int v, int n) { return (((v % n) + 3 * n / 2) % n) - n / 2; }
-
-template <class T>
-DevBuf upload_as(const std::vector<double> &v, hipStream_t s) {
-    if constexpr (std::is_same<T, double>::value) {
-        return upload(v, s);
-    } else {
-        std::vector<T> f(v.begin(), v.end());
-        DevBuf b = upload(f, s);
-        HIP_CHECK(hipStreamSynchronize(s));
-        return b;
-    }
 }
 }  // namespace
 
@@ -87,102 +77,19 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
     const auto &abf = R0.abf;
     const auto &cells = R0.cells;
     const hipStream_t st = R0.stream;
-    const int cell0 = R0.cell_index(0, 0, 0);
-
-    // ---- folded Cs, as in the chi0 plan ----
-    std::map<std::tuple<int, int, int>, std::vector<double>> folded;
-    for (const auto &kv : ds.cs) {
-        const int I = std::get<0>(kv.first), K = std::get<1>(kv.first);
-        const int rr = R0.fold_index(std::get<2>(kv.first), std::get<3>(kv.first), std::get<4>(kv.first));
-        auto &dst = folded[{I, K, rr}];
-        if (dst.empty()) dst = kv.second;
-        else for (size_t i = 0; i < dst.size(); ++i) dst[i] += kv.second[i];
-    }
-    auto cval = [&](int I, int K, int rr, int mu, int i, int k) -> double {
-        auto it = folded.find({I, K, rr});
-        if (it == folded.end()) return 0.0;
-        return it->second[((size_t)i * nb[K] + k) * na[I] + mu];
-    };
-    nbrs = R0.nbrs;
-    onsite.assign(natom, -1);
-    for (int I = 0; I < natom; ++I) {
-        for (size_t n = 0; n < nbrs[I].size(); ++n)
-            if (nbrs[I][n].K == I && nbrs[I][n].r == cell0) onsite[I] = (int)n;
-        if (onsite[I] < 0) { onsite[I] = (int)nbrs[I].size(); nbrs[I].push_back({I, cell0}); }
-    }
-    loff.assign(natom, {});
-    lsum.assign(natom, 0);
-    for (int I = 0; I < natom; ++I) {
-        long long l = 0;
-        for (const auto &n : nbrs[I]) { loff[I].push_back(l); l += nb[n.K]; }
-        lsum[I] = l;
-    }
-
-    // ---- packed Cs ----
-    {
-        cd_off.assign(natom + 1, 0);
-        cb_off.assign(natom + 1, 0);
-        ca_off.assign(natom + 1, 0);
-        for (int I = 0; I < natom; ++I) {
-            cd_off[I + 1] = cd_off[I] + (long long)nb[I] * na[I] * lsum[I];
-            cb_off[I + 1] = cb_off[I] + lsum[I] * na[I] * nb[I];
-            ca_off[I + 1] = ca_off[I] + (long long)nb[I] * na[I] * R0.lsum[I];
-        }
-        std::vector<double> cd(cd_off[natom]), cb(cb_off[natom]), ca(ca_off[natom]);
-        for (int I = 0; I < natom; ++I) {
-            const int ni = nb[I], nm = na[I];
-            const long long kd = (long long)nm * lsum[I];
-            for (size_t n = 0; n < nbrs[I].size(); ++n) {
-                const int K = nbrs[I][n].K, rr = nbrs[I][n].r;
-                for (int mu = 0; mu < nm; ++mu)
-                    for (int i = 0; i < ni; ++i)
-                        for (int k = 0; k < nb[K]; ++k) {
-                            const double v = cval(I, K, rr, mu, i, k);
-                            // CD_I[i][(n, mu, k)]
-                            cd[cd_off[I] + (size_t)i * kd + (size_t)nm * loff[I][n] + (size_t)mu * nb[K] + k] = v;
-                            // CB_I[(n, k)][(mu, i)]
-                            cb[cb_off[I] + (size_t)(loff[I][n] + k) * nm * ni + (size_t)mu * ni + i] = v;
-                        }
-            }
-            // CA_I[i][(mu, (n, k))] over the chi0 neighbour list of I (I in the role of J)
-            const long long ls = R0.lsum[I];
-            for (size_t n = 0; n < R0.nbrs[I].size(); ++n) {
-                const int K = R0.nbrs[I][n].K, rr = R0.nbrs[I][n].r;
-                for (int mu = 0; mu < nm; ++mu)
-                    for (int i = 0; i < ni; ++i)
-                        for (int k = 0; k < nb[K]; ++k)
-                            ca[ca_off[I] + (size_t)i * nm * ls + (size_t)mu * ls + R0.loff[I][n] + k] =
-                                cval(I, K, rr, mu, i, k);
-            }
-        }
-        if (prec == Prec::F64) {
-            d_CD = upload_as<double>(cd, st);
-            d_CB = upload_as<double>(cb, st);
-            d_CA = upload_as<double>(ca, st);
-        } else {
-            d_CD = upload_as<float>(cd, st);
-            d_CB = upload_as<float>(cb, st);
-            d_CA = upload_as<float>(ca, st);
-        }
-    }
-
     // ---- extended cell grid ----
     const int *p = R0.period;
     for (int a = 0; a < 3; ++a) E[a] = 2 * p[a] - 1;
     NE = E[0] * E[1] * E[2];
     c0 = linr(p[0] - 1, p[1] - 1, p[2] - 1);
-    ext_fold.assign(NE, 0);
-    ext_foldneg.assign(NE, 0);
+    std::vector<int> fold(NE), neg(nR);
     for (int x = 0; x < E[0]; ++x)
         for (int y = 0; y < E[1]; ++y)
-            for (int z = 0; z < E[2]; ++z) {
-                const int e = (x * E[1] + y) * E[2] + z;
-                const int dx = x - (p[0] - 1), dy = y - (p[1] - 1), dz = z - (p[2] - 1);
-                ext_fold[e] = R0.fold_index(dx, dy, dz);
-                ext_foldneg[e] = R0.fold_index(-dx, -dy, -dz);
-            }
-    d_fold = upload(ext_fold, st);
-    d_foldneg = upload(ext_foldneg, st);
+            for (int z = 0; z < E[2]; ++z)
+                fold[(x * E[1] + y) * E[2] + z] = R0.fold_index(x - (p[0] - 1), y - (p[1] - 1), z - (p[2] - 1));
+    for (int rr = 0; rr < nR; ++rr) neg[rr] = R0.fold_index(-cells[rr][0], -cells[rr][1], -cells[rr][2]);
+    d_fold = upload(fold, st);
+    d_neg = upload(neg, st);
     std::vector<long long> ext_cols(LD);
     for (int rr = 0; rr < nR; ++rr)
         for (int c = 0; c < NAO; ++c)
@@ -192,224 +99,214 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
 
-    // ---- U_J(S) for all J, S (resident) and the gathered G panels by chunks of J ----
+    // ---- U_J(S) for all J, S and signs (resident) and the gathered G panels by chunks of J ----
     u_off.assign((size_t)natom * nR + 1, 0);
     for (int J = 0; J < natom; ++J)
         for (int S = 0; S < nR; ++S)
             u_off[(size_t)J * nR + S + 1] = u_off[(size_t)J * nR + S] + (long long)NAO * nb[J] * na[J];
     u_elems = u_off[(size_t)natom * nR];
     const long long gpm_r = (long long)NAO * 2 * NAO;
+    max_ghat = 0;
     {
         const double budget = std::min(24e9, 0.08 * (double)free_b);
         int j = 0;
         while (j < natom) {
             UChunk c;
-            c.j0 = j;
-            long long g = 0;
-            int jj = j;
-            while (jj < natom) {
-                const long long g1 = (long long)nR * NAO * R0.lsum[jj];
-                if (jj > j && (double)(g + g1) * ts > budget) break;
-                g += g1;
-                ++jj;
-            }
-            c.j1 = jj;
-            c.ghat_elems = g;
-            long long go = 0;
-            for (int J = c.j0; J < c.j1; ++J)
-                for (int S = 0; S < nR; ++S) {
-                    c.ghat_off.push_back(go);
-                    go += (long long)NAO * R0.lsum[J];
-                }
-            for (int sg = 0; sg < 2; ++sg) {
-                for (int J = c.j0; J < c.j1; ++J)
-                    for (int S = 0; S < nR; ++S) {
+            const int j0 = j;
+            for (; j < natom; ++j) {
+                const long long g1 = (long long)nR * 2 * NAO * R0.lsum[j];
+                if (j > j0 && (double)(c.ghat_elems + g1) * ts > budget) break;
+                const long long ls = R0.lsum[j];
+                for (int S = 0; S < nR; ++S)
+                    for (int sg = 0; sg < 2; ++sg) {
                         GatherJob gj;
-                        gj.dst_off = c.ghat_off[(size_t)(J - c.j0) * nR + S];
-                        gj.ncol = (int)R0.lsum[J];
-                        gj.col_off = (int)c.colsrc[sg].size();
-                        for (const auto &n : R0.nbrs[J]) {
+                        gj.dst_off = c.ghat_elems;
+                        gj.ncol = (int)ls;
+                        gj.col_off = (int)c.colsrc.size();
+                        for (const auto &n : R0.nbrs[j]) {
                             const auto &R2 = cells[n.r];
                             const auto &Sv = cells[S];
                             const int rr = R0.fold_index(Sv[0] + R2[0], Sv[1] + R2[1], Sv[2] + R2[2]);
                             for (int l = 0; l < nb[n.K]; ++l)
-                                c.colsrc[sg].push_back(rr * gpm_r + 2 * ao[n.K] + (long long)sg * nb[n.K] + l);
+                                c.colsrc.push_back(rr * gpm_r + 2 * ao[n.K] + (long long)sg * nb[n.K] + l);
                         }
                         c.max_gcol = std::max(c.max_gcol, gj.ncol);
-                        c.jobs[sg].push_back(gj);
+                        c.jobs.push_back(gj);
+                        // K = 0 (an atom without Cs) writes zeros
+                        c.ub.add(make_prob(NAO, nb[j] * na[j], (int)ls, c.ghat_elems, (int)ls, R0.cwb_off[j],
+                                           nb[j] * na[j], sg * u_elems + u_off[(size_t)j * nR + S], nb[j] * na[j]));
+                        c.ghat_elems += (long long)NAO * ls;
                     }
-                c.d_jobs[sg] = upload(c.jobs[sg], st);
-                c.d_colsrc[sg] = upload(c.colsrc[sg], st);
             }
-            for (int J = c.j0; J < c.j1; ++J)
-                for (int S = 0; S < nR; ++S) {
-                    if (R0.lsum[J] == 0) continue;
-                    c.ub.add(make_prob(NAO, nb[J] * na[J], (int)R0.lsum[J], c.ghat_off[(size_t)(J - c.j0) * nR + S],
-                                       (int)R0.lsum[J], R0.cwb_off[J], nb[J] * na[J], u_off[(size_t)J * nR + S],
-                                       nb[J] * na[J]));
-                }
+            c.d_jobs = upload(c.jobs, st);
+            c.d_colsrc = upload(c.colsrc, st);
             // default tiles: the autotuner's choices on the 64-atom, 8-k cell (FP64)
             c.ub.finalize(prec == Prec::F64 ? T128x64w8 : big_tile(prec), st);
             flops_sigma += c.ub.flops;
+            max_ghat = std::max(max_ghat, c.ghat_elems);
             uchunks.push_back(std::move(c));
-            j = jj;
         }
     }
 
-    // ---- Y (partner-partner intermediate), GC, A1 / A2 / A3a ----
+    // ---- Y and its contraction ----
     y_off.assign(natom + 1, 0);
     for (int I = 0; I < natom; ++I) y_off[I + 1] = y_off[I] + (long long)na[I] * nb[I] * LD;
     y_elems = y_off[natom];
-    gc_elems = 0;
-    for (int J = 0; J < natom; ++J) gc_elems = std::max(gc_elems, (long long)na[J] * NAO * R0.lsum[J]);
-    a1.clear();
-    a2.clear();
-    a1.resize((size_t)natom * nR);
-    a2.resize((size_t)natom * nR);
-    for (int J = 0; J < natom; ++J) {
-        const long long ls = R0.lsum[J];
-        if (ls == 0) continue;
-        for (int rr = 0; rr < nR; ++rr) {
-            GemmBatch &b1 = a1[(size_t)J * nR + rr];
-            GemmBatch &b2 = a2[(size_t)J * nR + rr];
-            for (int I = 0; I < natom; ++I) {
-                // GC_I[nu][i][c] = sum_j G_IJ(R)(i, j) CA_J[j][(nu, c)]
-                GemmProb q1 = make_prob(nb[I], na[J] * (int)ls, nb[J], rr * gpm_r + ao[I] * 2LL * NAO + 2 * ao[J],
-                                        2 * NAO, ca_off[J], na[J] * (int)ls, (long long)na[J] * ls * ao[I], (int)ls);
-                q1.ncb = (int)ls;
-                q1.cbs = (long long)nb[I] * ls;
-                b1.add(q1);
-                // Y_I[(mu, i)][cols] += sum_nu W_IJ(R)(mu, nu) GC_I[nu][(i, c)]
-                GemmProb q2 = make_prob(na[I], nb[I] * (int)ls, na[J], (long long)rr * NABF * NABF + abf[I] * NABF + abf[J],
-                                        NABF, (long long)na[J] * ls * ao[I], nb[I] * (int)ls, y_off[I],
-                                        (int)(nb[I] * LD));
-                q2.ncb = (int)ls;
-                q2.cbs = LD;
-                q2.ct_off = 0;
-                b2.add(q2);
-            }
-            // column map of the (L, Rb, l) index of J into the (S = R + Rb, L, l) index
-            const auto &Rv = cells[rr];
-            for (size_t n = 0; n < R0.nbrs[J].size(); ++n) {
-                const auto &R2 = cells[R0.nbrs[J][n].r];
-                const int S = R0.fold_index(Rv[0] + R2[0], Rv[1] + R2[1], Rv[2] + R2[2]);
-                const int L = R0.nbrs[J][n].K;
-                for (int l = 0; l < nb[L]; ++l) b2.coltab.push_back((long long)S * NAO + ao[L] + l);
-            }
-            b1.finalize(prec == Prec::F64 ? T16x256 : T32x128, st);
-            b2.finalize(big_tile(prec), st);
-            flops_sigma += b1.flops + b2.flops;
-        }
-    }
-    auto add_a3 = [&](GemmBatch &b, int I, long long b_off) {
-        GemmProb q = make_prob(0, (int)LD, na[I] * nb[I], 0, 0, b_off, (int)LD, 0, 0);
-        q.rt_off = (int)(b.rowtab.size() / 2);
+    a3 = GemmBatch();
+    a3.atomic = true;
+    a3.trans_b = true;
+    a3.coltab = ext_cols;
+    for (int I = 0; I < natom; ++I) {
+        if (R0.lsum[I] == 0) continue;
+        GemmProb q = make_prob((int)R0.lsum[I], (int)LD, na[I] * nb[I], 0, 0, y_off[I], na[I] * nb[I], 0, 0);
+        q.rt_off = (int)(a3.rowtab.size() / 2);
         q.ct_off = 0;
-        int m = 0;
-        for (size_t n = 0; n < nbrs[I].size(); ++n) {
-            const int K = nbrs[I][n].K;
-            const auto &Ra = cells[nbrs[I][n].r];
+        for (size_t n = 0; n < R0.nbrs[I].size(); ++n) {
+            const int K = R0.nbrs[I][n].K;
+            const auto &Ra = cells[R0.nbrs[I][n].r];
             const long long lr = linr(Ra[0], Ra[1], Ra[2]);
             for (int k = 0; k < nb[K]; ++k) {
-                b.rowtab.push_back(cb_off[I] + (loff[I][n] + k) * na[I] * nb[I]);
-                b.rowtab.push_back((ao[K] + k) * NAO - lr * NAO * (long long)NAO);
-                ++m;
+                a3.rowtab.push_back(R0.cfin_off[I] + (R0.loff[I][n] + k) * nb[I] * na[I]);
+                a3.rowtab.push_back((ao[K] + k) * NAO - lr * NAO * (long long)NAO);
             }
         }
-        q.M = m;
-        b.add(q);
-    };
-    a3a = GemmBatch();
-    a3a.atomic = true;
-    a3a.coltab = ext_cols;
-    for (int I = 0; I < natom; ++I) add_a3(a3a, I, y_off[I]);
-    a3a.finalize(big_tile(prec), st);
-    flops_sigma += a3a.flops;
+        a3.add(q);
+    }
+    a3.finalize(big_tile(prec), st);
+    flops_sigma += 2 * a3.flops;
 
-    // ---- chunks of I for T^D ----
-    std::vector<std::vector<std::pair<int, int>>> rev(natom);  // K -> (I, n)
-    for (int I = 0; I < natom; ++I)
-        for (size_t n = 0; n < nbrs[I].size(); ++n) rev[nbrs[I][n].K].push_back({I, (int)n});
+    // ---- CW by chunks of atoms, and the passes over it ----
+    const double per_sign = (double)ts * (u_elems + max_ghat + y_elems + (2.0 * nR + NE) * NAO * (double)NAO);
+    double cw_total = 0, fl = 0;
+    std::vector<long long> cw_x(natom);  // CW of atom x in its chunk: [R][J][c][i][nu]
     {
-        const double fixed = (double)ts * (u_elems + y_elems + gc_elems + 4.0 * NE * NAO * (double)NAO) +
-                             8.0 * ntau * nR * (double)NABF * NABF;
+        const double fixed = 2.0 * per_sign + 8.0 * ntau * nR * (double)NABF * NABF;
         const double budget = std::max(4e9, std::min(96e9, 0.6 * (double)free_b - fixed));
-        int i = 0;
-        while (i < natom) {
-            IChunk c;
-            c.i0 = i;
-            long long t = 0;
-            int ii = i;
-            while (ii < natom) {
-                const long long t1 = (long long)na[ii] * lsum[ii] * LD;
-                if (ii > i && (double)(t + t1) * ts > budget) break;
-                t += t1;
-                ++ii;
+        int x = 0;
+        while (x < natom) {
+            XChunk c;
+            c.x0 = x;
+            for (; x < natom; ++x) {
+                const long long t = (long long)nR * R0.lsum[x] * nb[x] * NABF;
+                if (x > c.x0 && (double)(c.cw_elems + t) * ts > budget) break;
+                cw_x[x] = c.cw_elems;
+                c.cw_elems += t;
             }
-            c.i1 = ii;
-            c.td_elems = t;
-            long long o = 0;
-            for (int I = c.i0; I < c.i1; ++I) { c.td_off.push_back(o); o += (long long)na[I] * lsum[I] * LD; }
-            auto tdo = [&](int I) { return c.td_off[I - c.i0]; };
-            // T^D build: per (J, S, K), rows (I, n, mu) of atoms I of the chunk with K_n = K
-            c.tdb.trans_b = true;
-            for (int J = 0; J < natom; ++J)
-                for (int S = 0; S < nR; ++S)
-                    for (int K = 0; K < natom; ++K) {
-                        GemmProb q = make_prob(0, nb[K] * nb[J], na[J], 0, 0,
-                                               u_off[(size_t)J * nR + S] + ao[K] * nb[J] * (long long)na[J], na[J], 0,
-                                               0);
-                        q.ncb = nb[J];
-                        q.cbs = LD;
-                        q.rt_off = (int)(c.tdb.rowtab.size() / 2);
-                        int m = 0;
-                        const auto &Sv = cells[S];
-                        for (const auto &in : rev[K]) {
-                            const int I = in.first, n = in.second;
-                            if (I < c.i0 || I >= c.i1) continue;
-                            const auto &Ra = cells[nbrs[I][n].r];
-                            const int rr = R0.fold_index(Sv[0] + Ra[0], Sv[1] + Ra[1], Sv[2] + Ra[2]);
-                            for (int mu = 0; mu < na[I]; ++mu) {
-                                c.tdb.rowtab.push_back((long long)rr * NABF * NABF + (abf[I] + mu) * NABF + abf[J]);
-                                c.tdb.rowtab.push_back(tdo(I) + ((long long)na[I] * loff[I][n] + (long long)mu * nb[K]) * LD +
-                                                       (long long)rr * NAO + ao[J]);
-                                ++m;
-                            }
-                        }
-                        if (m == 0) { c.tdb.rowtab.resize((size_t)q.rt_off * 2); continue; }
-                        q.M = m;
-                        c.tdb.add(q);
-                    }
-            c.tdb.finalize(prec == Prec::F64 ? T128x64w8 : T128x64, st);
-            // label a0b0_a2b2: Sigma_I.(R)[i][(R, J, j)] = CD_I * T_I
-            for (int I = c.i0; I < c.i1; ++I) {
-                GemmProb q = make_prob(nb[I], (int)LD, (int)(na[I] * lsum[I]), cd_off[I], (int)(na[I] * lsum[I]), tdo(I),
-                                       (int)LD, ao[I] * NAO, NAO);
-                q.ncb = NAO;
-                q.cbs = (long long)NAO * NAO;
-                c.dcon.add(q);
-            }
-            c.dcon.finalize(prec == Prec::F64 ? T32x64 : T32x128, st);
-            // label a0b0_a1b2 from the on-site rows of T_I
-            c.a3b.atomic = true;
-            c.a3b.coltab = ext_cols;
-            for (int I = c.i0; I < c.i1; ++I) add_a3(c.a3b, I, tdo(I) + (long long)na[I] * loff[I][onsite[I]] * LD);
-            c.a3b.finalize(big_tile(prec), st);
-            flops_sigma += c.tdb.flops + c.dcon.flops + c.a3b.flops;
-            ichunks.push_back(std::move(c));
-            i = ii;
+            c.x1 = x;
+            cw_total += (double)c.cw_elems;
+            max_cw = std::max(max_cw, c.cw_elems);
+            xchunks.push_back(std::move(c));
         }
     }
-    flops_sigma *= 2.0 * nspin * ntau;  // both signs, all spins and tau
-
-    // ---- device buffers ----
-    long long max_g = 0, max_td = 0;
-    for (auto &c : uchunks) max_g = std::max(max_g, c.ghat_elems);
-    for (auto &c : ichunks) max_td = std::max(max_td, c.td_elems);
-    // work buffers of the Sigma phase are allocated when it starts (after W's temporaries are freed)
-    max_ghat = max_g;
-    max_tdc = max_td;
-    HIP_CHECK(hipStreamSynchronize(st));
+    std::vector<long long> seg_i(natom + 1, 0);  // segment table: atom, cell
+    for (int I = 0; I < natom; ++I) seg_i[I + 1] = seg_i[I] + nR * R0.lsum[I];
+    auto pack = [&](std::map<std::pair<int, int>, std::vector<SigTask>> &m, std::vector<Tasks> &out) {
+        for (auto &kv : m) {
+            Tasks t;
+            t.a = kv.first.first;
+            t.b = kv.first.second;
+            t.n = (int)kv.second.size();
+            t.d = upload(kv.second, st);
+            HIP_CHECK(hipStreamSynchronize(st));
+            out.push_back(std::move(t));
+        }
+    };
+    for (auto &c : xchunks) {
+        std::vector<SigBlk> blks;
+        for (int I = c.x0; I < c.x1; ++I) {
+            const long long lb = R0.lsum[I] * nb[I];
+            if (lb == 0) continue;
+            for (int rr = 0; rr < nR; ++rr)
+                for (int J = 0; J < natom; ++J) {
+                    const long long at = cw_x[I] + (rr * (long long)NABF + abf[J]) * lb;
+                    c.cwb.add(make_prob((int)lb, na[J], na[I], R0.cfin_off[I], na[I],
+                                        (long long)rr * NABF * NABF + abf[I] * NABF + abf[J], NABF, at, na[J]));
+                    blks.push_back({at, u_off[(size_t)J * nR], nb[I], nb[J], na[J], (int)R0.lsum[I], (int)ao[I],
+                                    (int)ao[J], rr, (int)(seg_i[I] + rr * R0.lsum[I])});
+                    fl += 8.0 * R0.lsum[I] * nb[I] * na[J] * nb[J] + 4.0 * nb[I] * na[I] * nb[J] * R0.lsum[J];
+                }
+        }
+        c.cwb.finalize(prec == Prec::F64 ? T128x64w8 : T128x64, st);
+        c.d_blks = upload(blks, st);
+        fl += c.cwb.flops / nspin;
+        HIP_CHECK(hipStreamSynchronize(st));
+    }
+    flops_sigma = (flops_sigma + fl) * nspin * ntau;
+    // tau points per pass, as in the chi0 build: up to about 120 GFLOP, and 12 GB
+    nbatch = 1;
+    if (uchunks.size() == 1 && xchunks.size() == 1)
+        nbatch = (int)std::max(1.0, std::min({(double)R0.nbatch, std::ceil(1.2e11 / std::max(1.0, flops_sigma / ntau)),
+                                              std::min(12e9, 0.1 * (double)free_b) / (ts * cw_total + 2.0 * per_sign)}));
+    nbatch = ceil_div(ntau, ceil_div(ntau, nbatch));
+    for (auto &c : xchunks) {
+        std::map<std::pair<int, int>, std::vector<SigTask>> td, tb;
+        int b = 0;
+        const double nblk = (double)(c.x1 - c.x0) * natom * nR * nbatch;
+        for (int I = c.x0; I < c.x1; ++I) {
+            const int l = (int)R0.lsum[I];
+            if (l == 0) continue;
+            // 2048 workgroups, each with at least 16 segments
+            const int parts = std::max(1, std::min(ceil_div(l, 16), (int)std::ceil(2048.0 / nblk)));
+            for (int rr = 0; rr < nR; ++rr)
+                for (int J = 0; J < natom; ++J, ++b) {
+                    const int fi = nb[I] > 16 ? 2 : 1, fj = nb[J] > 16 ? 2 : 1, fc = l > 64 ? 2 : 1;
+                    for (int j0 = 0; j0 < nb[J]; j0 += 16 * fj) {
+                        for (int i0 = 0; i0 < nb[I]; i0 += 16 * fi)
+                            for (int q = 0; q < parts; ++q)
+                                td[{fi, fj}].push_back({b, i0, j0, (int)((long long)l * q / parts),
+                                                        (int)((long long)l * (q + 1) / parts)});
+                        for (int t0 = 0; t0 < l; t0 += 64 * fc) tb[{fc, fj}].push_back({b, 0, j0, t0, l});
+                    }
+                }
+        }
+        pack(td, c.d);
+        pack(tb, c.b);
+    }
+    // entries (J, R) of every (S, L): J's neighbours L in the cell S - R
+    {
+        std::vector<SigYEnt> ents;
+        std::vector<int> e0((size_t)nR * natom + 1, 0);
+        std::vector<std::vector<int>> nbr_at(natom, std::vector<int>((size_t)natom * nR, -1));
+        for (int J = 0; J < natom; ++J)
+            for (size_t n = 0; n < R0.nbrs[J].size(); ++n)
+                nbr_at[J][(size_t)R0.nbrs[J][n].K * nR + R0.nbrs[J][n].r] = (int)n;
+        for (int S = 0; S < nR; ++S)
+            for (int L = 0; L < natom; ++L) {
+                for (int J = 0; J < natom; ++J)
+                    for (int rr = 0; rr < nR; ++rr) {
+                        const int r2 = R0.fold_index(cells[S][0] - cells[rr][0], cells[S][1] - cells[rr][1],
+                                                     cells[S][2] - cells[rr][2]);
+                        const int n = nbr_at[J][(size_t)L * nR + r2];
+                        if (n < 0) continue;
+                        const long long lb = R0.lsum[J] * nb[J];
+                        ents.push_back({rr * gpm_r + 2 * ao[J], cw_x[J] + neg[rr] * (long long)NABF * lb, (int)lb,
+                                        (int)(R0.loff[J][n] * nb[J]), nb[J], J});
+                    }
+                e0[(size_t)S * natom + L + 1] = (int)ents.size();
+            }
+        std::map<int, std::vector<SigYTask>> ty;
+        for (int S = 0; S < nR; ++S)
+            for (int L = 0; L < natom; ++L)
+                for (int I = 0; I < natom; ++I) {
+                    const int fi = nb[I] > 16 ? 2 : 1;
+                    for (int l0 = 0; l0 < nb[L]; l0 += 4)
+                        for (int mu0 = 0; mu0 < na[I]; mu0 += 64)
+                            for (int i0 = 0; i0 < nb[I]; i0 += 16 * fi)
+                                ty[fi].push_back({y_off[I] + ((long long)S * NAO + ao[L]) * nb[I] * na[I],
+                                                  e0[(size_t)S * natom + L], e0[(size_t)S * natom + L + 1], nb[I], na[I],
+                                                  (int)ao[I], (int)abf[I], l0, nb[L], mu0, i0});
+                }
+        for (auto &kv : ty) {
+            Tasks t;
+            t.a = kv.first;
+            t.n = (int)kv.second.size();
+            t.d = upload(kv.second, st);
+            HIP_CHECK(hipStreamSynchronize(st));
+            ytasks.push_back(std::move(t));
+        }
+        d_yent = upload(ents, st);
+        HIP_CHECK(hipStreamSynchronize(st));
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -810,152 +707,104 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
     HIP_CHECK(hipMemsetAsync(d_Sre.get(), 0, d_Sre.bytes(), st));
     HIP_CHECK(hipMemsetAsync(d_Sim.get(), 0, d_Sim.bytes(), st));
     if (w_zero) { HIP_CHECK(hipStreamSynchronize(st)); t_sigma = now_s() - t0; return; }
-    d_U.alloc(u_elems * ts);
-    d_Ghat.alloc(max_ghat * ts);
-    d_TD.alloc(max_tdc * ts);
-    d_Y.alloc(y_elems * ts);
-    d_GC.alloc(gc_elems * ts);
-    for (int sg = 0; sg < 2; ++sg) d_sig[sg].alloc((size_t)nR * NAO * NAO * ts);
-    d_extA.alloc((size_t)NE * NAO * NAO * ts);
-    d_extB.alloc((size_t)NE * NAO * NAO * ts);
-    if (prec != Prec::F64) d_Wf.alloc((size_t)nR * NABF * NABF * ts);
+    d_U.alloc(2 * (size_t)u_elems * nbatch * ts);
+    d_Ghat.alloc((size_t)max_ghat * nbatch * ts);
+    d_CW.alloc(((size_t)max_cw * nbatch + kChi0Pad) * ts);
+    d_Y.alloc(2 * (size_t)y_elems * nbatch * ts);
+    const size_t next = (size_t)NE * NAO * NAO;
+    d_sig.alloc(2 * (size_t)nbatch * (2 * nel + next) * ts);
+    if (prec != Prec::F64) d_Wf.alloc((size_t)nbatch * nR * NABF * NABF * ts);
     R0.prepare_gf(ds.mf, -1);  // all bands (get_gf_cplx_imagtimes_Rs, meanfield.cpp:309-365)
-    const long long gpm_r = (long long)NAO * 2 * NAO;
-    (void)gpm_r;
-    const size_t esz = ts;
-    const long long nn_abf = (long long)NABF * NABF;
-    // LIBRPA_AMD_TUNE_SIGMA=1 times the Sigma batches' candidate tiles on the first pass (the
+    const long long nn_abf = (long long)NABF * NABF, zg = (long long)nR * NAO * 2 * NAO;
+    DevBuf dcw = upload(g.cos_t2f, st), dsw = upload(g.sin_t2f, st);
+    // LIBRPA_AMD_TUNE_SIGMA=1 times the U and CW batches' candidate tiles on the first pass (the
     // trials cost about as much as they save in one G0W0 run, so the defaults are used otherwise)
     const char *tsg = std::getenv("LIBRPA_AMD_TUNE_SIGMA");
     const bool tune_sigma = R0.autotune && tsg && std::atoi(tsg) != 0;
-    for (int it = 0; it < g.n; ++it) {
-        const void *Wf;
-        if (prec == Prec::F64) {
-            Wf = d_Wrt.as<double>() + (size_t)it * nR * nn_abf;
-        } else {
-            launch_convert<double, float>(d_Wrt.as<double>() + (size_t)it * nR * nn_abf, d_Wf.as<float>(),
-                                          (long long)nR * nn_abf, st);
-            Wf = d_Wf.get();
-        }
-        std::vector<double> cw(nw), sw(nw);
-        for (int w = 0; w < nw; ++w) {
-            cw[w] = g.cos_t2f[(size_t)w * g.n + it];
-            sw[w] = g.sin_t2f[(size_t)w * g.n + it];
-        }
-        DevBuf dcw = upload(cw, st), dsw = upload(sw, st);
-        if (verbose) { fprintf(stderr, "[librpa-mi355x] Sigma_c: tau %d / %d (%.1f s)\n", it + 1, g.n, now_s() - t0); fflush(stderr); }
-        for (int s = 0; s < nspin; ++s) {
-            R0.build_gf(ds.mf, &g.tau[it], 1, s);
-            for (int sg = 0; sg < 2; ++sg) {
-                HIP_CHECK(hipMemsetAsync(d_sig[sg].get(), 0, d_sig[sg].bytes(), st));
-                HIP_CHECK(hipMemsetAsync(d_extA.get(), 0, d_extA.bytes(), st));
-                HIP_CHECK(hipMemsetAsync(d_extB.get(), 0, d_extB.bytes(), st));
-                HIP_CHECK(hipMemsetAsync(d_Y.get(), 0, d_Y.bytes(), st));
+    auto passes = [&](auto tag) {
+        using T = decltype(tag);
+        const T *G = R0.d_Gpm.as<T>();
+        for (int it = 0, nz = 1; it < g.n; it += nz) {
+            // tau points [it, it + nz) in one pass
+            nz = std::min(nbatch, g.n - it);
+            const void *Wf = d_Wrt.as<double>() + (size_t)it * nR * nn_abf;
+            if (prec != Prec::F64) {
+                launch_convert<double, float>(d_Wrt.as<double>() + (size_t)it * nR * nn_abf, d_Wf.as<float>(),
+                                              (long long)nz * nR * nn_abf, st);
+                Wf = d_Wf.get();
+            }
+            if (verbose) {
+                HIP_CHECK(hipStreamSynchronize(st));
+                fprintf(stderr, "[librpa-mi355x] Sigma_c: tau %d / %d (%.1f s)\n", it + 1, g.n, now_s() - t0);
+                fflush(stderr);
+            }
+            for (int s = 0; s < nspin; ++s) {
+                R0.build_gf(ds.mf, &g.tau[it], nz, s);
+                T *sig = d_sig.as<T>(), *s2 = sig + 2 * (size_t)nbatch * nel, *ext = s2 + 2 * (size_t)nbatch * nel;
+                HIP_CHECK(hipMemsetAsync(d_sig.get(), 0, d_sig.bytes(), st));
                 // U_J(S) for all J, S
                 for (auto &c : uchunks) {
                     prof.begin("gw_gather", st);
-                    if (prec == Prec::F64)
-                        launch_gather_cols<double>(R0.d_Gpm.as<double>(), 2LL * NAO, d_Ghat.as<double>(),
-                                                   c.d_jobs[sg].as<GatherJob>(), (int)c.jobs[sg].size(),
-                                                   c.d_colsrc[sg].as<long long>(), NAO, c.max_gcol, st);
-                    else
-                        launch_gather_cols<float>(R0.d_Gpm.as<float>(), 2LL * NAO, d_Ghat.as<float>(),
-                                                  c.d_jobs[sg].as<GatherJob>(), (int)c.jobs[sg].size(),
-                                                  c.d_colsrc[sg].as<long long>(), NAO, c.max_gcol, st);
-                    prof.end("gw_gather", st, 0, 2.0 * c.ghat_elems * esz);
+                    launch_gather_cols<T>(G, 2LL * NAO, d_Ghat.as<T>(), c.d_jobs.template as<GatherJob>(), (int)c.jobs.size(),
+                                          c.d_colsrc.template as<long long>(), NAO, c.max_gcol, st, nz, zg, c.ghat_elems);
+                    prof.end("gw_gather", st, 0, 2.0 * nz * c.ghat_elems * ts);
                     prof.begin("gw_U", st);
-                    if (tune_sigma && !sigma_tuned)
+                    c.ub.nz = nz;
+                    c.ub.za = c.ghat_elems;
+                    c.ub.zc = 2 * u_elems;
+                    if (tune_sigma && !c.ub.tuned)
                         c.ub.tune(prec, d_Ghat.get(), R0.d_CWb.get(), d_U.get(), 1.0, 0.0, st);
                     gemm_run(prec, c.ub, d_Ghat.get(), R0.d_CWb.get(), d_U.get(), 1.0, 0.0, st);
-                    prof.end("gw_U", st, c.ub.flops);
+                    prof.end("gw_U", st, nz * c.ub.flops);
                 }
-                if (tune_sigma && !sigma_tuned) {
-                    // time the candidate tiles once per batch shape; the trials leave garbage in
-                    // GC, Y, T^D and Sigma, which are reset before the real pass
-                    for (int J = 0; J < natom; ++J) {
-                        const char *gbase = R0.d_Gpm.as<char>() + (size_t)sg * R0.nb[J] * esz;
-                        for (int rr = 0; rr < nR; ++rr) {
-                            GemmBatch &b1 = a1[(size_t)J * nR + rr];
-                            GemmBatch &b2 = a2[(size_t)J * nR + rr];
-                            if (b1.empty()) continue;
-                            b1.tune(prec, gbase, d_CA.get(), d_GC.get(), 1.0, 0.0, st);
-                            gemm_run(prec, b1, gbase, d_CA.get(), d_GC.get(), 1.0, 0.0, st);
-                            b2.tune(prec, Wf, d_GC.get(), d_Y.get(), 1.0, 1.0, st);
-                        }
+                for (auto &c : xchunks) {
+                    if (s == 0 || xchunks.size() > 1) {
+                        prof.begin("gw_CW", st);
+                        c.cwb.nz = nz;
+                        c.cwb.zb = nR * nn_abf;
+                        c.cwb.zc = c.cw_elems;
+                        if (tune_sigma && !c.cwb.tuned)
+                            c.cwb.tune(prec, R0.d_Cfin.get(), Wf, d_CW.get(), 1.0, 0.0, st);
+                        gemm_run(prec, c.cwb, R0.d_Cfin.get(), Wf, d_CW.get(), 1.0, 0.0, st);
+                        prof.end("gw_CW", st, nz * c.cwb.flops);
                     }
-                    for (auto &c : ichunks) {
-                        c.tdb.tune(prec, Wf, d_U.get(), d_TD.get(), 1.0, 0.0, st);
-                        gemm_run(prec, c.tdb, Wf, d_U.get(), d_TD.get(), 1.0, 0.0, st);
-                        c.dcon.tune(prec, d_CD.get(), d_TD.get(), d_sig[sg].get(), 1.0, 1.0, st);
-                    }
-                    HIP_CHECK(hipMemsetAsync(d_Y.get(), 0, d_Y.bytes(), st));
-                    HIP_CHECK(hipMemsetAsync(d_sig[sg].get(), 0, d_sig[sg].bytes(), st));
-                    sigma_tuned = true;
-                    if (verbose) {
-                        auto nm = [](const GemmBatch &b) { return tile_name(b.cfg); };
-                        for (auto &c : uchunks) fprintf(stderr, "[librpa-mi355x] tile U %s\n", nm(c.ub));
-                        for (int J = 0; J < natom; ++J)
-                            if (!a1[(size_t)J * nR].empty())
-                                fprintf(stderr, "[librpa-mi355x] tile A1 J=%d %s A2 %s\n", J, nm(a1[(size_t)J * nR]),
-                                        nm(a2[(size_t)J * nR]));
-                        for (auto &c : ichunks)
-                            fprintf(stderr, "[librpa-mi355x] tile TD %s D %s\n", nm(c.tdb), nm(c.dcon));
-                        fflush(stderr);
-                    }
-                }
-                // partner-partner term: Y_I over all (J, R), then one contraction
-                prof.begin("gw_A12", st);
-                double fa = 0;
-                for (int J = 0; J < natom; ++J) {
-                    const char *gbase = R0.d_Gpm.as<char>() + (size_t)sg * R0.nb[J] * esz;
-                    for (int rr = 0; rr < nR; ++rr) {
-                        const GemmBatch &b1 = a1[(size_t)J * nR + rr];
-                        const GemmBatch &b2 = a2[(size_t)J * nR + rr];
-                        if (b1.empty()) continue;
-                        gemm_run(prec, b1, gbase, d_CA.get(), d_GC.get(), 1.0, 0.0, st);
-                        gemm_run(prec, b2, Wf, d_GC.get(), d_Y.get(), 1.0, 1.0, st);
-                        fa += b1.flops + b2.flops;
-                    }
-                }
-                prof.end("gw_A12", st, fa);
-                prof.begin("gw_A3", st);
-                gemm_run(prec, a3a, d_CB.get(), d_Y.get(), d_extA.get(), 1.0, 1.0, st);
-                prof.end("gw_A3", st, a3a.flops);
-                // owner-row terms by chunks of I
-                for (auto &c : ichunks) {
-                    prof.begin("gw_TD", st);
-                    gemm_run(prec, c.tdb, Wf, d_U.get(), d_TD.get(), 1.0, 0.0, st);
-                    prof.end("gw_TD", st, c.tdb.flops);
+                    const SigBlk *blks = c.d_blks.template as<SigBlk>();
+                    const Chi0Seg *segs = R0.d_segs.as<Chi0Seg>();
                     prof.begin("gw_D", st);
-                    gemm_run(prec, c.dcon, d_CD.get(), d_TD.get(), d_sig[sg].get(), 1.0, 1.0, st);
-                    prof.end("gw_D", st, c.dcon.flops);
-                    prof.begin("gw_A3", st);
-                    gemm_run(prec, c.a3b, d_CB.get(), d_TD.get(), d_extB.get(), 1.0, 1.0, st);
-                    prof.end("gw_A3", st, c.a3b.flops);
+                    for (auto &t : c.d)
+                        launch_sigma_d<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, d_CW.as<T>(), c.cw_elems,
+                                          d_U.as<T>(), u_elems, sig, nel, NAO, nz, st);
+                    prof.end("gw_D", st);
+                    prof.begin("gw_B", st);
+                    for (auto &t : c.b)
+                        launch_sigma_b<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, d_CW.as<T>(), c.cw_elems,
+                                          d_U.as<T>(), u_elems, s2, nel, NAO, nz, st);
+                    prof.end("gw_B", st);
+                    prof.begin("gw_Y", st);
+                    for (auto &t : ytasks)
+                        launch_sigma_y<T>(t.d.template as<SigYTask>(), t.n, t.a, d_yent.as<SigYEnt>(), d_CW.as<T>(), c.cw_elems,
+                                          G, zg, d_Y.as<T>(), y_elems, NAO, c.x0, c.x1, c.x0 == 0, nz, st);
+                    prof.end("gw_Y", st);
                 }
+                prof.begin("gw_A3", st);
+                a3.nz = 2 * nz;
+                a3.zb = y_elems;
+                a3.zc = (long long)next;
+                gemm_run(prec, a3, R0.d_Cfin.get(), d_Y.get(), ext, 1.0, 1.0, st);
+                prof.end("gw_A3", st, 2 * nz * a3.flops);
                 prof.begin("gw_fold", st);
-                if (prec == Prec::F64)
-                    launch_sigma_fold<double>(d_sig[sg].as<double>(), d_extA.as<double>(), d_extB.as<double>(),
-                                              d_fold.as<int>(), d_foldneg.as<int>(), NE, nR, NAO, st);
-                else
-                    launch_sigma_fold<float>(d_sig[sg].as<float>(), d_extA.as<float>(), d_extB.as<float>(),
-                                             d_fold.as<int>(), d_foldneg.as<int>(), NE, nR, NAO, st);
+                launch_sigma_fold<T>(sig, s2, ext, d_fold.as<int>(), d_neg.as<int>(), NE, nR, NAO, nz, st);
+                launch_sigma_freq<T>(sig, nel, dcw.as<double>(), dsw.as<double>(), nw, g.n, it, nz,
+                                     d_Sre.as<double>() + (size_t)s * nw * nel, d_Sim.as<double>() + (size_t)s * nw * nel,
+                                     st);
                 prof.end("gw_fold", st);
             }
-            prof.begin("gw_freq", st);
-            double *sre = d_Sre.as<double>() + (size_t)s * nw * nel;
-            double *sim = d_Sim.as<double>() + (size_t)s * nw * nel;
-            if (prec == Prec::F64)
-                launch_sigma_freq<double>(d_sig[0].as<double>(), d_sig[1].as<double>(), nel, dcw.as<double>(),
-                                          dsw.as<double>(), nw, sre, sim, st);
-            else
-                launch_sigma_freq<float>(d_sig[0].as<float>(), d_sig[1].as<float>(), nel, dcw.as<double>(),
-                                         dsw.as<double>(), nw, sre, sim, st);
-            prof.end("gw_freq", st);
         }
-        HIP_CHECK(hipStreamSynchronize(st));
-    }
-    for (DevBuf *b : {&d_U, &d_Ghat, &d_TD, &d_Y, &d_GC, &d_sig[0], &d_sig[1], &d_extA, &d_extB, &d_Wf}) b->release();
+    };
+    if (prec == Prec::F64) passes(double());
+    else passes(float());
+    HIP_CHECK(hipStreamSynchronize(st));
+    for (DevBuf *b : {&d_U, &d_Ghat, &d_CW, &d_Y, &d_sig, &d_Wf}) b->release();
     t_sigma = now_s() - t0;
 }
 

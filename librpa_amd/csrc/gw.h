@@ -9,6 +9,7 @@
 #include "../../include/librpa_options.h"
 #include "dataset.h"
 #include "gemm.h"
+#include "gw_kernels.h"
 #include "kernels.h"
 #include "rpa.h"
 
@@ -21,61 +22,52 @@ struct GwEngine {
     int natom = 0, NAO = 0, NABF = 0, nR = 0, nk = 0, nspin = 1, ntau = 0;
     long long LD = 0;  // nR * NAO: column count of the (cell, atom, orbital) index
 
-    // neighbour lists with the on-site block always present (zero if Cs has none)
-    std::vector<std::vector<RpaEngine::Nbr>> nbrs;
-    std::vector<std::vector<long long>> loff;
-    std::vector<long long> lsum;
-    std::vector<int> onsite;
-
     // cell differences R1 - R2 of two BvK cells on an extended (2p - 1)^3 grid
     int E[3] = {1, 1, 1};
     int NE = 1;
     long long c0 = 0;
-    std::vector<int> ext_fold, ext_foldneg;
     long long linr(int x, int y, int z) const { return ((long long)x * E[1] + y) * E[2] + z; }
 
-    // packed Cs (compute precision)
-    DevBuf d_CD, d_CB, d_CA;
-    std::vector<long long> cd_off, cb_off, ca_off;
+    int nbatch = 1;  // tau points per pass
 
-    // U_J(S) build
+    // U_J(S) build, both signs
     struct UChunk {
-        int j0 = 0, j1 = 0;
         long long ghat_elems = 0;
         int max_gcol = 0;
-        std::vector<long long> ghat_off;  // per (J - j0, S)
-        std::vector<GatherJob> jobs[2];
-        std::vector<long long> colsrc[2];
-        DevBuf d_jobs[2], d_colsrc[2];
+        std::vector<GatherJob> jobs;
+        std::vector<long long> colsrc;
+        DevBuf d_jobs, d_colsrc;
         GemmBatch ub;
     };
     std::vector<UChunk> uchunks;
     std::vector<long long> u_off;  // per (J, S)
     long long u_elems = 0;
 
-    // T^D and the owner-row contractions per chunk of atoms I
-    struct IChunk {
-        int i0 = 0, i1 = 0;
-        long long td_elems = 0;
-        std::vector<long long> td_off;  // per I - i0
-        GemmBatch tdb, dcon, a3b;
+    // CW of the atoms [x0, x1) and the contractions that read it
+    struct Tasks { int a = 1, b = 1, n = 0; DevBuf d; };  // fragments of a task
+    struct XChunk {
+        int x0 = 0, x1 = 0;
+        long long cw_elems = 0;
+        GemmBatch cwb;
+        DevBuf d_blks;
+        std::vector<Tasks> d, b;
     };
-    std::vector<IChunk> ichunks;
-
-    // partner-partner term: per (J, R) GC = G C^J and Y += W GC, then one contraction
-    std::vector<GemmBatch> a1, a2;
-    GemmBatch a3a;
+    std::vector<XChunk> xchunks;
+    std::vector<Tasks> ytasks;
+    DevBuf d_yent;
+    GemmBatch a3;
     std::vector<long long> y_off;
-    long long y_elems = 0, gc_elems = 0;
+    long long y_elems = 0;
 
-    DevBuf d_U, d_Ghat, d_TD, d_Y, d_GC, d_Wf;
-    DevBuf d_sig[2], d_extA, d_extB, d_fold, d_foldneg;
+    DevBuf d_U, d_Ghat, d_CW, d_Y, d_Wf;
+    DevBuf d_sig;  // sig, s2 and ext of every tau point and sign of a pass
+    DevBuf d_fold, d_neg;
     DevBuf d_Wrt;         // W(R, tau) [tau][R][NABF][NABF], FP64
     DevBuf d_Sre, d_Sim;  // Sigma(R, i omega) [spin][omega][R][NAO][NAO], FP64
     bool w_zero = false;  // no truncated Coulomb given: W = 0
 
     double flops_sigma = 0, flops_w = 0, t_w = 0, t_sigma = 0;
-    long long max_ghat = 0, max_tdc = 0;
+    long long max_ghat = 0, max_cw = 0;
     bool verbose = false;  // progress lines on stderr
     // eps_mac(i omega_w) per grid frequency: replaces the head of the dielectric matrix at q = 0
     // (replace_w_head with option_dielect_func 0); empty = no replacement

@@ -3,6 +3,7 @@
 // projection of Sigma(R, i omega).
 #pragma once
 
+#include "chi0.h"
 #include "common.h"
 
 namespace lra {
@@ -16,17 +17,48 @@ void launch_w_accum(const double *aug, long long aug_stride, int cnt, int n, int
                     const double *coef, int ntau, const double *cs_r, const double *sn_r, int nR, double *Wrt,
                     hipStream_t s);
 
-// sig[R][a][b] += sum_{e : fold[e] == R} (extA[e][a][b] + extB[e][a][b])
-//              + sum_{e : foldneg[e] == R} extB[e][b][a]
+// ---- self-energy contractions (gw.cpp) ----
+// CW_IJ(R)[c][i][nu] = sum_mu C^I[(c, i)][mu] W_IJ(R)[mu][nu] and U_J(S)[(X, x)][j][nu] per tau point; c
+// runs over the rows (K, R1, k) of atom I's neighbours (Chi0Seg order: (cell, row) of R - R1).
+// One (I, J, R).
+struct SigBlk {
+    long long cw, u;  // CW_IJ(R), U_J(cell 0) (cells NAO nj aj apart)
+    int ni, nj, aj, l;
+    int rowI, colJ, r;
+    int seg0;         // first entry of (I, R) in the segment table
+};
+// segments [c0, c1) of a block, rows from i0 (or all), columns from j0
+struct SigTask { int blk, i0, j0, c0, c1; };
+// sig[z][sign][R][NAO][NAO] += D, the label a0b0_a2b2: CW zcw elements per tau point, U two signs usg apart
 template <class T>
-void launch_sigma_fold(T *sig, const T *extA, const T *extB, const int *fold, const int *foldneg, int NE, int nR,
-                       int n, hipStream_t s);
+void launch_sigma_d(const SigTask *tasks, int ntask, int fi, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
+                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, hipStream_t s);
+// s2[z][sign][R][NAO][NAO] += the label a0b0_a1b2, 64 fc segments a task from c0
+template <class T>
+void launch_sigma_b(const SigTask *tasks, int ntask, int fc, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
+                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, hipStream_t s);
+// One (J, R) that reaches the columns (S, L, .): G_IJ(R) at g, CW_JI(-R)[(L, S - R, l)] at
+// b + abf(I) lb + (cb + l nj) ai
+struct SigYEnt { long long g, b; int lb, cb, nj, J; };
+struct SigYTask {
+    long long y;  // Y_I row of (S, L, 0)
+    int e0, e1;   // entries of (S, L)
+    int ni, ai, ao, abf, l0, nl, mu0, i0;
+};
+template <class T>
+void launch_sigma_y(const SigYTask *tasks, int ntask, int fi, const SigYEnt *ents, const T *CW, long long zcw, const T *G,
+                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, hipStream_t s);
 
-// Sigma(R, i w) += 0.5 (S+ + S-) cos_t2f(w) + i 0.5 (S+ - S-) sin_t2f(w) for all w
-// (sre / sim layout [w][R][n][n]).
+// for nz tau points and both signs: sig[R][a][b] += s2[R][a][b] + s2[-R][b][a] + sum_{e : fold[e] == R} ext[e][a][b]
 template <class T>
-void launch_sigma_freq(const T *sp, const T *sn, long long nelem, const double *cw, const double *sw, int nw,
-                       double *sre, double *sim, hipStream_t s);
+void launch_sigma_fold(T *sig, const T *s2, const T *ext, const int *fold, const int *neg, int NE, int nR, int n,
+                       int nz, hipStream_t s);
+
+// Sigma(R, i w) += 0.5 (S+ + S-) cos_t2f(w) + i 0.5 (S+ - S-) sin_t2f(w) for all w and the tau points
+// [it0, it0 + nz) (sig [z][sign][nelem], cw / sw [w][ntau], sre / sim [w][nelem]).
+template <class T>
+void launch_sigma_freq(const T *sig, long long nelem, const double *cw, const double *sw, int nw, int ntau, int it0,
+                       int nz, double *sre, double *sim, hipStream_t s);
 
 // Y[w][a][st] = sum_b sum_R ph[(I(a), J(b), R)] Sigma(R, w)[a][b] U[st][b] for one k point
 // (complex, st < nst <= 16); ph layout [I][J][R] (re, im interleaved), U [st][b] (re, im).

@@ -1,6 +1,8 @@
 // Streaming kernels of the G0W0 path (gfx950).
 #include "gw_kernels.h"
 
+#include <type_traits>
+
 namespace lra {
 
 constexpr int kWMax = 8;
@@ -50,60 +52,429 @@ void launch_w_accum(const double *aug, long long aug_stride, int cnt, int n, int
     HIP_CHECK(hipGetLastError());
 }
 
+// ------------------------------------------------------------------------------------
+// self-energy contractions
+// ------------------------------------------------------------------------------------
+namespace {
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+// 16-byte loads at element alignment (rows of odd basis sizes)
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <class T> struct SV;
+template <> struct SV<double> { using A = v4d; using V = d2u; static constexpr int VL = 2; };
+template <> struct SV<float> { using A = v4f; using V = f4u; static constexpr int VL = 4; };
+__device__ __forceinline__ v4d mfma(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ v4f mfma(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+// row of a 16 x 16 result that register r of lane group kq holds
+template <class T> __device__ __forceinline__ int acc_row(int r, int kq) { return sizeof(T) == 8 ? 4 * r + kq : 4 * kq + r; }
+
+// elements [0, n) of p (n <= 4), zero past them
 template <class T>
-__global__ void sigma_fold_kernel(T *__restrict__ sig, const T *__restrict__ extA, const T *__restrict__ extB,
-                                  const int *__restrict__ fold, const int *__restrict__ foldneg, int NE, int nR,
-                                  int n) {
+__device__ __forceinline__ void load4(T (&v)[4], const T *p, int n) {
+    using V = typename SV<T>::V;
+    constexpr int VL = SV<T>::VL;
+    if (n >= 4) {
+#pragma unroll
+        for (int g = 0; g < 4 / VL; ++g) {
+            const V x = *reinterpret_cast<const V *>(p + g * VL);
+#pragma unroll
+            for (int e = 0; e < VL; ++e) v[g * VL + e] = x[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = e < n ? p[e] : T(0);
+    }
+}
+}  // namespace
+
+// Sigma_IJ(R)[i][j] += sum_(c, nu) CW_IJ(R)[c][i][nu] U_J(S_c)[row_c][j][nu] over segments [c0, c1) of a
+// task, both signs at once: a wave takes every fourth segment, FI x FJ fragments of 16 x 16, and 16 nu
+// at a time, four consecutive ones a lane (any assignment of nu to the steps of an MFMA will do when
+// both operands share it).  The four waves are summed in LDS before one atomic add per element.
+// Bound by the reads of CW (each element once per pass) and, for small n_b, by U from L2: an MFMA
+// multiplies a fragment pair of 1 KB in 64 (FP64) cycles, so the next fragments are in flight
+// meanwhile.  8 atoms, 4 k: 24 such contractions of T = W U through an 8-workgroup GEMM took 35 ms.
+template <class T, int FI, int FJ>
+__global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restrict__ tasks, const SigBlk *__restrict__ blks,
+                                                         const Chi0Seg *__restrict__ segs, const T *__restrict__ CW,
+                                                         long long zcw, const T *__restrict__ U, long long usg,
+                                                         T *__restrict__ sig, long long ssg, int NAO) {
+    using A = typename SV<T>::A;
+    __shared__ __align__(16) T red[FI * FJ * 2 * 256];
+    const SigTask tk = tasks[blockIdx.x];
+    const SigBlk B = blks[tk.blk];
+    CW += blockIdx.y * zcw + B.cw;
+    U += blockIdx.y * 2 * usg + B.u;
+    sig += blockIdx.y * 2 * ssg;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, kq = lane >> 4;
+    const int ni = B.ni, nj = B.nj, aj = B.aj;
+    const Chi0Seg *st = segs + B.seg0;
+    int ao[FI], uo[FJ];
+#pragma unroll
+    for (int f = 0; f < FI; ++f) ao[f] = min(tk.i0 + 16 * f + c16, ni - 1) * aj + 4 * kq;
+#pragma unroll
+    for (int g = 0; g < FJ; ++g) uo[g] = min(tk.j0 + 16 * g + c16, nj - 1) * aj + 4 * kq;
+    A acc[FI][FJ][2];
+#pragma unroll
+    for (int f = 0; f < FI; ++f)
+#pragma unroll
+        for (int g = 0; g < FJ; ++g) acc[f][g][0] = acc[f][g][1] = A{0, 0, 0, 0};
+    struct Frag { T a[FI][4], u[2][FJ][4]; };
+    auto load = [&](Frag &x, int t, int k0) {
+        const Chi0Seg sg = st[t];
+        const T *ab = CW + (long long)sg.c * ni * aj + k0;
+        const T *ub = U + ((long long)sg.cell * NAO + sg.row) * nj * aj + k0;
+        const int n = aj - k0 - 4 * kq;
+#pragma unroll
+        for (int f = 0; f < FI; ++f) load4(x.a[f], ab + ao[f], n);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int g = 0; g < FJ; ++g) load4(x.u[s][g], ub + s * usg + uo[g], n);
+    };
+    auto use = [&](const Frag &x) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int f = 0; f < FI; ++f)
+#pragma unroll
+                    for (int g = 0; g < FJ; ++g) acc[f][g][s] = mfma(x.a[f][e], x.u[s][g][e], acc[f][g][s]);
+    };
+    int t = tk.c0 + wave, k0 = 0;
+    if (t < tk.c1) {
+        Frag x, y;
+        load(x, t, k0);
+        for (;;) {
+            k0 += 16;
+            if (k0 >= aj) { k0 = 0; t += 4; }
+            const bool more = t < tk.c1;
+            if (more) load(y, t, k0);
+            use(x);
+            if (!more) break;
+            x = y;
+        }
+    }
+    for (int w = 1; w < 4; ++w) {
+        __syncthreads();
+        if (wave == w)
+#pragma unroll
+            for (int f = 0; f < FI; ++f)
+#pragma unroll
+                for (int g = 0; g < FJ; ++g)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) *reinterpret_cast<A *>(&red[(((f * FJ + g) * 2 + s) * 64 + lane) * 4]) = acc[f][g][s];
+        __syncthreads();
+        if (wave == 0)
+#pragma unroll
+            for (int f = 0; f < FI; ++f)
+#pragma unroll
+                for (int g = 0; g < FJ; ++g)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) acc[f][g][s] += *reinterpret_cast<const A *>(&red[(((f * FJ + g) * 2 + s) * 64 + lane) * 4]);
+    }
+    if (wave != 0) return;
+#pragma unroll
+    for (int f = 0; f < FI; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = tk.i0 + 16 * f + acc_row<T>(r, kq);
+            if (i >= ni) continue;
+#pragma unroll
+            for (int g = 0; g < FJ; ++g) {
+                const int j = tk.j0 + 16 * g + c16;
+                if (j >= nj) continue;
+                T *dst = sig + ((long long)B.r * NAO + B.rowI + i) * NAO + B.colJ + j;
+                unsafeAtomicAdd(dst, acc[f][g][0][r]);
+                unsafeAtomicAdd(dst + ssg, acc[f][g][1][r]);
+            }
+        }
+}
+
+// S2(S_c)[row_c][j] += sum_(i, nu) CW_IJ(R)[c][(i, nu)] U_J(R)[(I, i)][j][nu] for the 16 FC segments of a
+// wave (64 FC of a task, from c0), FJ fragments of j and both signs; operands as in sigma_d_kernel.
+template <class T, int FC, int FJ>
+__global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restrict__ tasks, const SigBlk *__restrict__ blks,
+                                                         const Chi0Seg *__restrict__ segs, const T *__restrict__ CW,
+                                                         long long zcw, const T *__restrict__ U, long long usg,
+                                                         T *__restrict__ s2, long long ssg, int NAO) {
+    using A = typename SV<T>::A;
+    const SigTask tk = tasks[blockIdx.x];
+    const SigBlk B = blks[tk.blk];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, kq = lane >> 4;
+    const int ni = B.ni, nj = B.nj, aj = B.aj, t0 = tk.c0 + 16 * FC * wave;
+    if (t0 >= B.l) return;
+    CW += blockIdx.y * zcw + B.cw;
+    U += blockIdx.y * 2 * usg + B.u + ((long long)B.r * NAO + B.rowI) * nj * aj;
+    s2 += blockIdx.y * 2 * ssg;
+    const Chi0Seg *st = segs + B.seg0;
+    const T *ap[FC];
+#pragma unroll
+    for (int f = 0; f < FC; ++f) ap[f] = CW + (long long)st[min(t0 + 16 * f + c16, B.l - 1)].c * ni * aj + 4 * kq;
+    int uo[FJ];
+#pragma unroll
+    for (int g = 0; g < FJ; ++g) uo[g] = min(tk.j0 + 16 * g + c16, nj - 1) * aj + 4 * kq;
+    A acc[FC][FJ][2];
+#pragma unroll
+    for (int f = 0; f < FC; ++f)
+#pragma unroll
+        for (int g = 0; g < FJ; ++g) acc[f][g][0] = acc[f][g][1] = A{0, 0, 0, 0};
+    struct Frag { T a[FC][4], u[2][FJ][4]; };
+    auto load = [&](Frag &x, int i, int k0) {
+        const int n = aj - k0 - 4 * kq;
+        const T *ub = U + (long long)i * nj * aj + k0;
+#pragma unroll
+        for (int f = 0; f < FC; ++f) load4(x.a[f], ap[f] + i * aj + k0, n);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int g = 0; g < FJ; ++g) load4(x.u[s][g], ub + s * usg + uo[g], n);
+    };
+    int i = 0, k0 = 0;
+    Frag x, y;
+    load(x, i, k0);
+    for (;;) {
+        k0 += 16;
+        if (k0 >= aj) { k0 = 0; ++i; }
+        const bool more = i < ni;
+        if (more) load(y, i, k0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int f = 0; f < FC; ++f)
+#pragma unroll
+                    for (int g = 0; g < FJ; ++g) acc[f][g][s] = mfma(x.a[f][e], x.u[s][g][e], acc[f][g][s]);
+        if (!more) break;
+        x = y;
+    }
+#pragma unroll
+    for (int f = 0; f < FC; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = t0 + 16 * f + acc_row<T>(r, kq);
+            if (t >= B.l) continue;
+            const Chi0Seg sg = st[t];
+#pragma unroll
+            for (int g = 0; g < FJ; ++g) {
+                const int j = tk.j0 + 16 * g + c16;
+                if (j >= nj) continue;
+                T *dst = s2 + ((long long)sg.cell * NAO + sg.row) * NAO + B.colJ + j;
+                unsafeAtomicAdd(dst, acc[f][g][0][r]);
+                unsafeAtomicAdd(dst + ssg, acc[f][g][1][r]);
+            }
+        }
+}
+
+// Y_I[(S, L, l)][i][mu] (+)= sum_(J, R, j) G_IJ(R)[i][j] CW_JI(-R)[(L, S - R, l)][j][mu], both signs: a wave
+// takes one column (S, L, l), 16 FI rows i and 64 mu, and the entries (J, R) of (S, L) with J in
+// [x0, x1) (first chunk: Y is overwritten).  Each element of CW is read once, 16 bytes a lane, for
+// 2 FI MFMAs; G_IJ comes from L2.
+template <class T, int FI>
+__global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restrict__ tasks, const SigYEnt *__restrict__ ents,
+                                                         const T *__restrict__ CW, long long zcw, const T *__restrict__ G,
+                                                         long long zg, T *__restrict__ Y, long long ysg, int NAO, int x0,
+                                                         int x1, int first) {
+    using A = typename SV<T>::A;
+    using V = typename SV<T>::V;
+    constexpr int VL = SV<T>::VL, NV = 4 / VL;
+    const SigYTask tk = tasks[blockIdx.x];
+    const int lane = threadIdx.x & 63, c16 = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = tk.l0 + wave;
+    if (l >= tk.nl) return;
+    CW += blockIdx.y * zcw;
+    G += blockIdx.y * zg + (long long)tk.ao * 2 * NAO;
+    Y += blockIdx.y * 2 * ysg + tk.y;
+    const int ni = tk.ni, ai = tk.ai;
+    int go[FI], mo[NV];
+#pragma unroll
+    for (int f = 0; f < FI; ++f) go[f] = min(tk.i0 + 16 * f + c16, ni - 1) * 2 * NAO;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) mo[v] = min(tk.mu0 + (16 * v + c16) * VL, ai - 1);
+    A acc[FI][4][2];
+#pragma unroll
+    for (int f = 0; f < FI; ++f)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc[f][m][0] = acc[f][m][1] = A{0, 0, 0, 0};
+    struct Frag { T g[2][FI]; V w[NV]; };
+    int e = tk.e0 - 1, s = 0, ns = 0, nj = 0;
+    const T *pg = nullptr, *pw = nullptr;
+    auto next_entry = [&]() {
+        for (++e; e < tk.e1; ++e) {
+            const SigYEnt E = ents[e];
+            if (E.J < x0 || E.J >= x1) continue;
+            nj = E.nj;
+            ns = (nj + 3) / 4;
+            pg = G + E.g;
+            pw = CW + E.b + (long long)tk.abf * E.lb + (long long)(E.cb + l * nj) * ai;
+            return true;
+        }
+        return false;
+    };
+    auto load = [&](Frag &x) {
+        const int j = 4 * s + kq, jc = min(j, nj - 1);
+#pragma unroll
+        for (int f = 0; f < FI; ++f)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const T v = pg[go[f] + q * nj + jc];
+                x.g[q][f] = j < nj ? v : T(0);
+            }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) x.w[v] = *reinterpret_cast<const V *>(pw + (long long)jc * ai + mo[v]);
+    };
+    if (next_entry()) {
+        Frag x, y;
+        load(x);
+        for (;;) {
+            bool more = true;
+            if (++s >= ns) { s = 0; more = next_entry(); }
+            if (more) load(y);
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int f = 0; f < FI; ++f)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) acc[f][m][q] = mfma(x.g[q][f], x.w[m / VL][m % VL], acc[f][m][q]);
+            if (!more) break;
+            x = y;
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < FI; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = tk.i0 + 16 * f + acc_row<T>(r, kq);
+            if (i >= ni) continue;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                T *dst = Y + q * ysg + ((long long)l * ni + i) * ai;
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const int mu = tk.mu0 + (16 * (m / VL) + c16) * VL + m % VL;
+                    if (mu >= ai) continue;
+                    if (first) dst[mu] = acc[f][m][q][r];
+                    else dst[mu] += acc[f][m][q][r];
+                }
+            }
+        }
+}
+
+namespace {
+template <class F> void by_two(int a, int b, F f) {
+    if (a == 1 && b == 1) f(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+    else if (a == 1) f(std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+    else if (b == 1) f(std::integral_constant<int, 2>(), std::integral_constant<int, 1>());
+    else f(std::integral_constant<int, 2>(), std::integral_constant<int, 2>());
+}
+}  // namespace
+
+template <class T>
+void launch_sigma_d(const SigTask *tasks, int ntask, int fi, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
+                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, hipStream_t s) {
+    if (ntask <= 0) return;
+    by_two(fi, fj, [&](auto a, auto b) {
+        hipLaunchKernelGGL((sigma_d_kernel<T, decltype(a)::value, decltype(b)::value>), dim3(ntask, nz), dim3(256), 0, s,
+                           tasks, blks, segs, CW, zcw, U, usg, sig, ssg, NAO);
+    });
+    HIP_CHECK(hipGetLastError());
+}
+template <class T>
+void launch_sigma_b(const SigTask *tasks, int ntask, int fc, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
+                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, hipStream_t s) {
+    if (ntask <= 0) return;
+    by_two(fc, fj, [&](auto a, auto b) {
+        hipLaunchKernelGGL((sigma_b_kernel<T, decltype(a)::value, decltype(b)::value>), dim3(ntask, nz), dim3(256), 0, s,
+                           tasks, blks, segs, CW, zcw, U, usg, s2, ssg, NAO);
+    });
+    HIP_CHECK(hipGetLastError());
+}
+template <class T>
+void launch_sigma_y(const SigYTask *tasks, int ntask, int fi, const SigYEnt *ents, const T *CW, long long zcw, const T *G,
+                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, hipStream_t s) {
+    if (ntask <= 0) return;
+    if (fi == 1)
+        hipLaunchKernelGGL((sigma_y_kernel<T, 1>), dim3(ntask, nz), dim3(256), 0, s, tasks, ents, CW, zcw, G, zg, Y, ysg,
+                           NAO, x0, x1, (int)first);
+    else
+        hipLaunchKernelGGL((sigma_y_kernel<T, 2>), dim3(ntask, nz), dim3(256), 0, s, tasks, ents, CW, zcw, G, zg, Y, ysg,
+                           NAO, x0, x1, (int)first);
+    HIP_CHECK(hipGetLastError());
+}
+#define LRA_SIGMA(T)                                                                                                    \
+    template void launch_sigma_d<T>(const SigTask *, int, int, int, const SigBlk *, const Chi0Seg *, const T *, long long, \
+                                    const T *, long long, T *, long long, int, int, hipStream_t);                       \
+    template void launch_sigma_b<T>(const SigTask *, int, int, int, const SigBlk *, const Chi0Seg *, const T *, long long, \
+                                    const T *, long long, T *, long long, int, int, hipStream_t);                       \
+    template void launch_sigma_y<T>(const SigYTask *, int, int, const SigYEnt *, const T *, long long, const T *, long long, \
+                                    T *, long long, int, int, int, bool, int, hipStream_t);
+LRA_SIGMA(double)
+LRA_SIGMA(float)
+#undef LRA_SIGMA
+
+// blockIdx.y: tau point and sign
+template <class T>
+__global__ void sigma_fold_kernel(T *__restrict__ sig, const T *__restrict__ s2, const T *__restrict__ ext,
+                                  const int *__restrict__ fold, const int *__restrict__ neg, int NE, int nR, int n) {
     const long long nn = (long long)n * n;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nn * nR) return;
+    sig += blockIdx.y * nn * nR;
+    s2 += blockIdx.y * nn * nR;
+    ext += blockIdx.y * nn * NE;
     const int R = (int)(idx / nn);
     const long long ab = idx % nn;
     const int a = (int)(ab / n), b = (int)(ab % n);
-    T acc = 0;
-    for (int e = 0; e < NE; ++e) {
-        if (fold[e] == R) acc += extA[(long long)e * nn + ab] + extB[(long long)e * nn + ab];
-        if (foldneg[e] == R) acc += extB[(long long)e * nn + (long long)b * n + a];
-    }
+    T acc = s2[idx] + s2[neg[R] * nn + (long long)b * n + a];
+    for (int e = 0; e < NE; ++e)
+        if (fold[e] == R) acc += ext[(long long)e * nn + ab];
     sig[idx] += acc;
 }
 
 template <class T>
-void launch_sigma_fold(T *sig, const T *extA, const T *extB, const int *fold, const int *foldneg, int NE, int nR,
-                       int n, hipStream_t s) {
-    hipLaunchKernelGGL(sigma_fold_kernel<T>, dim3(ceil_div((long long)n * n * nR, 256)), dim3(256), 0, s, sig, extA,
-                       extB, fold, foldneg, NE, nR, n);
+void launch_sigma_fold(T *sig, const T *s2, const T *ext, const int *fold, const int *neg, int NE, int nR, int n,
+                       int nz, hipStream_t s) {
+    hipLaunchKernelGGL(sigma_fold_kernel<T>, dim3(ceil_div((long long)n * n * nR, 256), 2 * nz), dim3(256), 0, s, sig,
+                       s2, ext, fold, neg, NE, nR, n);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_sigma_fold<double>(double *, const double *, const double *, const int *, const int *, int, int,
-                                        int, hipStream_t);
-template void launch_sigma_fold<float>(float *, const float *, const float *, const int *, const int *, int, int,
+                                        int, int, hipStream_t);
+template void launch_sigma_fold<float>(float *, const float *, const float *, const int *, const int *, int, int, int,
                                        int, hipStream_t);
 
+// blockIdx.y: frequency; the tau points of a pass are added in their order
 template <class T>
-__global__ void sigma_freq_kernel(const T *__restrict__ sp, const T *__restrict__ sn, long long nelem,
-                                  const double *__restrict__ cw, const double *__restrict__ sw, int nw,
-                                  double *__restrict__ sre, double *__restrict__ sim) {
+__global__ void sigma_freq_kernel(const T *__restrict__ sig, long long nelem, const double *__restrict__ cw,
+                                  const double *__restrict__ sw, int ntau, int it0, int nz, double *__restrict__ sre,
+                                  double *__restrict__ sim) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nelem) return;
-    const double p = static_cast<double>(sp[i]), m = static_cast<double>(sn[i]);
-    const double c = 0.5 * (p + m), d = 0.5 * (p - m);
-    for (int w = 0; w < nw; ++w) {
-        sre[(long long)w * nelem + i] += c * cw[w];
-        sim[(long long)w * nelem + i] += d * sw[w];
+    const int w = blockIdx.y;
+    double re = sre[(long long)w * nelem + i], im = sim[(long long)w * nelem + i];
+    for (int z = 0; z < nz; ++z) {
+        const double p = static_cast<double>(sig[2ll * z * nelem + i]), m = static_cast<double>(sig[(2ll * z + 1) * nelem + i]);
+        re += 0.5 * (p + m) * cw[w * ntau + it0 + z];
+        im += 0.5 * (p - m) * sw[w * ntau + it0 + z];
     }
+    sre[(long long)w * nelem + i] = re;
+    sim[(long long)w * nelem + i] = im;
 }
 
 template <class T>
-void launch_sigma_freq(const T *sp, const T *sn, long long nelem, const double *cw, const double *sw, int nw,
-                       double *sre, double *sim, hipStream_t s) {
-    hipLaunchKernelGGL(sigma_freq_kernel<T>, dim3(ceil_div(nelem, 256)), dim3(256), 0, s, sp, sn, nelem, cw, sw, nw,
-                       sre, sim);
+void launch_sigma_freq(const T *sig, long long nelem, const double *cw, const double *sw, int nw, int ntau, int it0,
+                       int nz, double *sre, double *sim, hipStream_t s) {
+    hipLaunchKernelGGL(sigma_freq_kernel<T>, dim3(ceil_div(nelem, 256), nw), dim3(256), 0, s, sig, nelem, cw, sw, ntau,
+                       it0, nz, sre, sim);
     HIP_CHECK(hipGetLastError());
 }
-template void launch_sigma_freq<double>(const double *, const double *, long long, const double *, const double *,
-                                        int, double *, double *, hipStream_t);
-template void launch_sigma_freq<float>(const float *, const float *, long long, const double *, const double *, int,
+template void launch_sigma_freq<double>(const double *, long long, const double *, const double *, int, int, int, int,
+                                        double *, double *, hipStream_t);
+template void launch_sigma_freq<float>(const float *, long long, const double *, const double *, int, int, int, int,
                                        double *, double *, hipStream_t);
 
 constexpr int kStMax = 16;
