@@ -5,9 +5,10 @@
 // with v = L L^H (Cholesky) and M = 1 - L^H chi0 L, exact when the truncated Coulomb
 // equals the bare one.  L M^{-1} L^H - v is read off as minus the Schur complement of
 // the augmented matrix [[M, L^H], [L, v]] after eliminating its first block column with
-// the signed blocked Cholesky; complex q use the real embedding [[Re, -Im], [Im, Re]].
+// the signed blocked Cholesky; with k points all matrices are held as real and imaginary planes.
+// All frequencies of as many q as memory allows go through every step together.
 // W(R, tau) = Re sum_w gamma_f2t(tau, w) (1/N_k) sum_q e^{-i 2 pi q.R} Wc(q, w)
-// (CT_FT_Wc_freq_q, epsilon.cpp:2490-2666) is accumulated per q on the device.  With an IBZ
+// (CT_FT_Wc_freq_q, epsilon.cpp:2490-2666) is accumulated on the device.  With an IBZ
 // mapping only the irreducible q are formed; the others must be their time-reversal partners
 // (FT_Wc_freq_q, epsilon.cpp:2430-2452, takes W(-q) = conj W(q)), whose real parts of
 // e^{-i 2 pi q.R} W(q) are equal, so each irreducible q is weighted by its star size.
@@ -181,7 +182,9 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
     std::vector<long long> cw_x(natom);  // CW of atom x in its chunk: [R][J][c][i][nu]
     {
         const double fixed = 2.0 * per_sign + 8.0 * ntau * nR * (double)NABF * NABF;
-        const double budget = std::max(4e9, std::min(96e9, 0.6 * (double)free_b - fixed));
+        double budget = std::max(4e9, std::min(96e9, 0.6 * (double)free_b - fixed));
+        if (const char *cb = std::getenv("LIBRPA_AMD_CHUNK_BYTES"))
+            if (std::atof(cb) > 0) budget = std::min(budget, std::atof(cb));
         int x = 0;
         while (x < natom) {
             XChunk c;
@@ -313,44 +316,80 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
 // W(q, omega) -> W(R, tau)
 // ------------------------------------------------------------------------------------------
 namespace {
-// Principal square root of a symmetric positive-definite n x n matrix A (in place) by the coupled
-// Newton-Schulz iteration Y <- Y T, Z <- T Z, T = (3 I - Z Y) / 2 from Y = A / c, Z = I with
+// C = A B of nmat matrices, real or of two planes each, nn elements apart; the operands of matrix m at
+// a[m], b[m] (offsets), the results compact
+GemmBatch square_batch(int n, bool herm, const std::vector<long long> &a, const std::vector<long long> &b, hipStream_t st) {
+    GemmBatch out;
+    const long long plane = (long long)n * n, nn = plane * (herm ? 2 : 1);
+    for (size_t m = 0; m < a.size(); ++m)
+        for (int h = 0; h < (herm ? 2 : 1); ++h) {
+            GemmProb p = make_prob(n, n, n, a[m], n, b[m] + h * plane, n, (long long)m * nn + h * plane, n);
+            if (herm) {
+                p.sgn2 = h ? 1 : -1;
+                p.a_off2 = a[m] + plane;
+                p.b_off2 = b[m] + (1 - h) * plane;
+            }
+            out.add(p);
+        }
+    // a single small matrix on few workgroups is bound by one tile's K loop: smaller tiles
+    out.finalize((double)n * n * out.probs.size() < 64.0 * 64 * 512 ? T32x64 : T64x64, st);
+    return out;
+}
+
+// Principal square roots of the Hermitian positive-definite matrices A + sel[m] nn (in place) by the
+// coupled Newton-Schulz iteration Y <- Y T, Z <- T Z, T = (3 I - Z Y) / 2 from Y = A / c, Z = I with
 // c = ||A||_F >= lambda_max; Y -> (A / c)^{1/2}.  Equals the eigen-decomposition root of
-// power_hemat (src/math/matrix_m.h:916-970) for positive-definite input.  Runs to convergence.
-void ns_sqrt(double *A, int n, hipStream_t st) {
-    const size_t nn = (size_t)n * n;
-    DevBuf dY(nn * 8), dZ(nn * 8), dT(nn * 8), dP(nn * 8), dYn(nn * 8), dZn(nn * 8), dr(64);
-    GemmBatch b;
-    b.add(make_prob(n, n, n, 0, n, 0, n, 0, n));
-    b.finalize(T64x64, st);
-    launch_sumsq(A, (long long)nn, dr.as<double>(), st);
-    double h[2];
-    HIP_CHECK(hipMemcpyAsync(h, dr.get(), 8, hipMemcpyDeviceToHost, st));
+// power_hemat (src/math/matrix_m.h:916-970) for positive-definite input.  Runs to convergence, all
+// matrices together; the host looks at the changes of every fourth iteration's batch only.
+void ns_sqrt(double *A, int n, bool herm, const std::vector<int> &sel, hipStream_t st) {
+    if (sel.empty()) return;
+    const int nm = (int)sel.size(), pl = herm ? 2 : 1;
+    const size_t nn = (size_t)n * n * pl, all = nn * 8 * nm;
+    constexpr int kMax = 200, kLook = 4;
+    DevBuf dY(all), dZ(all), dP(all), dYn(all), dZn(all), dpart(32 * 8 * (size_t)nm), dscale(8 * (size_t)nm),
+        dchg(sizeof(unsigned long long) * 2 * nm * kMax);
+    DevBuf dsel = upload(sel, st);
+    std::vector<long long> at(nm);
+    for (int m = 0; m < nm; ++m) at[m] = (long long)m * (long long)nn;
+    GemmBatch b = square_batch(n, herm, at, at, st);
+    HIP_CHECK(hipMemsetAsync(dchg.get(), 0, dchg.bytes(), st));
+    launch_ns_init(A, dsel.as<int>(), nm, n, pl, dpart.as<double>(), dY.as<double>(), dZ.as<double>(),
+                   dscale.as<double>(), st);
+    std::vector<double> c(nm), h(2 * (size_t)nm * kLook), prev(nm, 1e300);
+    std::vector<int> stall(nm, 0);
+    std::vector<char> done(nm, 0);
+    HIP_CHECK(hipMemcpyAsync(c.data(), dscale.get(), 8 * (size_t)nm, hipMemcpyDeviceToHost, st));
     HIP_CHECK(hipStreamSynchronize(st));
-    const double c = std::sqrt(h[0]);
-    if (!(c > 0) || !std::isfinite(c)) LRA_THROW("Coulomb matrix is zero or not finite");
-    launch_scale_add_identity(A, dY.as<double>(), n, 1.0 / c, 0.0, st);
-    launch_scale_add_identity(A, dZ.as<double>(), n, 0.0, 1.0, st);
-    double prev = 1e300;
-    int stall = 0;
-    for (int k = 0; k < 200; ++k) {
-        gemm_run(Prec::F64, b, dZ.get(), dY.get(), dP.get(), 1.0, 0.0, st);
-        launch_scale_add_identity(dP.as<double>(), dT.as<double>(), n, -0.5, 1.5, st);
-        gemm_run(Prec::F64, b, dY.get(), dT.get(), dYn.get(), 1.0, 0.0, st);
-        gemm_run(Prec::F64, b, dT.get(), dZ.get(), dZn.get(), 1.0, 0.0, st);
-        launch_absmax_diff(dYn.as<double>(), dY.as<double>(), (long long)nn, dr.as<double>(), st);
-        HIP_CHECK(hipMemcpyAsync(h, dr.get(), 16, hipMemcpyDeviceToHost, st));
+    for (double x : c)
+        if (!(x > 0) || !std::isfinite(x)) LRA_THROW("Coulomb matrix is zero or not finite");
+    bool all_done = false;
+    for (int k0 = 0; k0 < kMax && !all_done; k0 += kLook) {
+        for (int k = k0; k < k0 + kLook; ++k) {
+            gemm_run(Prec::F64, b, dZ.get(), dY.get(), dP.get(), 1.0, 0.0, st);
+            launch_ns_step(dP.as<double>(), nm, n, pl, st);
+            gemm_run(Prec::F64, b, dY.get(), dP.get(), dYn.get(), 1.0, 0.0, st);
+            gemm_run(Prec::F64, b, dP.get(), dZ.get(), dZn.get(), 1.0, 0.0, st);
+            launch_ns_change(dYn.as<double>(), dY.as<double>(), nm, n, pl, dchg.as<unsigned long long>() + 2 * (size_t)nm * k, st);
+            std::swap(dY, dYn);
+            std::swap(dZ, dZn);
+        }
+        HIP_CHECK(hipMemcpyAsync(h.data(), dchg.as<unsigned long long>() + 2 * (size_t)nm * k0, 8 * h.size(),
+                                 hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
-        std::swap(dY, dYn);
-        std::swap(dZ, dZn);
-        const double rel = h[0] / std::max(h[1], 1e-300);
-        if (!std::isfinite(rel)) LRA_THROW("square root of the Coulomb matrix did not converge (not positive definite?)");
-        // quadratic phase ends at rounding level: stop once the update no longer shrinks
-        if (rel < 1e-13) { if (rel >= prev || ++stall >= 3) break; }
-        prev = rel;
-        if (k == 199) LRA_THROW("square root of the Coulomb matrix did not converge");
+        all_done = true;
+        for (int m = 0; m < nm; ++m) {
+            for (int k = 0; k < kLook && !done[m]; ++k) {
+                const double rel = h[2 * ((size_t)k * nm + m)] / std::max(h[2 * ((size_t)k * nm + m) + 1], 1e-300);
+                if (!std::isfinite(rel)) LRA_THROW("square root of the Coulomb matrix did not converge (not positive definite?)");
+                // quadratic phase ends at rounding level: stop once the update no longer shrinks
+                if (rel < 1e-13 && (rel >= prev[m] || ++stall[m] >= 3)) done[m] = 1;
+                prev[m] = rel;
+            }
+            all_done = all_done && done[m];
+        }
     }
-    launch_scale_add_identity(dY.as<double>(), A, n, std::sqrt(c), 0.0, st);
+    if (!all_done) LRA_THROW("square root of the Coulomb matrix did not converge");
+    launch_ns_finish(dY.as<double>(), dscale.as<double>(), dsel.as<int>(), nm, n, pl, A, st);
     HIP_CHECK(hipStreamSynchronize(st));
 }
 
@@ -413,32 +452,33 @@ std::pair<double, double> eig_sqrt(double *A, int n, double thr, double *top, in
     return {l0, l1};
 }
 
-// The upper atom-pair blocks (I <= J) of a Coulomb input for every k, staged on the device for
-// launch_v_scatter, with the largest |V| and |Im V| of each k.
+// The upper atom-pair blocks (I <= J) of a Coulomb input for the k points qs, staged on the device for
+// launch_v_scatter (VBlock::q: position in qs), with the largest |V| and |Im V| of each.
 struct CoulombStage {
     DevBuf blk, desc;
-    std::vector<int> first;  // descriptors of k: [first[k], first[k + 1])
+    std::vector<int> first;  // descriptors of qs[i]: [first[i], first[i + 1])
     std::vector<double> vmax, imax;
 };
-void stage_coulomb(const RpaEngine &R0, const std::map<std::tuple<int, int, int>, std::vector<cplx>> &store, int nk,
-                   CoulombStage &out, hipStream_t st) {
+void stage_coulomb(const RpaEngine &R0, const std::map<std::tuple<int, int, int>, std::vector<cplx>> &store,
+                   const std::vector<int> &qs, CoulombStage &out, hipStream_t st) {
     std::vector<VBlock> desc;
     std::vector<cplx> vals;
     out.first.assign(1, 0);
-    out.vmax.assign(nk, 0.0);
-    out.imax.assign(nk, 0.0);
-    for (int k = 0; k < nk; ++k) {
-        for (const auto &kv : store) {
-            const int ik = std::get<0>(kv.first), I = std::get<1>(kv.first), J = std::get<2>(kv.first);
-            if (ik != k || I > J) continue;
-            if (kv.second.size() != (size_t)R0.na[I] * R0.na[J]) LRA_THROW("Coulomb block of the wrong size");
-            for (const cplx &v : kv.second) {
-                out.vmax[k] = std::max(out.vmax[k], std::abs(v));
-                out.imax[k] = std::max(out.imax[k], std::fabs(v.imag()));
+    out.vmax.assign(qs.size(), 0.0);
+    out.imax.assign(qs.size(), 0.0);
+    for (size_t i = 0; i < qs.size(); ++i) {
+        for (auto it = store.lower_bound({qs[i], 0, 0}); it != store.end() && std::get<0>(it->first) == qs[i]; ++it) {
+            const int I = std::get<1>(it->first), J = std::get<2>(it->first);
+            if (I > J) continue;
+            if (it->second.size() != (size_t)R0.na[I] * R0.na[J]) LRA_THROW("Coulomb block of the wrong size");
+            for (const cplx &v : it->second) {
+                out.vmax[i] = std::max(out.vmax[i], std::norm(v));
+                out.imax[i] = std::max(out.imax[i], std::fabs(v.imag()));
             }
-            desc.push_back({(long long)vals.size(), (int)R0.abf[I], (int)R0.abf[J], R0.na[I], R0.na[J], I == J ? 1 : 0, 0});
-            vals.insert(vals.end(), kv.second.begin(), kv.second.end());
+            desc.push_back({(long long)vals.size(), (int)R0.abf[I], (int)R0.abf[J], R0.na[I], R0.na[J], I == J ? 1 : 0, (int)i});
+            vals.insert(vals.end(), it->second.begin(), it->second.end());
         }
+        out.vmax[i] = std::sqrt(out.vmax[i]);
         out.first.push_back((int)desc.size());
     }
     out.blk = upload(vals, st);
@@ -446,12 +486,12 @@ void stage_coulomb(const RpaEngine &R0, const std::map<std::tuple<int, int, int>
     HIP_CHECK(hipStreamSynchronize(st));
 }
 
-// dense (embedded when complex) Hermitian matrix of k point kq into V (device)
-void dense_coulomb(const CoulombStage &cs, int kq, int n, int n2, bool embed, bool real_part, double *V,
-                   hipStream_t st) {
-    HIP_CHECK(hipMemsetAsync(V, 0, sizeof(double) * (size_t)n2 * n2, st));
-    launch_v_scatter(cs.blk.as<double>(), cs.desc.as<VBlock>() + cs.first[kq], cs.first[kq + 1] - cs.first[kq], V, n,
-                     embed ? kEmbedded : kReal, real_part ? 1 : 0, 0, 0, st);
+// dense matrices of qs[i0, i0 + cnt) into V, stride elements apart
+void dense_coulomb(const CoulombStage &cs, int i0, int cnt, int n, DenseLayout lay, bool real_part, double *V,
+                   long long stride, hipStream_t st) {
+    HIP_CHECK(hipMemsetAsync(V, 0, sizeof(double) * (size_t)stride * cnt, st));
+    launch_v_scatter(cs.blk.as<double>(), cs.desc.as<VBlock>() + cs.first[i0], cs.first[i0 + cnt] - cs.first[i0], V, n,
+                     lay, real_part ? 1 : 0, i0, stride, st);
 }
 }  // namespace
 
@@ -495,43 +535,71 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
         auto it = ds.vq_cut.find(kv.first);
         same_cut = same_cut && it != ds.vq_cut.end() && it->second.size() == kv.second.size();
         for (size_t i = 0; same_cut && i < kv.second.size(); ++i)
-            same_cut = std::abs(it->second[i] - kv.second[i]) <= 1e-12 * (1.0 + std::abs(kv.second[i]));
+            same_cut = it->second[i] == kv.second[i] ||
+                       std::abs(it->second[i] - kv.second[i]) <= 1e-12 * (1.0 + std::abs(kv.second[i]));
     }
 
-    const bool embed = nk > 1;
-    const int n2 = embed ? 2 * n : n;
-    const int N = 2 * n2;
-    const size_t nn = (size_t)n2 * n2, NN = (size_t)N * N;
+    const bool herm = nk > 1;
+    const DenseLayout lay = herm ? kPlanar : kReal;
+    const int N = 2 * n, pl = herm ? 2 : 1;
+    const long long plane = (long long)n * n, nn = plane * pl, im = herm ? 4 * plane : 0, NN = 4 * plane * pl;
+    std::vector<int> qs;
+    for (int k = 0; k < nk; ++k)
+        if (mult[k] > 0) qs.push_back(k);
+    const int nq = (int)qs.size();
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
     // chi0(R, omega) once for all q when it fits in a quarter of the free memory
     if (!R0.chiw_ok && R0.form_chiw(g, 0.25 * (double)free_b, st)) HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    const double per_w = 8.0 * (NN + 2.0 * nn);
-    const double budget = std::min(160e9, 0.7 * (double)free_b) - 8.0 * 10 * nn;
+    // all frequencies of several q per pass (q is the inner loop of every launch), or some of one q
+    const double per_w = 8.0 * ((double)NN + 2.0 * nn) + 16.0 * pl * N * (N >= (herm ? 2048 : 4096) ? (herm ? 1024 : 2048) : (herm ? 256 : 512));
+    const double per_q = 8.0 * 14 * nn;
+    const double budget = std::min(160e9, 0.7 * (double)free_b) - per_q;
     const int WCH = std::max(1, std::min(nw, (int)(budget / per_w)));
-    DevBuf dV0(nn * 8), dL(nn * 8), dD(nn * 8 * WCH), dX(nn * 8 * WCH), dA(NN * 8 * WCH), dacc(sizeof(double) * (WCH + 8));
-    // pivot signs of v = L S L^T: a negative pivot means v^{1/2} must come from the eigen-decomposition
-    // with the negative eigenvalues dropped (power_hemat, matrix_m.h:916-970)
-    DevBuf dSg((size_t)n2 * 8), dProbe, dProbeFlag(16);
+    const int QG = WCH < nw ? 1 : std::max(1, std::min(nq, (int)((budget + per_q) / (nw * per_w + per_q))));
+    const int UCH = QG > 1 ? QG * nw : WCH;
+    // F: v and then its factor (Cholesky, or square root); C: v_c and then its root; V0: v_c, or S_c S_c
+    // when a root is filtered
+    DevBuf dFC(nn * 8 * 2 * QG), dV0(nn * 8 * QG), dD(nn * 8 * UCH), dX(nn * 8 * UCH), dA(NN * 8 * UCH), dacc(8 * (size_t)UCH),
+        dflag(16);
+    double *F = dFC.as<double>(), *C = F + nn * QG, *V0 = dV0.as<double>();
+    DevBuf dSg((size_t)n * 8 * 2 * QG), dProbe, dld(8 * 2 * (size_t)QG), dE;
     std::vector<double> hsg;
-    int *dflag = reinterpret_cast<int *>(dacc.as<double>() + WCH + 4);
     HIP_CHECK(hipMemsetAsync(dacc.get(), 0, dacc.bytes(), st));
+    HIP_CHECK(hipMemsetAsync(dflag.get(), 0, 16, st));
     CholWork cw;
-    DevBuf dSc;
-    auto negative_pivot = [&](const double *M) {
-        dProbe.reserve(nn * 8);
-        HIP_CHECK(hipMemcpyAsync(dProbe.get(), M, nn * 8, hipMemcpyDeviceToDevice, st));
-        HIP_CHECK(hipMemsetAsync(dProbeFlag.get(), 0, 16, st));
-        cholesky_logdet(dProbe.as<double>(), n2, n2, dProbeFlag.as<double>(), reinterpret_cast<int *>(dProbeFlag.as<double>() + 1),
-                        true, cw, st, dSg.as<double>());
-        hsg.resize(n2);
-        HIP_CHECK(hipMemcpyAsync(hsg.data(), dSg.get(), (size_t)n2 * 8, hipMemcpyDeviceToHost, st));
-        int zf = 0;
-        HIP_CHECK(hipMemcpyAsync(&zf, dProbeFlag.as<double>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIP_CHECK(hipStreamSynchronize(st));
-        bool neg = zf != 0;  // a zero pivot also needs the filtered root
-        for (double v : hsg) neg = neg || v < 0;
-        return neg;
+    // L S L^H of cnt matrices in place; which of them have a zero or negative pivot: v^{1/2} must then come
+    // from the eigen-decomposition with the negative eigenvalues dropped (power_hemat, matrix_m.h:916-970).
+    // A zero pivot raises the flag of the whole batch, whose matrices are then looked at one by one.
+    auto factor = [&](double *M, int cnt, std::vector<char> &neg) {
+        neg.assign(cnt, 0);
+        DevBuf keep;
+        if (cnt > 1) {
+            keep.alloc(nn * 8 * cnt);
+            HIP_CHECK(hipMemcpyAsync(keep.get(), M, nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
+        }
+        auto run = [&](int m0, int m1) {
+            HIP_CHECK(hipMemsetAsync(dld.get(), 0, dld.bytes(), st));
+            HIP_CHECK(hipMemsetAsync(dflag.as<int>() + 1, 0, sizeof(int), st));
+            cholesky_logdet_batched(M + m0 * nn, nn, m1 - m0, n, n, dld.as<double>(), 1, dflag.as<int>() + 1, true, cw, st,
+                                    -1, dSg.as<double>(), n, herm ? plane : 0);
+            hsg.resize((size_t)n * (m1 - m0));
+            int zf = 0;
+            HIP_CHECK(hipMemcpyAsync(hsg.data(), dSg.get(), 8 * hsg.size(), hipMemcpyDeviceToHost, st));
+            HIP_CHECK(hipMemcpyAsync(&zf, dflag.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
+            HIP_CHECK(hipStreamSynchronize(st));
+            for (int m = m0; m < m1; ++m)
+                for (int i = 0; i < n; ++i)
+                    if (!(hsg[(size_t)(m - m0) * n + i] > 0)) neg[m] = 1;
+            return zf != 0;
+        };
+        if (!run(0, cnt)) return;
+        if (cnt == 1) { neg[0] = 1; return; }
+        HIP_CHECK(hipMemcpyAsync(M, keep.get(), nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
+        for (int m = 0; m < cnt; ++m) {
+            neg[m] = 0;
+            if (run(m, m + 1)) neg[m] = 1;
+        }
     };
     // head replacement at q = 0: eps_mac per frequency and the leading eigenvector of Re v(0)
     DevBuf dHead, dU0((size_t)n * 8), dQ(sizeof(double) * (WCH + 1));
@@ -540,155 +608,191 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
         dHead = upload(head, st);
     }
     CoulombStage vst, vcst;
-    stage_coulomb(R0, ds.vq, nk, vst, st);
-    if (!same_cut) stage_coulomb(R0, ds.vq_cut, nk, vcst, st);
-    std::map<std::pair<int, bool>, std::pair<GemmBatch, GemmBatch>> batches;
-    auto get_batches = [&](int cnt, bool tri) -> std::pair<GemmBatch, GemmBatch> & {
-        auto it = batches.find({cnt, tri});
+    stage_coulomb(R0, ds.vq, qs, vst, st);
+    if (!same_cut) stage_coulomb(R0, ds.vq_cut, qs, vcst, st);
+    // filtered root of one matrix, through the real embedding when there are k points
+    auto eig_root = [&](double *M, double *top) {
+        if (!herm) return eig_sqrt(M, n, sqrt_threshold, top, 1, st);
+        dE.reserve(4 * plane * 8);
+        launch_planes_to_embedded(M, dE.as<double>(), n, st);
+        const auto r = eig_sqrt(dE.as<double>(), 2 * n, sqrt_threshold, top, 2, st);
+        launch_embedded_to_planes(dE.as<double>(), M, n, st);
+        HIP_CHECK(hipStreamSynchronize(st));
+        return r;
+    };
+    std::map<std::tuple<int, int, bool>, std::pair<GemmBatch, GemmBatch>> batches;
+    auto get_batches = [&](int qg, int cnt, bool tri) -> std::pair<GemmBatch, GemmBatch> & {
+        auto it = batches.find({qg, cnt, tri});
         if (it != batches.end()) return it->second;
-        auto &pr = batches[{cnt, tri}];
+        auto &pr = batches[{qg, cnt, tri}];
         GemmBatch &bx = pr.first, &bm = pr.second;
         bm.trans_a = true;
         bm.lower_only = true;
-        for (int w = 0; w < cnt; ++w) {
-            GemmProb px = make_prob(n2, n2, n2, (long long)w * nn, n2, 0, n2, (long long)w * nn, n2);
-            px.kmode = tri ? 1 : 0;  // triangular Cholesky factor, or the full square root
-            bx.add(px);
-            GemmProb pm = make_prob(n2, n2, n2, 0, n2, (long long)w * nn, n2, (long long)w * NN, N);
-            pm.kmode = tri ? 2 : 0;
-            bm.add(pm);
-        }
-        const int cfg = T64x64;
-        bx.finalize(cfg, st);
-        bm.finalize(cfg, st);
-        bx.flops = 2.0 * cnt * (double)n2 * n2 * n2 / 2.0;
-        bm.flops = 2.0 * cnt * (double)n2 * n2 * n2 / 6.0;
+        for (int qi = 0; qi < qg; ++qi)
+            for (int w = 0; w < cnt; ++w)
+                for (int h = 0; h < pl; ++h) {
+                    // plane h of X = D F and of F^H X
+                    const long long u = ((long long)qi * cnt + w), l = qi * nn;
+                    GemmProb px = make_prob(n, n, n, u * nn, n, l + h * plane, n, u * nn + h * plane, n);
+                    px.kmode = tri ? 1 : 0;  // triangular Cholesky factor, or the full square root
+                    GemmProb pm = make_prob(n, n, n, l, n, u * nn + h * plane, n, u * NN + h * im, N);
+                    pm.kmode = tri ? 2 : 0;
+                    if (herm) {
+                        px.sgn2 = h ? 1 : -1;
+                        px.a_off2 = u * nn + plane;
+                        px.b_off2 = l + (1 - h) * plane;
+                        pm.sgn2 = h ? -1 : 1;
+                        pm.a_off2 = l + plane;
+                        pm.b_off2 = u * nn + (1 - h) * plane;
+                    }
+                    bx.add(px);
+                    bm.add(pm);
+                }
+        bx.finalize(T64x64, st);
+        bm.finalize(T64x64, st);
         return pr;
     };
     const auto &cells = R0.cells;
-    for (int iq = 0; iq < nk; ++iq) {
-        if (mult[iq] == 0) continue;
-        const double *kf = &ds.kfrac[(size_t)iq * 3];
-        const bool gamma = std::fabs(kf[0]) < 1e-12 && std::fabs(kf[1]) < 1e-12 && std::fabs(kf[2]) < 1e-12;
-        const double vmax = vst.vmax[iq], imax = vst.imax[iq];
-        const bool head_q = gamma && !head.empty();
-        bool eig_v = sqrt_threshold > 0 || head_q, eig_vc = sqrt_threshold > 0;
-        bool chol = false;  // v_c = v with v = L S L^T, S = I: the Cholesky identity
-        // v^{1/2} from Re v at q = 0 (power_hemat_blacs_real, epsilon.cpp:2019-2024)
-        if (same_cut && gamma && imax > 1e-12 * std::max(vmax, 1e-300))
-            LRA_THROW("W at q = 0 with v_c = v needs a real Coulomb matrix (Im v(0) != 0)");
-        if (same_cut && !eig_v) {
-            dense_coulomb(vst, iq, n, n2, embed, gamma, dV0.as<double>(), st);
-            HIP_CHECK(hipMemcpyAsync(dL.get(), dV0.get(), nn * 8, hipMemcpyDeviceToDevice, st));
-            prof.begin("gw_w_chol_v", st);
-            HIP_CHECK(hipMemsetAsync(dProbeFlag.get(), 0, 16, st));
-            cholesky_logdet(dL.as<double>(), n2, n2, dProbeFlag.as<double>(),
-                            reinterpret_cast<int *>(dProbeFlag.as<double>() + 1), true, cw, st, dSg.as<double>());
-            hsg.resize(n2);
-            int zf = 0;
-            HIP_CHECK(hipMemcpyAsync(hsg.data(), dSg.get(), (size_t)n2 * 8, hipMemcpyDeviceToHost, st));
-            HIP_CHECK(hipMemcpyAsync(&zf, dProbeFlag.as<double>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-            HIP_CHECK(hipStreamSynchronize(st));
-            chol = zf == 0;  // a zero or negative pivot needs the filtered root
-            for (double v : hsg) chol = chol && v > 0;
-            eig_v = eig_vc = !chol;
-            prof.end("gw_w_chol_v", st, (double)n2 * n2 * n2 / 3.0);
+    for (int iq0 = 0; iq0 < nq; iq0 += QG) {
+        const int qg = std::min(QG, nq - iq0);
+        if (verbose) { fprintf(stderr, "[librpa-mi355x] W: q %d / %d (%.1f s)\n", qs[iq0] + 1, nk, now_s() - t0); fflush(stderr); }
+        std::vector<const double *> kfs(qg);
+        int gamma = -1;  // position of q = 0 in the pass
+        for (int i = 0; i < qg; ++i) {
+            kfs[i] = &ds.kfrac[(size_t)qs[iq0 + i] * 3];
+            if (std::fabs(kfs[i][0]) < 1e-12 && std::fabs(kfs[i][1]) < 1e-12 && std::fabs(kfs[i][2]) < 1e-12) gamma = i;
         }
-        if (!chol) {
-            // dL <- S = v^{1/2}; dSc <- S_c = v_c^{1/2} (complex v_c kept, as the reference does);
-            // dV0 <- v_c, or S_c S_c when a root is filtered
-            if (!same_cut && !embed && vcst.imax[iq] > 1e-12 * std::max(vcst.vmax[iq], 1e-300))
-                LRA_THROW("a complex truncated Coulomb matrix at Gamma-only sampling is outside this build");
+        const bool head_here = gamma >= 0 && !head.empty();
+        // v^{1/2} from Re v at q = 0 (power_hemat_blacs_real, epsilon.cpp:2019-2024)
+        if (gamma >= 0 && same_cut && vst.imax[iq0 + gamma] > 1e-12 * std::max(vst.vmax[iq0 + gamma], 1e-300))
+            LRA_THROW("W at q = 0 with v_c = v needs a real Coulomb matrix (Im v(0) != 0)");
+        auto fill_v = [&](double *dst) {
+            dense_coulomb(vst, iq0, qg, n, lay, false, dst, nn, st);
+            if (gamma >= 0) dense_coulomb(vst, iq0 + gamma, 1, n, lay, true, dst + gamma * nn, nn, st);
+        };
+        std::vector<char> neg(qg, 0), negc(qg, 0);
+        bool tri = same_cut && sqrt_threshold <= 0;  // every factor of the pass is a Cholesky factor
+        if (tri) {
+            // v_c = v with v = L S L^T, S = I: the Cholesky identity
+            prof.begin("gw_w_chol_v", st);
+            fill_v(V0);
+            HIP_CHECK(hipMemcpyAsync(F, V0, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+            factor(F, qg, neg);
+            prof.end("gw_w_chol_v", st, (herm ? 4.0 : 1.0) * qg * n * (double)n * n / 3.0);
+        }
+        std::vector<char> chol(qg, 0);
+        for (int i = 0; i < qg; ++i) {
+            chol[i] = same_cut && sqrt_threshold <= 0 && !neg[i] && !(head_here && i == gamma);
+            tri = tri && chol[i];
+        }
+        if (tri || (same_cut && std::count(chol.begin(), chol.end(), 1) > 0))
+            HIP_CHECK(hipMemcpyAsync(C, F, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+        if (!tri) {
+            // F <- S = v^{1/2}; C <- S_c = v_c^{1/2} (complex v_c kept, as the reference does);
+            // V0 <- v_c, or S_c S_c when a root is filtered
             prof.begin("gw_w_sqrt_v", st);
-            dense_coulomb(vst, iq, n, n2, embed, gamma, dL.as<double>(), st);
-            if (!eig_v) eig_v = negative_pivot(dL.as<double>());
-            if (eig_v) {
-                const auto top2 = eig_sqrt(dL.as<double>(), n2, sqrt_threshold, head_q ? dU0.as<double>() : nullptr,
-                                           embed ? 2 : 1, st);
-                if (head_q && !(top2.first - top2.second > 1e-8 * std::fabs(top2.first)))
-                    LRA_THROW("head of the dielectric matrix: the largest eigenvalue of v(0) is degenerate");
-            } else {
-                ns_sqrt(dL.as<double>(), n2, st);
+            std::vector<char> eig(qg, 0), eigc(qg, 0);
+            if (!same_cut) {
+                for (int i = 0; i < qg; ++i)
+                    if (!herm && vcst.imax[iq0 + i] > 1e-12 * std::max(vcst.vmax[iq0 + i], 1e-300))
+                        LRA_THROW("a complex truncated Coulomb matrix at Gamma-only sampling is outside this build");
+                fill_v(F);
+                dense_coulomb(vcst, iq0, qg, n, lay, false, C, nn, st);
+                HIP_CHECK(hipMemcpyAsync(V0, C, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+                if (sqrt_threshold <= 0) {
+                    dProbe.reserve(nn * 8 * qg);
+                    HIP_CHECK(hipMemcpyAsync(dProbe.get(), F, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+                    factor(dProbe.as<double>(), qg, neg);
+                    HIP_CHECK(hipMemcpyAsync(dProbe.get(), C, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+                    factor(dProbe.as<double>(), qg, negc);
+                }
+            } else if (sqrt_threshold > 0) {
+                fill_v(V0);
             }
-            dSc.reserve(nn * 8);
-            if (same_cut) {
-                eig_vc = eig_v;
-                HIP_CHECK(hipMemcpyAsync(dSc.get(), dL.get(), nn * 8, hipMemcpyDeviceToDevice, st));
-            } else {
-                dense_coulomb(vcst, iq, n, n2, embed, false, dV0.as<double>(), st);
-                HIP_CHECK(hipMemcpyAsync(dSc.get(), dV0.get(), nn * 8, hipMemcpyDeviceToDevice, st));
-                if (!eig_vc) eig_vc = negative_pivot(dSc.as<double>());
-                if (eig_vc) eig_sqrt(dSc.as<double>(), n2, sqrt_threshold, nullptr, 1, st);
-                else ns_sqrt(dSc.as<double>(), n2, st);
+            std::vector<int> sel;  // roots by iteration: F of i at i, C of i at QG + i
+            for (int i = 0; i < qg; ++i) {
+                if (chol[i]) continue;
+                if (same_cut) HIP_CHECK(hipMemcpyAsync(F + i * nn, V0 + i * nn, nn * 8, hipMemcpyDeviceToDevice, st));
+                const bool head_q = head_here && i == gamma;
+                // (with v_c = v a pivot that is not positive is the reason to be here, or the threshold, or the head)
+                eig[i] = same_cut || sqrt_threshold > 0 || head_q || neg[i];
+                eigc[i] = !same_cut && (sqrt_threshold > 0 || negc[i]);
+                if (!eig[i]) sel.push_back(i);
+                if (!same_cut && !eigc[i]) sel.push_back(QG + i);
             }
-            if (eig_v || eig_vc) {
-                GemmBatch sq;
-                sq.add(make_prob(n2, n2, n2, 0, n2, 0, n2, 0, n2));
-                sq.finalize(T64x64, st);
-                gemm_run(Prec::F64, sq, dSc.get(), dSc.get(), dV0.get(), 1.0, 0.0, st);
+            ns_sqrt(F, n, herm, sel, st);
+            std::vector<long long> sq;
+            std::vector<int> which;
+            for (int i = 0; i < qg; ++i) {
+                if (chol[i]) continue;
+                const bool head_q = head_here && i == gamma;
+                if (eig[i]) {
+                    const auto top2 = eig_root(F + i * nn, head_q ? dU0.as<double>() : nullptr);
+                    if (head_q && !(top2.first - top2.second > 1e-8 * std::fabs(top2.first)))
+                        LRA_THROW("head of the dielectric matrix: the largest eigenvalue of v(0) is degenerate");
+                }
+                if (same_cut) HIP_CHECK(hipMemcpyAsync(C + i * nn, F + i * nn, nn * 8, hipMemcpyDeviceToDevice, st));
+                else if (eigc[i]) eig_root(C + i * nn, nullptr);
+                if (eig[i] || eigc[i]) {
+                    GemmBatch b = square_batch(n, herm, {i * nn}, {i * nn}, st);
+                    gemm_run(Prec::F64, b, C, C, V0 + i * nn, 1.0, 0.0, st);
+                    HIP_CHECK(hipStreamSynchronize(st));  // b's problem list is freed here
+                }
             }
             prof.end("gw_w_sqrt_v", st);
         }
-        std::vector<double> csr(nR), snr(nR);
-        for (int rr = 0; rr < nR; ++rr) {
-            const double ang = 2 * M_PI * (kf[0] * cells[rr][0] + kf[1] * cells[rr][1] + kf[2] * cells[rr][2]);
-            csr[rr] = std::cos(ang);
-            snr[rr] = std::sin(ang);
-        }
-        DevBuf dcs = upload(csr, st), dsn = upload(snr, st);
-        if (verbose) { fprintf(stderr, "[librpa-mi355x] W: q %d / %d (%.1f s)\n", iq + 1, nk, now_s() - t0); fflush(stderr); }
-        for (int w0 = 0; w0 < nw; w0 += WCH) {
-            const int cnt = std::min(WCH, nw - w0);
-            prof.begin("gw_w_chi0q", st);
-            R0.assemble_dense(g, kf, w0, cnt, dD.get(), true, (long long)nn, embed ? kEmbedded : kReal, st);
-            prof.end("gw_w_chi0q", st);
-            auto &bb = get_batches(cnt, chol);
-            prof.begin("gw_w_gemm", st);
-            gemm_run(Prec::F64, bb.first, dD.get(), dL.get(), dX.get(), 1.0, 0.0, st);
-            HIP_CHECK(hipMemsetAsync(dA.get(), 0, (size_t)cnt * NN * 8, st));
-            for (int w = 0; w < cnt; ++w) {
-                double *A = dA.as<double>() + (size_t)w * NN;
-                launch_set_identity<double>(A, n2, N, st);
-                launch_copy_block(chol ? dL.as<double>() : dSc.as<double>(), n2, A + (size_t)n2 * N, N, n2, n2, st);
-                launch_copy_block(dV0.as<double>(), n2, A + (size_t)n2 * N + n2, N, n2, n2, st);
+        std::vector<double> ph((size_t)qg * nR * 2);
+        for (int i = 0; i < qg; ++i)
+            for (int rr = 0; rr < nR; ++rr) {
+                const double ang = 2 * M_PI * (kfs[i][0] * cells[rr][0] + kfs[i][1] * cells[rr][1] + kfs[i][2] * cells[rr][2]);
+                ph[((size_t)i * nR + rr) * 2] = std::cos(ang);
+                ph[((size_t)i * nR + rr) * 2 + 1] = std::sin(ang);
             }
-            gemm_run(Prec::F64, bb.second, dL.get(), dX.get(), dA.get(), -1.0, 1.0, st);
-            if (head_q) {
+        DevBuf dph = upload(ph, st);
+        const int cstep = qg > 1 ? nw : WCH;
+        for (int w0 = 0; w0 < nw; w0 += cstep) {
+            const int cnt = std::min(cstep, nw - w0), nu = qg * cnt;
+            prof.begin("gw_w_chi0q", st);
+            R0.assemble_dense_q(g, kfs, w0, cnt, dD.get(), true, nn, lay, st);
+            prof.end("gw_w_chi0q", st);
+            auto &bb = get_batches(qg, cnt, tri);
+            prof.begin("gw_w_gemm", st);
+            gemm_run(Prec::F64, bb.first, dD.get(), F, dX.get(), 1.0, 0.0, st);
+            launch_fill_aug(dA.as<double>(), NN, im, qg, cnt, n, C, V0, st);
+            gemm_run(Prec::F64, bb.second, F, dX.get(), dA.get(), -1.0, 1.0, st);
+            if (head_here) {
                 // eps += (eps_mac - u^T eps u) u u^T, u the leading eigenvector of Re v(0): the
-                // head overwrite of epsilon.cpp:2106-2181 in the eigenbasis of v
+                // head overwrite of epsilon.cpp:2106-2181 in the eigenbasis of v (real at q = 0)
+                double *A0 = dA.as<double>() + (long long)gamma * cnt * NN;
                 HIP_CHECK(hipMemsetAsync(dQ.get(), 0, sizeof(double) * cnt, st));
-                launch_head_quad(dA.as<double>(), (long long)NN, N, n, cnt, dU0.as<double>(), dQ.as<double>(), st);
-                launch_head_update(dA.as<double>(), (long long)NN, N, n, embed ? n : 0, cnt, dU0.as<double>(),
-                                   dHead.as<double>() + w0, dQ.as<double>(), st);
+                launch_head_quad(A0, NN, N, n, cnt, dU0.as<double>(), dQ.as<double>(), st);
+                launch_head_update(A0, NN, N, n, cnt, dU0.as<double>(), dHead.as<double>() + w0, dQ.as<double>(), st);
             }
             prof.end("gw_w_gemm", st, bb.first.flops + bb.second.flops);
             prof.begin("gw_w_schur", st);
-            cholesky_logdet_batched(dA.as<double>(), (long long)NN, cnt, N, N, dacc.as<double>(), 1, dflag, false, cw,
-                                    st, n2);
-            prof.end("gw_w_schur", st, (double)cnt * (7.0 / 3.0) * n2 * (double)n2 * n2);
-            // W(R, tau) += sum_w f2t(tau, w) / N_k (cos Re W + sin Im W)
+            cholesky_logdet_batched(dA.as<double>(), NN, nu, N, N, dacc.as<double>(), 1, dflag.as<int>(), false, cw, st, n,
+                                    nullptr, 0, im);
+            prof.end("gw_w_schur", st, (herm ? 4.0 : 1.0) * nu * (7.0 / 3.0) * n * (double)n * n);
+            // W(R, tau) += sum_(q, w) f2t(tau, w) / N_k (cos Re W + sin Im W)
             prof.begin("gw_w_accum", st);
-            for (int a0 = 0; a0 < cnt; a0 += 8) {
-                const int cw_n = std::min(8, cnt - a0);
-                std::vector<double> coef((size_t)cw_n * g.n);
-                for (int w = 0; w < cw_n; ++w)
+            std::vector<double> coef((size_t)nu * g.n);
+            for (int i = 0; i < qg; ++i)
+                for (int w = 0; w < cnt; ++w)
                     for (int t = 0; t < g.n; ++t)
-                        coef[(size_t)w * g.n + t] = g.cos_f2t[(size_t)t * g.n + w0 + a0 + w] * mult[iq] / nk;
-                DevBuf dcoef = upload(coef, st);
-                launch_w_accum(dA.as<double>() + (size_t)a0 * NN, (long long)NN, cw_n, n, n2, N, embed,
-                               dcoef.as<double>(), g.n, dcs.as<double>(), dsn.as<double>(), nR, d_Wrt.as<double>(), st);
-                HIP_CHECK(hipStreamSynchronize(st));
-            }
-            prof.end("gw_w_accum", st, 0, 8.0 * cnt * (double)n * n + 16.0 * g.n * nR * (double)n * n);
+                        coef[((size_t)i * cnt + w) * g.n + t] = g.cos_f2t[(size_t)t * g.n + w0 + w] * mult[qs[iq0 + i]] / nk;
+            DevBuf dcoef = upload(coef, st);
+            launch_w_accum(dA.as<double>(), NN, im, qg, cnt, n, dcoef.as<double>(), g.n, dph.as<double>(), nR,
+                           d_Wrt.as<double>(), st);
+            HIP_CHECK(hipStreamSynchronize(st));
+            prof.end("gw_w_accum", st, 0, 8.0 * nu * (double)nn * ceil_div(g.n, 4) + 16.0 * g.n * nR * (double)n * n);
         }
     }
-    int hflag[2] = {0, 0};
-    HIP_CHECK(hipMemcpyAsync(hflag, dflag, sizeof(hflag), hipMemcpyDeviceToHost, st));
+    int hflag = 0;
+    HIP_CHECK(hipMemcpyAsync(&hflag, dflag.get(), sizeof(hflag), hipMemcpyDeviceToHost, st));
     HIP_CHECK(hipStreamSynchronize(st));
-    if (hflag[0]) LRA_THROW("1 - v^1/2 chi0 v^1/2 is singular or not finite at some (q, omega)");
-    const double nq_w = (double)std::count_if(mult.begin(), mult.end(), [](int m) { return m > 0; });
-    flops_w = nq_w * ((double)n2 * n2 * n2 / 3.0 + nw * (2.0 * n2 * (double)n2 * n2 / 2.0 + 2.0 * n2 * (double)n2 * n2 / 6.0 +
-                                                       (7.0 / 3.0) * n2 * (double)n2 * n2));
+    if (hflag) LRA_THROW("1 - v^1/2 chi0 v^1/2 is singular or not finite at some (q, omega)");
+    const double n3 = (herm ? 4.0 : 1.0) * n * (double)n * n;
+    flops_w = nq * (n3 / 3.0 + nw * (n3 + n3 / 3.0 + (7.0 / 3.0) * n3));
     t_w = now_s() - t0;
 }
 

@@ -8,14 +8,17 @@
 
 namespace lra {
 
-// W(R, tau)[a][b] += sum_w coef[w][tau] (cos_R Re W_w(a, b) + sin_R Im W_w(a, b)) for all R, tau,
-// with W_w = -(trailing block of the partially factorised augmented matrix w), that block
-// starting at (n2, n2) of an N x N row-major matrix (lower triangle valid).  For complex q
-// the trailing block is the real embedding [[Re W, -Im W], [Im W, Re W]] (embed = true).
-// Wrt layout: [tau][R][n][n].  At most 8 omega per launch.
-void launch_w_accum(const double *aug, long long aug_stride, int cnt, int n, int n2, int N, bool embed,
-                    const double *coef, int ntau, const double *cs_r, const double *sn_r, int nR, double *Wrt,
-                    hipStream_t s);
+// Dense n x n matrices below are real, or Hermitian in two planes (Re, Im) of n x n (pl = 2, im > 0).
+
+// W(R, tau)[a][b] += sum_(q, w) coef[q][w][tau] (ph_qR.x Re W_qw(a, b) + ph_qR.y Im W_qw(a, b)) for all R
+// and tau, W_qw = -(trailing block of the partially factorised augmented matrix q * nw + w), that block
+// starting at (n, n) of a 2n x 2n matrix (lower triangle valid), matrices stride apart and the
+// imaginary plane im after the real one (0: none).  ph [q][R] (cos, sin); Wrt layout: [tau][R][n][n].
+void launch_w_accum(const double *aug, long long stride, long long im, int nq, int nw, int n, const double *coef,
+                    int ntau, const double *ph, int nR, double *Wrt, hipStream_t s);
+// lower triangle of every augmented matrix: [[I, .], [C_q, V_q]]
+void launch_fill_aug(double *A, long long stride, long long im, int nq, int nw, int n, const double *C, const double *V,
+                     hipStream_t s);
 
 // ---- self-energy contractions (gw.cpp) ----
 // CW_IJ(R)[c][i][nu] = sum_mu C^I[(c, i)][mu] W_IJ(R)[mu][nu] and U_J(S)[(X, x)][j][nu] per tau point; c
@@ -65,11 +68,17 @@ void launch_sigma_freq(const T *sig, long long nelem, const double *cw, const do
 void launch_sigma_ks_rows(const double *sre, const double *sim, int nw, int nR, int n, const int *atom_of,
                           int natom, const double *ph, const double *U, int nst, double *Y, hipStream_t s);
 
-// Dense helpers of the Newton-Schulz square root (FP64, row-major n x n, lda = n):
-// B = alpha A + beta I
-void launch_scale_add_identity(const double *A, double *B, int n, double alpha, double beta, hipStream_t s);
-// out[0] = max |A - B|, out[1] = max |B| (single workgroup, overwritten)
-void launch_absmax_diff(const double *A, const double *B, long long n, double *out, hipStream_t s);
+// Newton-Schulz square roots of the matrices A + sel[m] * nn, m < nmat (nn = pl n^2 elements each), on
+// compact work arrays Y, Z: Y = A / c, Z = I with c = ||A||_F in scale (part: 32 doubles a matrix) ...
+void launch_ns_init(const double *A, const int *sel, int nmat, int n, int pl, double *part, double *Y, double *Z,
+                    double *scale, hipStream_t s);
+// ... P <- 1.5 I - 0.5 P ...
+void launch_ns_step(double *P, int nmat, int n, int pl, hipStream_t s);
+// ... out[2 m], out[2 m + 1] = max |Yn - Y|, max |Y| (bits of doubles, cleared by the caller) ...
+void launch_ns_change(const double *Yn, const double *Y, int nmat, int n, int pl, unsigned long long *out, hipStream_t s);
+// ... and A + sel[m] * nn = sqrt(c) Y
+void launch_ns_finish(const double *Y, const double *scale, const int *sel, int nmat, int n, int pl, double *A,
+                      hipStream_t s);
 // A[i][:] *= f[i] (row-major n x n)
 void launch_scale_rows(double *A, int n, const double *f, hipStream_t s);
 
@@ -78,11 +87,8 @@ void launch_scale_rows(double *A, int n, const double *f, hipStream_t s);
 // origin (q is accumulated, clear it first) ...
 void launch_head_quad(const double *A, long long stride, int ld, int n, int cnt, const double *u, double *q,
                       hipStream_t s);
-// ... then eps_w += (eps_mac[w] - q[w]) u u^T on the lower triangle of that block and, when
-// off2 > 0, of the copy at (off2, off2) (the real embedding of a q = 0 matrix).
-void launch_head_update(double *A, long long stride, int ld, int n, int off2, int cnt, const double *u,
-                        const double *eps_mac, const double *q, hipStream_t s);
-// out[0] = sum A^2 (overwritten)
-void launch_sumsq(const double *A, long long n, double *out, hipStream_t s);
+// ... then eps_w += (eps_mac[w] - q[w]) u u^T on the lower triangle of that block.
+void launch_head_update(double *A, long long stride, int ld, int n, int cnt, const double *u, const double *eps_mac,
+                        const double *q, hipStream_t s);
 
 }  // namespace lra

@@ -1,54 +1,87 @@
 // Streaming kernels of the G0W0 path (gfx950).
 #include "gw_kernels.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace lra {
 
-constexpr int kWMax = 8;
-
-__global__ __launch_bounds__(256) void w_accum_kernel(const double *__restrict__ aug, long long aug_stride, int cnt,
-                                                      int n, int n2, int N, int embed, const double *__restrict__ coef,
-                                                      int ntau, const double *__restrict__ cs_r,
-                                                      const double *__restrict__ sn_r, int nR,
-                                                      double *__restrict__ Wrt) {
+// One element of (a, b), kWTau tau points and kWCells cells a thread: sums over the frequencies of each q
+// of the pass first, then over q with its phases, so that W(q, omega) is read once per four tau points
+// and eight cells and W(R, tau) is written once per pass over q (it was read and written again for
+// every q and eight frequencies).
+constexpr int kWTau = 4, kWCells = 8;
+__global__ __launch_bounds__(256) void w_accum_kernel(const double *__restrict__ aug, long long stride, long long im,
+                                                      int nq, int nw, int n, const double *__restrict__ coef, int ntau,
+                                                      const double *__restrict__ ph, int nR, double *__restrict__ Wrt) {
     const long long nn = (long long)n * n;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nn) return;
-    const int a = (int)(idx / n), b = (int)(idx % n);
-    const int hi = a > b ? a : b, lo = a > b ? b : a;
-    double re[kWMax], im[kWMax];
+    const int a = (int)(idx / n), b = (int)(idx % n), N = 2 * n;
+    const int t0 = blockIdx.y * kWTau, r0 = blockIdx.z * kWCells;
+    const long long at = (long long)(n + max(a, b)) * N + n + min(a, b);
+    const double sgn = a < b ? -1.0 : 1.0;  // Im W_ab = -Im W_ba
+    double acc[kWTau][kWCells];
 #pragma unroll
-    for (int w = 0; w < kWMax; ++w) {
-        re[w] = 0;
-        im[w] = 0;
-        if (w < cnt) {
-            const double *A = aug + (long long)w * aug_stride;
-            re[w] = -A[(long long)(n2 + hi) * N + n2 + lo];
-            if (embed) im[w] = -A[(long long)(n2 + n + a) * N + n2 + b];
-        }
-    }
-    for (int t = 0; t < ntau; ++t) {
-        double x = 0, y = 0;
+    for (int t = 0; t < kWTau; ++t)
 #pragma unroll
-        for (int w = 0; w < kWMax; ++w) {
-            if (w < cnt) {
-                const double c = coef[w * ntau + t];
-                x += c * re[w];
-                y += c * im[w];
+        for (int r = 0; r < kWCells; ++r) acc[t][r] = 0;
+    for (int q = 0; q < nq; ++q) {
+        double x[kWTau], y[kWTau];
+#pragma unroll
+        for (int t = 0; t < kWTau; ++t) x[t] = y[t] = 0;
+        for (int w = 0; w < nw; ++w) {
+            const double *A = aug + ((long long)q * nw + w) * stride + at;
+            const double re = -A[0], ii = im ? -sgn * A[im] : 0.0;
+#pragma unroll
+            for (int t = 0; t < kWTau; ++t) {
+                const double c = coef[((long long)q * nw + w) * ntau + min(t0 + t, ntau - 1)];
+                x[t] += c * re;
+                y[t] += c * ii;
             }
         }
-        double *dst = Wrt + (long long)t * nR * nn + idx;
-        for (int R = 0; R < nR; ++R) dst[(long long)R * nn] += cs_r[R] * x + sn_r[R] * y;
+#pragma unroll
+        for (int r = 0; r < kWCells; ++r) {
+            const double *p = ph + 2 * ((long long)q * nR + min(r0 + r, nR - 1));
+#pragma unroll
+            for (int t = 0; t < kWTau; ++t) acc[t][r] += p[0] * x[t] + p[1] * y[t];
+        }
     }
+#pragma unroll
+    for (int t = 0; t < kWTau; ++t)
+#pragma unroll
+        for (int r = 0; r < kWCells; ++r)
+            if (t0 + t < ntau && r0 + r < nR) Wrt[((long long)(t0 + t) * nR + r0 + r) * nn + idx] += acc[t][r];
 }
 
-void launch_w_accum(const double *aug, long long aug_stride, int cnt, int n, int n2, int N, bool embed,
-                    const double *coef, int ntau, const double *cs_r, const double *sn_r, int nR, double *Wrt,
-                    hipStream_t s) {
-    if (cnt < 1 || cnt > kWMax) LRA_THROW("w_accum: 1..8 frequencies per launch");
-    hipLaunchKernelGGL(w_accum_kernel, dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, aug, aug_stride, cnt,
-                       n, n2, N, (int)embed, coef, ntau, cs_r, sn_r, nR, Wrt);
+void launch_w_accum(const double *aug, long long stride, long long im, int nq, int nw, int n, const double *coef,
+                    int ntau, const double *ph, int nR, double *Wrt, hipStream_t s) {
+    hipLaunchKernelGGL(w_accum_kernel, dim3(ceil_div((long long)n * n, 256), ceil_div(ntau, kWTau), ceil_div(nR, kWCells)),
+                       dim3(256), 0, s, aug, stride, im, nq, nw, n, coef, ntau, ph, nR, Wrt);
+    HIP_CHECK(hipGetLastError());
+}
+
+// lower triangle (whole rows of the lower left block) of matrix blockIdx.y = q * nw + w, plane blockIdx.z
+__global__ __launch_bounds__(256) void fill_aug_kernel(double *__restrict__ A, long long stride, long long im, int nw, int n,
+                                                       const double *__restrict__ C, const double *__restrict__ V,
+                                                       long long nn) {
+    const int N = 2 * n;
+    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (long long)N * N) return;
+    const int i = (int)(idx / N), j = (int)(idx % N);
+    if (j > i) return;
+    const long long src = (blockIdx.y / nw) * nn + blockIdx.z * (long long)n * n;
+    double v;
+    if (i < n) v = (i == j && blockIdx.z == 0) ? 1.0 : 0.0;
+    else if (j < n) v = C[src + (long long)(i - n) * n + j];
+    else v = V[src + (long long)(i - n) * n + j - n];
+    A[blockIdx.y * stride + blockIdx.z * im + idx] = v;
+}
+void launch_fill_aug(double *A, long long stride, long long im, int nq, int nw, int n, const double *C, const double *V,
+                     hipStream_t s) {
+    const int pl = im ? 2 : 1;
+    hipLaunchKernelGGL(fill_aug_kernel, dim3(ceil_div(4LL * n * n, 256), nq * nw, pl), dim3(256), 0, s, A, stride, im, nw,
+                       n, C, V, (long long)pl * n * n);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -539,16 +572,104 @@ void launch_sigma_ks_rows(const double *sre, const double *sim, int nw, int nR, 
     HIP_CHECK(hipGetLastError());
 }
 
-__global__ void scale_add_identity_kernel(const double *__restrict__ A, double *__restrict__ B, int n, double alpha,
-                                          double beta) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)n * n) return;
-    const int i = (int)(idx / n), j = (int)(idx % n);
-    B[idx] = alpha * A[idx] + (i == j ? beta : 0.0);
+// ------------------------------------------------------------------------------------
+// Newton-Schulz square roots of several matrices (blockIdx.y), pl planes of n x n each
+// ------------------------------------------------------------------------------------
+constexpr int kNsBlocks = 32;  // partial sums and maxima per matrix
+
+__global__ __launch_bounds__(256) void ns_norm_kernel(const double *__restrict__ A, const int *__restrict__ sel,
+                                                      long long nn, double *__restrict__ part) {
+    __shared__ double red[256];
+    const double *M = A + sel[blockIdx.y] * nn;
+    double v = 0;
+    for (long long i = blockIdx.x * 256 + threadIdx.x; i < nn; i += kNsBlocks * 256) v += M[i] * M[i];
+    red[threadIdx.x] = v;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) part[blockIdx.y * kNsBlocks + blockIdx.x] = red[0];
 }
-void launch_scale_add_identity(const double *A, double *B, int n, double alpha, double beta, hipStream_t s) {
-    hipLaunchKernelGGL(scale_add_identity_kernel, dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, A, B, n, alpha,
-                       beta);
+
+__device__ __forceinline__ double ns_scale(const double *part) {
+    double v = 0;
+    for (int i = 0; i < kNsBlocks; ++i) v += part[i];
+    return sqrt(v);
+}
+
+// Y = A / c, Z = I with c = ||A||_F (kept in scale)
+__global__ __launch_bounds__(256) void ns_init_kernel(const double *__restrict__ A, const int *__restrict__ sel, int n,
+                                                      long long nn, const double *__restrict__ part,
+                                                      double *__restrict__ Y, double *__restrict__ Z,
+                                                      double *__restrict__ scale) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nn) return;
+    const double c = ns_scale(part + blockIdx.y * kNsBlocks);
+    if (i == 0) scale[blockIdx.y] = c;
+    Y[blockIdx.y * nn + i] = A[sel[blockIdx.y] * nn + i] * (1.0 / c);
+    Z[blockIdx.y * nn + i] = (i < (long long)n * n && i / n == i % n) ? 1.0 : 0.0;
+}
+void launch_ns_init(const double *A, const int *sel, int nmat, int n, int pl, double *part, double *Y, double *Z,
+                    double *scale, hipStream_t s) {
+    const long long nn = (long long)pl * n * n;
+    hipLaunchKernelGGL(ns_norm_kernel, dim3(kNsBlocks, nmat), dim3(256), 0, s, A, sel, nn, part);
+    HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(ns_init_kernel, dim3(ceil_div(nn, 256), nmat), dim3(256), 0, s, A, sel, n, nn, part, Y, Z, scale);
+    HIP_CHECK(hipGetLastError());
+}
+
+// T = 1.5 I - 0.5 P, in place
+__global__ __launch_bounds__(256) void ns_step_kernel(double *P, int n, long long nn) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nn) return;
+    const bool diag = i < (long long)n * n && i / n == i % n;
+    P[blockIdx.y * nn + i] = -0.5 * P[blockIdx.y * nn + i] + (diag ? 1.5 : 0.0);
+}
+void launch_ns_step(double *P, int nmat, int n, int pl, hipStream_t s) {
+    const long long nn = (long long)pl * n * n;
+    hipLaunchKernelGGL(ns_step_kernel, dim3(ceil_div(nn, 256), nmat), dim3(256), 0, s, P, n, nn);
+    HIP_CHECK(hipGetLastError());
+}
+
+// out[2 m] = max |Yn - Y|, out[2 m + 1] = max |Y| of matrix m, as the bits of non-negative doubles (which
+// order as integers); a NaN counts as infinity.  out starts from zero.
+__global__ __launch_bounds__(256) void ns_change_kernel(const double *__restrict__ Yn, const double *__restrict__ Y,
+                                                        long long nn, unsigned long long *__restrict__ out) {
+    double d = 0, m = 0;
+    const auto up = [](double &m_, double v) {
+        v = fabs(v);
+        if (!(v <= m_)) m_ = v < INFINITY ? v : INFINITY;
+    };
+    for (long long i = blockIdx.x * 256 + threadIdx.x; i < nn; i += kNsBlocks * 256) {
+        const double y = Y[blockIdx.y * nn + i];
+        up(d, Yn[blockIdx.y * nn + i] - y);
+        up(m, y);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        d = fmax(d, __shfl_xor(d, o, 64));
+        m = fmax(m, __shfl_xor(m, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(out + 2 * blockIdx.y, (unsigned long long)__double_as_longlong(d));
+        atomicMax(out + 2 * blockIdx.y + 1, (unsigned long long)__double_as_longlong(m));
+    }
+}
+void launch_ns_change(const double *Yn, const double *Y, int nmat, int n, int pl, unsigned long long *out, hipStream_t s) {
+    hipLaunchKernelGGL(ns_change_kernel, dim3(kNsBlocks, nmat), dim3(256), 0, s, Yn, Y, (long long)pl * n * n, out);
+    HIP_CHECK(hipGetLastError());
+}
+
+// A[sel] = sqrt(c) Y
+__global__ __launch_bounds__(256) void ns_finish_kernel(const double *__restrict__ Y, const double *__restrict__ scale,
+                                                        const int *__restrict__ sel, long long nn, double *__restrict__ A) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < nn) A[sel[blockIdx.y] * nn + i] = sqrt(scale[blockIdx.y]) * Y[blockIdx.y * nn + i];
+}
+void launch_ns_finish(const double *Y, const double *scale, const int *sel, int nmat, int n, int pl, double *A,
+                      hipStream_t s) {
+    const long long nn = (long long)pl * n * n;
+    hipLaunchKernelGGL(ns_finish_kernel, dim3(ceil_div(nn, 256), nmat), dim3(256), 0, s, Y, scale, sel, nn, A);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -586,65 +707,18 @@ void launch_head_quad(const double *A, long long stride, int ld, int n, int cnt,
     HIP_CHECK(hipGetLastError());
 }
 
-__global__ __launch_bounds__(256) void head_update_kernel(double *__restrict__ A, long long stride, int ld, int off2,
+__global__ __launch_bounds__(256) void head_update_kernel(double *__restrict__ A, long long stride, int ld,
                                                           const double *__restrict__ u,
                                                           const double *__restrict__ eps_mac,
                                                           const double *__restrict__ q) {
     const int i = blockIdx.x, w = blockIdx.y;
     const double d = (eps_mac[w] - q[w]) * u[i];
     double *row = A + (long long)w * stride + (long long)i * ld;
-    for (int j = threadIdx.x; j <= i; j += blockDim.x) {
-        const double add = d * u[j];
-        row[j] += add;
-        if (off2 > 0) row[(long long)off2 * ld + off2 + j] += add;
-    }
+    for (int j = threadIdx.x; j <= i; j += blockDim.x) row[j] += d * u[j];
 }
-void launch_head_update(double *A, long long stride, int ld, int n, int off2, int cnt, const double *u,
-                        const double *eps_mac, const double *q, hipStream_t s) {
-    hipLaunchKernelGGL(head_update_kernel, dim3(n, cnt), dim3(256), 0, s, A, stride, ld, off2, u, eps_mac, q);
-    HIP_CHECK(hipGetLastError());
-}
-
-// single workgroup of 1024 threads: deterministic reductions without atomics
-__global__ __launch_bounds__(1024) void absmax_diff_kernel(const double *__restrict__ A, const double *__restrict__ B,
-                                                           long long n, double *out) {
-    __shared__ double r0[1024], r1[1024];
-    double d = 0, m = 0;
-    for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-        d = fmax(d, fabs(A[i] - B[i]));
-        m = fmax(m, fabs(B[i]));
-    }
-    r0[threadIdx.x] = d;
-    r1[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            r0[threadIdx.x] = fmax(r0[threadIdx.x], r0[threadIdx.x + o]);
-            r1[threadIdx.x] = fmax(r1[threadIdx.x], r1[threadIdx.x + o]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) { out[0] = r0[0]; out[1] = r1[0]; }
-}
-void launch_absmax_diff(const double *A, const double *B, long long n, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(absmax_diff_kernel, dim3(1), dim3(1024), 0, s, A, B, n, out);
-    HIP_CHECK(hipGetLastError());
-}
-
-__global__ __launch_bounds__(1024) void sumsq_kernel(const double *__restrict__ A, long long n, double *out) {
-    __shared__ double r[1024];
-    double v = 0;
-    for (long long i = threadIdx.x; i < n; i += blockDim.x) v += A[i] * A[i];
-    r[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) r[threadIdx.x] += r[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = r[0];
-}
-void launch_sumsq(const double *A, long long n, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(sumsq_kernel, dim3(1), dim3(1024), 0, s, A, n, out);
+void launch_head_update(double *A, long long stride, int ld, int n, int cnt, const double *u, const double *eps_mac,
+                        const double *q, hipStream_t s) {
+    hipLaunchKernelGGL(head_update_kernel, dim3(n, cnt), dim3(256), 0, s, A, stride, ld, u, eps_mac, q);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -38,9 +38,8 @@ void launch_gather_cols(const T *src, long long src_ld, T *dst, const GatherJob 
 // tau -> omega and R -> q of chi0s into dense Hermitian matrices ---------------------
 // For each pair p = (I <= J) with element count na_I * na_J and each omega w of the
 // chunk: val = (2 / nspin) sum_t sum_r gamma[w][t] e^{i 2 pi q.R_r} chi0s[t][eoff[p][r] + e].
-// Output by layout: real (Gamma) n x n, the real embedding [[Re, -Im], [Im, Re]] (2n x 2n), or the
-// planes Re and Im (n x n each).
-enum DenseLayout : int { kReal = 0, kEmbedded = 1, kPlanar = 2 };
+// Output by layout: real (Gamma) n x n, or the planes Re and Im (n x n each).
+enum DenseLayout : int { kReal = 0, kPlanar = 1 };
 struct PairDesc {
     int I, J;
     int naI, naJ;
@@ -74,7 +73,9 @@ void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *p
                           TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s);
 
 // Dense helpers --------------------------------------------------------------------
-template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s);
+// planes Re, Im (n x n each) of a complex matrix <-> its real embedding [[Re, -Im], [Im, Re]] (2n x 2n)
+void launch_planes_to_embedded(const double *M, double *E, int n, hipStream_t s);
+void launch_embedded_to_planes(const double *E, double *M, int n, hipStream_t s);
 template <class TS, class TD> void launch_convert(const TS *src, TD *dst, long long n, hipStream_t s);
 // lower triangles of nmat n x n matrices, stride elements apart (pitch n)
 void launch_copy_lower_f2d(const float *src, double *dst, int n, long long nmat, long long stride, hipStream_t s);
@@ -95,7 +96,6 @@ void launch_v_scatter(const double *blk, const VBlock *d, int nblk, double *V, i
 // S = signs + (u / per) * n
 void launch_add_signs_trace(double *A, int n, long long nmat, long long stride, const double *signs, int per, double *acc,
                             hipStream_t s);
-void launch_copy_block(const double *src, int lds, double *dst, int ldd, int rows, int cols, hipStream_t s);
 
 // Blocked Cholesky with signed pivots (lower, row-major, FP64): A = L S L^H in place, S = diag(+-1);
 // equal to Cholesky for positive-definite A.  A is real, or Hermitian with its imaginary plane im
@@ -105,9 +105,7 @@ void launch_copy_block(const double *src, int lds, double *dst, int ldd, int row
 struct CholWork {
     DevBuf linv, panel;
 };
-void cholesky_logdet(double *A, int n, int lda, double *logdet, int *flag, bool keep_L, CholWork &w,
-                     hipStream_t s, double *signs = nullptr);
-// The same for nbatch matrices at A + b * strideA, all factorised in the same launches;
+// nbatch matrices at A + b * strideA are factorised in the same launches;
 // matrix b adds its ln|det| to logdet[b * ld_stride].  With ncols in (0, n) only the
 // first ncols columns are eliminated: the lower triangle of the trailing block then
 // holds its Schur complement A22 - A21 A11^{-1} A21^T and logdet gets ln|det A11|.

@@ -138,25 +138,11 @@ template void launch_gather_cols<float>(const float *, long long, float *, const
 template <class TD>
 __device__ __forceinline__ void put_dense(TD *__restrict__ D, long long n, long long row, long long col, double re,
                                           double im, bool mirror, int lay) {
-    if (lay != kEmbedded) {
-        D[row * n + col] = static_cast<TD>(re);
-        if (mirror) D[col * n + row] = static_cast<TD>(re);
-        if (lay == kPlanar) {
-            D[(n + row) * n + col] = static_cast<TD>(im);
-            if (mirror) D[(n + col) * n + row] = static_cast<TD>(-im);
-        }
-        return;
-    }
-    const long long ld = 2 * n;
-    D[row * ld + col] = static_cast<TD>(re);
-    D[(n + row) * ld + n + col] = static_cast<TD>(re);
-    D[(n + row) * ld + col] = static_cast<TD>(im);
-    D[row * ld + n + col] = static_cast<TD>(-im);
-    if (mirror) {
-        D[col * ld + row] = static_cast<TD>(re);
-        D[(n + col) * ld + n + row] = static_cast<TD>(re);
-        D[(n + col) * ld + row] = static_cast<TD>(-im);
-        D[col * ld + n + row] = static_cast<TD>(im);
+    D[row * n + col] = static_cast<TD>(re);
+    if (mirror) D[col * n + row] = static_cast<TD>(re);
+    if (lay == kPlanar) {
+        D[(n + row) * n + col] = static_cast<TD>(im);
+        if (mirror) D[(n + col) * n + row] = static_cast<TD>(-im);
     }
 }
 
@@ -372,18 +358,31 @@ template void launch_chi0_rq_multi<float>(const double *, long long, const PairD
 // ------------------------------------------------------------------------------------
 // dense helpers
 // ------------------------------------------------------------------------------------
-template <class T>
-__global__ void set_identity_kernel(T *A, int n, int lda) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)n * n) return;
-    const int i = (int)(idx / n), j = (int)(idx % n);
-    A[(long long)i * lda + j] = i == j ? T(1) : T(0);
+// (Re, Im) planes <-> the real embedding [[Re, -Im], [Im, Re]]
+__global__ void planes_to_embedded_kernel(const double *__restrict__ M, double *__restrict__ E, int n) {
+    const long long nn = (long long)n * n, idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= nn) return;
+    const long long i = idx / n, j = idx % n, ld = 2 * n;
+    const double re = M[idx], im = M[nn + idx];
+    E[i * ld + j] = E[(n + i) * ld + n + j] = re;
+    E[(n + i) * ld + j] = im;
+    E[i * ld + n + j] = -im;
 }
-template <class T> void launch_set_identity(T *A, int n, int lda, hipStream_t s) {
-    hipLaunchKernelGGL((set_identity_kernel<T>), dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, A, n, lda);
+void launch_planes_to_embedded(const double *M, double *E, int n, hipStream_t s) {
+    hipLaunchKernelGGL(planes_to_embedded_kernel, dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, M, E, n);
     HIP_CHECK(hipGetLastError());
 }
-template void launch_set_identity<double>(double *, int, int, hipStream_t);
+__global__ void embedded_to_planes_kernel(const double *__restrict__ E, double *__restrict__ M, int n) {
+    const long long nn = (long long)n * n, idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= nn) return;
+    const long long i = idx / n, j = idx % n, ld = 2 * n;
+    M[idx] = E[i * ld + j];
+    M[nn + idx] = E[(n + i) * ld + j];
+}
+void launch_embedded_to_planes(const double *E, double *M, int n, hipStream_t s) {
+    hipLaunchKernelGGL(embedded_to_planes_kernel, dim3(ceil_div((long long)n * n, 256)), dim3(256), 0, s, E, M, n);
+    HIP_CHECK(hipGetLastError());
+}
 
 // zero above the diagonal; the diagonal too on odd planes (blockIdx.y counts matrices, .z planes im apart)
 __global__ void zero_upper_kernel(double *A, int n, int lda, long long stride, long long im) {
@@ -470,20 +469,6 @@ void launch_add_signs_trace(double *A, int n, long long nmat, long long stride, 
                             hipStream_t s) {
     if (nmat <= 0) return;
     hipLaunchKernelGGL(add_signs_trace_kernel, dim3((unsigned)nmat), dim3(256), 0, s, A, n, stride, signs, per, acc);
-    HIP_CHECK(hipGetLastError());
-}
-
-__global__ void copy_block_kernel(const double *__restrict__ src, int lds, double *__restrict__ dst, int ldd,
-                                  int rows, int cols) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)rows * cols) return;
-    const int i = (int)(idx / cols), j = (int)(idx % cols);
-    dst[(long long)i * ldd + j] = src[(long long)i * lds + j];
-}
-void launch_copy_block(const double *src, int lds, double *dst, int ldd, int rows, int cols, hipStream_t s) {
-    if (rows <= 0 || cols <= 0) return;
-    hipLaunchKernelGGL(copy_block_kernel, dim3(ceil_div((long long)rows * cols, 256)), dim3(256), 0, s, src, lds,
-                       dst, ldd, rows, cols);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -833,11 +818,6 @@ void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, in
                            strideA, im);
         HIP_CHECK(hipGetLastError());
     }
-}
-
-void cholesky_logdet(double *A, int n, int lda, double *logdet, int *flag, bool keep_L, CholWork &w, hipStream_t s,
-                     double *signs) {
-    cholesky_logdet_batched(A, 0, 1, n, lda, logdet, 0, flag, keep_L, w, s, -1, signs, 0);
 }
 
 }  // namespace lra
