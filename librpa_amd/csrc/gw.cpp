@@ -341,19 +341,24 @@ GemmBatch square_batch(int n, bool herm, const std::vector<long long> &a, const 
 // c = ||A||_F >= lambda_max; Y -> (A / c)^{1/2}.  Equals the eigen-decomposition root of
 // power_hemat (src/math/matrix_m.h:916-970) for positive-definite input.  Runs to convergence, all
 // matrices together; the host looks at the changes of every fourth iteration's batch only.
-void ns_sqrt(double *A, int n, bool herm, const std::vector<int> &sel, hipStream_t st) {
+// work: at least 5 matrices per root, or memory is allocated.
+void ns_sqrt(double *A, int n, bool herm, const std::vector<int> &sel, double *work, size_t work_elems, hipStream_t st) {
     if (sel.empty()) return;
     const int nm = (int)sel.size(), pl = herm ? 2 : 1;
     const size_t nn = (size_t)n * n * pl, all = nn * 8 * nm;
     constexpr int kMax = 200, kLook = 4;
-    DevBuf dY(all), dZ(all), dP(all), dYn(all), dZn(all), dpart(32 * 8 * (size_t)nm), dscale(8 * (size_t)nm),
-        dchg(sizeof(unsigned long long) * 2 * nm * kMax);
+    DevBuf own, dpart(32 * 8 * (size_t)nm), dscale(8 * (size_t)nm), dchg(sizeof(unsigned long long) * 2 * nm * kMax);
+    if (work_elems < 5 * nn * nm) {
+        own.alloc(5 * all);
+        work = own.as<double>();
+    }
+    double *dY = work, *dZ = dY + nn * nm, *dP = dZ + nn * nm, *dYn = dP + nn * nm, *dZn = dYn + nn * nm;
     DevBuf dsel = upload(sel, st);
     std::vector<long long> at(nm);
     for (int m = 0; m < nm; ++m) at[m] = (long long)m * (long long)nn;
     GemmBatch b = square_batch(n, herm, at, at, st);
     HIP_CHECK(hipMemsetAsync(dchg.get(), 0, dchg.bytes(), st));
-    launch_ns_init(A, dsel.as<int>(), nm, n, pl, dpart.as<double>(), dY.as<double>(), dZ.as<double>(),
+    launch_ns_init(A, dsel.as<int>(), nm, n, pl, dpart.as<double>(), dY, dZ,
                    dscale.as<double>(), st);
     std::vector<double> c(nm), h(2 * (size_t)nm * kLook), prev(nm, 1e300);
     std::vector<int> stall(nm, 0);
@@ -365,11 +370,11 @@ void ns_sqrt(double *A, int n, bool herm, const std::vector<int> &sel, hipStream
     bool all_done = false;
     for (int k0 = 0; k0 < kMax && !all_done; k0 += kLook) {
         for (int k = k0; k < k0 + kLook; ++k) {
-            gemm_run(Prec::F64, b, dZ.get(), dY.get(), dP.get(), 1.0, 0.0, st);
-            launch_ns_step(dP.as<double>(), nm, n, pl, st);
-            gemm_run(Prec::F64, b, dY.get(), dP.get(), dYn.get(), 1.0, 0.0, st);
-            gemm_run(Prec::F64, b, dP.get(), dZ.get(), dZn.get(), 1.0, 0.0, st);
-            launch_ns_change(dYn.as<double>(), dY.as<double>(), nm, n, pl, dchg.as<unsigned long long>() + 2 * (size_t)nm * k, st);
+            gemm_run(Prec::F64, b, dZ, dY, dP, 1.0, 0.0, st);
+            launch_ns_step(dP, nm, n, pl, st);
+            gemm_run(Prec::F64, b, dY, dP, dYn, 1.0, 0.0, st);
+            gemm_run(Prec::F64, b, dP, dZ, dZn, 1.0, 0.0, st);
+            launch_ns_change(dYn, dY, nm, n, pl, dchg.as<unsigned long long>() + 2 * (size_t)nm * k, st);
             std::swap(dY, dYn);
             std::swap(dZ, dZn);
         }
@@ -389,7 +394,7 @@ void ns_sqrt(double *A, int n, bool herm, const std::vector<int> &sel, hipStream
         }
     }
     if (!all_done) LRA_THROW("square root of the Coulomb matrix did not converge");
-    launch_ns_finish(dY.as<double>(), dscale.as<double>(), dsel.as<int>(), nm, n, pl, A, st);
+    launch_ns_finish(dY, dscale.as<double>(), dsel.as<int>(), nm, n, pl, A, st);
     HIP_CHECK(hipStreamSynchronize(st));
 }
 
@@ -452,13 +457,7 @@ std::pair<double, double> eig_sqrt(double *A, int n, double thr, double *top, in
     return {l0, l1};
 }
 
-// The upper atom-pair blocks (I <= J) of a Coulomb input for the k points qs, staged on the device for
-// launch_v_scatter (VBlock::q: position in qs), with the largest |V| and |Im V| of each.
-struct CoulombStage {
-    DevBuf blk, desc;
-    std::vector<int> first;  // descriptors of qs[i]: [first[i], first[i + 1])
-    std::vector<double> vmax, imax;
-};
+// the blocks of the k points qs
 void stage_coulomb(const RpaEngine &R0, const std::map<std::tuple<int, int, int>, std::vector<cplx>> &store,
                    const std::vector<int> &qs, CoulombStage &out, hipStream_t st) {
     std::vector<VBlock> desc;
@@ -495,7 +494,28 @@ void dense_coulomb(const CoulombStage &cs, int i0, int cnt, int n, DenseLayout l
 }
 }  // namespace
 
-void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
+namespace {
+// at_least: what a later phase will take of the same buffer
+template <class F> void carve(DevBuf &buf, F layout, size_t at_least = 0) {
+    Carve count{nullptr};
+    layout(count);
+    buf.reserve(std::max(count.at, at_least));
+    Carve c{buf.as<char>()};
+    layout(c);
+}
+}  // namespace
+
+void GwEngine::sigma_layout(Carve &c, SigmaWork &w) const {
+    const size_t nel = (size_t)nR * NAO * NAO, next = (size_t)NE * NAO * NAO;
+    w.U = c.take<char>(2 * (size_t)u_elems * nbatch * ts);
+    w.Ghat = c.take<char>((size_t)max_ghat * nbatch * ts);
+    w.CW = c.take<char>(((size_t)max_cw * nbatch + kChi0Pad) * ts);
+    w.Y = c.take<char>(2 * (size_t)y_elems * nbatch * ts);
+    w.sigma = c.take<char>(2 * (size_t)nbatch * (2 * nel + next) * ts);
+    w.Wlow = prec != Prec::F64 ? c.take<char>((size_t)nbatch * nR * NABF * NABF * ts) : nullptr;
+}
+
+void GwEngine::build_w(const Dataset &ds, const TFGrid &g, Result &out) {
     auto &prof = profiler();
     const double t0 = now_s();
     RpaEngine &R0 = *rpa;
@@ -504,11 +524,11 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
     const int nw = g.n;
     if (R0.ntau_done != g.n) LRA_THROW("chi0 must be built on the same grid before W");
     if (R0.host_staged) LRA_THROW("G0W0 needs the device-resident chi0 store (too large for this device)");
-    d_Wrt.alloc(sizeof(double) * (size_t)g.n * nR * n * n);
-    HIP_CHECK(hipMemsetAsync(d_Wrt.get(), 0, d_Wrt.bytes(), st));
+    out.Wrt.alloc(sizeof(double) * (size_t)g.n * nR * n * n);
+    HIP_CHECK(hipMemsetAsync(out.Wrt.get(), 0, out.Wrt.bytes(), st));
     // no truncated Coulomb: v_c^{1/2} = 0 and W = 0 (epsilon.cpp:1862-1879)
-    w_zero = ds.vq_cut.empty();
-    if (w_zero) { HIP_CHECK(hipStreamSynchronize(st)); t_w = now_s() - t0; return; }
+    out.w_zero = ds.vq_cut.empty();
+    if (out.w_zero) { HIP_CHECK(hipStreamSynchronize(st)); t_w = now_s() - t0; return; }
     // irreducible q and their star sizes; a reducible q must be the time-reversal partner of its
     // irreducible q (the assumption of FT_Wc_freq_q, epsilon.cpp:2430-2452)
     std::vector<int> mult(nk, 0);
@@ -528,17 +548,6 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
         }
         mult[r]++;
     }
-    // v_c = v lets W = L M^{-1} L^T - v use the Cholesky factor of v; otherwise the square roots
-    // of v and v_c are formed (Newton-Schulz) and W = v_c^{1/2} eps^{-1} v_c^{1/2} - v_c
-    bool same_cut = ds.vq_cut.size() == ds.vq.size();
-    for (const auto &kv : ds.vq) {
-        auto it = ds.vq_cut.find(kv.first);
-        same_cut = same_cut && it != ds.vq_cut.end() && it->second.size() == kv.second.size();
-        for (size_t i = 0; same_cut && i < kv.second.size(); ++i)
-            same_cut = it->second[i] == kv.second[i] ||
-                       std::abs(it->second[i] - kv.second[i]) <= 1e-12 * (1.0 + std::abs(kv.second[i]));
-    }
-
     const bool herm = nk > 1;
     const DenseLayout lay = herm ? kPlanar : kReal;
     const int N = 2 * n, pl = herm ? 2 : 1;
@@ -547,10 +556,31 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
     for (int k = 0; k < nk; ++k)
         if (mult[k] > 0) qs.push_back(k);
     const int nq = (int)qs.size();
+    // the Coulomb inputs go to the device once per plan and list of q (the engine goes with the inputs).
+    // v_c = v lets W = L M^{-1} L^T - v use the Cholesky factor of v; otherwise the square roots
+    // of v and v_c are formed and W = v_c^{1/2} eps^{-1} v_c^{1/2} - v_c
+    if (v_qs != qs) {
+        v_qs.clear();
+        same_cut = ds.vq_cut.size() == ds.vq.size();
+        for (const auto &kv : ds.vq) {
+            auto it = ds.vq_cut.find(kv.first);
+            same_cut = same_cut && it != ds.vq_cut.end() && it->second.size() == kv.second.size();
+            for (size_t i = 0; same_cut && i < kv.second.size(); ++i)
+                same_cut = it->second[i] == kv.second[i] ||
+                           std::abs(it->second[i] - kv.second[i]) <= 1e-12 * (1.0 + std::abs(kv.second[i]));
+        }
+        stage_coulomb(R0, ds.vq, qs, vst, st);
+        if (!same_cut) stage_coulomb(R0, ds.vq_cut, qs, vcst, st);
+        v_qs = qs;
+    }
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    free_b += work.bytes();
     // chi0(R, omega) once for all q when it fits in a quarter of the free memory
-    if (!R0.chiw_ok && R0.form_chiw(g, 0.25 * (double)free_b, st)) HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    if (!R0.chiw_ok && R0.form_chiw(g, 0.25 * (double)free_b, st)) {
+        HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+        free_b += work.bytes();
+    }
     // all frequencies of several q per pass (q is the inner loop of every launch), or some of one q
     const double per_w = 8.0 * ((double)NN + 2.0 * nn) + 16.0 * pl * N * (N >= (herm ? 2048 : 4096) ? (herm ? 1024 : 2048) : (herm ? 256 : 512));
     const double per_q = 8.0 * 14 * nn;
@@ -560,33 +590,49 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
     const int UCH = QG > 1 ? QG * nw : WCH;
     // F: v and then its factor (Cholesky, or square root); C: v_c and then its root; V0: v_c, or S_c S_c
     // when a root is filtered
-    DevBuf dFC(nn * 8 * 2 * QG), dV0(nn * 8 * QG), dD(nn * 8 * UCH), dX(nn * 8 * UCH), dA(NN * 8 * UCH), dacc(8 * (size_t)UCH),
-        dflag(16);
-    double *F = dFC.as<double>(), *C = F + nn * QG, *V0 = dV0.as<double>();
-    DevBuf dSg((size_t)n * 8 * 2 * QG), dProbe, dld(8 * 2 * (size_t)QG), dE;
+    double *F, *C, *V0, *D, *X, *A, *acc, *Sg, *ld, *U0, *Q, *dph, *dcoef;
+    int *flag;
+    const auto layout = [&](Carve &c) {
+        F = c.take<double>(2 * nn * QG);
+        C = F + nn * QG;
+        V0 = c.take<double>(nn * QG);
+        D = c.take<double>(nn * UCH);
+        X = c.take<double>(nn * UCH);
+        A = c.take<double>(NN * UCH);
+        acc = c.take<double>(UCH);
+        Sg = c.take<double>((size_t)n * QG);
+        ld = c.take<double>(QG);
+        U0 = c.take<double>(n);
+        Q = c.take<double>(WCH);
+        dph = c.take<double>(2 * (size_t)nR * QG);
+        dcoef = c.take<double>((size_t)UCH * g.n);
+        flag = c.take<int>(2);
+    };
+    SigmaWork later;
+    Carve count{nullptr};
+    sigma_layout(count, later);
+    carve(work, layout, count.at);
+    DevBuf dE;
     std::vector<double> hsg;
-    HIP_CHECK(hipMemsetAsync(dacc.get(), 0, dacc.bytes(), st));
-    HIP_CHECK(hipMemsetAsync(dflag.get(), 0, 16, st));
-    CholWork cw;
+    HIP_CHECK(hipMemsetAsync(acc, 0, 8 * (size_t)UCH, st));
+    HIP_CHECK(hipMemsetAsync(flag, 0, 2 * sizeof(int), st));
+    CholWork &cw = R0.ec_cw;
     // L S L^H of cnt matrices in place; which of them have a zero or negative pivot: v^{1/2} must then come
     // from the eigen-decomposition with the negative eigenvalues dropped (power_hemat, matrix_m.h:916-970).
     // A zero pivot raises the flag of the whole batch, whose matrices are then looked at one by one.
     auto factor = [&](double *M, int cnt, std::vector<char> &neg) {
         neg.assign(cnt, 0);
-        DevBuf keep;
-        if (cnt > 1) {
-            keep.alloc(nn * 8 * cnt);
-            HIP_CHECK(hipMemcpyAsync(keep.get(), M, nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
-        }
+        // (X is free until chi0's products)
+        if (cnt > 1) HIP_CHECK(hipMemcpyAsync(X, M, nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
         auto run = [&](int m0, int m1) {
-            HIP_CHECK(hipMemsetAsync(dld.get(), 0, dld.bytes(), st));
-            HIP_CHECK(hipMemsetAsync(dflag.as<int>() + 1, 0, sizeof(int), st));
-            cholesky_logdet_batched(M + m0 * nn, nn, m1 - m0, n, n, dld.as<double>(), 1, dflag.as<int>() + 1, true, cw, st,
-                                    -1, dSg.as<double>(), n, herm ? plane : 0);
+            HIP_CHECK(hipMemsetAsync(ld, 0, 8 * (size_t)QG, st));
+            HIP_CHECK(hipMemsetAsync(flag + 1, 0, sizeof(int), st));
+            cholesky_logdet_batched(M + m0 * nn, nn, m1 - m0, n, n, ld, 1, flag + 1, true, cw, st,
+                                    -1, Sg, n, herm ? plane : 0);
             hsg.resize((size_t)n * (m1 - m0));
             int zf = 0;
-            HIP_CHECK(hipMemcpyAsync(hsg.data(), dSg.get(), 8 * hsg.size(), hipMemcpyDeviceToHost, st));
-            HIP_CHECK(hipMemcpyAsync(&zf, dflag.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
+            HIP_CHECK(hipMemcpyAsync(hsg.data(), Sg, 8 * hsg.size(), hipMemcpyDeviceToHost, st));
+            HIP_CHECK(hipMemcpyAsync(&zf, flag + 1, sizeof(int), hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
             for (int m = m0; m < m1; ++m)
                 for (int i = 0; i < n; ++i)
@@ -595,21 +641,18 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
         };
         if (!run(0, cnt)) return;
         if (cnt == 1) { neg[0] = 1; return; }
-        HIP_CHECK(hipMemcpyAsync(M, keep.get(), nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
+        HIP_CHECK(hipMemcpyAsync(M, X, nn * 8 * cnt, hipMemcpyDeviceToDevice, st));
         for (int m = 0; m < cnt; ++m) {
             neg[m] = 0;
             if (run(m, m + 1)) neg[m] = 1;
         }
     };
     // head replacement at q = 0: eps_mac per frequency and the leading eigenvector of Re v(0)
-    DevBuf dHead, dU0((size_t)n * 8), dQ(sizeof(double) * (WCH + 1));
+    DevBuf dHead;
     if (!head.empty()) {
         if ((int)head.size() != nw) LRA_THROW("dielectric function: one value per frequency of the grid is needed");
         dHead = upload(head, st);
     }
-    CoulombStage vst, vcst;
-    stage_coulomb(R0, ds.vq, qs, vst, st);
-    if (!same_cut) stage_coulomb(R0, ds.vq_cut, qs, vcst, st);
     // filtered root of one matrix, through the real embedding when there are k points
     auto eig_root = [&](double *M, double *top) {
         if (!herm) return eig_sqrt(M, n, sqrt_threshold, top, 1, st);
@@ -700,11 +743,11 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
                 dense_coulomb(vcst, iq0, qg, n, lay, false, C, nn, st);
                 HIP_CHECK(hipMemcpyAsync(V0, C, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
                 if (sqrt_threshold <= 0) {
-                    dProbe.reserve(nn * 8 * qg);
-                    HIP_CHECK(hipMemcpyAsync(dProbe.get(), F, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
-                    factor(dProbe.as<double>(), qg, neg);
-                    HIP_CHECK(hipMemcpyAsync(dProbe.get(), C, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
-                    factor(dProbe.as<double>(), qg, negc);
+                    // (D is free until chi0 is assembled)
+                    HIP_CHECK(hipMemcpyAsync(D, F, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+                    factor(D, qg, neg);
+                    HIP_CHECK(hipMemcpyAsync(D, C, nn * 8 * qg, hipMemcpyDeviceToDevice, st));
+                    factor(D, qg, negc);
                 }
             } else if (sqrt_threshold > 0) {
                 fill_v(V0);
@@ -720,14 +763,14 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
                 if (!eig[i]) sel.push_back(i);
                 if (!same_cut && !eigc[i]) sel.push_back(QG + i);
             }
-            ns_sqrt(F, n, herm, sel, st);
+            ns_sqrt(F, n, herm, sel, A, (size_t)NN * UCH, st);
             std::vector<long long> sq;
             std::vector<int> which;
             for (int i = 0; i < qg; ++i) {
                 if (chol[i]) continue;
                 const bool head_q = head_here && i == gamma;
                 if (eig[i]) {
-                    const auto top2 = eig_root(F + i * nn, head_q ? dU0.as<double>() : nullptr);
+                    const auto top2 = eig_root(F + i * nn, head_q ? U0 : nullptr);
                     if (head_q && !(top2.first - top2.second > 1e-8 * std::fabs(top2.first)))
                         LRA_THROW("head of the dielectric matrix: the largest eigenvalue of v(0) is degenerate");
                 }
@@ -748,29 +791,29 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
                 ph[((size_t)i * nR + rr) * 2] = std::cos(ang);
                 ph[((size_t)i * nR + rr) * 2 + 1] = std::sin(ang);
             }
-        DevBuf dph = upload(ph, st);
+        HIP_CHECK(hipMemcpyAsync(dph, ph.data(), 8 * ph.size(), hipMemcpyHostToDevice, st));
         const int cstep = qg > 1 ? nw : WCH;
         for (int w0 = 0; w0 < nw; w0 += cstep) {
             const int cnt = std::min(cstep, nw - w0), nu = qg * cnt;
             prof.begin("gw_w_chi0q", st);
-            R0.assemble_dense_q(g, kfs, w0, cnt, dD.get(), true, nn, lay, st);
+            R0.assemble_dense_q(g, kfs, w0, cnt, D, true, nn, lay, st);
             prof.end("gw_w_chi0q", st);
             auto &bb = get_batches(qg, cnt, tri);
             prof.begin("gw_w_gemm", st);
-            gemm_run(Prec::F64, bb.first, dD.get(), F, dX.get(), 1.0, 0.0, st);
-            launch_fill_aug(dA.as<double>(), NN, im, qg, cnt, n, C, V0, st);
-            gemm_run(Prec::F64, bb.second, F, dX.get(), dA.get(), -1.0, 1.0, st);
+            gemm_run(Prec::F64, bb.first, D, F, X, 1.0, 0.0, st);
+            launch_fill_aug(A, NN, im, qg, cnt, n, C, V0, st);
+            gemm_run(Prec::F64, bb.second, F, X, A, -1.0, 1.0, st);
             if (head_here) {
                 // eps += (eps_mac - u^T eps u) u u^T, u the leading eigenvector of Re v(0): the
                 // head overwrite of epsilon.cpp:2106-2181 in the eigenbasis of v (real at q = 0)
-                double *A0 = dA.as<double>() + (long long)gamma * cnt * NN;
-                HIP_CHECK(hipMemsetAsync(dQ.get(), 0, sizeof(double) * cnt, st));
-                launch_head_quad(A0, NN, N, n, cnt, dU0.as<double>(), dQ.as<double>(), st);
-                launch_head_update(A0, NN, N, n, cnt, dU0.as<double>(), dHead.as<double>() + w0, dQ.as<double>(), st);
+                double *A0 = A + (long long)gamma * cnt * NN;
+                HIP_CHECK(hipMemsetAsync(Q, 0, sizeof(double) * cnt, st));
+                launch_head_quad(A0, NN, N, n, cnt, U0, Q, st);
+                launch_head_update(A0, NN, N, n, cnt, U0, dHead.as<double>() + w0, Q, st);
             }
             prof.end("gw_w_gemm", st, bb.first.flops + bb.second.flops);
             prof.begin("gw_w_schur", st);
-            cholesky_logdet_batched(dA.as<double>(), NN, nu, N, N, dacc.as<double>(), 1, dflag.as<int>(), false, cw, st, n,
+            cholesky_logdet_batched(A, NN, nu, N, N, acc, 1, flag, false, cw, st, n,
                                     nullptr, 0, im);
             prof.end("gw_w_schur", st, (herm ? 4.0 : 1.0) * nu * (7.0 / 3.0) * n * (double)n * n);
             // W(R, tau) += sum_(q, w) f2t(tau, w) / N_k (cos Re W + sin Im W)
@@ -780,15 +823,15 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
                 for (int w = 0; w < cnt; ++w)
                     for (int t = 0; t < g.n; ++t)
                         coef[((size_t)i * cnt + w) * g.n + t] = g.cos_f2t[(size_t)t * g.n + w0 + w] * mult[qs[iq0 + i]] / nk;
-            DevBuf dcoef = upload(coef, st);
-            launch_w_accum(dA.as<double>(), NN, im, qg, cnt, n, dcoef.as<double>(), g.n, dph.as<double>(), nR,
-                           d_Wrt.as<double>(), st);
+            HIP_CHECK(hipMemcpyAsync(dcoef, coef.data(), 8 * coef.size(), hipMemcpyHostToDevice, st));
+            launch_w_accum(A, NN, im, qg, cnt, n, dcoef, g.n, dph, nR,
+                           out.Wrt.as<double>(), st);
             HIP_CHECK(hipStreamSynchronize(st));
             prof.end("gw_w_accum", st, 0, 8.0 * nu * (double)nn * ceil_div(g.n, 4) + 16.0 * g.n * nR * (double)n * n);
         }
     }
     int hflag = 0;
-    HIP_CHECK(hipMemcpyAsync(&hflag, dflag.get(), sizeof(hflag), hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipMemcpyAsync(&hflag, flag, sizeof(hflag), hipMemcpyDeviceToHost, st));
     HIP_CHECK(hipStreamSynchronize(st));
     if (hflag) LRA_THROW("1 - v^1/2 chi0 v^1/2 is singular or not finite at some (q, omega)");
     const double n3 = (herm ? 4.0 : 1.0) * n * (double)n * n;
@@ -799,25 +842,22 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g) {
 // ------------------------------------------------------------------------------------------
 // Sigma(R, i omega)
 // ------------------------------------------------------------------------------------------
-void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
+void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g, Result &out) {
     auto &prof = profiler();
     const double t0 = now_s();
     RpaEngine &R0 = *rpa;
     const hipStream_t st = R0.stream;
     const int nw = g.n;
     const long long nel = (long long)nR * NAO * NAO;
-    d_Sre.alloc(sizeof(double) * (size_t)nspin * nw * nel);
-    d_Sim.alloc(sizeof(double) * (size_t)nspin * nw * nel);
-    HIP_CHECK(hipMemsetAsync(d_Sre.get(), 0, d_Sre.bytes(), st));
-    HIP_CHECK(hipMemsetAsync(d_Sim.get(), 0, d_Sim.bytes(), st));
-    if (w_zero) { HIP_CHECK(hipStreamSynchronize(st)); t_sigma = now_s() - t0; return; }
-    d_U.alloc(2 * (size_t)u_elems * nbatch * ts);
-    d_Ghat.alloc((size_t)max_ghat * nbatch * ts);
-    d_CW.alloc(((size_t)max_cw * nbatch + kChi0Pad) * ts);
-    d_Y.alloc(2 * (size_t)y_elems * nbatch * ts);
-    const size_t next = (size_t)NE * NAO * NAO;
-    d_sig.alloc(2 * (size_t)nbatch * (2 * nel + next) * ts);
-    if (prec != Prec::F64) d_Wf.alloc((size_t)nbatch * nR * NABF * NABF * ts);
+    out.Sre.alloc(sizeof(double) * (size_t)nspin * nw * nel);
+    out.Sim.alloc(sizeof(double) * (size_t)nspin * nw * nel);
+    HIP_CHECK(hipMemsetAsync(out.Sre.get(), 0, out.Sre.bytes(), st));
+    HIP_CHECK(hipMemsetAsync(out.Sim.get(), 0, out.Sim.bytes(), st));
+    if (out.w_zero) { HIP_CHECK(hipStreamSynchronize(st)); t_sigma = now_s() - t0; return; }
+    const size_t next = (size_t)NE * NAO * NAO, sig_elems = 2 * (size_t)nbatch * (2 * nel + next);
+    SigmaWork w;
+    carve(work, [&](Carve &c) { sigma_layout(c, w); });
+    char *const U = w.U, *const Ghat = w.Ghat, *const CW = w.CW, *const Y = w.Y, *const sigma = w.sigma, *const Wlow = w.Wlow;
     R0.prepare_gf(ds.mf, -1);  // all bands (get_gf_cplx_imagtimes_Rs, meanfield.cpp:309-365)
     const long long nn_abf = (long long)NABF * NABF, zg = (long long)nR * NAO * 2 * NAO;
     DevBuf dcw = upload(g.cos_t2f, st), dsw = upload(g.sin_t2f, st);
@@ -828,14 +868,15 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
     auto passes = [&](auto tag) {
         using T = decltype(tag);
         const T *G = R0.d_Gpm.as<T>();
+        T *const tU = reinterpret_cast<T *>(U), *const tCW = reinterpret_cast<T *>(CW), *const tY = reinterpret_cast<T *>(Y);
         for (int it = 0, nz = 1; it < g.n; it += nz) {
             // tau points [it, it + nz) in one pass
             nz = std::min(nbatch, g.n - it);
-            const void *Wf = d_Wrt.as<double>() + (size_t)it * nR * nn_abf;
+            const void *Wf = out.Wrt.as<double>() + (size_t)it * nR * nn_abf;
             if (prec != Prec::F64) {
-                launch_convert<double, float>(d_Wrt.as<double>() + (size_t)it * nR * nn_abf, d_Wf.as<float>(),
+                launch_convert<double, float>(out.Wrt.as<double>() + (size_t)it * nR * nn_abf, reinterpret_cast<float *>(Wlow),
                                               (long long)nz * nR * nn_abf, st);
-                Wf = d_Wf.get();
+                Wf = Wlow;
             }
             if (verbose) {
                 HIP_CHECK(hipStreamSynchronize(st));
@@ -844,12 +885,12 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
             }
             for (int s = 0; s < nspin; ++s) {
                 R0.build_gf(ds.mf, &g.tau[it], nz, s);
-                T *sig = d_sig.as<T>(), *s2 = sig + 2 * (size_t)nbatch * nel, *ext = s2 + 2 * (size_t)nbatch * nel;
-                HIP_CHECK(hipMemsetAsync(d_sig.get(), 0, d_sig.bytes(), st));
+                T *sig = reinterpret_cast<T *>(sigma), *s2 = sig + 2 * (size_t)nbatch * nel, *ext = s2 + 2 * (size_t)nbatch * nel;
+                HIP_CHECK(hipMemsetAsync(sigma, 0, sig_elems * ts, st));
                 // U_J(S) for all J, S
                 for (auto &c : uchunks) {
                     prof.begin("gw_gather", st);
-                    launch_gather_cols<T>(G, 2LL * NAO, d_Ghat.as<T>(), c.d_jobs.template as<GatherJob>(), (int)c.jobs.size(),
+                    launch_gather_cols<T>(G, 2LL * NAO, reinterpret_cast<T *>(Ghat), c.d_jobs.template as<GatherJob>(), (int)c.jobs.size(),
                                           c.d_colsrc.template as<long long>(), NAO, c.max_gcol, st, nz, zg, c.ghat_elems);
                     prof.end("gw_gather", st, 0, 2.0 * nz * c.ghat_elems * ts);
                     prof.begin("gw_U", st);
@@ -857,8 +898,8 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
                     c.ub.za = c.ghat_elems;
                     c.ub.zc = 2 * u_elems;
                     if (tune_sigma && !c.ub.tuned)
-                        c.ub.tune(prec, d_Ghat.get(), R0.d_CWb.get(), d_U.get(), 1.0, 0.0, st);
-                    gemm_run(prec, c.ub, d_Ghat.get(), R0.d_CWb.get(), d_U.get(), 1.0, 0.0, st);
+                        c.ub.tune(prec, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
+                    gemm_run(prec, c.ub, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
                     prof.end("gw_U", st, nz * c.ub.flops);
                 }
                 for (auto &c : xchunks) {
@@ -868,38 +909,38 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
                         c.cwb.zb = nR * nn_abf;
                         c.cwb.zc = c.cw_elems;
                         if (tune_sigma && !c.cwb.tuned)
-                            c.cwb.tune(prec, R0.d_Cfin.get(), Wf, d_CW.get(), 1.0, 0.0, st);
-                        gemm_run(prec, c.cwb, R0.d_Cfin.get(), Wf, d_CW.get(), 1.0, 0.0, st);
+                            c.cwb.tune(prec, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
+                        gemm_run(prec, c.cwb, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
                         prof.end("gw_CW", st, nz * c.cwb.flops);
                     }
                     const SigBlk *blks = c.d_blks.template as<SigBlk>();
                     const Chi0Seg *segs = R0.d_segs.as<Chi0Seg>();
                     prof.begin("gw_D", st);
                     for (auto &t : c.d)
-                        launch_sigma_d<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, d_CW.as<T>(), c.cw_elems,
-                                          d_U.as<T>(), u_elems, sig, nel, NAO, nz, st);
+                        launch_sigma_d<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
+                                          tU, u_elems, sig, nel, NAO, nz, st);
                     prof.end("gw_D", st);
                     prof.begin("gw_B", st);
                     for (auto &t : c.b)
-                        launch_sigma_b<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, d_CW.as<T>(), c.cw_elems,
-                                          d_U.as<T>(), u_elems, s2, nel, NAO, nz, st);
+                        launch_sigma_b<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
+                                          tU, u_elems, s2, nel, NAO, nz, st);
                     prof.end("gw_B", st);
                     prof.begin("gw_Y", st);
                     for (auto &t : ytasks)
-                        launch_sigma_y<T>(t.d.template as<SigYTask>(), t.n, t.a, d_yent.as<SigYEnt>(), d_CW.as<T>(), c.cw_elems,
-                                          G, zg, d_Y.as<T>(), y_elems, NAO, c.x0, c.x1, c.x0 == 0, nz, st);
+                        launch_sigma_y<T>(t.d.template as<SigYTask>(), t.n, t.a, d_yent.as<SigYEnt>(), tCW, c.cw_elems,
+                                          G, zg, tY, y_elems, NAO, c.x0, c.x1, c.x0 == 0, nz, st);
                     prof.end("gw_Y", st);
                 }
                 prof.begin("gw_A3", st);
                 a3.nz = 2 * nz;
                 a3.zb = y_elems;
                 a3.zc = (long long)next;
-                gemm_run(prec, a3, R0.d_Cfin.get(), d_Y.get(), ext, 1.0, 1.0, st);
+                gemm_run(prec, a3, R0.d_Cfin.get(), Y, ext, 1.0, 1.0, st);
                 prof.end("gw_A3", st, 2 * nz * a3.flops);
                 prof.begin("gw_fold", st);
                 launch_sigma_fold<T>(sig, s2, ext, d_fold.as<int>(), d_neg.as<int>(), NE, nR, NAO, nz, st);
                 launch_sigma_freq<T>(sig, nel, dcw.as<double>(), dsw.as<double>(), nw, g.n, it, nz,
-                                     d_Sre.as<double>() + (size_t)s * nw * nel, d_Sim.as<double>() + (size_t)s * nw * nel,
+                                     out.Sre.as<double>() + (size_t)s * nw * nel, out.Sim.as<double>() + (size_t)s * nw * nel,
                                      st);
                 prof.end("gw_fold", st);
             }
@@ -908,7 +949,7 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g) {
     if (prec == Prec::F64) passes(double());
     else passes(float());
     HIP_CHECK(hipStreamSynchronize(st));
-    for (DevBuf *b : {&d_U, &d_Ghat, &d_CW, &d_Y, &d_sig, &d_Wf}) b->release();
+    if ((double)work.bytes() > kKeepBytes) work.release();
     t_sigma = now_s() - t0;
 }
 
@@ -918,7 +959,7 @@ void GwEngine::w_block(int it, int I, int J, int r, double *out) const {
     std::vector<double> row(R0.na[J]);
     for (int mu = 0; mu < R0.na[I]; ++mu) {
         const size_t off = ((size_t)it * nR + r) * nn + (size_t)(R0.abf[I] + mu) * NABF + R0.abf[J];
-        HIP_CHECK(hipMemcpy(out + (size_t)mu * R0.na[J], d_Wrt.as<double>() + off, sizeof(double) * R0.na[J],
+        HIP_CHECK(hipMemcpy(out + (size_t)mu * R0.na[J], res->Wrt.as<double>() + off, sizeof(double) * R0.na[J],
                             hipMemcpyDeviceToHost));
     }
 }
@@ -929,9 +970,9 @@ void GwEngine::sigma_block(int spin, int iw, int I, int J, int r, double *re, do
     for (int i = 0; i < R0.nb[I]; ++i) {
         const size_t off = ((size_t)spin * ntau + iw) * nel + (size_t)r * NAO * NAO + (size_t)(R0.ao[I] + i) * NAO +
                            R0.ao[J];
-        HIP_CHECK(hipMemcpy(re + (size_t)i * R0.nb[J], d_Sre.as<double>() + off, sizeof(double) * R0.nb[J],
+        HIP_CHECK(hipMemcpy(re + (size_t)i * R0.nb[J], res->Sre.as<double>() + off, sizeof(double) * R0.nb[J],
                             hipMemcpyDeviceToHost));
-        HIP_CHECK(hipMemcpy(im + (size_t)i * R0.nb[J], d_Sim.as<double>() + off, sizeof(double) * R0.nb[J],
+        HIP_CHECK(hipMemcpy(im + (size_t)i * R0.nb[J], res->Sim.as<double>() + off, sizeof(double) * R0.nb[J],
                             hipMemcpyDeviceToHost));
     }
 }
@@ -973,29 +1014,34 @@ std::vector<std::vector<cplx>> GwEngine::ks_diag(const Dataset &ds, int spin, in
                 ph[(((size_t)I * natom + J) * nR + rr) * 2] = std::cos(ang);
                 ph[(((size_t)I * natom + J) * nR + rr) * 2 + 1] = std::sin(ang);
             }
-    std::vector<int> atom_of(NAO);
-    for (int I = 0; I < natom; ++I)
-        for (int i = 0; i < R0.nb[I]; ++i) atom_of[R0.ao[I] + i] = I;
-    DevBuf dph = upload(ph, st), dat = upload(atom_of, st);
+    // one upload and one download per 16 states, in buffers that stay
+    std::lock_guard<std::mutex> lk(ks_mu);
     const auto &Uk = ds.mf.wfc[(size_t)spin * nk + ik];
     std::vector<std::vector<cplx>> out(states.size(), std::vector<cplx>(nw));
     const long long nel = (long long)nR * NAO * NAO;
     for (size_t s0 = 0; s0 < states.size(); s0 += 16) {
         const int ns = (int)std::min<size_t>(16, states.size() - s0);
-        std::vector<double> U((size_t)ns * NAO * 2);
+        std::vector<double> in(ph);
+        in.resize(ph.size() + (size_t)ns * NAO * 2 + NAO);
+        double *U = in.data() + ph.size();
         for (int a = 0; a < ns; ++a)
             for (int b = 0; b < NAO; ++b) {
                 const cplx u = Uk[(size_t)states[s0 + a] * NAO + b];
                 U[((size_t)a * NAO + b) * 2] = u.real();
                 U[((size_t)a * NAO + b) * 2 + 1] = u.imag();
             }
-        DevBuf dU = upload(U, st);
-        DevBuf dY(sizeof(double) * (size_t)nw * NAO * ns * 2);
-        launch_sigma_ks_rows(d_Sre.as<double>() + (size_t)spin * nw * nel, d_Sim.as<double>() + (size_t)spin * nw * nel,
-                             nw, nR, NAO, dat.as<int>(), natom, dph.as<double>(), dU.as<double>(), ns, dY.as<double>(),
-                             st);
+        int *atom_of = reinterpret_cast<int *>(U + (size_t)ns * NAO * 2);
+        for (int I = 0; I < natom; ++I)
+            for (int i = 0; i < R0.nb[I]; ++i) atom_of[R0.ao[I] + i] = I;
         std::vector<double> Y((size_t)nw * NAO * ns * 2);
-        HIP_CHECK(hipMemcpyAsync(Y.data(), dY.get(), Y.size() * 8, hipMemcpyDeviceToHost, st));
+        ks_in.reserve(8 * in.size());
+        ks_out.reserve(8 * Y.size());
+        const double *dph = ks_in.as<double>(), *dU = dph + ph.size();
+        HIP_CHECK(hipMemcpyAsync(ks_in.get(), in.data(), 8 * in.size(), hipMemcpyHostToDevice, st));
+        launch_sigma_ks_rows(res->Sre.as<double>() + (size_t)spin * nw * nel, res->Sim.as<double>() + (size_t)spin * nw * nel,
+                             nw, nR, NAO, reinterpret_cast<const int *>(dU + (size_t)ns * NAO * 2), natom, dph, dU, ns,
+                             ks_out.as<double>(), st);
+        HIP_CHECK(hipMemcpyAsync(Y.data(), ks_out.get(), Y.size() * 8, hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
         for (int a = 0; a < ns; ++a)
             for (int w = 0; w < nw; ++w) {
@@ -1091,16 +1137,21 @@ void gw_build_sigma(Dataset &d, const LibrpaOptions &o) {
         eng->plan(d, d.chi0_prec, d.ec_prec, d.grid.n);
         d.rpa = eng;
     }
+    // the plan and the work memory stay with the inputs they were made for
+    auto gw = d.gw;
+    if (!gw || gw->rpa != eng) gw = std::make_shared<GwEngine>();
     eng->build_chi0(d, d.grid, o.n_bands_chi0);
-    eng->release_work();  // chi0(R, tau) stays; the chi0 work buffers are rebuilt on demand
-    eng->release_ec();    // an earlier Ec evaluation's buffers
-    auto gw = std::make_shared<GwEngine>();
+    // chi0(R, tau) stays; large chi0 work buffers and those of an earlier Ec evaluation are rebuilt on demand
+    if (eng->work_bytes() > GwEngine::kKeepBytes) eng->release_work();
+    if (eng->ec_bytes() > GwEngine::kKeepBytes) eng->release_ec();
     gw->verbose = o.output_level >= LIBRPA_VERBOSE_DEBUG;
     gw->head = head;
     gw->sqrt_threshold = o.sqrt_coulomb_threshold;
-    gw->plan(d, eng);
-    gw->build_w(d, d.grid);
-    gw->build_sigma(d, d.grid);
+    if (gw->rpa != eng) gw->plan(d, eng);
+    auto res = std::make_shared<GwEngine::Result>();
+    gw->build_w(d, d.grid, *res);
+    gw->build_sigma(d, d.grid, *res);
+    gw->res = res;
     d.gw = gw;
 }
 

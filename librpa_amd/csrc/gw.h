@@ -4,6 +4,7 @@
 
 #include <cstdio>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "../../include/librpa_options.h"
@@ -14,6 +15,25 @@
 #include "rpa.h"
 
 namespace lra {
+
+// The upper atom-pair blocks (I <= J) of a Coulomb input for a list of k points, on the device for
+// launch_v_scatter (VBlock::q: position in the list), with the largest |V| and |Im V| of each.
+struct CoulombStage {
+    DevBuf blk, desc;
+    std::vector<int> first;  // descriptors of point i: [first[i], first[i + 1])
+    std::vector<double> vmax, imax;
+};
+
+// consecutive 256-byte aligned pieces of a buffer (a null base counts the bytes)
+struct Carve {
+    char *base;
+    size_t at = 0;
+    template <class T> T *take(size_t n) {
+        T *p = reinterpret_cast<T *>(base + at);
+        at += (n * sizeof(T) + 255) / 256 * 256;
+        return p;
+    }
+};
 
 struct GwEngine {
     std::shared_ptr<RpaEngine> rpa;  // geometry, G(R, +-tau) builder, chi0(R, tau)
@@ -59,12 +79,26 @@ struct GwEngine {
     std::vector<long long> y_off;
     long long y_elems = 0;
 
-    DevBuf d_U, d_Ghat, d_CW, d_Y, d_Wf;
-    DevBuf d_sig;  // sig, s2 and ext of every tau point and sign of a pass
     DevBuf d_fold, d_neg;
-    DevBuf d_Wrt;         // W(R, tau) [tau][R][NABF][NABF], FP64
-    DevBuf d_Sre, d_Sim;  // Sigma(R, i omega) [spin][omega][R][NAO][NAO], FP64
-    bool w_zero = false;  // no truncated Coulomb given: W = 0
+    // Work memory of W and of Sigma, one after the other in the same bytes.  Kept for the next build up to
+    // kKeepBytes (allocating and freeing 3 GB took 30 of the 86 ms of a build on 8 atoms and 4 k), as are
+    // the chi0 build's buffers beside it; larger systems give it back after every build.
+    DevBuf work;
+    static constexpr double kKeepBytes = 12e9;
+    struct SigmaWork { char *U, *Ghat, *CW, *Y, *sigma, *Wlow; };  // sigma: sig, s2 and ext of each tau and sign
+    void sigma_layout(Carve &c, SigmaWork &w) const;
+    CoulombStage vst, vcst;          // the Coulomb inputs of the q in v_qs
+    std::vector<int> v_qs;
+    bool same_cut = false;           // v_c = v
+    // What a build leaves for the getters; replaced when the next one is complete.
+    struct Result {
+        DevBuf Wrt;       // W(R, tau) [tau][R][NABF][NABF], FP64
+        DevBuf Sre, Sim;  // Sigma(R, i omega) [spin][omega][R][NAO][NAO], FP64
+        bool w_zero = false;  // no truncated Coulomb given: W = 0
+    };
+    std::shared_ptr<Result> res;
+    mutable std::mutex ks_mu;  // ks_diag's buffers
+    DevBuf ks_in, ks_out;
 
     double flops_sigma = 0, flops_w = 0, t_w = 0, t_sigma = 0;
     long long max_ghat = 0, max_cw = 0;
@@ -73,11 +107,10 @@ struct GwEngine {
     // (replace_w_head with option_dielect_func 0); empty = no replacement
     std::vector<double> head;
     double sqrt_threshold = 0.0;  // sqrt_coulomb_threshold: eigenvalues of v, v_c below it are dropped
-    bool sigma_tuned = false;  // Sigma batches' tiles timed (LIBRPA_AMD_TUNE_SIGMA=1) on the first pass
 
     void plan(const Dataset &ds, std::shared_ptr<RpaEngine> r);
-    void build_w(const Dataset &ds, const TFGrid &g);
-    void build_sigma(const Dataset &ds, const TFGrid &g);
+    void build_w(const Dataset &ds, const TFGrid &g, Result &out);
+    void build_sigma(const Dataset &ds, const TFGrid &g, Result &out);
     void w_block(int it, int I, int J, int r, double *out) const;
     void sigma_block(int spin, int iw, int I, int J, int r, double *re, double *im) const;
     // Sigma_KS(k, i omega)_nn for the given states: [state][omega]

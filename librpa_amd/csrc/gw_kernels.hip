@@ -550,6 +550,7 @@ __global__ __launch_bounds__(256) void sigma_ks_rows_kernel(const double *__rest
     const int lane = t & 63, wave = t >> 6;
 #pragma unroll
     for (int st = 0; st < kStMax; ++st) {
+        if (st >= nst) break;
         double x = ar[st], y = ai[st];
         for (int o = 32; o > 0; o >>= 1) {
             x += __shfl_xor(x, o, 64);

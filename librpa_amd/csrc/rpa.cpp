@@ -652,10 +652,7 @@ RpaResult RpaEngine::ec(const Dataset &ds, const TFGrid &g) {
     // enough matrices to fill the device
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
     // the Ec buffers kept from an earlier call count as free here (they are reused or regrown)
-    double held = 0;
-    for (const DevBuf *b : {&ec_V, &ec_L32, &ec_D, &ec_X, &ec_M, &ec_M64, &ec_S, &ec_Vld, &ec_acc, &ec_cw.linv,
-                            &ec_cw.panel})
-        held += (double)b->bytes();
+    const double held = ec_bytes();
     const double panel_w = 16.0 * n * (n >= (herm ? 2048 : 4096) ? 2048 : 512);  // Cholesky panels per matrix
     const double per_w = (double)nn * (3 * es + (f64 ? 0 : 8)) + panel_w;
     const double per_q = (double)nn * 12 + panel_w;
@@ -941,6 +938,14 @@ void RpaEngine::assemble_dense(const TFGrid &g, const double *kf, int w0, int cn
                                                dgp.as<double>(), cw_n, (float *)Dd, nn, n, lay, s);
         HIP_CHECK(hipStreamSynchronize(s));  // dgp is freed on return
     }
+}
+
+double RpaEngine::ec_bytes() const {
+    double held = 0;
+    for (const DevBuf *b : {&ec_V, &ec_L32, &ec_D, &ec_X, &ec_M, &ec_M64, &ec_S, &ec_Vld, &ec_acc, &ec_cw.linv,
+                            &ec_cw.panel})
+        held += (double)b->bytes();
+    return held;
 }
 
 void RpaEngine::release_ec() {

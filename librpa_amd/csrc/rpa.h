@@ -136,6 +136,8 @@ struct RpaEngine {
     void build_gf(const MeanField &mf, const double *taus, int nz, int s);
     void build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g);
     void release_work();  // free the gathered-G and W work buffers (rebuilt by build_chi0)
+    double ec_bytes() const;
+    double work_bytes() const { return (double)d_Ghat.bytes() + (double)d_W.bytes(); }
     void release_ec();    // free the Ec work buffers (rebuilt by ec)
     // chi0(R, omega) = sum_tau (2 / nspin) gamma_c(omega, tau) chi0(R, tau) of the last build, FP64
     // [omega][E], formed once per Ec / W evaluation when it fits in max_bytes (returns whether it
