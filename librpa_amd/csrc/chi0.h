@@ -13,7 +13,7 @@ namespace lra {
 struct Chi0Out {
     long long cfin;    // Cfin_I [(K, R1, k, i)][mu]
     long long gpm;     // G_IJ(R) in Gpm: element (i, q) at gpm + i * 2 NAO + q, q = (s, j)
-    long long wseg;    // W(., J, cell 0); cell S at + S * 2 nj NAO * aj
+    long long wseg;    // W(., J, cell 0); cell S at + S * NAO * 2 nj * aj
     long long xa, xb;  // W(I, -R) rows of J and W(J, R) rows of I (the direct term's operands)
     long long eoff;    // chi0s block, row-major ai x aj
     int ni, nj, ai, aj;
@@ -21,7 +21,7 @@ struct Chi0Out {
     int lsum;          // segments: rows (K, R1, k) of atom I
     int segtab;        // first entry of (I, R) in the segment table
 };
-// Segment t of (I, R): W(K, J, R - R1) row k is at wseg + (cell * 2 nj NAO + row) * aj, its rows
+// Segment t of (I, R): W(K, J, R - R1) row k is at wseg + (cell * NAO + row) * 2 nj * aj, its rows
 // of Cfin_I start at c * ni.  In the order of (cell, row): the outputs of one R then walk through
 // the rows of W and of Cs in step, whatever their I and J.
 struct Chi0Seg { int cell, row, c, pad; };

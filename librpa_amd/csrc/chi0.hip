@@ -16,9 +16,9 @@
 // the loop; only G_IJ, which every segment reuses, is in LDS.  An operand register is loaded again
 // as soon as the MFMAs that read it are issued, so a load has 1 to 4 thousand cycles of MFMA to
 // arrive.  Measured against the two GEMMs with T between them (38 GB of it per tau point on a
-// 64-atom cell), X and T_A and contraction together: 526 -> 448 ms on 64 atoms at Gamma (42 TF/s of
-// the sums' own flops, the MFMA pipes 75% busy; 60- and 120-row blocks and 13- and 27-row T
-// fragments pad the rest), 52 -> 34 ms on 16 atoms and 8 k (45 TF/s, 84% busy).
+// 64-atom cell), X and T_A and contraction together: 526 -> 411 ms on 64 atoms at Gamma (46 TF/s of
+// the sums' own flops; 60- and 120-row blocks and 13- and 27-row T fragments pad the rest), 52 -> 32.7 ms
+// on 16 atoms and 8 k (47 TF/s).
 #include "chi0.h"
 
 #include <algorithm>
@@ -30,9 +30,9 @@ namespace lra {
 namespace {
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-// 16-byte loads at element alignment (rows of odd basis sizes)
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+// 16-byte buffer loads need dword alignment only (rows of odd basis sizes)
+typedef double d2u __attribute__((ext_vector_type(2)));
+typedef float f4u __attribute__((ext_vector_type(4)));
 
 template <class T> struct CT;
 template <> struct CT<double> { using V = d2u; using A = v4d; static constexpr int VL = 2; };
@@ -79,17 +79,19 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
     const bool active = ta < tb && n0 < O.aj;
     const int ni = O.ni, ai = O.ai, aj = O.aj, qn = 2 * O.nj;
     const int QS = (qn + 3) / 4;
-    // byte offsets of a lane: row kq of the four rows of a step of W and of Cs, clamped in the last
-    // step (G, and so T, is zero past the end); the rest of each address is wave-uniform
-    const long long qstride = (long long)NAO * aj;
+    // byte offsets of a lane: its column, and row kq of the four rows of a step of W and of Cs, clamped
+    // to the last row (G, and so T, is zero past the end); the base of a segment is wave-uniform
     const unsigned nul = min(n0 + c * VL, aj - 1) * TS;
-    const unsigned qo = (unsigned)(kq * qstride) * TS + nul, qol = (unsigned)(min(kq, (qn - 1) & 3) * qstride) * TS + nul;
-    const unsigned co = kq * ai * TS, col = min(kq, (ni - 1) & 3) * ai * TS;
+    const unsigned qstep = 4 * aj * TS, qo = kq * aj * TS + nul, qmax = (qn - 1) * aj * TS + nul;
+    const unsigned cstep = 4 * ai * TS, co = kq * ai * TS;
     unsigned mul[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) mul[g] = min(tk.m0 + (g * 16 + c) * VL, ai - 1) * TS;
+    // 16 bytes at base + o: base in scalar registers, o one vector register (a 64-bit lane address per step
+    // and fragment, worked out ahead of the loop, took 64 registers and two moves per load)
     const auto at = [](const T *b, unsigned o) {
-        return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(b) + o);
+        const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(b), 0, -1, 0x00027000);
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0));
     };
 
     A acc[FM][FN];
@@ -117,18 +119,15 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
         const int CS = min(4 * FI, (ni - i0 + 3) / 4);
         const Chi0Seg *st = segs + O.segtab;
         const auto q_base = [&](const Chi0Seg &sg) {
-            return W + O.wseg + ((long long)sg.cell * qn * NAO + sg.row) * aj;
+            return W + O.wseg + ((long long)sg.cell * NAO + sg.row) * qn * aj;
         };
         const auto c_base = [&](const Chi0Seg &sg) { return Cfin + O.cfin + ((long long)sg.c * ni + i0) * ai; };
-        const auto load_q = [&](const T *qb, int s) {
-            s = min(s, QS - 1);
-            return at(qb + 4 * s * qstride, s == QS - 1 ? qol : qo);
-        };
+        const unsigned cmax = (ni - 1 - i0) * ai * TS;
+        const auto load_q = [&](const T *qb, int s) { return at(qb, min(qo + s * qstep, qmax)); };
         const auto load_c = [&](V *cc, const T *cb, int s) {
-            s = min(s, CS - 1);
-            const unsigned o = i0 + 4 * s + 4 >= ni ? col : co;
+            const unsigned o = min(co + s * cstep, cmax);
 #pragma unroll
-            for (int g = 0; g < G; ++g) cc[g] = at(cb + (long long)4 * s * ai, o + mul[g]);
+            for (int g = 0; g < G; ++g) cc[g] = at(cb, o + mul[g]);
         };
         A tf[FI][FN];
         const auto zero_t = [&]() {
@@ -167,6 +166,10 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
             for (int s = 0; s < RQ; ++s) qr[s] = load_q(qb, s);
             load_p(0);
             for (int t = ta; t < mb; ++t) {
+                // (opaque: comparisons with the steps stay in the loop, two scalar instructions each; ahead of it
+                // they were two dozen masks, spilled)
+                int qsteps = QS, csteps = CS;
+                asm volatile("" : "+s"(qsteps), "+s"(csteps));
                 const T *qn_ = q_base(s1), *cn_ = c_base(s1);
                 s1 = st[min(t + 2, mb - 1)];
 #pragma unroll
@@ -178,13 +181,13 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
 #pragma unroll
                     for (int f = 0; f < FI; ++f) pc[f] = pn[f];
                     load_p(s + 1 < NQ ? s + 1 : 0);
-                    if (s < QS) t_step(pc, qr[s % RQ]);
+                    if (s < qsteps) t_step(pc, qr[s % RQ]);
                     if (s + RQ < NQ) qr[s % RQ] = load_q(qb, s + RQ);
                     else qr[s % RQ] = load_q(qn_, s + RQ - NQ);
                 }
 #pragma unroll
                 for (int s = 0; s < 4 * FI; ++s) {
-                    if (s < CS) c_step(cr[s % RC], s);
+                    if (s < csteps) c_step(cr[s % RC], s);
                     if (s + RC < 4 * FI) load_c(cr[s % RC], cb, s + RC);
                 }
                 qb = qn_;
@@ -228,9 +231,8 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
         }
     }
     // direct term: segment lsum + (s', j) contracts over i
-    const long long astride = (long long)NAO * ai;
-    const unsigned ao_ = (unsigned)(kq * astride) * TS, aol = (unsigned)(min(kq, (ni - 1) & 3) * astride) * TS;
-    const unsigned bo = kq * aj * TS + nul, bol = min(kq, (ni - 1) & 3) * aj * TS + nul;
+    const unsigned ao_ = kq * ai * TS, aol = min(kq, (ni - 1) & 3) * ai * TS;
+    const unsigned bo = kq * qn * aj * TS + nul, bol = min(kq, (ni - 1) & 3) * qn * aj * TS + nul;
     const int xa0 = max(ta, O.lsum) - O.lsum, nic = (ni + 4 * RC - 1) / (4 * RC), nu = active ? max(0, (tb - O.lsum - xa0) * nic) : 0;
     if (nu > 0) {
         V ar[RC][G], br[RC];
@@ -240,8 +242,8 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
             const int sp = x >= O.nj ? 1 : 0, j = x - sp * O.nj;
             const int is = min(i0 + 4 * s, (ni - 1) & ~3);
             const bool last = is + 4 >= ni;
-            const T *ab = W + O.xa + ((long long)((1 - sp) * ni + is) * NAO + j) * ai;
-            const T *bb = W + O.xb + ((long long)(sp * O.nj + j) * NAO + is) * aj;
+            const T *ab = W + O.xa + ((long long)j * 2 * ni + (1 - sp) * ni + is) * ai;
+            const T *bb = W + O.xb + ((long long)is * qn + sp * O.nj + j) * aj;
 #pragma unroll
             for (int g = 0; g < G; ++g) ar[s][g] = at(ab, (last ? aol : ao_) + mul[g]);
             br[s] = at(bb, last ? bol : bo);

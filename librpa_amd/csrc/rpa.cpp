@@ -7,7 +7,7 @@
 //      (build_gf_Rt_libri_serial, chi0.cpp:303-426).  G(+tau) and G(-tau) are
 //      stored side by side per atom column block: Gpm[R][row][2*ao(J) + s*nb(J) + j].
 //   2. W(K, J, S)[k, (j, nu)] = sum_{(L,R2) in N(J)} G(S+R2)_KL C^J(L,R2): one GEMM
-//      per (J, S, sign) on a gathered G panel, written as W[(s, j)][(K, k)][nu].
+//      per (J, S, sign) on a gathered G panel, written as W[(K, k)][(s, j)][nu].
 //   3. chi0s(I,J,R) = sum_(K,R1,k) C^I [G_IJ W(K,J,R-R1)] + W(I,-R)^T W(J,R), one launch per tile
 //      class (chi0.hip): the bracket is formed in registers and never stored.
 // The four terms of LibRI's labels a1b1_a2b2 and a1b2_a2b1 called with
@@ -173,7 +173,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
         flops_chi0_alg = f * ntau;
     }
 
-    // ---- W(K, J, S) of every J stays resident: [(s', j)][(K, k)][nu] per (J, S) ----
+    // ---- W(K, J, S) of every J stays resident: [(K, k)][(s', j)][nu] per (J, S) ----
     w_off.assign((size_t)natom * nR + 1, 0);
     for (int J = 0; J < natom; ++J)
         for (int S = 0; S < nR; ++S)
@@ -251,16 +251,14 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
                     c.max_gcol = std::max(c.max_gcol, gj.ncol);
                     c.jobs.push_back(gj);
                 }
-        // W build: W[(s', j)][(K,k)][nu], s' = 1 holds W+ (from G+), s' = 0 holds W- (from G-)
+        // W build: W[(K,k)][(s', j)][nu], s' = 1 holds W+ (from G+), s' = 0 holds W- (from G-)
         for (int J = c.j_begin; J < c.j_end; ++J)
             for (int S = 0; S < nR; ++S)
                 for (int sg = 0; sg < 2; ++sg) {
                     const int sp = (sg == 0) ? 1 : 0;
                     GemmProb pr = make_prob(NAO, nb[J] * na[J], (int)lsum[J], ghat_at(J, S, sg), (int)lsum[J],
                                             cwb_off[J], nb[J] * na[J],
-                                            w_at(J, S) + (long long)sp * nb[J] * NAO * na[J], na[J]);
-                    pr.ncb = na[J];
-                    pr.cbs = (long long)NAO * na[J];
+                                            w_at(J, S) + (long long)sp * nb[J] * na[J], 2 * nb[J] * na[J]);
                     c.wb.add(pr);  // K = 0 (an atom without Cs) writes zeros
                 }
         c.wb.finalize(big_tile(prec), stream);
@@ -298,8 +296,8 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
             c.cfin = cfin_off[O.I];
             c.gpm = O.r * gpm_r + ao[O.I] * 2LL * NAO + 2 * ao[O.J];
             c.wseg = w_off[(size_t)O.J * nR];
-            c.xa = w_off[(size_t)O.I * nR + mr] + ao[O.J] * na[O.I];
-            c.xb = w_off[(size_t)O.J * nR + O.r] + ao[O.I] * na[O.J];
+            c.xa = w_off[(size_t)O.I * nR + mr] + ao[O.J] * 2 * nb[O.I] * na[O.I];
+            c.xb = w_off[(size_t)O.J * nR + O.r] + ao[O.I] * 2 * nb[O.J] * na[O.J];
             c.eoff = O.eoff;
             c.I = O.I; c.J = O.J; c.r = O.r;
             c.ni = nb[O.I]; c.nj = nb[O.J]; c.ai = na[O.I]; c.aj = na[O.J];
