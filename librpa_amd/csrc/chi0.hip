@@ -41,13 +41,18 @@ template <> struct CT<float> { using V = f4u; using A = v4f; static constexpr in
 __device__ __forceinline__ v4d mfma(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ v4f mfma(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+// One wave a SIMD with long rings, or two with short ones: two hide the instructions between the MFMAs
+// (FP32, 120-row blocks of 27-row fragments: 18.7 -> 17.0 ms a 32-atom build) as long as the accumulators
+// leave registers for them; 128 + 32 FP64 ones do not (38 spilled: 205 -> 258 ms on 64 atoms).
+template <class T> constexpr bool one_wave(int fm, int fi) { return sizeof(T) == 8 && fm * fi >= 16; }
+
 constexpr int kQsMax = 64;  // G steps kept in LDS (n_b(J) <= 128); later ones are read from memory
 }  // namespace
 
 // NQ: steps of W held in registers (n_b(J) <= 2 NQ); NQ = 0 for larger n_b(J), whose steps are
 // read four at a time.
 template <class T, class TO, int FM, int FI, int NQ>
-__global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_contract_kernel(
+__global__ __launch_bounds__(256, one_wave<T>(FM, FI) ? 1 : 2) void chi0_contract_kernel(
     const Chi0Task *__restrict__ tasks, const Chi0Out *__restrict__ outs, int nout, const Chi0Seg *__restrict__ segs,
     const T *__restrict__ Gpm, long long zg, const T *__restrict__ W, long long zw, const T *__restrict__ Cfin,
     TO *__restrict__ chi, long long zc, int NAO, int qsl, int single, const unsigned char *__restrict__ skip) {
@@ -55,7 +60,8 @@ __global__ __launch_bounds__(256, FM * FI >= 12 || FM == 8 ? 1 : 2) void chi0_co
     using A = typename CT<T>::A;
     constexpr int VL = CT<T>::VL, FN = VL, G = FM / VL;
     constexpr unsigned TS = sizeof(T);
-    constexpr int RQ = NQ > 0 ? (FM * FI >= 12 || FM == 8 ? 8 : 4) : 1, RC = 4;
+    constexpr bool ONE = one_wave<T>(FM, FI);
+    constexpr int RQ = NQ > 0 ? (ONE ? 8 : 4) : 1, RC = !ONE && (FM * FI >= 12 || FM == 8) ? 2 : 4;
     static_assert(NQ % RQ == 0 && (4 * FI) % RC == 0, "rings");
     static_assert(G * VL == FM, "row fragments come in vectors");
     extern __shared__ __align__(16) char smem[];
