@@ -81,8 +81,10 @@ struct GemmBatch {
     int nz = 1;                        // copies of the batch in one launch
     long long za = 0, zb = 0, zc = 0;  // operand distances of a copy, in elements
     int total_tiles = 0;
+    std::vector<int> tile_prob;
+    int per_prob = 0;      // tiles of every problem where that is one number, else 0: d_tile_prob maps a tile
     double flops = 0;      // flops of one launch: 2 M N K summed, less the skipped triangular work
-    DevBuf d_probs, d_rowtab, d_coltab;
+    DevBuf d_probs, d_rowtab, d_coltab, d_tile_prob;
 
     bool tuned = false;
     float tuned_ms = 0;    // time of the chosen tile shape in the tuning run

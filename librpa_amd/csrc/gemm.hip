@@ -1,7 +1,8 @@
 // Grouped MFMA GEMM kernels for gfx950.
 //
-// One workgroup (4 or 8 waves) computes a BM x BN tile of one problem.  Tiles of all problems of a batch form one flat grid; a binary
-// search over the per-problem tile prefix finds the problem.  The flat tile
+// One workgroup (4 or 8 waves) computes a BM x BN tile of one problem.  Tiles of all problems of a batch form one flat grid; the problem of
+// a tile is a division where all have the same number of tiles, else one entry of a table (a binary search over
+// the problems is a chain of up to ten loads, 2 to 5 us of launches that take 13).  The flat tile
 // index is remapped so that each XCD (8 per MI355X, workgroups dispatched
 // round-robin) receives a contiguous range of tiles, which keeps tiles that
 // share A or B panels in the same L2.
@@ -47,15 +48,6 @@ __device__ __forceinline__ unsigned short f2bf_rne(float x) {
 }
 __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(static_cast<unsigned int>(h) << 16); }
 
-__device__ __forceinline__ int find_prob(const GemmProb *__restrict__ probs, int nprob, int t) {
-    int lo = 0, hi = nprob - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (probs[mid].tile0 <= t) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 // XCD-aware remap of the dispatch index: XCD x (= bid % 8) gets a contiguous
 // chunk of logical tiles.
 __device__ __forceinline__ int xcd_remap(int bid, int G) {
@@ -67,7 +59,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int G) {
 // VAR selects the extras compiled in: 0 plain, 1 second segment, 2 column table and atomic epilogue
 // (kept out of the plain kernels, where they cost registers and 5% of the time).  blockIdx.y is the copy of the batch.
 template <int MODE, int BM, int BN, int WM, int WN, bool TA, bool TB, int VAR>
-__global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__restrict__ probs, int nprob, int total,
+__global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__restrict__ probs, const int *__restrict__ tile_prob,
+                                                    int per_prob, int total,
                                                     const typename ModeTraits<MODE>::T *__restrict__ A,
                                                     const typename ModeTraits<MODE>::T *__restrict__ B,
                                                     typename ModeTraits<MODE>::T *__restrict__ C,
@@ -98,7 +91,7 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
 
     const int tile = xcd_remap(blockIdx.x, gridDim.x);
     if (tile >= total) return;
-    const int pi = find_prob(probs, nprob, tile);
+    const int pi = per_prob > 0 ? tile / per_prob : tile_prob[tile];
     const GemmProb P = probs[pi];
     A += blockIdx.y * za;
     B += blockIdx.y * zb;
@@ -369,6 +362,18 @@ void GemmBatch::finalize(int cfg_, hipStream_t s) {
         }
     }
     total_tiles = t0;
+    tile_prob.clear();
+    per_prob = probs.empty() ? 0 : t0 / (int)probs.size();
+    if (per_prob * (int)probs.size() != t0) per_prob = 0;
+    for (size_t i = 0; i < probs.size(); ++i)
+        if (probs[i].tile0 != (int)i * per_prob) { per_prob = 0; break; }
+    if (per_prob == 0) {
+        tile_prob.resize(t0);
+        for (size_t i = 0; i < probs.size(); ++i)
+            std::fill(tile_prob.begin() + probs[i].tile0,
+                      i + 1 < probs.size() ? tile_prob.begin() + probs[i + 1].tile0 : tile_prob.end(), (int)i);
+    }
+    d_tile_prob = upload(tile_prob, s);
     d_probs = upload(probs, s);
     // the tables do not depend on the tile shape: upload once
     if (!rowtab.empty() && d_rowtab.bytes() != rowtab.size() * sizeof(long long)) d_rowtab = upload(rowtab, s);
@@ -388,7 +393,7 @@ static void launch_one(const GemmBatch &b, const void *A, const void *B, void *C
     constexpr int WN = (CFG == 7) ? 4 : (CFG == 8) ? 2 : 4 / WM;
     hipLaunchKernelGGL((ggemm_kernel<MODE, BM, BN, WM, WN, TA, TB, VAR>), dim3(b.total_tiles, b.nz),
                        dim3(WM * WN * 64), 0, s,
-                       b.d_probs.as<GemmProb>(), (int)b.probs.size(), b.total_tiles, static_cast<const T *>(A),
+                       b.d_probs.as<GemmProb>(), b.d_tile_prob.as<int>(), b.per_prob, b.total_tiles, static_cast<const T *>(A),
                        static_cast<const T *>(B), static_cast<T *>(C), b.d_rowtab.as<long long>(),
                        b.d_coltab.as<long long>(), (T)alpha, (T)beta, (int)b.lower_only, (int)b.atomic, b.za, b.zb,
                        b.zc);

@@ -214,18 +214,20 @@ template void launch_chi0_assemble<double, float>(const double *, long long, int
                                                   int, DenseLayout, hipStream_t);
 
 // chiw[w][i] = sum_t coef[w][t] chi0s[t][i] for every element i of the chi0(R, tau) store: the
-// cosine tau -> omega transform, done once for all q.  Coefficients in LDS; each thread owns one
-// element and re-reads its ntau values once per group of 8 frequencies.
+// cosine tau -> omega transform, done once for all q.  Coefficients in LDS; a thread owns one element
+// and re-reads its ntau values once per group of 8 frequencies.  Where the elements alone are under 1024
+// workgroups the groups go over the grid (a molecule: 17 us of load latency in one thread's two groups).
 template <class TS>
 __global__ __launch_bounds__(256) void tau_to_omega_kernel(const TS *__restrict__ chi0s, long long E_tot, int ntau,
-                                                           const double *__restrict__ coef, int nw,
+                                                           const double *__restrict__ coef, int nw, int wper,
                                                            double *__restrict__ chiw) {
     __shared__ double c[kTauOmegaMax * kTauOmegaMax];
-    for (int k = threadIdx.x; k < nw * ntau; k += blockDim.x) c[k] = coef[k];
+    const int wb = blockIdx.y * wper, we = min(nw, wb + wper);
+    for (int k = wb * ntau + threadIdx.x; k < we * ntau; k += blockDim.x) c[k] = coef[k];
     __syncthreads();
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < E_tot;
          i += (long long)gridDim.x * blockDim.x) {
-        for (int w0 = 0; w0 < nw; w0 += 8) {
+        for (int w0 = wb; w0 < we; w0 += 8) {
             double acc[8];
 #pragma unroll
             for (int w = 0; w < 8; ++w) acc[w] = 0.0;
@@ -233,11 +235,11 @@ __global__ __launch_bounds__(256) void tau_to_omega_kernel(const TS *__restrict_
                 const double v = static_cast<double>(chi0s[(long long)t * E_tot + i]);
 #pragma unroll
                 for (int w = 0; w < 8; ++w)
-                    if (w0 + w < nw) acc[w] += c[(w0 + w) * ntau + t] * v;
+                    if (w0 + w < we) acc[w] += c[(w0 + w) * ntau + t] * v;
             }
 #pragma unroll
             for (int w = 0; w < 8; ++w)
-                if (w0 + w < nw) chiw[(long long)(w0 + w) * E_tot + i] = acc[w];
+                if (w0 + w < we) chiw[(long long)(w0 + w) * E_tot + i] = acc[w];
         }
     }
 }
@@ -246,14 +248,18 @@ void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const d
                          hipStream_t s) {
     if (ntau > kTauOmegaMax || nw > kTauOmegaMax) LRA_THROW("tau -> omega: grid too large");
     const int bx = (int)std::min<long long>(ceil_div(E_tot, 256), 8192);
-    hipLaunchKernelGGL(tau_to_omega_kernel<double>, dim3(bx), dim3(256), 0, s, chi0s, E_tot, ntau, coef, nw, chiw);
+    const int wper = bx >= 1024 ? nw : 8;
+    hipLaunchKernelGGL(tau_to_omega_kernel<double>, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s, E_tot, ntau, coef,
+                       nw, wper, chiw);
     HIP_CHECK(hipGetLastError());
 }
 void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
                          hipStream_t s) {
     if (ntau > kTauOmegaMax || nw > kTauOmegaMax) LRA_THROW("tau -> omega: grid too large");
     const int bx = (int)std::min<long long>(ceil_div(E_tot, 256), 8192);
-    hipLaunchKernelGGL(tau_to_omega_kernel<float>, dim3(bx), dim3(256), 0, s, chi0s, E_tot, ntau, coef, nw, chiw);
+    const int wper = bx >= 1024 ? nw : 8;
+    hipLaunchKernelGGL(tau_to_omega_kernel<float>, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s, E_tot, ntau, coef,
+                       nw, wper, chiw);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -510,7 +516,7 @@ __global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long 
     constexpr int NB = chol_nb(CPLX), PL = CPLX ? 2 : 1, PN = NB / 16, NX = PN * (PN + 1) / 2;
     __shared__ double L[PL][NB][NB + 1];
     __shared__ double X[PL][NX][16][17];
-    __shared__ double sg[NB];
+    __shared__ double sg[NB], dinv[NB];  // pivot signs, 1 / L_jj
     double *A = A0 + strideA * blockIdx.x;
     double *Linv = work + chol_work(CPLX) * blockIdx.x, *SLinv = Linv + (long long)PL * NB * NB;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, kq = lane >> 4;
@@ -524,7 +530,7 @@ __global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long 
     bool bad = false;
     for (int p = 0; p < PN; ++p) {
         if (wave == 0) {
-            double a[16];
+            double a[16], own = 1.0;
 #pragma unroll
             for (int k = 0; k < 16; ++k) a[k] = L[half][t][16 * p + k];
 #pragma unroll
@@ -532,10 +538,16 @@ __global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long 
                 const int jj = 16 * p + j;
                 double d = readlane_f64(a[j], jj);
                 if (!(fabs(d) > 0.0)) { bad = true; d = 1.0; }
-                const double s = d > 0 ? 1.0 : -1.0, r = sqrt(fabs(d));
+                const double s = d > 0 ? 1.0 : -1.0, q = fabs(d);
+                // 1 / sqrt(q) from the hardware's approximation by one step of third order: short, where
+                // sqrt and a division are a chain of 300 cycles in each of the columns.  sqrt(q) itself is only
+                // written, once per panel
+                double y = __builtin_amdgcn_rsq(q);
+                const double e = fma(-(q * y), y, 1.0);
+                y = q < INFINITY ? fma(y * e, fma(0.375, e, 0.5), y) : 0.0;
                 // L_tj = a_tj / (s r), so that A = L S L^H also for a negative pivot
-                const double l = t > jj ? a[j] * (s / r) : 0.0;
-                if (t == jj) { a[j] = half ? 0.0 : r; if (!half) { my_r = r; sg[t] = s; } }
+                const double l = t > jj ? a[j] * (s * y) : 0.0;
+                if (t == jj) { own = q; if (!half) { sg[t] = s; dinv[t] = y; } }
                 if (t > jj) a[j] = l;
                 const double f1 = s * l;
                 if constexpr (CPLX) {
@@ -549,9 +561,13 @@ __global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long 
                     for (int k = j + 1; k < 16; ++k) a[k] -= f1 * readlane_f64(a[j], 16 * p + k);
                 }
             }
-            if (t >= 16 * p)
+            const double r = sqrt(own);
+            if (t >= 16 * p) {
+                const int dk = t - 16 * p;
+                if (half == 0 && dk < 16) my_r = r;
 #pragma unroll
-                for (int k = 0; k < 16; ++k) L[half][t][16 * p + k] = a[k];
+                for (int k = 0; k < 16; ++k) L[half][t][16 * p + k] = k == dk ? (half ? 0.0 : r) : a[k];
+            }
         }
         __syncthreads();
         // tiles right of the panel: L_ij -= L_ip S L_jp^H
@@ -592,7 +608,7 @@ __global__ __launch_bounds__(256) void potrf_block_kernel(double *A0, long long 
         for (int r = 0; r < 16; ++r) x[r] = (r == c && hx == 0) ? 1.0 : 0.0;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            x[r] *= 1.0 / L[0][b + r][b + r];
+            x[r] *= dinv[b + r];
             double xp = 0;
             if constexpr (CPLX) {
                 xp = __shfl_xor(x[r], 16, 64);
