@@ -1,6 +1,8 @@
 // Host wrappers of the streaming / small kernels of the chi0 -> Ec path.
 #pragma once
 
+#include <vector>
+
 #include "common.h"
 
 namespace lra {
@@ -56,10 +58,15 @@ void launch_chi0_assemble(const TS *chi0s, long long E_tot, int ntau, const Pair
 // chi0s[t][i] once for all q (coef = (2 / nspin) gamma_c, nw x ntau, row-major), then per q and
 // frequency chunk the R -> q phase sum ph[r] = (cos, sin)(2 pi q.R_r) into dense matrices.
 constexpr int kTauOmegaMax = kTauMax;
-void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
-                         hipStream_t s);
-void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
-                         hipStream_t s);
+// A small host table of a launch: up to kArgTable doubles go with the kernel's arguments, larger ones are
+// uploaded to a buffer of the caller's (which must outlive the launch, as must the table then).  An upload of its
+// own cost each of these launches an allocation, a copy, a wait and a free: 40 to 60 us.
+constexpr int kArgTable = 448;
+struct ArgTable { double v[kArgTable]; };
+void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const std::vector<double> &coef, DevBuf &buf, int nw,
+                         double *chiw, hipStream_t s);
+void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const std::vector<double> &coef, DevBuf &buf, int nw,
+                         double *chiw, hipStream_t s);
 // chiw[w][i] = sum_{t' <= t} coef[w][t'] slice_t'[i], one slice per call (t = 0 overwrites)
 template <class TS>
 void launch_tau_accumulate(const TS *slice, long long E_tot, int t, int ntau, const double *coef, int nw, double *chiw,
@@ -69,8 +76,8 @@ void launch_tau_accumulate(const TS *slice, long long E_tot, int t, int ntau, co
 constexpr int kChi0RqMaxQ = 8;
 template <class TD>
 void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs,
-                          long long n_pair_elems, const long long *eoff, int nR, const double *ph, int nq, int nw,
-                          TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s);
+                          long long n_pair_elems, const long long *eoff, int nR, const std::vector<double> &ph,
+                          DevBuf &buf, int nq, int nw, TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s);
 
 // Dense helpers --------------------------------------------------------------------
 // planes Re, Im (n x n each) of a complex matrix <-> its real embedding [[Re, -Im], [Im, Re]] (2n x 2n)

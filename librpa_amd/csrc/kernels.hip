@@ -1,6 +1,7 @@
 // Streaming and small kernels of the chi0 -> Ec path (gfx950).
 #include "kernels.h"
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <tuple>
@@ -217,13 +218,30 @@ template void launch_chi0_assemble<double, float>(const double *, long long, int
 // cosine tau -> omega transform, done once for all q.  Coefficients in LDS; a thread owns one element
 // and re-reads its ntau values once per group of 8 frequencies.  Where the elements alone are under 1024
 // workgroups the groups go over the grid (a molecule: 17 us of load latency in one thread's two groups).
-template <class TS>
+// TAB: an ArgTable, or a pointer
+__device__ __forceinline__ double table_at(const ArgTable &t, int i) { return t.v[i]; }
+__device__ __forceinline__ double table_at(const double *t, int i) { return t[i]; }
+// the table of a launch to the launch itself
+template <class F> void with_table(const std::vector<double> &v, DevBuf &buf, hipStream_t s, F f) {
+    if (v.size() <= (size_t)kArgTable) {
+        ArgTable t;
+        std::copy(v.begin(), v.end(), t.v);
+        f(t);
+        return;
+    }
+    buf.reserve(v.size() * sizeof(double));
+    HIP_CHECK(hipMemcpyAsync(buf.get(), v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, s));
+    f(static_cast<const double *>(buf.as<double>()));
+    HIP_CHECK(hipStreamSynchronize(s));  // the next table may go to the same buffer
+}
+
+template <class TS, class TAB>
 __global__ __launch_bounds__(256) void tau_to_omega_kernel(const TS *__restrict__ chi0s, long long E_tot, int ntau,
-                                                           const double *__restrict__ coef, int nw, int wper,
+                                                           const TAB coef, int nw, int wper,
                                                            double *__restrict__ chiw) {
     __shared__ double c[kTauOmegaMax * kTauOmegaMax];
     const int wb = blockIdx.y * wper, we = min(nw, wb + wper);
-    for (int k = wb * ntau + threadIdx.x; k < we * ntau; k += blockDim.x) c[k] = coef[k];
+    for (int k = wb * ntau + threadIdx.x; k < we * ntau; k += blockDim.x) c[k] = table_at(coef, k);
     __syncthreads();
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < E_tot;
          i += (long long)gridDim.x * blockDim.x) {
@@ -244,23 +262,25 @@ __global__ __launch_bounds__(256) void tau_to_omega_kernel(const TS *__restrict_
     }
 }
 
-void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
-                         hipStream_t s) {
+template <class TS>
+static void tau_to_omega(const TS *chi0s, long long E_tot, int ntau, const std::vector<double> &coef, DevBuf &buf, int nw,
+                         double *chiw, hipStream_t s) {
     if (ntau > kTauOmegaMax || nw > kTauOmegaMax) LRA_THROW("tau -> omega: grid too large");
     const int bx = (int)std::min<long long>(ceil_div(E_tot, 256), 8192);
     const int wper = bx >= 1024 ? nw : 8;
-    hipLaunchKernelGGL(tau_to_omega_kernel<double>, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s, E_tot, ntau, coef,
-                       nw, wper, chiw);
-    HIP_CHECK(hipGetLastError());
+    with_table(coef, buf, s, [&](auto table) {
+        hipLaunchKernelGGL((tau_to_omega_kernel<TS, decltype(table)>), dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s,
+                           E_tot, ntau, table, nw, wper, chiw);
+        HIP_CHECK(hipGetLastError());
+    });
 }
-void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const double *coef, int nw, double *chiw,
-                         hipStream_t s) {
-    if (ntau > kTauOmegaMax || nw > kTauOmegaMax) LRA_THROW("tau -> omega: grid too large");
-    const int bx = (int)std::min<long long>(ceil_div(E_tot, 256), 8192);
-    const int wper = bx >= 1024 ? nw : 8;
-    hipLaunchKernelGGL(tau_to_omega_kernel<float>, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s, E_tot, ntau, coef,
-                       nw, wper, chiw);
-    HIP_CHECK(hipGetLastError());
+void launch_tau_to_omega(const double *chi0s, long long E_tot, int ntau, const std::vector<double> &coef, DevBuf &buf, int nw,
+                         double *chiw, hipStream_t s) {
+    tau_to_omega(chi0s, E_tot, ntau, coef, buf, nw, chiw, s);
+}
+void launch_tau_to_omega(const float *chi0s, long long E_tot, int ntau, const std::vector<double> &coef, DevBuf &buf, int nw,
+                         double *chiw, hipStream_t s) {
+    tau_to_omega(chi0s, E_tot, ntau, coef, buf, nw, chiw, s);
 }
 
 // chiw[w][i] (+)= coef[w][t] slice[i] for one tau slice t (the first slice overwrites): the same
@@ -298,11 +318,11 @@ template void launch_tau_accumulate<float>(const float *, long long, int, int, c
 // alone are under 1024 workgroups: with all 16 in the loop the 2-atom cell (120 functions, 43
 // workgroups) took 168 us where its bytes take 15; with one each the 64-atom cell takes 6.2 ms, not 4.7.
 // q point qi writes its nw matrices at dense + qi * qstride.
-template <class TD, int NQ>
+template <class TD, int NQ, class TAB>
 __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__ chiw, long long E_tot,
                                                       const PairDesc *__restrict__ pairs, int npairs, long long nelem,
                                                       const long long *__restrict__ eoff, int nR,
-                                                      const double *__restrict__ ph, int nq, int nw, int wper,
+                                                      const TAB ph, int nq, int nw, int wper,
                                                       TD *__restrict__ dense, long long dstride, long long qstride,
                                                       int n, int lay) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -327,8 +347,8 @@ __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 if (q < nq) {
-                    re[q] += ph[2 * ((long long)q * nR + r)] * v;
-                    im[q] += ph[2 * ((long long)q * nR + r) + 1] * v;
+                    re[q] += table_at(ph, 2 * (q * nR + r)) * v;
+                    im[q] += table_at(ph, 2 * (q * nR + r) + 1) * v;
                 }
             }
         }
@@ -342,24 +362,28 @@ __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__
 
 template <class TD>
 void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *pairs, int npairs,
-                          long long n_pair_elems, const long long *eoff, int nR, const double *ph, int nq, int nw,
-                          TD *dense, long long dense_stride, long long q_stride, int n, DenseLayout lay, hipStream_t s) {
+                          long long n_pair_elems, const long long *eoff, int nR, const std::vector<double> &ph,
+                          DevBuf &buf, int nq, int nw, TD *dense, long long dense_stride, long long q_stride, int n,
+                          DenseLayout lay, hipStream_t s) {
     if (nq < 1 || nq > kChi0RqMaxQ) LRA_THROW("chi0_rq_multi: 1 to kChi0RqMaxQ q points per launch");
     const int bx = ceil_div(n_pair_elems, 256), wper = bx >= 1024 ? nw : 1;
-    const auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chiw, E_tot, pairs, npairs,
-                           n_pair_elems, eoff, nR, ph, nq, nw, wper, dense, dense_stride, q_stride, n, (int)lay);
-    };
-    if (nq == 1) go(chi0_rq_kernel<TD, 1>);
-    else go(chi0_rq_kernel<TD, kChi0RqMaxQ>);
-    HIP_CHECK(hipGetLastError());
+    with_table(ph, buf, s, [&](auto table) {
+        using TAB = decltype(table);
+        const auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chiw, E_tot, pairs, npairs,
+                               n_pair_elems, eoff, nR, table, nq, nw, wper, dense, dense_stride, q_stride, n, (int)lay);
+        };
+        if (nq == 1) go(chi0_rq_kernel<TD, 1, TAB>);
+        else go(chi0_rq_kernel<TD, kChi0RqMaxQ, TAB>);
+        HIP_CHECK(hipGetLastError());
+    });
 }
 template void launch_chi0_rq_multi<double>(const double *, long long, const PairDesc *, int, long long,
-                                           const long long *, int, const double *, int, int, double *, long long,
-                                           long long, int, DenseLayout, hipStream_t);
+                                           const long long *, int, const std::vector<double> &, DevBuf &, int, int,
+                                           double *, long long, long long, int, DenseLayout, hipStream_t);
 template void launch_chi0_rq_multi<float>(const double *, long long, const PairDesc *, int, long long,
-                                          const long long *, int, const double *, int, int, float *, long long,
-                                          long long, int, DenseLayout, hipStream_t);
+                                           const long long *, int, const std::vector<double> &, DevBuf &, int, int,
+                                           float *, long long, long long, int, DenseLayout, hipStream_t);
 
 // ------------------------------------------------------------------------------------
 // dense helpers

@@ -418,6 +418,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
 
 void RpaEngine::prepare_gf(const MeanField &mf, int nbands_g) {
     // band ranges with non-zero weight for each sign
+    bool same = !gb.empty();
     for (int sg = 0; sg < 2; ++sg) {
         int lo = nbands, hi = 0;
         for (int s = 0; s < nspin; ++s)
@@ -430,9 +431,12 @@ void RpaEngine::prepare_gf(const MeanField &mf, int nbands_g) {
                     if (w > 0) { lo = std::min(lo, b); hi = std::max(hi, b + 1); }
                 }
         if (hi <= lo) { lo = 0; hi = 0; }
+        same = same && band_lo[sg] == lo && band_hi[sg] == hi;
         band_lo[sg] = lo;
         band_hi[sg] = hi;
     }
+    gf_nbands = nbands_g;
+    if (same) return;
     // both signs in one batch; a sign without bands has K = 0 and gets zeros
     gb = GemmBatch();
     gb.trans_a = true;
@@ -445,7 +449,6 @@ void RpaEngine::prepare_gf(const MeanField &mf, int nbands_g) {
     gb.zb = 2 * nk * zs_k;
     gb.zc = 2 * nk * mst_k;
     gb.finalize(T64x64, stream);
-    gf_nbands = nbands_g;
 }
 
 void RpaEngine::build_gf(const MeanField &mf, const double *taus, int nz, int s) {
@@ -832,8 +835,8 @@ bool RpaEngine::form_chiw(const TFGrid &g, double max_bytes, hipStream_t s) {
     std::vector<double> coef((size_t)g.n * g.n);
     for (int w = 0; w < g.n; ++w)
         for (int t = 0; t < g.n; ++t) coef[(size_t)w * g.n + t] = g.cos_t2f[(size_t)w * g.n + t] * 2.0 / nspin;
-    DevBuf dc = upload(coef, s);
     if (host_staged) {
+        DevBuf dc = upload(coef, s);
         // slices back through the one-slice device buffer, accumulated tau by tau
         for (int t = 0; t < ntau_done; ++t) {
             HIP_CHECK(hipMemcpyAsync(d_chi0s.get(), h_chi0s[t].data(), ts * (size_t)E_tot, hipMemcpyHostToDevice, s));
@@ -849,10 +852,9 @@ bool RpaEngine::form_chiw(const TFGrid &g, double max_bytes, hipStream_t s) {
         return true;
     }
     if (prec == Prec::F64)
-        launch_tau_to_omega(d_chi0s.as<double>(), E_tot, ntau_done, dc.as<double>(), g.n, d_chiw.as<double>(), s);
+        launch_tau_to_omega(d_chi0s.as<double>(), E_tot, ntau_done, coef, d_table, g.n, d_chiw.as<double>(), s);
     else
-        launch_tau_to_omega(d_chi0s.as<float>(), E_tot, ntau_done, dc.as<double>(), g.n, d_chiw.as<double>(), s);
-    HIP_CHECK(hipStreamSynchronize(s));  // dc is freed on return
+        launch_tau_to_omega(d_chi0s.as<float>(), E_tot, ntau_done, coef, d_table, g.n, d_chiw.as<double>(), s);
     chiw_ok = true;
     return true;
 }
@@ -877,18 +879,16 @@ void RpaEngine::assemble_dense_q(const TFGrid &g, const std::vector<const double
                 ph[((size_t)qi * nR + r) * 2 + 1] = std::sin(ang);
             }
         }
-        DevBuf dph = upload(ph, s);
         const double *cw = d_chiw.as<double>() + (size_t)w0 * E_tot;
         char *Dd = static_cast<char *>(dense) + q0 * cnt * nn * es;
         if (f64)
             launch_chi0_rq_multi<double>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
-                                         d_pair_eoff.as<long long>(), nR, dph.as<double>(), nq, cnt, (double *)Dd, nn,
+                                         d_pair_eoff.as<long long>(), nR, ph, d_table, nq, cnt, (double *)Dd, nn,
                                          (long long)cnt * nn, n, lay, s);
         else
             launch_chi0_rq_multi<float>(cw, E_tot, d_pairs.as<PairDesc>(), (int)pairs.size(), n_pair_elems,
-                                        d_pair_eoff.as<long long>(), nR, dph.as<double>(), nq, cnt, (float *)Dd, nn,
+                                        d_pair_eoff.as<long long>(), nR, ph, d_table, nq, cnt, (float *)Dd, nn,
                                         (long long)cnt * nn, n, lay, s);
-        HIP_CHECK(hipStreamSynchronize(s));  // dph is freed on return
     }
 }
 

@@ -55,6 +55,7 @@ struct RpaEngine {
     Chi0Tasks ctasks[2];
     int nbatch = 1;  // tau points per pass: G, gathered G and W are held for that many
     DevBuf d_couts, d_segs, d_skip;
+    DevBuf d_table;  // tables of launches past kArgTable entries
     std::vector<double> out_flops;  // per output and tau point
     double contract_flops = 0, contract_bytes = 0;
 
