@@ -726,14 +726,16 @@ static std::map<std::tuple<int, int, int, long long, hipStream_t, int, long long
     return p;
 }
 
-// Right-looking blocked L S L^H factorisation in three levels.  Steps of one diagonal block (64 real
-// or 32 complex columns, by potrf_block_kernel; Q = A21 L11^-H and Q S by one GEMM launch) update only
-// the rest of their middle panel (512 real or 256 complex columns); after each middle panel one GEMM
-// updates the remaining columns of its outer panel; after each outer panel one lower-triangular GEMM
-// updates the trailing matrix (2048 real or 1024 complex columns for n >= 4096 / 2048, else the middle
-// level is the outer one).  Few, deep trailing updates read and write the trailing matrix four times
-// less often.  Q and Q S of the outer panel's columns are kept in wide buffers per matrix (pitch =
-// outer panel width, indexed by global row).
+// Right-looking blocked L S L^H factorisation in three levels.  Steps of one diagonal block (64 real or 32
+// complex columns, by potrf_block_kernel; Q = A21 L11^-H and Q S by one GEMM launch) update only the rest
+// of their middle panel (512 real or 256 complex columns); after each middle panel one GEMM updates the
+// remaining columns of its outer panel; after each outer panel one lower-triangular GEMM updates the
+// trailing matrix (2048 real or 1024 complex columns for n >= 4096 / 2048, else the middle level is the
+// outer one).  Few, deep trailing updates read and write the trailing matrix four times less often.  All of
+// them on 64x64 tiles: 128x128 ones waste half of every diagonal tile and run FP64 at 42 TF/s, not 50 (16
+// atoms and 8 k, n = 960: 7.5 -> 4.2 ms of trailing updates; n = 5760: 24.8 -> 21.0).  Q and Q S of the
+// outer panel's columns are kept in wide buffers per matrix (pitch = outer panel width, indexed by global
+// row).
 //
 // A Hermitian matrix is factored as such, from its two planes, each product as two real segments:
 // 4/3 n^3 real multiply-adds, where the real embedding [[Re, -Im], [Im, Re]] (2n x 2n) needs 8/3 n^3.
@@ -803,7 +805,7 @@ void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, in
                             add(md, n - pend, oend - pend, pend - p0, wq + qs_off, qplane, PO, wq, qplane, PO,
                                 strideA * b + (long long)pend * lda + pend, im, lda);
                         }
-                        md.finalize(T128x128w8, s);
+                        md.finalize(T64x64, s);
                     }
                     const int mt = n - oend;
                     if (j0 + nb == oend && mt > 0) {
@@ -815,7 +817,7 @@ void cholesky_logdet_batched(double *A, long long strideA, int nbatch, int n, in
                             add(tl, mt, mt, oend - o0, wq + qs_off, qplane, PO, wq, qplane, PO,
                                 strideA * b + (long long)oend * lda + oend, im, lda);
                         }
-                        tl.finalize(T128x128w8, s);
+                        tl.finalize(T64x64, s);
                     }
                     cp.trsm.push_back(std::move(tr));
                     cp.inpanel.push_back(std::move(ip));
