@@ -512,7 +512,8 @@ template void launch_sigma_freq<float>(const float *, long long, const double *,
 
 constexpr int kStMax = 16;
 
-// one workgroup per (row a, omega); threads stride over the columns b
+// one workgroup per (row a, omega); threads stride over the columns b.  Under 256 columns the threads left over
+// share the cells of a column (26 functions on 8 k kept 26 threads waiting for 8 cells in turn).
 __global__ __launch_bounds__(256) void sigma_ks_rows_kernel(const double *__restrict__ sre,
                                                             const double *__restrict__ sim, int nR, int n,
                                                             const int *__restrict__ atom_of, int natom,
@@ -526,11 +527,11 @@ __global__ __launch_bounds__(256) void sigma_ks_rows_kernel(const double *__rest
 #pragma unroll
     for (int st = 0; st < kStMax; ++st) { ar[st] = 0; ai[st] = 0; }
     const long long nn = (long long)n * n;
-    for (int b = t; b < n; b += blockDim.x) {
-        const int J = atom_of[b];
-        const double *p = ph + ((long long)I * natom + J) * nR * 2;
+    const int G = n >= 256 ? 1 : min(nR, 256 / n), g = G > 1 ? t / n : 0;
+    for (int b = G > 1 ? t % n : t; b < n && g < G; b += G > 1 ? n : 256) {
+        const double *p = ph + ((long long)I * natom + atom_of[b]) * nR * 2;
         double vr = 0, vi = 0;
-        for (int R = 0; R < nR; ++R) {
+        for (int R = g; R < nR; R += G) {
             const long long e = ((long long)w * nR + R) * nn + (long long)a * n + b;
             const double sr = sre[e], si = sim[e];
             const double cr = p[2 * R], ci = p[2 * R + 1];
