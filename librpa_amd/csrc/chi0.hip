@@ -18,7 +18,8 @@
 // arrive.  Measured against the two GEMMs with T between them (38 GB of it per tau point on a
 // 64-atom cell), X and T_A and contraction together: 526 -> 411 ms on 64 atoms at Gamma (46 TF/s of
 // the sums' own flops; 60- and 120-row blocks and 13- and 27-row T fragments pad the rest), 52 -> 32.7 ms
-// on 16 atoms and 8 k (47 TF/s).
+// on 16 atoms and 8 k (47 TF/s).  On 128 atoms (46 TF/s FP64, 121 ms a tau point) the operands come through
+// the L2 at 3.9 TB/s (FP64) and 5.0 TB/s (FP32, 61 ms): FP32 is bound by that, FP64 nearly.
 #include "chi0.h"
 
 #include <algorithm>
@@ -380,7 +381,8 @@ void Chi0Tasks::build(const std::vector<Chi0Out> &outs, bool f64, int nz, int sp
         }
     }
     // workgroups that run side by side: one J, the same share of the segments, different I and R.
-    // (Blocks of 4 to 16 I x 4 to 16 J of one R measured the same within 1%, 16 x 16 10% slower.)
+    // (Blocks of 4 to 16 I x 4 to 16 J of one R measured the same within 1%, 16 x 16 10% slower; one I and R
+    // with different J, which share Cs and walk in step, 4% slower.)
     for (auto &cl : classes) {
         std::stable_sort(cl.tasks.begin(), cl.tasks.end(), [&](const Chi0Task &a, const Chi0Task &b) {
             const auto key = [&](const Chi0Task &t) {
