@@ -18,12 +18,12 @@ void launch_scale_bands(const double *wre, const double *wim, const double *eps,
                         int nbands, int nbasis, const int b0[2], const int b1[2], const TauList &taus, double efermi,
                         int nspin, int nbands_g, hipStream_t s);
 
-// Gpm[z][R][row][gcol[sg][col]] = (sg ? -1 : 1) sum_k (cs[R][k] Mre_k[row][col] + sn[R][k] Mim_k[row][col]),
-// Mstack[z][sg][k] laid out [Re rows; Im rows] (2 nbasis x nbasis), for nz tau points and both
-// signs.  T = double or float.
+// Gpm[z][R][row][gcol[sg][col]] = (t < 0 ? -1 : 1) sum_k (cs[R][k] Mre_k[row][col] + sn[R][k] Mim_k[row][col]),
+// t = +-taus.t[z] by sg, Mstack[z][sg][k] laid out [Re rows; Im rows] (2 nbasis x nbasis), for the tau
+// points of taus and both signs.  T = double or float.
 template <class T>
 void launch_k2r(const double *Mstack, const double *cs, const double *sn, const int *gcol, T *Gpm, int nk, int nR,
-                int nbasis, int nz, hipStream_t s);
+                int nbasis, const TauList &taus, hipStream_t s);
 
 // Column gather: dst[job][row][c] = src[colsrc[job_cols + c] + row * src_ld] for row < nrows, for nz
 // sources zs and destinations zd elements apart.

@@ -63,11 +63,13 @@ constexpr int kK2rCells = 4;
 template <class T>
 __global__ __launch_bounds__(256) void k2r_kernel(const double *__restrict__ M, const double *__restrict__ cs,
                                                   const double *__restrict__ sn, const int *__restrict__ gcol,
-                                                  T *__restrict__ G, int nk, int nR, int nbasis) {
+                                                  T *__restrict__ G, int nk, int nR, int nbasis, TauList taus) {
     const long long nn = (long long)nbasis * nbasis;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nn) return;
     const int r0 = blockIdx.y * kK2rCells, z = blockIdx.z >> 1, sg = blockIdx.z & 1;
+    // by the time itself, not by sg: a grid may hold tau = 0, where neither G changes sign
+    const bool neg = sg ? taus.t[z] > 0 : taus.t[z] < 0;
     M += (long long)blockIdx.z * nk * 2 * nn;
     G += (long long)z * nR * 2 * nn;
     const int row = (int)(idx / nbasis), col = (int)(idx % nbasis);
@@ -85,21 +87,21 @@ __global__ __launch_bounds__(256) void k2r_kernel(const double *__restrict__ M, 
     }
 #pragma unroll
     for (int i = 0; i < kK2rCells; ++i)
-        if (r0 + i < nR) G[(long long)(r0 + i) * 2 * nn + dst] = static_cast<T>(sg ? -acc[i] : acc[i]);
+        if (r0 + i < nR) G[(long long)(r0 + i) * 2 * nn + dst] = static_cast<T>(neg ? -acc[i] : acc[i]);
 }
 
 template <class T>
 void launch_k2r(const double *Mstack, const double *cs, const double *sn, const int *gcol, T *Gpm, int nk, int nR,
-                int nbasis, int nz, hipStream_t s) {
+                int nbasis, const TauList &taus, hipStream_t s) {
     const long long nn = (long long)nbasis * nbasis;
-    hipLaunchKernelGGL((k2r_kernel<T>), dim3(ceil_div(nn, 256), ceil_div(nR, kK2rCells), 2 * nz), dim3(256), 0, s,
-                       Mstack, cs, sn, gcol, Gpm, nk, nR, nbasis);
+    hipLaunchKernelGGL((k2r_kernel<T>), dim3(ceil_div(nn, 256), ceil_div(nR, kK2rCells), 2 * taus.n), dim3(256), 0, s,
+                       Mstack, cs, sn, gcol, Gpm, nk, nR, nbasis, taus);
     HIP_CHECK(hipGetLastError());
 }
 template void launch_k2r<double>(const double *, const double *, const double *, const int *, double *, int, int,
-                                 int, int, hipStream_t);
+                                 int, const TauList &, hipStream_t);
 template void launch_k2r<float>(const double *, const double *, const double *, const int *, float *, int, int,
-                                int, int, hipStream_t);
+                                int, const TauList &, hipStream_t);
 
 template <class T>
 __global__ void gather_cols_kernel(const T *__restrict__ src, long long src_ld, T *__restrict__ dst,

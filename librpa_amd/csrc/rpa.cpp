@@ -469,10 +469,10 @@ void RpaEngine::build_gf(const MeanField &mf, const double *taus, int nz, int s)
     gemm_run(Prec::F64, gb, d_ZZ.as<double>() + zz_s, d_Zs.get(), d_Mst.get(), 1.0, 0.0, stream);
     if (cur == Prec::F64)
         launch_k2r<double>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(), d_gcol.as<int>(),
-                           d_Gpm.as<double>(), nk, nR, NAO, nz, stream);
+                           d_Gpm.as<double>(), nk, nR, NAO, tl, stream);
     else
         launch_k2r<float>(d_Mst.as<double>(), d_cs.as<double>(), d_sn.as<double>(), d_gcol.as<int>(), d_Gpm.as<float>(),
-                          nk, nR, NAO, nz, stream);
+                          nk, nR, NAO, tl, stream);
     prof.end("gf_build", stream, nz * gb.flops, (double)gpm_bytes);
 }
 
