@@ -12,7 +12,7 @@ namespace lra {
 // Zs[z][sg][k][(2b + c)][j] = s_b * (c == 0 ? Re U[b][j] : Im U[b][j]) for b in [b0[sg], b1[sg]),
 // s_b = exp(min(0, -t (eps_b - mu))) * w_b with the occupation weights of
 // build_gf_Rt_libri_serial (src/core/chi0.cpp:333-355).  U, eps, wg per k.
-constexpr int kTauMax = 34;  // the largest minimax grid
+constexpr int kTauMax = 34;  // tau points of a pass: the largest minimax grid (others may be longer)
 struct TauList { int n; double t[kTauMax]; };
 void launch_scale_bands(const double *wre, const double *wim, const double *eps, const double *wg, double *Zs, int nk,
                         int nbands, int nbasis, const int b0[2], const int b1[2], const TauList &taus, double efermi,

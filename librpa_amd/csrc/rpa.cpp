@@ -315,14 +315,15 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
         d_segs = upload(segs, stream);
         d_couts = upload(co, stream);
         // tau points per launch: one tau point of a small system leaves the device idle between its
-        // launches, so several run as copies of one batch, up to about 120 GFLOP (2 ms) and 8 GB
+        // launches, so several run as copies of one batch, up to about 120 GFLOP (2 ms), 8 GB and the
+        // kTauMax that a kernel's arguments hold (an evenly spaced grid may have more points)
         double wflops = 0;
         for (const auto &c : chunks) wflops += c.wb.flops;
         const double per_tau = 8.0 * (2.0 * nk * (2.0 * nbands * NAO + 2.0 * NAO * NAO)) +
                                ts * ((double)nR * 2 * NAO * NAO + ghat_max + (double)w_off.back());
         nbatch = 1;
         if (!host_staged && chunks.size() == 1)
-            nbatch = (int)std::max(1.0, std::min({(double)ntau, std::ceil(1.2e11 / std::max(1.0, contract_flops + wflops)),
+            nbatch = (int)std::max(1.0, std::min({(double)ntau, (double)kTauMax, std::ceil(1.2e11 / std::max(1.0, contract_flops + wflops)),
                                                   std::min(8e9, 0.1 * (double)free_b) / per_tau}));
         if (const char *e = std::getenv("LIBRPA_AMD_TAU_BATCH")) nbatch = std::max(1, std::min(nbatch, std::atoi(e)));
         nbatch = ceil_div(ntau, ceil_div(ntau, nbatch));
