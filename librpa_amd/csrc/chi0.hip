@@ -319,11 +319,14 @@ void Chi0Tasks::build(const std::vector<Chi0Out> &outs, bool f64, int nz, int sp
     const int VL = f64 ? 2 : 4, FN = VL;
     auto fm_of = [&](int ai, int &strips) {
         const int fr = ceil_div(ai, 16);
-        strips = ceil_div(fr, 8);
+        strips = std::max(1, ceil_div(fr, 8));
         return std::max(VL, ceil_div(ceil_div(fr, strips), VL) * VL);
     };
     // MFMAs of one wave over all segments of a strip
     auto cost = [&](const Chi0Out &o, int fm, double &main, double &direct) {
+        main = direct = 0;
+        // an atom without basis or auxiliary functions: no sum, and no rows for the kernel to clamp to
+        if (o.ni == 0 || o.nj == 0 || o.ai == 0 || o.aj == 0) return 0.0;
         const int qs = (2 * o.nj + 3) / 4;
         main = (double)ceil_div(o.ni, 16) * FN * qs + (double)fm * FN * ceil_div(o.ni, 4);
         direct = (double)fm * FN * ceil_div(o.ni, 4);

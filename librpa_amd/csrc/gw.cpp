@@ -247,7 +247,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
         const double nblk = (double)(c.x1 - c.x0) * natom * nR * nbatch;
         for (int I = c.x0; I < c.x1; ++I) {
             const int l = (int)R0.lsum[I];
-            if (l == 0) continue;
+            if (l * nb[I] == 0) continue;  // (as where the blocks that tasks count were made)
             // 2048 workgroups, each with at least 16 segments
             const int parts = std::max(1, std::min(ceil_div(l, 16), (int)std::ceil(2048.0 / nblk)));
             for (int rr = 0; rr < nR; ++rr)
@@ -276,7 +276,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
         for (int S = 0; S < nR; ++S)
             for (int L = 0; L < natom; ++L) {
                 for (int J = 0; J < natom; ++J)
-                    for (int rr = 0; rr < nR; ++rr) {
+                    for (int rr = 0; rr < nR && nb[J] > 0; ++rr) {
                         const int r2 = R0.fold_index(cells[S][0] - cells[rr][0], cells[S][1] - cells[rr][1],
                                                      cells[S][2] - cells[rr][2]);
                         const int n = nbr_at[J][(size_t)L * nR + r2];
