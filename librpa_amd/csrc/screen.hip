@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256, 2) void mlp_tile_grad_kernel(const float *__re
         for (int m = 0; m < 4; ++m) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                gw3[m][r] += dy * h2[m][r];
+                gw3[m][r] += s < n ? dy * h2[m][r] : 0.0f;  // (h2 of a padding lane can overflow where no sample's does)
                 d[m][r] = s < n ? d[m][r] * dy * w3[m][r] : 0.0f;
                 gb2[m][r] += d[m][r];
             }
