@@ -47,6 +47,12 @@ __device__ __forceinline__ v4f mfma(float a, float b, v4f c) { return __builtin_
 // leave registers for them; 128 + 32 FP64 ones do not (38 spilled: 205 -> 258 ms on 64 atoms).
 template <class T> constexpr bool one_wave(int fm, int fi) { return sizeof(T) == 8 && fm * fi >= 16; }
 
+// An FP32 accumulator takes at most this many steps (of four products) before it is added to chi.  Diagonal
+// blocks of the 128-atom cell against FP64: off by 1.28e-6 of their norm (rms) with a segment list in two to
+// four accumulators (up to 6400 steps each), by 0.77e-6 with this limit, and the launches 5% shorter (977 ->
+// 931 ms for 16 tau points).  The GEMMs over a stored T that took quarters of the list were off by 0.86e-6.
+constexpr double kMaxStepsF32 = 1600;
+
 constexpr int kQsMax = 64;  // G steps kept in LDS (n_b(J) <= 128); later ones are read from memory
 }  // namespace
 
@@ -368,6 +374,7 @@ void Chi0Tasks::build(const std::vector<Chi0Out> &outs, bool f64, int nz, int sp
             const int left = strips - n, ns = left >= 4 ? 4 : left >= 2 ? 2 : 1;
             const int kp = single ? 1 : 4 / ns;
             int parts = splitk > 0 ? ceil_div(splitk, kp) : (int)std::max(1.0, std::min(cst / (per * kp) + 0.5, 4096.0));
+            if (!f64 && splitk == 0) parts = std::max(parts, (int)std::ceil((double)o.lsum * ceil_div(o.ni, 4) / (kp * kMaxStepsF32)));
             parts = std::min(parts, std::max(1, nseg / kp));
             // segment where the share f of the cost is reached
             auto seg_at = [&](double f) {
