@@ -32,7 +32,7 @@ struct Chi0Task { int out, m0, n0, ns, kp, t0, t1, part; };
 // The task lists of one element type (FP64 or FP32), by tile class.
 struct Chi0Tasks {
     struct Class {
-        int fm, fi, nq;  // row fragments of mu per wave and of i per pass, W steps in registers
+        int fm, fn, fi, nq;  // row fragments of mu, columns of a lane, fragments of i per pass, unrolled W steps
         std::vector<Chi0Task> tasks;
         int qs = 0;  // LDS steps of the G operand
         DevBuf d_tasks;
