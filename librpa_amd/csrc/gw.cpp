@@ -505,6 +505,11 @@ template <class F> void carve(DevBuf &buf, F layout, size_t at_least = 0) {
 }
 }  // namespace
 
+double GwEngine::keep_bytes() {
+    const char *e = std::getenv("LIBRPA_AMD_KEEP_BYTES");
+    return e ? std::atof(e) : 12e9;
+}
+
 void GwEngine::sigma_layout(Carve &c, SigmaWork &w) const {
     const size_t nel = (size_t)nR * NAO * NAO, next = (size_t)NE * NAO * NAO;
     w.U = c.take<char>(2 * (size_t)u_elems * nbatch * ts);
@@ -949,7 +954,6 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g, Result &out) {
     if (prec == Prec::F64) passes(double());
     else passes(float());
     HIP_CHECK(hipStreamSynchronize(st));
-    if ((double)work.bytes() > kKeepBytes) work.release();
     t_sigma = now_s() - t0;
 }
 
@@ -1140,10 +1144,21 @@ void gw_build_sigma(Dataset &d, const LibrpaOptions &o) {
     // the plan and the work memory stay with the inputs they were made for
     auto gw = d.gw;
     if (!gw || gw->rpa != eng) gw = std::make_shared<GwEngine>();
+    // what is large goes back however the build ends
+    struct Trim {
+        GwEngine &gw;
+        RpaEngine &eng;
+        ~Trim() {
+            const double keep = GwEngine::keep_bytes();
+            if ((double)gw.work.bytes() > keep) gw.work.release();
+            if (eng.work_bytes() > keep) eng.release_work();
+            if (eng.ec_bytes() > keep) eng.release_ec();
+        }
+    } trim{*gw, *eng};
     eng->build_chi0(d, d.grid, o.n_bands_chi0);
     // chi0(R, tau) stays; large chi0 work buffers and those of an earlier Ec evaluation are rebuilt on demand
-    if (eng->work_bytes() > GwEngine::kKeepBytes) eng->release_work();
-    if (eng->ec_bytes() > GwEngine::kKeepBytes) eng->release_ec();
+    if (eng->work_bytes() > GwEngine::keep_bytes()) eng->release_work();
+    if (eng->ec_bytes() > GwEngine::keep_bytes()) eng->release_ec();
     gw->verbose = o.output_level >= LIBRPA_VERBOSE_DEBUG;
     gw->head = head;
     gw->sqrt_threshold = o.sqrt_coulomb_threshold;

@@ -81,10 +81,11 @@ struct GwEngine {
 
     DevBuf d_fold, d_neg;
     // Work memory of W and of Sigma, one after the other in the same bytes.  Kept for the next build up to
-    // kKeepBytes (allocating and freeing 3 GB took 30 of the 86 ms of a build on 8 atoms and 4 k), as are
-    // the chi0 build's buffers beside it; larger systems give it back after every build.
+    // keep_bytes (allocating and freeing 3 GB took 30 of the 86 ms of a build on 8 atoms and 4 k), as are
+    // the chi0 build's buffers and the Cholesky workspace beside it; larger systems give each of them back
+    // after every build, finished or failed.
     DevBuf work;
-    static constexpr double kKeepBytes = 12e9;
+    static double keep_bytes();  // 12 GB, or LIBRPA_AMD_KEEP_BYTES
     struct SigmaWork { char *U, *Ghat, *CW, *Y, *sigma, *Wlow; };  // sigma: sig, s2 and ext of each tau and sign
     void sigma_layout(Carve &c, SigmaWork &w) const;
     CoulombStage vst, vcst;          // the Coulomb inputs of the q in v_qs

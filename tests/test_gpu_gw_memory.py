@@ -1,0 +1,82 @@
+"""Device memory of G0W0 builds: what a handle keeps between builds, after a failed build, and beside
+another handle.  Free device memory is asked of the driver; sizes are chosen so that the kept buffers (over
+100 MB) stand out against its granularity (2 MB a buffer)."""
+import numpy as np
+import pytest
+import torch
+
+import librpa_amd as L
+from librpa_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def _system(nabf=220):
+    s = synth.tiny(natom=2, period=(2, 1, 1), nao=(12, 9), nabf=(nabf, nabf - 20), nocc=(2, 1), a=7.0, nfreq=12,
+                   real_gamma_v=True)
+    n = s.nabf_tot
+    s.vq[:] = np.eye(n)  # its largest eigenvalue is degenerate: no head can be replaced
+    return s
+
+
+def _options(s, **kw):
+    return L.Options(nfreq=s.nfreq, tfgrids_type=L.MINIMAX, parallel_routing=L.LIBRI, **kw)
+
+
+def _fail(h, s):
+    h.set_dielect_func_imagfreq(h.get_tfgrids(_options(s))["omega"], np.full(s.nfreq, 2.0))
+    with pytest.raises(L.LibrpaError, match="degenerate"):
+        h.build_g0w0_sigma(_options(s, replace_w_head=1))
+
+
+def test_failed_build(lib, monkeypatch):
+    """With nothing to be kept, a build that fails gives the memory back as one that ends does."""
+    print("failed G0W0 build", flush=True)
+    monkeypatch.setenv("LIBRPA_AMD_KEEP_BYTES", "0")
+    s = _system()
+    h = L.Handler()
+    L.load_system(h, s, vq_cut=True)
+    _fail(h, s)  # (the eigen-solver library takes its own work memory on first use)
+    h.free()
+    h = L.Handler()
+    L.load_system(h, s, vq_cut=True)
+    h.build_g0w0_sigma(_options(s))
+    good = np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    before = _free()
+    _fail(h, s)
+    after = _free()
+    print(f"  free memory {before / MB:.0f} MB before, {after / MB:.0f} MB after the failed build", flush=True)
+    assert after >= before - 8 * MB
+    # the earlier results stay, and the next build needs nothing of the failed one
+    assert np.array_equal(np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)]), good)
+    h.build_g0w0_sigma(_options(s))
+    again = np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    assert np.abs(again - good).max() <= 1e-11 * np.abs(good).max()
+
+
+def test_nothing_kept(lib, monkeypatch):
+    """LIBRPA_AMD_KEEP_BYTES=0: a second build leaves as much free as the first; by default it keeps its buffers."""
+    s = _system()
+    used = {}
+    for keep in ("0", None):
+        if keep:
+            monkeypatch.setenv("LIBRPA_AMD_KEEP_BYTES", keep)
+        else:
+            monkeypatch.delenv("LIBRPA_AMD_KEEP_BYTES")
+        h = L.Handler()
+        L.load_system(h, s, vq_cut=True)
+        start = _free()
+        h.build_g0w0_sigma(_options(s))
+        used[keep] = start - _free()
+        h.build_g0w0_sigma(_options(s))
+        assert abs(start - _free() - used[keep]) <= 8 * MB
+        h.free()
+    print(f"  kept: {used['0'] / MB:.0f} MB with a limit of 0, {used[None] / MB:.0f} MB by default", flush=True)
+    assert used[None] - used["0"] > 100 * MB
