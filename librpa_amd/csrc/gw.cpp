@@ -1135,6 +1135,13 @@ void gw_build_sigma(Dataset &d, const LibrpaOptions &o) {
         head = interpolate_dielec(o.option_dielect_func, d.dielect_omega, d.dielect_val, d.grid.omega);
     auto eng = d.rpa;
     if (!eng || eng->prec != d.chi0_prec || eng->mixed != d.chi0_mixed || eng->planned_ntau != d.grid.n) {
+        // the new plan sizes itself by the free memory: what the old engines hold beside the results that
+        // the getters read goes back first (the results stay, should the new build fail)
+        if (eng) eng->release_stores();
+        if (d.gw) {
+            d.gw->work.release();
+            d.gw->rpa->release_stores();
+        }
         d.rpa.reset();
         eng = std::make_shared<RpaEngine>();
         eng->mixed = d.chi0_mixed;

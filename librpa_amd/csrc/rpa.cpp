@@ -957,6 +957,16 @@ void RpaEngine::release_work() {
     d_W.release();
 }
 
+void RpaEngine::release_stores() {
+    release_work();
+    release_ec();
+    for (DevBuf *b : {&d_chi0s, &d_chiw, &d_Cfin, &d_CWb, &d_Cfin32, &d_CWb32, &d_ZZ, &d_Zs, &d_Mst, &d_Gpm, &d_wre, &d_wim, &d_vblk})
+        b->release();
+    free_host_store();
+    ntau_done = 0;
+    chiw_ok = false;
+}
+
 void RpaEngine::free_host_store() {
     h_chi0s.clear();
     h_chi0s.shrink_to_fit();

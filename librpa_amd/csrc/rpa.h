@@ -140,6 +140,7 @@ struct RpaEngine {
     double ec_bytes() const;
     double work_bytes() const { return (double)d_Ghat.bytes() + (double)d_W.bytes(); }
     void release_ec();    // free the Ec work buffers (rebuilt by ec)
+    void release_stores();  // free everything large; the engine then only says how its system is laid out
     // chi0(R, omega) = sum_tau (2 / nspin) gamma_c(omega, tau) chi0(R, tau) of the last build, FP64
     // [omega][E], formed once per Ec / W evaluation when it fits in max_bytes (returns whether it
     // was formed); the R -> q sums then read it once per q instead of chi0(R, tau) per chunk of 8

@@ -80,3 +80,29 @@ def test_nothing_kept(lib, monkeypatch):
         h.free()
     print(f"  kept: {used['0'] / MB:.0f} MB with a limit of 0, {used[None] / MB:.0f} MB by default", flush=True)
     assert used[None] - used["0"] > 100 * MB
+
+
+def test_changed_precision(lib):
+    """A build in another precision plans with the old engine's memory free: after one that failed there is the
+    new engine (half the bytes) beside the old results, not both engines."""
+    print("G0W0 in another precision", flush=True)
+    s = _system()
+    h = L.Handler()
+    L.load_system(h, s, vq_cut=True)
+    _fail(h, s)
+    h.free()
+    h = L.Handler()
+    L.load_system(h, s, vq_cut=True)
+    start = _free()
+    h.build_g0w0_sigma(_options(s))
+    good = np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    both = start - _free()
+    h.set_precision(L.FP32, L.FP32)
+    _fail(h, s)
+    used = start - _free()
+    print(f"  {both / MB:.0f} MB after the FP64 build, {used / MB:.0f} MB after the failed FP32 one", flush=True)
+    assert used <= both + 8 * MB
+    assert np.array_equal(np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)]), good)
+    h.build_g0w0_sigma(_options(s))
+    low = np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    assert 0 < np.abs(low - good).max() <= 1e-2 * np.abs(good).max()
