@@ -512,8 +512,10 @@ double librpa_get_rpa_correlation_energy(LibrpaHandler *h, const LibrpaOptions *
                 eng = std::make_shared<RpaEngine>();
                 eng->mixed = d.chi0_mixed;
                 eng->verbose = o.output_level >= LIBRPA_VERBOSE_DEBUG;
+                KeptMemory::InUse planning(*eng);
                 eng->plan(d, d.chi0_prec, d.ec_prec, d.grid.n);
             }
+            KeptMemory::InUse use(*eng);
             eng->ec_prec = d.ec_prec;
             eng->mixed_low = d.chi0_mixed_low;
             eng->verbose = o.output_level >= LIBRPA_VERBOSE_DEBUG;

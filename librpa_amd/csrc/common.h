@@ -28,6 +28,9 @@ struct Error : std::runtime_error {
             LRA_THROW(std::string("HIP error ") + hipGetErrorString(e_) + " in " #expr); \
     } while (0)
 
+// Frees the work memory that idle engines keep for their next call (KeptMemory in rpa.h).
+void reclaim_kept_memory();
+
 // Owning device allocation.
 class DevBuf {
   public:
@@ -44,7 +47,14 @@ class DevBuf {
     void alloc(size_t bytes) {
         release();
         if (bytes == 0) return;
-        HIP_CHECK(hipMalloc(&p_, bytes));
+        hipError_t rc = hipMalloc(&p_, bytes);
+        if (rc == hipErrorOutOfMemory) {  // once more with what other handles keep
+            (void)hipGetLastError();
+            reclaim_kept_memory();
+            rc = hipMalloc(&p_, bytes);
+        }
+        if (rc != hipSuccess) p_ = nullptr;
+        HIP_CHECK(rc);
         n_ = bytes;
     }
     // grow-only reallocation (contents not preserved)

@@ -97,6 +97,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
             ext_cols[(size_t)rr * NAO + c] =
                 (linr(cells[rr][0], cells[rr][1], cells[rr][2]) + c0) * NAO * (long long)NAO + c;
 
+    reclaim_if_low();
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
 
@@ -1137,20 +1138,29 @@ void gw_build_sigma(Dataset &d, const LibrpaOptions &o) {
     if (!eng || eng->prec != d.chi0_prec || eng->mixed != d.chi0_mixed || eng->planned_ntau != d.grid.n) {
         // the new plan sizes itself by the free memory: what the old engines hold beside the results that
         // the getters read goes back first (the results stay, should the new build fail)
-        if (eng) eng->release_stores();
+        if (eng) {
+            KeptMemory::InUse use(*eng);
+            eng->release_stores();
+        }
         if (d.gw) {
+            KeptMemory::InUse use(*d.gw);
             d.gw->work.release();
+        }
+        if (d.gw && d.gw->rpa != eng) {
+            KeptMemory::InUse use(*d.gw->rpa);
             d.gw->rpa->release_stores();
         }
         d.rpa.reset();
         eng = std::make_shared<RpaEngine>();
         eng->mixed = d.chi0_mixed;
+        KeptMemory::InUse planning(*eng);
         eng->plan(d, d.chi0_prec, d.ec_prec, d.grid.n);
         d.rpa = eng;
     }
     // the plan and the work memory stay with the inputs they were made for
     auto gw = d.gw;
     if (!gw || gw->rpa != eng) gw = std::make_shared<GwEngine>();
+    KeptMemory::InUse use_eng(*eng), use_gw(*gw);
     // what is large goes back however the build ends
     struct Trim {
         GwEngine &gw;

@@ -35,7 +35,9 @@ struct Carve {
     }
 };
 
-struct GwEngine {
+struct GwEngine : KeptMemory {
+    void give_back() override { work.release(); }
+    ~GwEngine() override { hold(); }
     std::shared_ptr<RpaEngine> rpa;  // geometry, G(R, +-tau) builder, chi0(R, tau)
     Prec prec = Prec::F64;
     size_t ts = 8;

@@ -28,7 +28,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <set>
+#include <thread>
 
 namespace lra {
 
@@ -38,6 +40,47 @@ double now_s() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 }  // namespace
+
+namespace {
+struct KeptList {
+    std::mutex mu;
+    std::set<KeptMemory *> all;
+};
+// (never destroyed: handles may outlive the statics of this file)
+KeptList &kept() {
+    static KeptList *l = new KeptList;
+    return *l;
+}
+}  // namespace
+
+KeptMemory::KeptMemory() {
+    std::lock_guard<std::mutex> lk(kept().mu);
+    kept().all.insert(this);
+}
+
+KeptMemory::~KeptMemory() {
+    std::lock_guard<std::mutex> lk(kept().mu);
+    kept().all.erase(this);
+}
+
+void KeptMemory::hold() {
+    while (held.exchange(true)) std::this_thread::yield();  // (a reclaim in another thread)
+}
+
+void reclaim_kept_memory() {
+    std::lock_guard<std::mutex> lk(kept().mu);
+    for (KeptMemory *k : kept().all) {
+        if (k->held.exchange(true)) continue;
+        k->give_back();
+        k->held = false;
+    }
+}
+
+void reclaim_if_low() {
+    size_t free_b = 0, total_b = 0;
+    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    if (free_b < total_b / 2) reclaim_kept_memory();
+}
 
 int RpaEngine::cell_index(int x, int y, int z) const {
     const int x0 = -(period[0] / 2), y0 = -(period[1] / 2), z0 = -(period[2] / 2);
@@ -179,6 +222,7 @@ void RpaEngine::plan(const Dataset &ds, Prec p, Prec pe, int ntau) {
         for (int S = 0; S < nR; ++S)
             w_off[(size_t)J * nR + S + 1] = w_off[(size_t)J * nR + S] + 2LL * nb[J] * NAO * na[J];
     // ---- chunking over J by memory budget (gathered G panels) ----
+    reclaim_if_low();
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
     // chi0(R, tau) of every tau beside the W slabs, or staged through pinned host memory
@@ -973,6 +1017,7 @@ void RpaEngine::free_host_store() {
 }
 
 RpaEngine::~RpaEngine() {
+    hold();
     free_host_store();
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <array>
+#include <atomic>
 #include <map>
 #include <tuple>
 #include <vector>
@@ -19,7 +20,26 @@ struct RpaResult {
     std::vector<cplx> qcontrib;  // per IBZ k
 };
 
-struct RpaEngine {
+// Work memory that an engine keeps between calls and that another handle may take back while the engine is
+// idle: every call holds it by InUse; reclaim_kept_memory leaves a held engine alone, from whatever thread.
+struct KeptMemory {
+    KeptMemory();
+    virtual ~KeptMemory();
+    KeptMemory(const KeptMemory &) = delete;
+    KeptMemory &operator=(const KeptMemory &) = delete;
+    virtual void give_back() = 0;
+    std::atomic<bool> held{false};
+    void hold();  // for good: the destructors of derived classes begin with it
+    struct InUse {
+        KeptMemory &k;
+        explicit InUse(KeptMemory &m) : k(m) { k.hold(); }
+        ~InUse() { k.held = false; }
+    };
+};
+// reclaim_kept_memory when less than half of the device is free: a plan sizes itself by the free memory
+void reclaim_if_low();
+
+struct RpaEngine : KeptMemory {
     // ---- static plan (tau independent) ----
     Prec prec = Prec::F64, ec_prec = Prec::F64;
     int natom = 0, NAO = 0, NABF = 0, nR = 0, nk = 0, nspin = 1, nbands = 0;
@@ -78,9 +98,8 @@ struct RpaEngine {
     DevBuf d_wre, d_wim, d_eps, d_wg, d_cs, d_sn, d_gcol;
     hipStream_t stream = 0;
     RpaEngine() = default;
-    RpaEngine(const RpaEngine &) = delete;
-    RpaEngine &operator=(const RpaEngine &) = delete;
-    ~RpaEngine();
+    ~RpaEngine() override;
+    void give_back() override { release_work(); release_ec(); }
 
     // transform / Ec
     std::vector<PairDesc> pairs;

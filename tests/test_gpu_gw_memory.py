@@ -106,3 +106,41 @@ def test_changed_precision(lib):
     h.build_g0w0_sigma(_options(s))
     low = np.array([h.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
     assert 0 < np.abs(low - good).max() <= 1e-2 * np.abs(good).max()
+
+
+def test_given_back_to_another_handle(lib):
+    """What an idle handle keeps goes back when another plans with less than half of the device free, and not
+    before; the idle handle's next calls allocate again."""
+    print("two handles", flush=True)
+    s = _system()
+    a = L.Handler()
+    L.load_system(a, s, vq_cut=True)
+    a.build_g0w0_sigma(_options(s))
+    ec = a.get_rpa_correlation_energy(_options(s), s.nk)[0]
+    good = np.array([a.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    small = synth.tiny(natom=2, period=(2, 1, 1), nao=(3, 2), nabf=(4, 3), nocc=(1, 1), a=7.0, nfreq=6)
+
+    def plan():
+        h = L.Handler()
+        L.load_system(h, small)
+        h.get_rpa_correlation_energy(_options(small), small.nk)
+        h.free()
+
+    plan()
+    free = _free()
+    plan()
+    assert abs(_free() - free) <= 8 * MB
+    total = torch.cuda.mem_get_info()[1]
+    fill = torch.empty(max(0, free - int(0.4 * total)), dtype=torch.uint8, device="cuda")
+    free = _free()
+    plan()
+    got = _free() - free
+    del fill
+    torch.cuda.empty_cache()
+    print(f"  {got / MB:.0f} MB came back", flush=True)
+    assert got > 100 * MB
+    again = a.get_rpa_correlation_energy(_options(s), s.nk)[0]
+    assert abs(again - ec) <= 1e-11 * abs(ec)
+    a.build_g0w0_sigma(_options(s))
+    again = np.array([a.get_sigc_ks(0, 0, n, s.nfreq) for n in range(3)])
+    assert np.abs(again - good).max() <= 1e-11 * np.abs(good).max()
