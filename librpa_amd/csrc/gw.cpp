@@ -107,20 +107,29 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
         for (int S = 0; S < nR; ++S)
             u_off[(size_t)J * nR + S + 1] = u_off[(size_t)J * nR + S] + (long long)NAO * nb[J] * na[J];
     u_elems = u_off[(size_t)natom * nR];
+    y_off.assign(natom + 1, 0);
+    for (int I = 0; I < natom; ++I) y_off[I + 1] = y_off[I] + (long long)na[I] * nb[I] * LD;
+    y_elems = y_off[natom];
+    const double ghat_budget = std::min(24e9, 0.08 * (double)free_b), wrt = 8.0 * ntau * nR * (double)NABF * NABF;
+    double cw_least = 0;  // CW of one atom
+    for (int x = 0; x < natom; ++x) cw_least = std::max(cw_least, (double)ts * nR * R0.lsum[x] * nb[x] * NABF);
+    signs = 2.0 * ts * (u_elems + y_elems) + ghat_budget + wrt + std::max(4e9, cw_least) > 0.85 * (double)free_b ? 1 : 2;
+    if (const char *e = std::getenv("LIBRPA_AMD_SIGMA_SIGNS")) signs = std::atoi(e) == 1 ? 1 : signs;
     const long long gpm_r = (long long)NAO * 2 * NAO;
     max_ghat = 0;
-    {
-        const double budget = std::min(24e9, 0.08 * (double)free_b);
+    for (int only = signs == 2 ? -1 : 0; only < (signs == 2 ? 0 : 2); ++only) {
         int j = 0;
         while (j < natom) {
             UChunk c;
+            c.sg = only;
             const int j0 = j;
             for (; j < natom; ++j) {
-                const long long g1 = (long long)nR * 2 * NAO * R0.lsum[j];
-                if (j > j0 && (double)(c.ghat_elems + g1) * ts > budget) break;
+                const long long g1 = (long long)nR * signs * NAO * R0.lsum[j];
+                if (j > j0 && (double)(c.ghat_elems + g1) * ts > ghat_budget) break;
                 const long long ls = R0.lsum[j];
                 for (int S = 0; S < nR; ++S)
                     for (int sg = 0; sg < 2; ++sg) {
+                        if (only >= 0 && sg != only) continue;
                         GatherJob gj;
                         gj.dst_off = c.ghat_elems;
                         gj.ncol = (int)ls;
@@ -136,7 +145,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
                         c.jobs.push_back(gj);
                         // K = 0 (an atom without Cs) writes zeros
                         c.ub.add(make_prob(NAO, nb[j] * na[j], (int)ls, c.ghat_elems, (int)ls, R0.cwb_off[j],
-                                           nb[j] * na[j], sg * u_elems + u_off[(size_t)j * nR + S], nb[j] * na[j]));
+                                           nb[j] * na[j], (only < 0 ? sg * u_elems : 0) + u_off[(size_t)j * nR + S], nb[j] * na[j]));
                         c.ghat_elems += (long long)NAO * ls;
                     }
             }
@@ -150,10 +159,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
         }
     }
 
-    // ---- Y and its contraction ----
-    y_off.assign(natom + 1, 0);
-    for (int I = 0; I < natom; ++I) y_off[I + 1] = y_off[I] + (long long)na[I] * nb[I] * LD;
-    y_elems = y_off[natom];
+    // ---- the contraction of Y ----
     a3 = GemmBatch();
     a3.atomic = true;
     a3.trans_b = true;
@@ -182,8 +188,7 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
     double cw_total = 0, fl = 0;
     std::vector<long long> cw_x(natom);  // CW of atom x in its chunk: [R][J][c][i][nu]
     {
-        const double fixed = 2.0 * per_sign + 8.0 * ntau * nR * (double)NABF * NABF;
-        double budget = std::max(4e9, std::min(96e9, 0.6 * (double)free_b - fixed));
+        double budget = std::max(4e9, std::min(96e9, 0.6 * (double)free_b - signs * per_sign - wrt));
         if (const char *cb = std::getenv("LIBRPA_AMD_CHUNK_BYTES"))
             if (std::atof(cb) > 0) budget = std::min(budget, std::atof(cb));
         int x = 0;
@@ -238,9 +243,9 @@ void GwEngine::plan(const Dataset &ds, std::shared_ptr<RpaEngine> r) {
     flops_sigma = (flops_sigma + fl) * nspin * ntau;
     // tau points per pass, as in the chi0 build: up to about 120 GFLOP, and 12 GB
     nbatch = 1;
-    if (uchunks.size() == 1 && xchunks.size() == 1)
+    if (signs == 2 && uchunks.size() == 1 && xchunks.size() == 1)
         nbatch = (int)std::max(1.0, std::min({(double)R0.nbatch, std::ceil(1.2e11 / std::max(1.0, flops_sigma / ntau)),
-                                              std::min(12e9, 0.1 * (double)free_b) / (ts * cw_total + 2.0 * per_sign)}));
+                                              std::min(12e9, 0.1 * (double)free_b) / (ts * cw_total + signs * per_sign)}));
     nbatch = ceil_div(ntau, ceil_div(ntau, nbatch));
     for (auto &c : xchunks) {
         std::map<std::pair<int, int>, std::vector<SigTask>> td, tb;
@@ -513,10 +518,10 @@ double GwEngine::keep_bytes() {
 
 void GwEngine::sigma_layout(Carve &c, SigmaWork &w) const {
     const size_t nel = (size_t)nR * NAO * NAO, next = (size_t)NE * NAO * NAO;
-    w.U = c.take<char>(2 * (size_t)u_elems * nbatch * ts);
+    w.U = c.take<char>(signs * (size_t)u_elems * nbatch * ts);
     w.Ghat = c.take<char>((size_t)max_ghat * nbatch * ts);
     w.CW = c.take<char>(((size_t)max_cw * nbatch + kChi0Pad) * ts);
-    w.Y = c.take<char>(2 * (size_t)y_elems * nbatch * ts);
+    w.Y = c.take<char>(signs * (size_t)y_elems * nbatch * ts);
     w.sigma = c.take<char>(2 * (size_t)nbatch * (2 * nel + next) * ts);
     w.Wlow = prec != Prec::F64 ? c.take<char>((size_t)nbatch * nR * NABF * NABF * ts) : nullptr;
 }
@@ -893,56 +898,59 @@ void GwEngine::build_sigma(const Dataset &ds, const TFGrid &g, Result &out) {
                 R0.build_gf(ds.mf, &g.tau[it], nz, s);
                 T *sig = reinterpret_cast<T *>(sigma), *s2 = sig + 2 * (size_t)nbatch * nel, *ext = s2 + 2 * (size_t)nbatch * nel;
                 HIP_CHECK(hipMemsetAsync(sigma, 0, sig_elems * ts, st));
-                // U_J(S) for all J, S
-                for (auto &c : uchunks) {
-                    prof.begin("gw_gather", st);
-                    launch_gather_cols<T>(G, 2LL * NAO, reinterpret_cast<T *>(Ghat), c.d_jobs.template as<GatherJob>(), (int)c.jobs.size(),
-                                          c.d_colsrc.template as<long long>(), NAO, c.max_gcol, st, nz, zg, c.ghat_elems);
-                    prof.end("gw_gather", st, 0, 2.0 * nz * c.ghat_elems * ts);
-                    prof.begin("gw_U", st);
-                    c.ub.nz = nz;
-                    c.ub.za = c.ghat_elems;
-                    c.ub.zc = 2 * u_elems;
-                    if (tune_sigma && !c.ub.tuned)
-                        c.ub.tune(prec, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
-                    gemm_run(prec, c.ub, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
-                    prof.end("gw_U", st, nz * c.ub.flops);
-                }
-                for (auto &c : xchunks) {
-                    if (s == 0 || xchunks.size() > 1) {
-                        prof.begin("gw_CW", st);
-                        c.cwb.nz = nz;
-                        c.cwb.zb = nR * nn_abf;
-                        c.cwb.zc = c.cw_elems;
-                        if (tune_sigma && !c.cwb.tuned)
-                            c.cwb.tune(prec, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
-                        gemm_run(prec, c.cwb, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
-                        prof.end("gw_CW", st, nz * c.cwb.flops);
+                for (int sg0 = 0; sg0 < 2; sg0 += signs) {
+                    // U_J(S) for all J, S
+                    for (auto &c : uchunks) {
+                        if (c.sg >= 0 && c.sg != sg0) continue;
+                        prof.begin("gw_gather", st);
+                        launch_gather_cols<T>(G, 2LL * NAO, reinterpret_cast<T *>(Ghat), c.d_jobs.template as<GatherJob>(), (int)c.jobs.size(),
+                                              c.d_colsrc.template as<long long>(), NAO, c.max_gcol, st, nz, zg, c.ghat_elems);
+                        prof.end("gw_gather", st, 0, 2.0 * nz * c.ghat_elems * ts);
+                        prof.begin("gw_U", st);
+                        c.ub.nz = nz;
+                        c.ub.za = c.ghat_elems;
+                        c.ub.zc = signs * u_elems;
+                        if (tune_sigma && !c.ub.tuned)
+                            c.ub.tune(prec, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
+                        gemm_run(prec, c.ub, Ghat, R0.d_CWb.get(), U, 1.0, 0.0, st);
+                        prof.end("gw_U", st, nz * c.ub.flops);
                     }
-                    const SigBlk *blks = c.d_blks.template as<SigBlk>();
-                    const Chi0Seg *segs = R0.d_segs.as<Chi0Seg>();
-                    prof.begin("gw_D", st);
-                    for (auto &t : c.d)
-                        launch_sigma_d<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
-                                          tU, u_elems, sig, nel, NAO, nz, st);
-                    prof.end("gw_D", st);
-                    prof.begin("gw_B", st);
-                    for (auto &t : c.b)
-                        launch_sigma_b<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
-                                          tU, u_elems, s2, nel, NAO, nz, st);
-                    prof.end("gw_B", st);
-                    prof.begin("gw_Y", st);
-                    for (auto &t : ytasks)
-                        launch_sigma_y<T>(t.d.template as<SigYTask>(), t.n, t.a, d_yent.as<SigYEnt>(), tCW, c.cw_elems,
-                                          G, zg, tY, y_elems, NAO, c.x0, c.x1, c.x0 == 0, nz, st);
-                    prof.end("gw_Y", st);
+                    for (auto &c : xchunks) {
+                        if ((s == 0 && sg0 == 0) || xchunks.size() > 1) {
+                            prof.begin("gw_CW", st);
+                            c.cwb.nz = nz;
+                            c.cwb.zb = nR * nn_abf;
+                            c.cwb.zc = c.cw_elems;
+                            if (tune_sigma && !c.cwb.tuned)
+                                c.cwb.tune(prec, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
+                            gemm_run(prec, c.cwb, R0.d_Cfin.get(), Wf, CW, 1.0, 0.0, st);
+                            prof.end("gw_CW", st, nz * c.cwb.flops);
+                        }
+                        const SigBlk *blks = c.d_blks.template as<SigBlk>();
+                        const Chi0Seg *segs = R0.d_segs.as<Chi0Seg>();
+                        prof.begin("gw_D", st);
+                        for (auto &t : c.d)
+                            launch_sigma_d<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
+                                              tU, u_elems, sig + sg0 * nel, nel, NAO, nz, signs, st);
+                        prof.end("gw_D", st);
+                        prof.begin("gw_B", st);
+                        for (auto &t : c.b)
+                            launch_sigma_b<T>(t.d.template as<SigTask>(), t.n, t.a, t.b, blks, segs, tCW, c.cw_elems,
+                                              tU, u_elems, s2 + sg0 * nel, nel, NAO, nz, signs, st);
+                        prof.end("gw_B", st);
+                        prof.begin("gw_Y", st);
+                        for (auto &t : ytasks)
+                            launch_sigma_y<T>(t.d.template as<SigYTask>(), t.n, t.a, d_yent.as<SigYEnt>(), tCW, c.cw_elems,
+                                              G, zg, tY, y_elems, NAO, c.x0, c.x1, c.x0 == 0, nz, signs, sg0, st);
+                        prof.end("gw_Y", st);
+                    }
+                    prof.begin("gw_A3", st);
+                    a3.nz = signs * nz;
+                    a3.zb = y_elems;
+                    a3.zc = (2 / signs) * (long long)next;
+                    gemm_run(prec, a3, R0.d_Cfin.get(), Y, ext + sg0 * next, 1.0, 1.0, st);
+                    prof.end("gw_A3", st, signs * nz * a3.flops);
                 }
-                prof.begin("gw_A3", st);
-                a3.nz = 2 * nz;
-                a3.zb = y_elems;
-                a3.zc = (long long)next;
-                gemm_run(prec, a3, R0.d_Cfin.get(), Y, ext, 1.0, 1.0, st);
-                prof.end("gw_A3", st, 2 * nz * a3.flops);
                 prof.begin("gw_fold", st);
                 launch_sigma_fold<T>(sig, s2, ext, d_fold.as<int>(), d_neg.as<int>(), NE, nR, NAO, nz, st);
                 launch_sigma_freq<T>(sig, nel, dcw.as<double>(), dsw.as<double>(), nw, g.n, it, nz,

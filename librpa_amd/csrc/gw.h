@@ -51,9 +51,11 @@ struct GwEngine : KeptMemory {
     long long linr(int x, int y, int z) const { return ((long long)x * E[1] + y) * E[2] + z; }
 
     int nbatch = 1;  // tau points per pass
+    int signs = 2;   // signs of tau per pass: U and Y of both are held, or of one at a time when two do not fit
 
-    // U_J(S) build, both signs
+    // U_J(S) build
     struct UChunk {
+        int sg = -1;  // its sign of tau (0: +, 1: -), -1: both
         long long ghat_elems = 0;
         int max_gcol = 0;
         std::vector<GatherJob> jobs;

@@ -32,14 +32,15 @@ struct SigBlk {
 };
 // segments [c0, c1) of a block, rows from i0 (or all), columns from j0
 struct SigTask { int blk, i0, j0, c0, c1; };
-// sig[z][sign][R][NAO][NAO] += D, the label a0b0_a2b2: CW zcw elements per tau point, U two signs usg apart
+// For nsg signs of tau (2, or 1 at a time: sig, s2 start at that sign then, U and Y hold it alone):
+// sig[z][sign][R][NAO][NAO] += D, the label a0b0_a2b2: CW zcw elements per tau point, U's signs usg apart
 template <class T>
 void launch_sigma_d(const SigTask *tasks, int ntask, int fi, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
-                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, hipStream_t s);
+                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, int nsg, hipStream_t s);
 // s2[z][sign][R][NAO][NAO] += the label a0b0_a1b2, 64 fc segments a task from c0
 template <class T>
 void launch_sigma_b(const SigTask *tasks, int ntask, int fc, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
-                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, hipStream_t s);
+                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, int nsg, hipStream_t s);
 // One (J, R) that reaches the columns (S, L, .): G_IJ(R) at g, CW_JI(-R)[(L, S - R, l)] at
 // b + abf(I) lb + (cb + l nj) ai
 struct SigYEnt { long long g, b; int lb, cb, nj, J; };
@@ -50,7 +51,7 @@ struct SigYTask {
 };
 template <class T>
 void launch_sigma_y(const SigYTask *tasks, int ntask, int fi, const SigYEnt *ents, const T *CW, long long zcw, const T *G,
-                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, hipStream_t s);
+                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, int nsg, int sg0, hipStream_t s);
 
 // for nz tau points and both signs: sig[R][a][b] += s2[R][a][b] + s2[-R][b][a] + sum_{e : fold[e] == R} ext[e][a][b]
 template <class T>

@@ -128,17 +128,17 @@ __device__ __forceinline__ void load4(T (&v)[4], const T *p, int n) {
 // Bound by the reads of CW (each element once per pass) and, for small n_b, by U from L2: an MFMA
 // multiplies a fragment pair of 1 KB in 64 (FP64) cycles, so the next fragments are in flight
 // meanwhile.  8 atoms, 4 k: 24 such contractions of T = W U through an 8-workgroup GEMM took 35 ms.
-template <class T, int FI, int FJ>
+template <class T, int FI, int FJ, int NSG>
 __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restrict__ tasks, const SigBlk *__restrict__ blks,
                                                          const Chi0Seg *__restrict__ segs, const T *__restrict__ CW,
                                                          long long zcw, const T *__restrict__ U, long long usg,
                                                          T *__restrict__ sig, long long ssg, int NAO) {
     using A = typename SV<T>::A;
-    __shared__ __align__(16) T red[FI * FJ * 2 * 256];
+    __shared__ __align__(16) T red[FI * FJ * NSG * 256];
     const SigTask tk = tasks[blockIdx.x];
     const SigBlk B = blks[tk.blk];
     CW += blockIdx.y * zcw + B.cw;
-    U += blockIdx.y * 2 * usg + B.u;
+    U += blockIdx.y * NSG * usg + B.u;
     sig += blockIdx.y * 2 * ssg;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, kq = lane >> 4;
     const int ni = B.ni, nj = B.nj, aj = B.aj;
@@ -148,12 +148,14 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
     for (int f = 0; f < FI; ++f) ao[f] = min(tk.i0 + 16 * f + c16, ni - 1) * aj + 4 * kq;
 #pragma unroll
     for (int g = 0; g < FJ; ++g) uo[g] = min(tk.j0 + 16 * g + c16, nj - 1) * aj + 4 * kq;
-    A acc[FI][FJ][2];
+    A acc[FI][FJ][NSG];
 #pragma unroll
     for (int f = 0; f < FI; ++f)
 #pragma unroll
-        for (int g = 0; g < FJ; ++g) acc[f][g][0] = acc[f][g][1] = A{0, 0, 0, 0};
-    struct Frag { T a[FI][4], u[2][FJ][4]; };
+        for (int g = 0; g < FJ; ++g)
+#pragma unroll
+            for (int s = 0; s < NSG; ++s) acc[f][g][s] = A{0, 0, 0, 0};
+    struct Frag { T a[FI][4], u[NSG][FJ][4]; };
     auto load = [&](Frag &x, int t, int k0) {
         const Chi0Seg sg = st[t];
         const T *ab = CW + (long long)sg.c * ni * aj + k0;
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
 #pragma unroll
         for (int f = 0; f < FI; ++f) load4(x.a[f], ab + ao[f], n);
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = 0; s < NSG; ++s)
 #pragma unroll
             for (int g = 0; g < FJ; ++g) load4(x.u[s][g], ub + s * usg + uo[g], n);
     };
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
+            for (int s = 0; s < NSG; ++s)
 #pragma unroll
                 for (int f = 0; f < FI; ++f)
 #pragma unroll
@@ -198,7 +200,7 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
 #pragma unroll
                 for (int g = 0; g < FJ; ++g)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) *reinterpret_cast<A *>(&red[(((f * FJ + g) * 2 + s) * 64 + lane) * 4]) = acc[f][g][s];
+                    for (int s = 0; s < NSG; ++s) *reinterpret_cast<A *>(&red[(((f * FJ + g) * NSG + s) * 64 + lane) * 4]) = acc[f][g][s];
         __syncthreads();
         if (wave == 0)
 #pragma unroll
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
 #pragma unroll
                 for (int g = 0; g < FJ; ++g)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) acc[f][g][s] += *reinterpret_cast<const A *>(&red[(((f * FJ + g) * 2 + s) * 64 + lane) * 4]);
+                    for (int s = 0; s < NSG; ++s) acc[f][g][s] += *reinterpret_cast<const A *>(&red[(((f * FJ + g) * NSG + s) * 64 + lane) * 4]);
     }
     if (wave != 0) return;
 #pragma unroll
@@ -220,15 +222,15 @@ __global__ __launch_bounds__(256, 2) void sigma_d_kernel(const SigTask *__restri
                 const int j = tk.j0 + 16 * g + c16;
                 if (j >= nj) continue;
                 T *dst = sig + ((long long)B.r * NAO + B.rowI + i) * NAO + B.colJ + j;
-                unsafeAtomicAdd(dst, acc[f][g][0][r]);
-                unsafeAtomicAdd(dst + ssg, acc[f][g][1][r]);
+#pragma unroll
+                for (int s = 0; s < NSG; ++s) unsafeAtomicAdd(dst + s * ssg, acc[f][g][s][r]);
             }
         }
 }
 
 // S2(S_c)[row_c][j] += sum_(i, nu) CW_IJ(R)[c][(i, nu)] U_J(R)[(I, i)][j][nu] for the 16 FC segments of a
 // wave (64 FC of a task, from c0), FJ fragments of j and both signs; operands as in sigma_d_kernel.
-template <class T, int FC, int FJ>
+template <class T, int FC, int FJ, int NSG>
 __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restrict__ tasks, const SigBlk *__restrict__ blks,
                                                          const Chi0Seg *__restrict__ segs, const T *__restrict__ CW,
                                                          long long zcw, const T *__restrict__ U, long long usg,
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restri
     const int ni = B.ni, nj = B.nj, aj = B.aj, t0 = tk.c0 + 16 * FC * wave;
     if (t0 >= B.l) return;
     CW += blockIdx.y * zcw + B.cw;
-    U += blockIdx.y * 2 * usg + B.u + ((long long)B.r * NAO + B.rowI) * nj * aj;
+    U += blockIdx.y * NSG * usg + B.u + ((long long)B.r * NAO + B.rowI) * nj * aj;
     s2 += blockIdx.y * 2 * ssg;
     const Chi0Seg *st = segs + B.seg0;
     const T *ap[FC];
@@ -249,19 +251,21 @@ __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restri
     int uo[FJ];
 #pragma unroll
     for (int g = 0; g < FJ; ++g) uo[g] = min(tk.j0 + 16 * g + c16, nj - 1) * aj + 4 * kq;
-    A acc[FC][FJ][2];
+    A acc[FC][FJ][NSG];
 #pragma unroll
     for (int f = 0; f < FC; ++f)
 #pragma unroll
-        for (int g = 0; g < FJ; ++g) acc[f][g][0] = acc[f][g][1] = A{0, 0, 0, 0};
-    struct Frag { T a[FC][4], u[2][FJ][4]; };
+        for (int g = 0; g < FJ; ++g)
+#pragma unroll
+            for (int s = 0; s < NSG; ++s) acc[f][g][s] = A{0, 0, 0, 0};
+    struct Frag { T a[FC][4], u[NSG][FJ][4]; };
     auto load = [&](Frag &x, int i, int k0) {
         const int n = aj - k0 - 4 * kq;
         const T *ub = U + (long long)i * nj * aj + k0;
 #pragma unroll
         for (int f = 0; f < FC; ++f) load4(x.a[f], ap[f] + i * aj + k0, n);
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = 0; s < NSG; ++s)
 #pragma unroll
             for (int g = 0; g < FJ; ++g) load4(x.u[s][g], ub + s * usg + uo[g], n);
     };
@@ -276,7 +280,7 @@ __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restri
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
+            for (int s = 0; s < NSG; ++s)
 #pragma unroll
                 for (int f = 0; f < FC; ++f)
 #pragma unroll
@@ -296,8 +300,8 @@ __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restri
                 const int j = tk.j0 + 16 * g + c16;
                 if (j >= nj) continue;
                 T *dst = s2 + ((long long)sg.cell * NAO + sg.row) * NAO + B.colJ + j;
-                unsafeAtomicAdd(dst, acc[f][g][0][r]);
-                unsafeAtomicAdd(dst + ssg, acc[f][g][1][r]);
+#pragma unroll
+                for (int s = 0; s < NSG; ++s) unsafeAtomicAdd(dst + s * ssg, acc[f][g][s][r]);
             }
         }
 }
@@ -306,11 +310,11 @@ __global__ __launch_bounds__(256, 2) void sigma_b_kernel(const SigTask *__restri
 // takes one column (S, L, l), 16 FI rows i and 64 mu, and the entries (J, R) of (S, L) with J in
 // [x0, x1) (first chunk: Y is overwritten).  Each element of CW is read once, 16 bytes a lane, for
 // 2 FI MFMAs; G_IJ comes from L2.
-template <class T, int FI>
+template <class T, int FI, int NSG>
 __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restrict__ tasks, const SigYEnt *__restrict__ ents,
                                                          const T *__restrict__ CW, long long zcw, const T *__restrict__ G,
                                                          long long zg, T *__restrict__ Y, long long ysg, int NAO, int x0,
-                                                         int x1, int first) {
+                                                         int x1, int first, int sg0) {
     using A = typename SV<T>::A;
     using V = typename SV<T>::V;
     constexpr int VL = SV<T>::VL, NV = 4 / VL;
@@ -321,19 +325,21 @@ __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restr
     if (l >= tk.nl) return;
     CW += blockIdx.y * zcw;
     G += blockIdx.y * zg + (long long)tk.ao * 2 * NAO;
-    Y += blockIdx.y * 2 * ysg + tk.y;
+    Y += blockIdx.y * NSG * ysg + tk.y;
     const int ni = tk.ni, ai = tk.ai;
     int go[FI], mo[NV];
 #pragma unroll
     for (int f = 0; f < FI; ++f) go[f] = min(tk.i0 + 16 * f + c16, ni - 1) * 2 * NAO;
 #pragma unroll
     for (int v = 0; v < NV; ++v) mo[v] = min(tk.mu0 + (16 * v + c16) * VL, ai - 1);
-    A acc[FI][4][2];
+    A acc[FI][4][NSG];
 #pragma unroll
     for (int f = 0; f < FI; ++f)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[f][m][0] = acc[f][m][1] = A{0, 0, 0, 0};
-    struct Frag { T g[2][FI]; V w[NV]; };
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int q = 0; q < NSG; ++q) acc[f][m][q] = A{0, 0, 0, 0};
+    struct Frag { T g[NSG][FI]; V w[NV]; };
     int e = tk.e0 - 1, s = 0, ns = 0, nj = 0;
     const T *pg = nullptr, *pw = nullptr;
     auto next_entry = [&]() {
@@ -353,8 +359,8 @@ __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restr
 #pragma unroll
         for (int f = 0; f < FI; ++f)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const T v = pg[go[f] + q * nj + jc];
+            for (int q = 0; q < NSG; ++q) {
+                const T v = pg[go[f] + (sg0 + q) * nj + jc];
                 x.g[q][f] = j < nj ? v : T(0);
             }
 #pragma unroll
@@ -368,7 +374,7 @@ __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restr
             if (++s >= ns) { s = 0; more = next_entry(); }
             if (more) load(y);
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
+            for (int q = 0; q < NSG; ++q)
 #pragma unroll
                 for (int f = 0; f < FI; ++f)
 #pragma unroll
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restr
             const int i = tk.i0 + 16 * f + acc_row<T>(r, kq);
             if (i >= ni) continue;
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+            for (int q = 0; q < NSG; ++q) {
                 T *dst = Y + q * ysg + ((long long)l * ni + i) * ai;
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
@@ -398,53 +404,61 @@ __global__ __launch_bounds__(256, 2) void sigma_y_kernel(const SigYTask *__restr
 }
 
 namespace {
-template <class F> void by_two(int a, int b, F f) {
-    if (a == 1 && b == 1) f(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
-    else if (a == 1) f(std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
-    else if (b == 1) f(std::integral_constant<int, 2>(), std::integral_constant<int, 1>());
-    else f(std::integral_constant<int, 2>(), std::integral_constant<int, 2>());
+// f of a, b and n (1 or 2 each) as constants
+template <class F> void by_two(int a, int b, int n, F f) {
+    const auto with_b = [&](auto ca) {
+        const auto with_n = [&](auto cb) {
+            if (n == 1) f(ca, cb, std::integral_constant<int, 1>());
+            else f(ca, cb, std::integral_constant<int, 2>());
+        };
+        if (b == 1) with_n(std::integral_constant<int, 1>());
+        else with_n(std::integral_constant<int, 2>());
+    };
+    if (a == 1) with_b(std::integral_constant<int, 1>());
+    else with_b(std::integral_constant<int, 2>());
 }
 }  // namespace
 
 template <class T>
 void launch_sigma_d(const SigTask *tasks, int ntask, int fi, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
-                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, hipStream_t s) {
+                    long long zcw, const T *U, long long usg, T *sig, long long ssg, int NAO, int nz, int nsg,
+                    hipStream_t s) {
     if (ntask <= 0) return;
-    by_two(fi, fj, [&](auto a, auto b) {
-        hipLaunchKernelGGL((sigma_d_kernel<T, decltype(a)::value, decltype(b)::value>), dim3(ntask, nz), dim3(256), 0, s,
-                           tasks, blks, segs, CW, zcw, U, usg, sig, ssg, NAO);
+    by_two(fi, fj, nsg, [&](auto a, auto b, auto n) {
+        hipLaunchKernelGGL((sigma_d_kernel<T, decltype(a)::value, decltype(b)::value, decltype(n)::value>),
+                           dim3(ntask, nz), dim3(256), 0, s, tasks, blks, segs, CW, zcw, U, usg, sig, ssg, NAO);
     });
     HIP_CHECK(hipGetLastError());
 }
 template <class T>
 void launch_sigma_b(const SigTask *tasks, int ntask, int fc, int fj, const SigBlk *blks, const Chi0Seg *segs, const T *CW,
-                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, hipStream_t s) {
+                    long long zcw, const T *U, long long usg, T *s2, long long ssg, int NAO, int nz, int nsg,
+                    hipStream_t s) {
     if (ntask <= 0) return;
-    by_two(fc, fj, [&](auto a, auto b) {
-        hipLaunchKernelGGL((sigma_b_kernel<T, decltype(a)::value, decltype(b)::value>), dim3(ntask, nz), dim3(256), 0, s,
-                           tasks, blks, segs, CW, zcw, U, usg, s2, ssg, NAO);
+    by_two(fc, fj, nsg, [&](auto a, auto b, auto n) {
+        hipLaunchKernelGGL((sigma_b_kernel<T, decltype(a)::value, decltype(b)::value, decltype(n)::value>),
+                           dim3(ntask, nz), dim3(256), 0, s, tasks, blks, segs, CW, zcw, U, usg, s2, ssg, NAO);
     });
     HIP_CHECK(hipGetLastError());
 }
 template <class T>
 void launch_sigma_y(const SigYTask *tasks, int ntask, int fi, const SigYEnt *ents, const T *CW, long long zcw, const T *G,
-                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, hipStream_t s) {
+                    long long zg, T *Y, long long ysg, int NAO, int x0, int x1, bool first, int nz, int nsg, int sg0,
+                    hipStream_t s) {
     if (ntask <= 0) return;
-    if (fi == 1)
-        hipLaunchKernelGGL((sigma_y_kernel<T, 1>), dim3(ntask, nz), dim3(256), 0, s, tasks, ents, CW, zcw, G, zg, Y, ysg,
-                           NAO, x0, x1, (int)first);
-    else
-        hipLaunchKernelGGL((sigma_y_kernel<T, 2>), dim3(ntask, nz), dim3(256), 0, s, tasks, ents, CW, zcw, G, zg, Y, ysg,
-                           NAO, x0, x1, (int)first);
+    by_two(fi, 1, nsg, [&](auto a, auto, auto n) {
+        hipLaunchKernelGGL((sigma_y_kernel<T, decltype(a)::value, decltype(n)::value>), dim3(ntask, nz), dim3(256), 0, s,
+                           tasks, ents, CW, zcw, G, zg, Y, ysg, NAO, x0, x1, (int)first, sg0);
+    });
     HIP_CHECK(hipGetLastError());
 }
 #define LRA_SIGMA(T)                                                                                                    \
     template void launch_sigma_d<T>(const SigTask *, int, int, int, const SigBlk *, const Chi0Seg *, const T *, long long, \
-                                    const T *, long long, T *, long long, int, int, hipStream_t);                       \
+                                    const T *, long long, T *, long long, int, int, int, hipStream_t);                  \
     template void launch_sigma_b<T>(const SigTask *, int, int, int, const SigBlk *, const Chi0Seg *, const T *, long long, \
-                                    const T *, long long, T *, long long, int, int, hipStream_t);                       \
+                                    const T *, long long, T *, long long, int, int, int, hipStream_t);                  \
     template void launch_sigma_y<T>(const SigYTask *, int, int, const SigYEnt *, const T *, long long, const T *, long long, \
-                                    T *, long long, int, int, int, bool, int, hipStream_t);
+                                    T *, long long, int, int, int, bool, int, int, int, hipStream_t);
 LRA_SIGMA(double)
 LRA_SIGMA(float)
 #undef LRA_SIGMA
