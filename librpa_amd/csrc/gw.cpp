@@ -596,8 +596,12 @@ void GwEngine::build_w(const Dataset &ds, const TFGrid &g, Result &out) {
     const double per_w = 8.0 * ((double)NN + 2.0 * nn) + 16.0 * pl * N * (N >= (herm ? 2048 : 4096) ? (herm ? 1024 : 2048) : (herm ? 256 : 512));
     const double per_q = 8.0 * 14 * nn;
     const double budget = std::min(160e9, 0.7 * (double)free_b) - per_q;
-    const int WCH = std::max(1, std::min(nw, (int)(budget / per_w)));
-    const int QG = WCH < nw ? 1 : std::max(1, std::min(nq, (int)((budget + per_q) / (nw * per_w + per_q))));
+    const auto cap = [](const char *name, int v) {
+        const char *e = std::getenv(name);
+        return e ? std::max(1, std::min(v, std::atoi(e))) : v;
+    };
+    const int WCH = cap("LIBRPA_AMD_W_FREQS", std::max(1, std::min(nw, (int)(budget / per_w))));
+    const int QG = WCH < nw ? 1 : cap("LIBRPA_AMD_W_QGROUP", std::max(1, std::min(nq, (int)((budget + per_q) / (nw * per_w + per_q)))));
     const int UCH = QG > 1 ? QG * nw : WCH;
     // F: v and then its factor (Cholesky, or square root); C: v_c and then its root; V0: v_c, or S_c S_c
     // when a root is filtered
