@@ -116,11 +116,10 @@ def _profiled_traffic(kernel, workload, prec_name):
 
 def dominant_kernel(prof, prec_name, workload):
     """Largest-time region among the single-kernel GEMM regions, placed on its roofline."""
-    cands = {k: v for k, v in prof.items() if k.startswith(("chi0_W", "chi0_TA", "chi0_X", "chi0_contract",
-                                                            "ec_gemm")) and v[2] > 0}
+    cands = {k: v for k, v in prof.items() if k.startswith(("chi0_W", "chi0_contract", "ec_gemm")) and v[2] > 0}
     name, (ms, calls, flops, nbytes) = max(cands.items(), key=lambda kv: kv[1][0])
     # regions named for the precision they ran in (_f32, _bf16x3: low-weight tau points of the mixed
-    # modes, and the small-K GEMMs that stay in FP32 under BF16x3)
+    # modes, and the contraction, which stays in FP32 under BF16x3)
     if name.endswith("_bf16x3"):
         prec_name = "bf16x3"
     elif name.endswith("_f32"):

@@ -17,14 +17,13 @@ extern "C" {
  * matrix has an entry above 1e3 (the transform multiplies their chi0 errors
  * by up to that much), FP32 at the others; chi0(R, tau) is stored in FP64. */
 #define LIBRPA_AMD_MIXED 3
-/* chi0 only: as LIBRPA_AMD_MIXED with BF16x3 instead of FP32 at the low-weight tau points (their
- * small-K X and T_A GEMMs stay FP32). */
+/* chi0 only: as LIBRPA_AMD_MIXED with BF16x3 instead of FP32 at the low-weight tau points, in their
+ * W products (the contraction runs in FP32 there, as it does under LIBRPA_AMD_BF16X3). */
 #define LIBRPA_AMD_MIXED_BF16 4
 
-/* Contraction precision of the chi0 build (G, W, T and the final Cs.T
- * contraction) and of the Ec transforms (chi0 L and L^T X).  The Cholesky
- * log-determinant, the tau->omega quadrature and all accumulation of Ec stay
- * in FP64.  Default FP64 / FP64. */
+/* Contraction precision of the chi0 build (G, W and the contraction with Cs) and of
+ * the Ec transforms (chi0 L and L^T X).  The Cholesky log-determinant, the
+ * tau->omega quadrature and all accumulation of Ec stay in FP64.  Default FP64 / FP64. */
 void librpa_amd_set_precision(LibrpaHandler *h, int chi0_prec, int ec_prec);
 
 /* 0 (default): errors are C++ exceptions thrown through the C ABI as in

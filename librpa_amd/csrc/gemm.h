@@ -7,10 +7,8 @@
 // generalisations needed by the atom-pair layouts:
 //   * row indirection: row m of A and C may come from a table of absolute
 //     element offsets (gathered rows, scattered outputs);
-//   * column split on C: output column c goes to (c / ncb) * cbs + c % ncb,
-//     which writes a [j][rows][nu] layout directly from a [rows][(j, nu)] GEMM;
-//   * column table on C: the within-block part c % ncb may be replaced by an
-//     entry of a table of element offsets (scattered output columns);
+//   * column table on C: column c may be replaced by an entry of a table of element
+//     offsets (scattered output columns);
 //   * atomic epilogue: C += alpha A B with atomic adds, for outputs that several
 //     problems of one launch accumulate into;
 //   * second segment: A B may be followed by sgn2 A2 B2 of the same shape and strides in the same
@@ -19,7 +17,6 @@
 // small system), so that few problems still fill the device.
 #pragma once
 
-#include <functional>
 #include <vector>
 
 #include "common.h"
@@ -36,8 +33,6 @@ struct GemmProb {
     int M, N, K;
     int tiles_n;   // filled by GemmBatch::finalize
     int tile0;     // first global tile of this problem (filled by finalize)
-    int ncb;       // C column-split block (>= N means none)
-    long long cbs; // C column-split stride
     long long a_off, b_off, c_off;
     int lda, ldb, ldc;
     int rt_off;    // offset into the row table, -1 if not row-indirect
@@ -81,7 +76,6 @@ struct GemmBatch {
     int nz = 1;                        // copies of the batch in one launch
     long long za = 0, zb = 0, zc = 0;  // operand distances of a copy, in elements
     int total_tiles = 0;
-    std::vector<int> tile_prob;
     int per_prob = 0;      // tiles of every problem where that is one number, else 0: d_tile_prob maps a tile
     double flops = 0;      // flops of one launch: 2 M N K summed, less the skipped triangular work
     DevBuf d_probs, d_rowtab, d_coltab, d_tile_prob;
@@ -102,10 +96,8 @@ struct GemmBatch {
     bool empty() const { return probs.empty(); }
     // Autotuner: time one launch of every tile shape this batch can use (after a warm-up
     // launch) on the real operands and keep the fastest.  The launches must be harmless
-    // to repeat (overwriting outputs); `before` runs before every launch (e.g. to reset an
-    // accumulated output).  Returns the chosen tile configuration.
-    int tune(Prec prec, const void *A, const void *B, void *C, double alpha, double beta, hipStream_t s,
-             const std::function<void()> &before = nullptr);
+    // to repeat (overwriting outputs).  Returns the chosen tile configuration.
+    int tune(Prec prec, const void *A, const void *B, void *C, double alpha, double beta, hipStream_t s);
 };
 
 GemmProb make_prob(int M, int N, int K, long long a_off, int lda, long long b_off, int ldb,

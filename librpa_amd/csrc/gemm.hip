@@ -257,21 +257,13 @@ __global__ __launch_bounds__(WM * WN * 64) void ggemm_kernel(const GemmProb *__r
     }
 
     // epilogue: acc[a][b][r] holds C[row][n0 + wn*WTN + b*16 + lane%16].  The output column of
-    // each b (column split and table included) depends on the lane only: worked out once here,
-    // not for every row (a split's division by ncb is some thirty VALU instructions)
-    const bool split = P.ncb < P.N;
+    // each b (column table included) depends on the lane only: worked out once here
     const bool ct = VAR == 2 && P.ct_off >= 0;
     long long ccol[FN];
 #pragma unroll
     for (int b = 0; b < FN; ++b) {
         const int gn = n0 + wn * WTN + b * 16 + (lane & 15);
-        ccol[b] = -1;
-        if (gn < P.N) {
-            const int inner = split ? gn % P.ncb : gn;
-            long long col = ct ? coltab[P.ct_off + inner] : inner;
-            if (split) col += (long long)(gn / P.ncb) * P.cbs;
-            ccol[b] = col;
-        }
+        ccol[b] = gn >= P.N ? -1 : ct ? coltab[P.ct_off + gn] : gn;
     }
     // a full tile with alpha = 1, beta = 0 and plain stores (the chi0 build's W GEMMs): no
     // per-element checks, scaling or reads of C
@@ -330,7 +322,6 @@ GemmProb make_prob(int M, int N, int K, long long a_off, int lda, long long b_of
     GemmProb p;
     std::memset(&p, 0, sizeof(p));
     p.M = M; p.N = N; p.K = K;
-    p.ncb = 1 << 30; p.cbs = 0;
     p.a_off = a_off; p.lda = lda; p.b_off = b_off; p.ldb = ldb; p.c_off = c_off; p.ldc = ldc;
     p.rt_off = -1;
     p.ct_off = -1;
@@ -362,7 +353,7 @@ void GemmBatch::finalize(int cfg_, hipStream_t s) {
         }
     }
     total_tiles = t0;
-    tile_prob.clear();
+    std::vector<int> tile_prob;
     per_prob = probs.empty() ? 0 : t0 / (int)probs.size();
     if (per_prob * (int)probs.size() != t0) per_prob = 0;
     for (size_t i = 0; i < probs.size(); ++i)
@@ -374,6 +365,7 @@ void GemmBatch::finalize(int cfg_, hipStream_t s) {
                       i + 1 < probs.size() ? tile_prob.begin() + probs[i + 1].tile0 : tile_prob.end(), (int)i);
     }
     d_tile_prob = upload(tile_prob, s);
+    if (!tile_prob.empty()) HIP_CHECK(hipStreamSynchronize(s));  // (tile_prob is freed here)
     d_probs = upload(probs, s);
     // the tables do not depend on the tile shape: upload once
     if (!rowtab.empty() && d_rowtab.bytes() != rowtab.size() * sizeof(long long)) d_rowtab = upload(rowtab, s);
@@ -453,7 +445,7 @@ std::map<std::vector<long long>, std::pair<int, float>> &tune_cache() {
 std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
     std::vector<long long> k = {(long long)prec, b.nz, b.trans_a, b.trans_b, b.lower_only,
                                 (long long)b.rowtab.size(), (long long)b.coltab.size()};
-    k.reserve(k.size() + 8 * b.probs.size());
+    k.reserve(k.size() + 7 * b.probs.size());
     for (const auto &p : b.probs) {
         k.push_back(p.M);
         k.push_back(p.N);
@@ -462,14 +454,12 @@ std::vector<long long> tune_key(Prec prec, const GemmBatch &b) {
         k.push_back(p.ldb);
         k.push_back(p.ldc);
         k.push_back(p.kmode + 4 * (p.rt_off >= 0) + 8 * (p.ct_off >= 0) + 16 * (p.sgn2 != 0));
-        k.push_back(p.ncb < p.N ? p.ncb : 0);
     }
     return k;
 }
 }  // namespace
 
-int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alpha, double beta, hipStream_t s,
-                    const std::function<void()> &before) {
+int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alpha, double beta, hipStream_t s) {
     if (probs.empty() || atomic) return cfg;
     const auto key = tune_key(prec, *this);
     {
@@ -490,7 +480,6 @@ int GemmBatch::tune(Prec prec, const void *A, const void *B, void *C, double alp
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     auto timed = [&](void) {
-        if (before) before();
         HIP_CHECK(hipEventRecord(e0, s));
         gemm_run(prec, *this, A, B, C, alpha, beta, s);
         HIP_CHECK(hipEventRecord(e1, s));

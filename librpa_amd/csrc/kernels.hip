@@ -435,8 +435,6 @@ template <class TS, class TD> void launch_convert(const TS *src, TD *dst, long l
     HIP_CHECK(hipGetLastError());
 }
 template void launch_convert<double, float>(const double *, float *, long long, hipStream_t);
-template void launch_convert<float, double>(const float *, double *, long long, hipStream_t);
-template void launch_convert<double, double>(const double *, double *, long long, hipStream_t);
 
 __global__ void copy_lower_f2d_kernel(const float *__restrict__ src, double *__restrict__ dst, int n, long long stride) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -527,7 +527,7 @@ void RpaEngine::build_chi0(const Dataset &ds, const TFGrid &g, int nbands_g) {
     const double t0 = now_s();
     const int ntau = g.n;
     chiw_ok = false;  // chi0(R, omega) of an earlier build is stale
-    if (host_staged) d_chiw.release();  // its room goes back to W and T (reformed for Ec)
+    if (host_staged) d_chiw.release();  // its room goes back to G and W (reformed for Ec)
     prepare_gf(mf, nbands_g);
     d_Ghat.reserve(ghat_max * nbatch * ts);
     d_W.reserve((size_t)(w_off.back() * nbatch + kChi0Pad) * ts);
