@@ -220,30 +220,33 @@ template void launch_chi0_assemble<double, float>(const double *, long long, int
 // cosine tau -> omega transform, done once for all q.  Coefficients in LDS; a thread owns one element
 // and re-reads its ntau values once per group of 8 frequencies.  Where the elements alone are under 1024
 // workgroups the groups go over the grid (a molecule: 17 us of load latency in one thread's two groups).
-// TAB: an ArgTable, or a pointer
-__device__ __forceinline__ double table_at(const ArgTable &t, int i) { return t.v[i]; }
-__device__ __forceinline__ double table_at(const double *t, int i) { return t[i]; }
+// A kernel takes its table as TAB (the ArgTable itself, or nothing) and a __restrict__ pointer: without
+// that word a table in memory is read again by every lane after each store (16 atoms, 64 k: the R -> q sums
+// 98 ms an evaluation, 76 with scalar loads).
+struct NoArgTable {};
+__device__ __forceinline__ double table_at(const ArgTable &t, const double *, int i) { return t.v[i]; }
+__device__ __forceinline__ double table_at(const NoArgTable &, const double *p, int i) { return p[i]; }
 // the table of a launch to the launch itself
 template <class F> void with_table(const std::vector<double> &v, DevBuf &buf, hipStream_t s, F f) {
     if (v.size() <= (size_t)kArgTable) {
         ArgTable t;
         std::copy(v.begin(), v.end(), t.v);
-        f(t);
+        f(t, static_cast<const double *>(nullptr));
         return;
     }
     buf.reserve(v.size() * sizeof(double));
     HIP_CHECK(hipMemcpyAsync(buf.get(), v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    f(static_cast<const double *>(buf.as<double>()));
+    f(NoArgTable(), static_cast<const double *>(buf.as<double>()));
     HIP_CHECK(hipStreamSynchronize(s));  // the next table may go to the same buffer
 }
 
 template <class TS, class TAB>
 __global__ __launch_bounds__(256) void tau_to_omega_kernel(const TS *__restrict__ chi0s, long long E_tot, int ntau,
-                                                           const TAB coef, int nw, int wper,
+                                                           const TAB tab, const double *__restrict__ coef, int nw, int wper,
                                                            double *__restrict__ chiw) {
     __shared__ double c[kTauOmegaMax * kTauOmegaMax];
     const int wb = blockIdx.y * wper, we = min(nw, wb + wper);
-    for (int k = wb * ntau + threadIdx.x; k < we * ntau; k += blockDim.x) c[k] = table_at(coef, k);
+    for (int k = wb * ntau + threadIdx.x; k < we * ntau; k += blockDim.x) c[k] = table_at(tab, coef, k);
     __syncthreads();
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < E_tot;
          i += (long long)gridDim.x * blockDim.x) {
@@ -270,9 +273,9 @@ static void tau_to_omega(const TS *chi0s, long long E_tot, int ntau, const std::
     if (ntau > kTauOmegaMax || nw > kTauOmegaMax) LRA_THROW("tau -> omega: grid too large");
     const int bx = (int)std::min<long long>(ceil_div(E_tot, 256), 8192);
     const int wper = bx >= 1024 ? nw : 8;
-    with_table(coef, buf, s, [&](auto table) {
+    with_table(coef, buf, s, [&](auto table, const double *p) {
         hipLaunchKernelGGL((tau_to_omega_kernel<TS, decltype(table)>), dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chi0s,
-                           E_tot, ntau, table, nw, wper, chiw);
+                           E_tot, ntau, table, p, nw, wper, chiw);
         HIP_CHECK(hipGetLastError());
     });
 }
@@ -320,11 +323,11 @@ template void launch_tau_accumulate<float>(const float *, long long, int, int, c
 // alone are under 1024 workgroups: with all 16 in the loop the 2-atom cell (120 functions, 43
 // workgroups) took 168 us where its bytes take 15; with one each the 64-atom cell takes 6.2 ms, not 4.7.
 // q point qi writes its nw matrices at dense + qi * qstride.
-template <class TD, int NQ, class TAB>
+template <class TD, int NQ, int WU, class TAB>
 __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__ chiw, long long E_tot,
                                                       const PairDesc *__restrict__ pairs, int npairs, long long nelem,
                                                       const long long *__restrict__ eoff, int nR,
-                                                      const TAB ph, int nq, int nw, int wper,
+                                                      const TAB tab, const double *__restrict__ ph, int nq, int nw, int wper,
                                                       TD *__restrict__ dense, long long dstride, long long qstride,
                                                       int n, int lay) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -337,28 +340,40 @@ __global__ __launch_bounds__(256) void chi0_rq_kernel(const double *__restrict__
     const PairDesc P = pairs[lo];
     const long long e = idx - P.e0;
     const int mu = (int)(e / P.naJ), nu = (int)(e % P.naJ);
-    for (int w = blockIdx.y * wper; w < min(nw, (int)(blockIdx.y + 1) * wper); ++w) {
-        double re[NQ], im[NQ];
+    const int we = min(nw, (int)(blockIdx.y + 1) * wper);
+    for (int w0 = blockIdx.y * wper; w0 < we; w0 += WU) {
+        double re[WU][NQ], im[WU][NQ];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) re[q] = im[q] = 0.0;
-        const double *cw = chiw + (long long)w * E_tot + e;
+        for (int u = 0; u < WU; ++u)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) re[u][q] = im[u][q] = 0.0;
+        const double *cw = chiw + (long long)w0 * E_tot + e;
         for (int r = 0; r < nR; ++r) {
             const long long off = eoff[(long long)lo * nR + r];
             if (off < 0) continue;
-            const double v = cw[off];
+            double v[WU];
+#pragma unroll
+            for (int u = 0; u < WU; ++u) v[u] = cw[off + (w0 + u < we ? u * E_tot : 0)];
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 if (q < nq) {
-                    re[q] += table_at(ph, 2 * (q * nR + r)) * v;
-                    im[q] += table_at(ph, 2 * (q * nR + r) + 1) * v;
+                    const double c = table_at(tab, ph, 2 * (q * nR + r)), d = table_at(tab, ph, 2 * (q * nR + r) + 1);
+#pragma unroll
+                    for (int u = 0; u < WU; ++u) {
+                        re[u][q] += c * v[u];
+                        im[u][q] += d * v[u];
+                    }
                 }
             }
         }
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            if (q >= nq) break;
-            put_dense(dense + q * qstride + w * dstride, n, P.rowI + mu, P.colJ + nu, re[q], im[q], P.I != P.J, lay);
-        }
+        for (int u = 0; u < WU; ++u)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                if (q >= nq || w0 + u >= we) break;
+                put_dense(dense + q * qstride + (w0 + u) * dstride, n, P.rowI + mu, P.colJ + nu, re[u][q], im[u][q],
+                          P.I != P.J, lay);
+            }
     }
 }
 
@@ -369,14 +384,16 @@ void launch_chi0_rq_multi(const double *chiw, long long E_tot, const PairDesc *p
                           DenseLayout lay, hipStream_t s) {
     if (nq < 1 || nq > kChi0RqMaxQ) LRA_THROW("chi0_rq_multi: 1 to kChi0RqMaxQ q points per launch");
     const int bx = ceil_div(n_pair_elems, 256), wper = bx >= 1024 ? nw : 1;
-    with_table(ph, buf, s, [&](auto table) {
+    with_table(ph, buf, s, [&](auto table, const double *p) {
         using TAB = decltype(table);
         const auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(bx, ceil_div(nw, wper)), dim3(256), 0, s, chiw, E_tot, pairs, npairs,
-                               n_pair_elems, eoff, nR, table, nq, nw, wper, dense, dense_stride, q_stride, n, (int)lay);
+                               n_pair_elems, eoff, nR, table, p, nq, nw, wper, dense, dense_stride, q_stride, n, (int)lay);
         };
-        if (nq == 1) go(chi0_rq_kernel<TD, 1, TAB>);
-        else go(chi0_rq_kernel<TD, kChi0RqMaxQ, TAB>);
+        // one q: four frequencies at a time, whose loads are in flight together (128 atoms: 20.6 -> 19.0 ms)
+        if (nq > 1) go(chi0_rq_kernel<TD, kChi0RqMaxQ, 1, TAB>);
+        else if (wper > 1) go(chi0_rq_kernel<TD, 1, 4, TAB>);
+        else go(chi0_rq_kernel<TD, 1, 1, TAB>);
         HIP_CHECK(hipGetLastError());
     });
 }
