@@ -222,7 +222,7 @@ template void launch_chi0_assemble<double, float>(const double *, long long, int
 // workgroups the groups go over the grid (a molecule: 17 us of load latency in one thread's two groups).
 // A kernel takes its table as TAB (the ArgTable itself, or nothing) and a __restrict__ pointer: without
 // that word a table in memory is read again by every lane after each store (16 atoms, 64 k: the R -> q sums
-// 98 ms an evaluation, 76 with scalar loads).
+// 98 ms an evaluation, 44 to 50 with scalar loads).
 struct NoArgTable {};
 __device__ __forceinline__ double table_at(const ArgTable &t, const double *, int i) { return t.v[i]; }
 __device__ __forceinline__ double table_at(const NoArgTable &, const double *p, int i) { return p[i]; }
